@@ -1,0 +1,642 @@
+"""Workloads whose time matters to a user of this framework.
+
+Each case is one call sequence of a solver program through the Python host API (tarang_amd.api) on device fields:
+time steps of every basis, the energy-transfer and spectrum diagnostics, the plain transforms and the adjoint, from
+64^3 to 512^3, in FP64 and with FP32 transforms, on power-of-two and radix-3/5 grids.
+
+listed()/draw(rng)  the cases, as dicts of plain values
+prepare(case, seed) fields, plan and solver objects a program holds before the call
+run(state)          one pass, returning its whole outputs
+exact(case, seed)   the same outputs in plain torch, 64 bits, where that is quick
+work(case)          bytes and operations a pass cannot do without
+"""
+import math
+
+import numpy as np
+import torch
+
+from tarang_amd import api
+
+DEALIAS = {"none": api.DEALIAS_NONE, "corner": api.DEALIAS_REF_CORNER, "twothirds": api.DEALIAS_TWOTHIRDS}
+SHELLS = 20                  # default log-spaced spheres and shells of the transfer diagnostics
+RA, PR = 1e8, 1.0            # Rayleigh-Benard parameters
+BAND = (2.0, 3.0)            # forcing band
+EXACT_POINTS = 4_000_000     # largest grid whose time step exact() evaluates
+EXACT_SMALL = 300_000        # the same for the adjoint and the transfers (tens of evaluations)
+
+
+def _case(name, kind, n, prec="fp64", dealias="corner", force=0, steps=1, every=1):
+    return {"name": name, "kind": kind, "nx": n[0], "ny": n[1], "nz": n[2], "prec": prec, "dealias": dealias,
+            "force": force, "steps": steps, "every": every}
+
+
+def listed():
+    return [
+        # the 64^3 run whose energy, dissipation and spectrum are printed after every step: the smallest calls, each
+        # waited for
+        _case("ns_64_step_outputs", "ns_outputs", (64, 64, 64), dealias="twothirds"),
+        # parameter studies and spin-up runs at moderate resolution, transforms in FP32
+        _case("ns_128_fp32", "ns", (128, 128, 128), prec="fp32", force=1),
+        # a box of unequal sides on radix-3/5 lengths
+        _case("ns_240x160x96", "ns", (240, 160, 96)),
+        # the production run: 512^3 with band-limited random forcing, FP64 ...
+        _case("ns_512", "ns", (512, 512, 512), force=2),
+        # ... and with FP32 transforms
+        _case("ns_512_fp32", "ns", (512, 512, 512), prec="fp32", force=2),
+        # MHD turbulence at the same resolution with FP32 transforms
+        _case("mhd_512_fp32", "mhd", (512, 512, 512), prec="fp32"),
+        # Rayleigh-Benard convection between walls, FP32 transforms, half the production grid per axis
+        _case("rbc_256x512x512_fp32", "rbc", (256, 512, 512), prec="fp32"),
+        # initial-condition gradients: forward sweep with checkpoints, backward sweep with recomputation
+        _case("adjoint_256", "adjoint", (256, 256, 256), steps=4, every=2),
+        # flux over 20 spheres and the shell-to-shell matrix of one snapshot
+        _case("transfer_256", "transfer", (256, 256, 256), dealias="twothirds"),
+        # energy, dissipation and shell spectra of one snapshot
+        _case("spectra_256", "spectra", (256, 256, 256)),
+        # user code that forms its own terms: one field to real space and back
+        _case("transforms_256", "transforms", (256, 256, 256)),
+        # channel flow on the Chebyshev basis, implicit-explicit Euler step
+        _case("chff_64x128x128", "chff", (64, 128, 128), dealias="none"),
+    ]
+
+
+_FP64_LENGTHS = sorted({r * 2 ** a for r in (1, 3, 5, 15) for a in range(3, 10) if 16 <= r * 2 ** a <= 512})
+_FP32_LENGTHS = [16, 32, 64, 128, 256, 512]
+#   kind: share of the draws, FP32 too, largest number of grid points, dealias modes
+_KINDS = {"ns": (4, True, 1 << 25, ("corner", "twothirds", "none")), "ns_outputs": (1, True, 1 << 22, ("twothirds", "corner")),
+          "mhd": (2, True, 1 << 24, ("corner", "twothirds")), "rbc": (2, True, 1 << 24, ("corner", "twothirds")),
+          "adjoint": (1, True, 1 << 23, ("corner", "twothirds")), "transfer": (1, True, 1 << 22, ("twothirds", "corner")),
+          "spectra": (1, False, 1 << 25, ("corner",)), "transforms": (1, True, 1 << 25, ("corner",)),
+          "chff": (1, False, 1 << 20, ("none",))}
+
+
+def draw(rng):
+    kind = rng.choice([k for k, v in _KINDS.items() for _ in range(v[0])])
+    _, fp32, most, dealias = _KINDS[kind]
+    prec = rng.choice(["fp64", "fp32"]) if fp32 else "fp64"
+    lengths = _FP32_LENGTHS if prec == "fp32" else _FP64_LENGTHS
+    # a target number of points, spread over its logarithm, and sides about it
+    points = 2 ** rng.uniform(14, math.log2(most))
+    while True:
+        n = [min(lengths, key=lambda v, t=points ** (1 / 3) * 2 ** rng.uniform(-0.8, 0.8): abs(math.log(v / t))) for _ in range(3)]
+        if n[2] % 16 == 0 and points / 4 <= n[0] * n[1] * n[2] <= most:
+            break
+    if kind == "chff":
+        n[0] = min(n[0], 64)
+    c = _case("", kind, n, prec, rng.choice(dealias))
+    del c["name"]
+    if kind == "ns":
+        c["force"] = rng.choice([0, 1, 2]) if min(n) >= 16 else 0
+        c["steps"] = rng.choice([1, 2])
+    if kind == "adjoint":
+        c["steps"] = rng.choice([2, 3])
+    return c
+
+
+# ---------------------------------------------------------------------------------------------------------------------
+# inputs
+# ---------------------------------------------------------------------------------------------------------------------
+def _size(c):
+    return c["nx"], c["ny"], c["nz"]
+
+
+def _kfactor(c):
+    return (math.pi, math.pi / math.sqrt(2.0), math.pi / math.sqrt(2.0)) if c["kind"] == "rbc" else (1.0, 1.0, 1.0)
+
+
+def _k(n, kf, device, sine_x=False):
+    """Wavenumbers (kx, ky, kz) as broadcastable FP64 tensors; the Nyquist index counts as positive."""
+    out = []
+    for d in range(3):
+        i = torch.arange(n[d] if d < 2 else n[2] // 2 + 1, dtype=torch.float64, device=device)
+        if d < 2 and not (d == 0 and sine_x):
+            i = torch.where(i <= n[d] // 2, i, i - n[d])
+        shape = [1, 1, 1]
+        shape[d] = -1
+        out.append((i * kf[d]).reshape(shape))
+    return out
+
+
+def _hermitian_plane(a, sine_x=False):
+    """kz = 0 plane of a real field's spectrum, Nyquist planes empty."""
+    p = a[:, :, 0]
+    m = torch.roll(torch.flip(p, (1,) if sine_x else (0, 1)), 1 if sine_x else (1, 1), (1,) if sine_x else (0, 1))
+    a[:, :, 0] = (p + m.conj()) / math.sqrt(2.0)
+    if not sine_x:
+        a[a.shape[0] // 2] = 0
+    a[:, a.shape[1] // 2] = 0
+    a[:, :, -1] = 0
+
+
+def _noise(shape, gen, device):
+    return torch.complex(torch.randn(shape, generator=gen, device=device, dtype=torch.float64),
+                         torch.randn(shape, generator=gen, device=device, dtype=torch.float64))
+
+
+def _turbulence(n, kf, seed, energy, device="cuda"):
+    """Solenoidal field with E(k) ~ k^-5/3 on 2 <= k <= N/3, random phases, given energy."""
+    gen = torch.Generator(device=device).manual_seed(seed)
+    kx, ky, kz = _k(n, kf, device)
+    k2 = kx * kx + ky * ky + kz * kz
+    kmax = min(n[d] * kf[d] for d in range(3)) / 3
+    amp = torch.where((k2 >= 4) & (k2 <= kmax * kmax), k2.clamp(min=1.0) ** (-11 / 12), torch.zeros_like(k2))
+    v = []
+    for _ in range(3):
+        a = _noise((n[0], n[1], n[2] // 2 + 1), gen, device)
+        _hermitian_plane(a)
+        v.append(a.mul_(amp))
+    del amp
+    p = (kx * v[0] + ky * v[1] + kz * v[2]) / k2.clamp(min=1e-300)
+    for a, k in zip(v, (kx, ky, kz)):
+        a -= k * p
+    e = sum(float((a.real ** 2 + a.imag ** 2).sum() - 0.5 * (a[:, :, 0].real ** 2 + a[:, :, 0].imag ** 2).sum()) for a in v)
+    for a in v:
+        a *= math.sqrt(energy / e)
+    return v
+
+
+def _convection(n, kf, seed, device="cuda"):
+    """Weak solenoidal motion and temperature noise in the first 32 modes per axis (sin/cos along x)."""
+    gen = torch.Generator(device=device).manual_seed(seed)
+    kx, ky, kz = _k(n, kf, device, sine_x=True)
+    k2 = kx * kx + ky * ky + kz * kz
+    m = [min(32, n[0] * 2 // 3), min(32, n[1] // 3), min(32, n[2] // 3)]
+    keep = (kx < m[0] * kf[0]) & (ky.abs() < m[1] * kf[1]) & (kz < m[2] * kf[2])
+    f = []
+    for c in range(4):
+        a = _noise((n[0], n[1], n[2] // 2 + 1), gen, device)
+        _hermitian_plane(a, sine_x=True)
+        a *= keep * (1e-4 if c < 3 else 1e-3) / (1 + k2)
+        if c in (0, 3):
+            a[0] = 0   # sine series
+        f.append(a)
+    p = (kx * f[0] + 1j * ky * f[1] + 1j * kz * f[2]) / k2.clamp(min=1e-300)
+    f[0] -= kx * p
+    f[1] += 1j * ky * p
+    f[2] += 1j * kz * p
+    return f[:3], f[3]
+
+
+def _cheb_matrices(nx, device):
+    """d/dx and multiplication by 1 - x^2 on Chebyshev coefficients."""
+    d = torch.zeros((nx, nx), dtype=torch.float64)
+    for k in range(nx):
+        for j in range(k + 1, nx, 2):
+            d[k, j] = (1.0 if k == 0 else 2.0) * j
+    w = 0.5 * torch.eye(nx, dtype=torch.float64)
+    for j in range(nx):
+        for t in (j + 2, abs(j - 2)):
+            if t < nx:
+                w[t, j] -= 0.25
+    return d.to(device), w.to(device)
+
+
+def _channel(n, seed, device="cuda"):
+    """Solenoidal no-slip field: phi = (1 - x^2)^2 h and chi = (1 - x^2) q per (ky, kz) line."""
+    gen = torch.Generator(device=device).manual_seed(seed)
+    _, ky, kz = _k(n, (1.0, 1.0, 1.0), device)
+    k2 = ky * ky + kz * kz
+    d, w = (m.to(torch.complex128) for m in _cheb_matrices(n[0], device))
+    keep = (k2 > 0) & (ky.abs() <= n[1] // 3) & (kz <= n[2] // 3)
+    low = (torch.arange(n[0], device=device) < n[0] // 4).to(torch.float64).reshape(-1, 1, 1)
+    h, q = (_noise((n[0], n[1], n[2] // 2 + 1), gen, device) * (keep * low * 1e-2 / (1 + k2)) for _ in range(2))
+    mul = lambda m, a: torch.tensordot(m, a, dims=([1], [0]))
+    phi, chi = mul(w, mul(w, h)), mul(w, q)
+    dphi = mul(d, phi) / k2.clamp(min=1e-300)
+    v = [phi, 1j * ky * dphi + 1j * kz * chi, 1j * kz * dphi - 1j * ky * chi]
+    for a in v:
+        _hermitian_plane_y(a)
+    return v
+
+
+def _hermitian_plane_y(a):
+    p = a[:, :, 0]
+    a[:, :, 0] = 0.5 * (p + torch.roll(torch.flip(p, (1,)), 1, 1).conj())
+
+
+def _inputs(c, seed):
+    n, kf, kind = _size(c), _kfactor(c), c["kind"]
+    if kind == "rbc":
+        v, t = _convection(n, kf, seed)
+        return v + [t]
+    if kind == "chff":
+        return _channel(n, seed)
+    if kind == "transforms":
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        a = _noise((n[0], n[1], n[2] // 2 + 1), gen, "cuda")
+        _hermitian_plane(a)
+        kx, ky, kz = _k(n, kf, "cuda")
+        return [a / (1 + kx * kx + ky * ky + kz * kz)]
+    v = _turbulence(n, kf, 2 * seed, 0.5)
+    if kind == "mhd":
+        v += _turbulence(n, kf, 2 * seed + 1, 0.25)
+    return v
+
+
+def _nu(c):
+    return 0.01 if c["nx"] * c["ny"] * c["nz"] <= 1 << 20 else 1e-3
+
+
+def _radii(c):
+    n = _size(c)
+    top = min(n) // 2
+    r = np.concatenate([[0.0, 2.0, 4.0], np.geomspace(4.0, top, SHELLS - 3 + 1)[1:], [np.inf]])
+    return r
+
+
+def prepare(case, seed):
+    c, kind, n = case, case["kind"], _size(case)
+    prec = api.PREC_FP32 if c["prec"] == "fp32" else api.PREC_FP64
+    x = _inputs(c, seed)
+    s = {"case": c}
+    if kind == "rbc":
+        b = api.SFF_Basis(n, kfactor=_kfactor(c), precision=prec, dealias=DEALIAS[c["dealias"]], reality=2)
+    elif kind == "chff":
+        b = api.ChFF_Basis(n)
+    else:
+        b = api.FFF_Basis(n, precision=prec, dealias=DEALIAS[c["dealias"]], strong_reality=kind != "adjoint")
+    s["basis"] = b
+    if kind == "transforms":
+        s["A"], s["R"], s["B"] = x[0], b.real_array(), b.complex_array()
+        return s
+    u = api.FluidVF(b, _nu(c))
+    u.set_field(x[:3])
+    s["U"] = u
+    if kind in ("ns", "ns_outputs"):
+        f = {0: {}, 1: {"force_kind": 1, "force_eps": 0.1}, 2: {"force_kind": 2, "force_eps": 0.1, "force_tau": 0.01, "force_seed": 1 + seed}}[c["force"]]
+        if f:
+            f.update(force_r_in=BAND[0], force_r_out=BAND[1])
+        s["ta"] = api.Time_advance_incompress(u, 1e-3, **f)
+    elif kind == "mhd":
+        w = api.FluidVF(b, _nu(c), name="W")
+        w.set_field(x[3:])
+        s["W"], s["ta"] = w, api.Time_advance_incompress_MHD(u, w, 1e-3)
+    elif kind == "rbc":
+        t = api.FluidSF(b)
+        t.set_field(x[3])
+        s["T"], s["ta"] = t, api.Time_advance_incompress_RBC(u, t, RA, PR, 1e-3)
+    elif kind == "chff":
+        s["ta"] = api.Time_advance_incompress_BDF1(u, 1e-3)
+    elif kind == "adjoint":
+        s["ta"] = api.Adjoint_incompress(u, 1e-3, checkpoint_every=c["every"])
+        s["weight"] = _loss_weight(n, "cuda")
+    elif kind == "transfer":
+        s["et"] = api.EnergyTr(b, flux_radii=_radii(c), shell_radii=_radii(c))
+    return s
+
+
+def _loss_weight(n, device):
+    """d/dA of the energy in 4 <= k < 8: 2 w A on the shell, w = 1/2 at kz = 0."""
+    kx, ky, kz = _k(n, (1.0, 1.0, 1.0), device)
+    k2 = kx * kx + ky * ky + kz * kz
+    return ((k2 >= 16) & (k2 < 64)) * torch.where(kz == 0, 1.0, 2.0).to(torch.float64)
+
+
+def run(state):
+    c = state["case"]
+    kind, b = c["kind"], state["basis"]
+    if kind == "transforms":
+        b.Inverse_transform(state["A"], state["R"])
+        b.Forward_transform(state["R"], state["B"])
+        return [state["R"], state["B"]]
+    u = state["U"]
+    if kind == "ns":
+        state["ta"].Time_advance_step(c["steps"])
+        return u.cvf
+    if kind == "ns_outputs":
+        state["ta"].Time_advance_step(1)
+        return u.cvf + _outputs(u)
+    if kind == "spectra":
+        return _outputs(u)
+    if kind == "mhd":
+        state["ta"].Time_advance_step(c["steps"])
+        return u.cvf + state["W"].cvf
+    if kind == "rbc":
+        state["ta"].Time_advance_step(c["steps"])
+        return u.cvf + [state["T"].F]
+    if kind == "chff":
+        state["ta"].Time_advance_step(1)
+        return u.cvf + [state["ta"].P]
+    if kind == "adjoint":
+        state["ta"].Forward(c["steps"])
+        lam = [a * state["weight"] for a in u.cvf]
+        return u.cvf + state["ta"].Backward(lam)
+    flux, s = state["et"].Compute_flux_and_shell_tr(u)
+    return [flux, s]
+
+
+def _outputs(u):
+    """What a run prints after a step: energy, dissipation and the shell spectrum of each component."""
+    return [u.Compute_total_energy(), u.dissipation(), np.stack([u.basis.Compute_shell_spectrum(a) for a in u.cvf])]
+
+
+# ---------------------------------------------------------------------------------------------------------------------
+# the same in plain torch
+# ---------------------------------------------------------------------------------------------------------------------
+class _Fourier:
+    def __init__(self, c):
+        self.n, self.kf = _size(c), _kfactor(c)
+        self.k = _k(self.n, self.kf, "cpu")
+        self.k2 = sum(k * k for k in self.k)
+        nx, ny, nz = self.n
+        ix, iy = torch.arange(nx).reshape(-1, 1, 1), torch.arange(ny).reshape(1, -1, 1)
+        iz = torch.arange(nz // 2 + 1).reshape(1, 1, -1)
+        self.keep = torch.ones((nx, ny, nz // 2 + 1), dtype=torch.float64)
+        if c["dealias"] == "corner":
+            z0, z1 = nz // 3 + 1, max(nz // 2, nz // 3 + 1)
+            y0 = ny // 3 + 1
+            y1 = max(2 * ny // 3 - 1, y0)
+            self.keep = 1.0 - ((ix > nx // 3) & (ix < 2 * nx // 3) & (iy >= y0) & (iy <= y1) & (iz >= z0) & (iz <= z1)).double()
+        elif c["dealias"] == "twothirds":
+            kx, ky = (torch.minimum(ix, nx - ix)), (torch.minimum(iy, ny - iy))
+            self.keep = ((kx <= nx // 3) & (ky <= ny // 3) & (iz <= nz // 3)).double()
+
+    def inv(self, a):
+        return torch.fft.irfftn(a, s=self.n, dim=(0, 1, 2), norm="forward")
+
+    def fwd(self, r):
+        return torch.fft.rfftn(r, dim=(0, 1, 2), norm="forward")
+
+    def div(self, u, w):
+        """F[d_j(u_j w_i)] for i = 0, 1, 2 from real fields."""
+        return [1j * sum(self.k[j] * self.fwd(u[j] * w[i]) for j in range(3)) for i in range(3)]
+
+    def solenoidal(self, n):
+        p = sum(k * a for k, a in zip(self.k, n)) / self.k2.clamp(min=1e-300)
+        return [a - k * p for a, k in zip(n, self.k)]
+
+    def reality(self, a):
+        """Hermitian kz = 0 plane from its first half, empty kz = Nz/2 plane."""
+        nx, ny, _ = self.n
+        a = a.clone()
+        p = a[:, :, 0].clone()
+        m = torch.roll(torch.flip(p, (0, 1)), (1, 1), (0, 1)).conj()
+        lower = torch.zeros((nx, ny), dtype=torch.bool)
+        lower[nx // 2 + 1:] = True
+        lower[:, ny // 2] = False
+        lower[0, ny // 2 + 1:] = True
+        a[:, :, 0] = torch.where(lower, m, p)
+        a[:, :, -1] = 0
+        return a
+
+    def force(self, c, v):
+        k = self.k2.sqrt()
+        band = ((k > BAND[0]) & (k <= BAND[1])).double()
+        w = torch.where(self.k[2] == 0, 0.5, 1.0).double() * band
+        e = sum(float((w * (a.real ** 2 + a.imag ** 2)).sum()) for a in v)
+        return [0.1 / (2 * e) * band * a if e > 0 else 0 * a for a in v]
+
+
+def _lawson(v0, rates, rhs, dt, k2, keep):
+    """Lawson RK4 step: rhs(stage fields, the fields its force sees); the first stage advances the dealiased state."""
+    eh = [torch.exp(-r * k2 * 0.5 * dt) for r in rates]
+    k1 = rhs(v0)
+    v = [e * (keep * a + 0.5 * dt * r) for e, a, r in zip(eh, v0, k1)]
+    acc = [e * e * r * (dt / 6) for e, r in zip(eh, k1)]
+    k = rhs(v)
+    v = [e * a + 0.5 * dt * r for e, a, r in zip(eh, v0, k)]
+    acc = [s + e * r * (dt / 3) for s, e, r in zip(acc, eh, k)]
+    k = rhs(v)
+    v = [e * (e * a + dt * r) for e, a, r in zip(eh, v0, k)]
+    acc = [s + e * r * (dt / 3) for s, e, r in zip(acc, eh, k)]
+    k = rhs(v)
+    return [e * e * a + s + r * (dt / 6) for e, a, s, r in zip(eh, v0, acc, k)]
+
+
+def _ns_rhs(f, c):
+    def rhs(v):
+        u = [f.inv(f.keep * a) for a in v]
+        n = f.div(u, u)
+        if c["force"] == 1:
+            n = [a - b for a, b in zip(n, f.force(c, v))]
+        return [-a for a in f.solenoidal(n)]
+    return rhs
+
+
+def _mhd_rhs(f):
+    def rhs(z):
+        u, b = ([f.inv(f.keep * a) for a in z[:3]], [f.inv(f.keep * a) for a in z[3:]])
+        nu = f.solenoidal([p - q for p, q in zip(f.div(u, u), f.div(b, b))])
+        nb = [p - q for p, q in zip(f.div(u, b), f.div(b, u))]
+        return [-a for a in nu + nb]
+    return rhs
+
+
+def _sc_inv(a, sine):
+    """Sum over modes of w_m A_m phi_m(x_j), phi = sin or cos of pi m (j + 1/2) / N, w_0 = 1, w_m = 2."""
+    n = a.shape[0]
+    m, j = torch.arange(n, dtype=torch.int64).reshape(1, -1), torch.arange(n, dtype=torch.int64).reshape(-1, 1)
+    ph = math.pi * ((m * (2 * j + 1)) % (4 * n)).double() / (2 * n)
+    t = (torch.sin(ph) if sine else torch.cos(ph)) * torch.where(m == 0, 0.0 if sine else 1.0, 2.0)
+    return torch.tensordot(t.to(a.dtype), a, dims=([1], [0]))
+
+
+def _sc_fwd(a, sine):
+    n = a.shape[0]
+    m, j = torch.arange(n, dtype=torch.int64).reshape(-1, 1), torch.arange(n, dtype=torch.int64).reshape(1, -1)
+    ph = math.pi * ((m * (2 * j + 1)) % (4 * n)).double() / (2 * n)
+    t = (torch.sin(ph) if sine else torch.cos(ph)) / n
+    return torch.tensordot(t.to(a.dtype), a, dims=([1], [0]))
+
+
+def _wall_inv(a, n, sine):
+    return torch.fft.irfftn(_sc_inv(a, sine), s=n[1:], dim=(1, 2), norm="forward")
+
+
+def _wall_fwd(r, sine):
+    return _sc_fwd(torch.fft.rfftn(r, dim=(1, 2), norm="forward"), sine)
+
+
+def _rbc_exact(c, x):
+    n, kf = _size(c), _kfactor(c)
+    k = _k(n, kf, "cpu", sine_x=True)
+    k2 = sum(a * a for a in k)
+    ix, iy, iz = (torch.arange(n[0]).reshape(-1, 1, 1), torch.arange(n[1]).reshape(1, -1, 1), torch.arange(n[2] // 2 + 1).reshape(1, 1, -1))
+    if c["dealias"] == "corner":
+        y0, z0 = n[1] // 3 + 1, n[2] // 3 + 1
+        cut = (ix > 2 * n[0] // 3) & (iy >= y0) & (iy <= max(2 * n[1] // 3 - 1, y0)) & (iz >= z0) & (iz <= max(n[2] // 2, z0))
+    else:
+        cut = (ix > 2 * n[0] // 3) | (torch.minimum(iy, n[1] - iy) > n[1] // 3) | (iz > n[2] // 3)
+    keep = 1.0 - cut.double()
+    sine = (True, False, False, True)
+    dx = lambda a, s: (k[0] if s else -k[0]) * a
+
+    def rhs(v):
+        r = [_wall_inv(keep * a, n, s) for a, s in zip(v, sine)]
+        out = []
+        for i in range(4):
+            t = 0
+            for j in range(3):
+                s = sine[i] != sine[j]          # the product of a sine and a cosine series is a sine series
+                p = _wall_fwd(r[j] * r[i], s)
+                t = t + (dx(p, s) if j == 0 else 1j * k[j] * p)
+            out.append(t)
+        out[0] = out[0] - v[3]
+        out[3] = out[3] - v[0]
+        p = (k[0] * out[0] + 1j * k[1] * out[1] + 1j * k[2] * out[2]) / k2.clamp(min=1e-300)
+        p[0, 0, 0] = 0
+        return [-(out[0] - k[0] * p), -(out[1] + 1j * k[1] * p), -(out[2] + 1j * k[2] * p), -out[3]]
+
+    rates = [math.sqrt(PR / RA)] * 3 + [1 / math.sqrt(PR * RA)]
+    for _ in range(c["steps"]):
+        x = _lawson(x, rates, rhs, 1e-3, k2, keep)
+        for a in x:
+            a[:, :, -1] = 0
+    return x
+
+
+def _chff_exact(c, v):
+    """One BDF1 step with dense tau solves per (ky, kz) line and the influence matrix of the wall pressure."""
+    n, nu, dt = _size(c), _nu(c), 1e-3
+    nx = n[0]
+    _, ky, kz = _k(n, (1.0, 1.0, 1.0), "cpu")
+    k2 = (ky * ky + kz * kz).reshape(-1)
+    d, _ = _cheb_matrices(nx, "cpu")
+    wt = torch.where(torch.arange(nx) == 0, 1.0, 2.0).double().reshape(-1, 1, 1)
+    inv = lambda a: _wall_inv(a / wt, n, False)
+    fwd = lambda r: wt * _wall_fwd(r, False)
+    dx = lambda a: torch.tensordot(d.to(a.dtype), a, dims=([1], [0]))
+    der = lambda a, j: dx(a) if j == 0 else 1j * (ky if j == 1 else kz) * a
+    u = [inv(a) for a in v]
+    nl = [sum(der(fwd(u[j] * u[i]), j) for j in range(3)) for i in range(3)]
+
+    def solver(lam):
+        m = (d @ d).unsqueeze(0) - lam.reshape(-1, 1, 1) * torch.eye(nx, dtype=torch.float64)
+        m[:, nx - 2] = 1.0                                                                   # u(+1)
+        m[:, nx - 1] = torch.where(torch.arange(nx) % 2 == 0, 1.0, -1.0).double()            # u(-1)
+        # the rows grow as nx^4: each is divided by its largest entry
+        sc = m.abs().amax(dim=2, keepdim=True)
+        lu = torch.linalg.lu_factor(m / sc)
+
+        def solve(r, plus=0.0, minus=0.0):
+            b = -r.reshape(nx, -1).T.clone()
+            b[:, nx - 2], b[:, nx - 1] = plus, minus
+            b = torch.view_as_real(b) / sc if b.is_complex() else b.unsqueeze(-1) / sc
+            z = torch.linalg.lu_solve(*lu, b)
+            z = torch.view_as_complex(z.contiguous()) if z.shape[-1] == 2 else z.squeeze(-1)
+            return z.T.reshape(r.shape)
+        return solve
+
+    pres, vel = solver(k2), solver(k2 + 1 / (dt * nu))
+    shape = (nx, n[1], n[2] // 2 + 1)
+    zero = torch.zeros(shape, dtype=torch.float64)
+    p = pres(sum(der(nl[j], j) for j in range(3)))
+    implicit = lambda i: vel((nl[i] - v[i] / dt + der(p, i)) / -nu)
+    ux = implicit(0)
+    hom = [pres(zero, 1.0, 0.0), pres(zero, 0.0, 1.0)]
+    hv = [vel(dx(h) / -nu) for h in hom]
+    top = (torch.arange(nx).double() ** 2).reshape(-1, 1, 1)
+    bot = top * torch.where(torch.arange(nx) % 2 == 0, -1.0, 1.0).double().reshape(-1, 1, 1)
+    g = lambda a: ((top * a).sum(0), (bot * a).sum(0))
+    (a00, a10), (a01, a11), (r0, r1) = g(hv[0]), g(hv[1]), g(ux)
+    det = a00 * a11 - a01 * a10
+    ok = det.abs() > 1e-15
+    det = torch.where(ok, det, torch.ones_like(det))
+    cp, cm = (ok * (a01 * r1 - a11 * r0) / det, ok * (a10 * r0 - a00 * r1) / det)
+    p = p + cp * hom[0] + cm * hom[1]
+    ux = ux + cp * hv[0] + cm * hv[1]
+    p[:, 0, 0] = 0
+    ux[:, 0, 0] = 0
+    # u_y and u_z see the corrected pressure
+    return [ux, implicit(1), implicit(2), p]
+
+
+def _multiplicity(f):
+    nx, ny, _ = f.n
+    m = torch.where(f.k[2] > 0, 1.0, 0.5).double()
+    edge = (torch.arange(nx).reshape(-1, 1, 1) == nx // 2) | (torch.arange(ny).reshape(1, -1, 1) == ny // 2)
+    return m * torch.where(edge, 2.0, 1.0).double()
+
+
+def _outputs_exact(f, c, v):
+    m, k2 = _multiplicity(f), f.k2
+    k = k2.sqrt()
+    top = math.ceil(math.sqrt(sum(((s // 2) * q) ** 2 for s, q in zip(f.n, f.kf))))
+    w = torch.where(f.k[2] > 0, 1.0, 0.5).double()
+    mag = [a.real ** 2 + a.imag ** 2 for a in v]
+    energy = sum(float((w * a).sum()) for a in mag)
+    diss = _nu(c) * 2 * sum(float((m * k2 * a * (k <= top)).sum()) for a in mag)
+    idx = torch.ceil(k).long().reshape(-1)
+    cnt = torch.bincount(idx, (2 * m).expand_as(k2).reshape(-1), minlength=top + 1)[:top + 1]
+    sp = [torch.bincount(idx, (m * a * k2).reshape(-1), minlength=top + 1)[:top + 1] * (4 * math.pi) / cnt.clamp(min=1e-300) for a in mag]
+    return [energy, diss, np.stack([torch.where(cnt > 0, s, torch.zeros_like(s)).numpy() for s in sp])]
+
+
+def _transfer_exact(f, c, v):
+    r = _radii(c)
+    v = [f.keep * a for a in v]
+    u = [f.inv(a) for a in v]
+    k, m = f.k2.sqrt().expand(v[0].shape), _multiplicity(f)
+    shell = torch.searchsorted(torch.from_numpy(r), k.contiguous(), right=False).reshape(-1)
+    inside = (k <= min(f.n) // 2).double()
+    nr = len(r)
+    s, t = np.zeros((nr, nr)), np.zeros((nr, nr))
+    for g in range(1, nr - 1):
+        w = [f.inv(((k > r[g - 1]) & (k <= r[g])).double() * a) for a in v]
+        d = 2 * m * sum((a * b.conj()).real for a, b in zip(f.div(u, w), v))
+        t[g] = -torch.bincount(shell, d.reshape(-1), minlength=nr).numpy()
+        s[g] = -torch.bincount(shell, (d * inside).reshape(-1), minlength=nr).numpy()
+    flux = np.array([0.0] + [t[1:i + 1, i + 1:].sum() for i in range(1, nr)])
+    return [flux, s]
+
+
+def exact(case, seed):
+    c, kind, n = case, case["kind"], _size(case)
+    points = n[0] * n[1] * n[2]
+    most = {"adjoint": EXACT_SMALL, "transfer": EXACT_SMALL, "spectra": 1 << 25, "transforms": 1 << 25, "chff": 1 << 20}.get(kind, EXACT_POINTS)
+    if points > most or c["force"] == 2 or (kind == "mhd" and points > EXACT_POINTS // 2) or (kind == "rbc" and points > EXACT_POINTS // 4):
+        return None
+    x = [a.cpu() for a in _inputs(c, seed)]
+    if kind == "chff":
+        return _chff_exact(c, x)
+    if kind == "rbc":
+        return _rbc_exact(c, x)
+    f = _Fourier(c)
+    if kind == "transforms":
+        r = f.inv(x[0])
+        pad = torch.zeros((n[0], n[1], n[2] + 2), dtype=torch.float64)
+        pad[:, :, :n[2]] = r
+        return [pad, f.fwd(r)]
+    if kind == "spectra":
+        return _outputs_exact(f, c, x)
+    if kind == "transfer":
+        return _transfer_exact(f, c, x)
+    dt, nu = 1e-3, _nu(c)
+    if kind == "adjoint":
+        v0 = [a.requires_grad_(True) for a in x]
+        v, rhs = v0, _ns_rhs(f, c)
+        for _ in range(c["steps"]):
+            v = _lawson(v, [nu] * 3, rhs, dt, f.k2, f.keep)
+        lam = [(a * _loss_weight(n, "cpu")).detach() for a in v]
+        grad = torch.autograd.grad(v, v0, lam)
+        return [a.detach() for a in v] + list(grad)
+    if kind == "mhd":
+        rhs, rates = _mhd_rhs(f), [nu] * 6
+    else:
+        rhs, rates = _ns_rhs(f, c), [nu] * 3
+    for _ in range(c["steps"]):
+        x = [f.reality(a) for a in _lawson(x, rates, rhs, dt, f.k2, f.keep)]
+    return x + _outputs_exact(f, c, x) if kind == "ns_outputs" else x
+
+
+def work(case):
+    """Inputs read once, outputs written once; 2.5 N log2 N operations a real transform."""
+    n = case["nx"] * case["ny"] * case["nz"]
+    field = 16 * case["nx"] * case["ny"] * (case["nz"] // 2 + 1)
+    fft = 2.5 * n * math.log2(n)
+    kind, steps = case["kind"], case["steps"]
+    if kind == "transforms":
+        return {"bytes": 2 * field + 2 * 8 * n, "flops": 2 * fft}
+    if kind == "spectra":
+        return {"bytes": 3 * field, "flops": 10 * 3 * n}
+    if kind == "transfer":
+        # the field's transforms once, per giver shell its three and the nine products
+        return {"bytes": 3 * field, "flops": (3 + (SHELLS - 1) * 12) * fft}
+    if kind == "chff":
+        return {"bytes": 7 * field, "flops": 9 * fft + 100 * n}
+    fields, per_stage = {"mhd": (6, 14), "rbc": (4, 12)}.get(kind, (3, 8))
+    if kind == "adjoint":
+        # forward, recomputation of all but the last segment, backward (five inverse, three forward a stage)
+        again = steps - ((steps - 1) % case["every"] + 1)
+        return {"bytes": 4 * fields * field, "flops": 4 * 8 * (2 * steps + again) * fft}
+    return {"bytes": 2 * fields * field, "flops": 4 * per_stage * steps * fft}
