@@ -35,6 +35,27 @@ template <typename T>
 __device__ __forceinline__ cpx<T> operator*(T s, cpx<T> a) { return mk<T>(s * a.x, s * a.y); }
 template <typename T>
 __device__ __forceinline__ cpx<T> conj(cpx<T> a) { return mk<T>(a.x, -a.y); }
+// Global loads and stores of one complex value; NT: the non-temporal hint, for
+// passes that stream fields far larger than the caches.
+template <typename T>
+using vec2 = T __attribute__((ext_vector_type(2)));
+template <bool NT, typename T>
+__device__ __forceinline__ cpx<T> gload(const cpx<T> *p)
+{
+    vec2<T> t;
+    if constexpr (NT) t = __builtin_nontemporal_load((const vec2<T> *)p);
+    else t = *(const vec2<T> *)p;
+    return mk<T>(t.x, t.y);
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void gstore(cpx<T> *p, cpx<T> v)
+{
+    vec2<T> t;
+    t.x = v.x;
+    t.y = v.y;
+    if constexpr (NT) __builtin_nontemporal_store(t, (vec2<T> *)p);
+    else *(vec2<T> *)p = t;
+}
 // multiply by i*s (s real): i*s*(x+iy) = -s*y + i*s*x
 template <typename T>
 __device__ __forceinline__ cpx<T> mul_i(T s, cpx<T> a) { return mk<T>(-s * a.y, s * a.x); }
@@ -259,13 +280,64 @@ __device__ __forceinline__ void line_sync()
 __device__ __forceinline__ int lpad(int i) { return i + (i >> 4); }
 __host__ __device__ constexpr int lpad_len(int L) { return L + L / 16 + 1; }
 
+// Exchange of a line's points between the threads that share it, as the FFT
+// passes use it: w(i) is point i of the buffer being written, r(i) of the one
+// being read, publish() makes what was written readable, release() ends the
+// reading (the buffer may be written again).
+//
+// LineX: each line's points consecutive in LDS, one buffer (lpad_len(L)
+// entries), consecutive threads of one line (line_sync).
+template <typename T, int L>
+struct LineX {
+    cpx<T> *p;
+    __device__ __forceinline__ cpx<T> &w(int i) const { return p[lpad(i)]; }
+    __device__ __forceinline__ cpx<T> &r(int i) const { return p[lpad(i)]; }
+    __device__ __forceinline__ void publish() const { line_sync<L / 8>(); }
+    __device__ __forceinline__ void release() const { line_sync<L / 8>(); }
+};
+
+// ColX: the CB lines of a block interleaved (point i of line c at row i,
+// column c), consecutive threads on consecutive lines: thread t holds line
+// t % CB at positions t / CB + TPL s, which is also how it reads a row
+// segment of CB columns from global memory, so a column tile goes from memory
+// to registers and back without passing through LDS; only the exchanges
+// between the FFT passes do, behind block barriers.  Rows of fewer than 128
+// bytes take one pad row in 8 (the first radix-8 pass writes rows 8 apart).
+// NBUF 2: a second buffer, so that an exchange takes one barrier instead of
+// two (a buffer is written again only after the other one's barrier, which
+// every thread reaches after its reads of the first).
+template <typename T, int L, int CB, int NBUF>
+struct ColX {
+    static constexpr bool PAD = CB * sizeof(cpx<T>) < 128;
+    static constexpr int ROWS = PAD ? L + L / 8 : L;
+    static constexpr int SIZE = ROWS * CB;   // entries of one buffer
+    cpx<T> *a, *b;   // buffer to write next, buffer to read (NBUF 1: the same)
+    __device__ __forceinline__ ColX(cpx<T> *lds, int c) : a(lds + c), b(NBUF == 2 ? lds + SIZE + c : lds + c) {}
+    static __device__ __forceinline__ int row(int i) { return (PAD ? i + (i >> 3) : i) * CB; }
+    __device__ __forceinline__ cpx<T> &w(int i) const { return a[row(i)]; }
+    __device__ __forceinline__ cpx<T> &r(int i) const { return b[row(i)]; }
+    __device__ __forceinline__ void publish()
+    {
+        lds_barrier();
+        if constexpr (NBUF == 2) {
+            cpx<T> *t = a;
+            a = b;
+            b = t;
+        }
+    }
+    __device__ __forceinline__ void release() const
+    {
+        if constexpr (NBUF == 1) lds_barrier();
+    }
+};
+
 // One Stockham pass, radix R, stride NS (product of the earlier radices),
 // over a line of L points; thread j of TPL = L/8.  v[] holds positions
 // j + TPL*s on entry.  If LAST, the results stay in v[] at the same
-// positions; otherwise they are written to the LDS line buffer (the caller
-// synchronises and reloads).
-template <int L, int R, int NS, int DIR, bool LAST, typename T>
-__device__ __forceinline__ void stockham_pass(cpx<T> *v, cpx<T> *lds, const cpx<T> *__restrict__ tw, int j)
+// positions; otherwise they are written to the exchange buffer (the caller
+// publishes and reloads).
+template <int L, int R, int NS, int DIR, bool LAST, typename X, typename T>
+__device__ __forceinline__ void stockham_pass(cpx<T> *v, const X &x, const cpx<T> *__restrict__ tw, int j)
 {
     constexpr int TPL = L / 8;
     constexpr int Q = 8 / R;
@@ -288,7 +360,7 @@ __device__ __forceinline__ void stockham_pass(cpx<T> *v, cpx<T> *lds, const cpx<
         } else {
             const int base = (b / NS) * NS * R + k;
 #pragma unroll
-            for (int r = 0; r < R; r++) lds[lpad(base + r * NS)] = a[r];
+            for (int r = 0; r < R; r++) x.w(base + r * NS) = a[r];
         }
     }
 }
@@ -296,8 +368,8 @@ __device__ __forceinline__ void stockham_pass(cpx<T> *v, cpx<T> *lds, const cpx<
 // One odd-radix Stockham pass (R = 3 or 5), LDS to LDS: the L/R butterflies
 // are spread over the TPL threads (ceil(8/R) each, the last round partial);
 // every input is read before the first output is written.
-template <int L, int R, int NS, int DIR, typename T>
-__device__ __forceinline__ void odd_pass(cpx<T> *lds, const cpx<T> *__restrict__ tw, int j)
+template <int L, int R, int NS, int DIR, typename X, typename T>
+__device__ __forceinline__ void odd_pass(X &x, const cpx<T> *__restrict__ tw, int j)
 {
     constexpr int TPL = L / 8, NB = L / R, QM = (NB + TPL - 1) / TPL;
     cpx<T> a[QM][R];
@@ -306,10 +378,10 @@ __device__ __forceinline__ void odd_pass(cpx<T> *lds, const cpx<T> *__restrict__
         const int b = j + TPL * q;
         if (b < NB) {
 #pragma unroll
-            for (int r = 0; r < R; r++) a[q][r] = lds[lpad(b + r * NB)];
+            for (int r = 0; r < R; r++) a[q][r] = x.r(b + r * NB);
         }
     }
-    line_sync<TPL>();
+    x.release();
 #pragma unroll
     for (int q = 0; q < QM; q++) {
         const int b = j + TPL * q;
@@ -323,66 +395,73 @@ __device__ __forceinline__ void odd_pass(cpx<T> *lds, const cpx<T> *__restrict__
             dftR<R, DIR>(a[q]);
             const int base = (b / NS) * NS * R + k;
 #pragma unroll
-            for (int r = 0; r < R; r++) lds[lpad(base + r * NS)] = a[q][r];
+            for (int r = 0; r < R; r++) x.w(base + r * NS) = a[q][r];
         }
     }
-    line_sync<TPL>();
+    x.publish();
 }
 
-template <int L, int DIR, int P, int NS, typename T>
-__device__ __forceinline__ void odd_passes(cpx<T> *lds, const cpx<T> *__restrict__ tw, int j)
+template <int L, int DIR, int P, int NS, typename X, typename T>
+__device__ __forceinline__ void odd_passes(X &x, const cpx<T> *__restrict__ tw, int j)
 {
     if constexpr (P < num_odd_passes(L)) {
         constexpr int R = odd_radix(L, P);
-        odd_pass<L, R, NS, DIR>(lds, tw, j);
-        odd_passes<L, DIR, P + 1, NS * R>(lds, tw, j);
+        odd_pass<L, R, NS, DIR>(x, tw, j);
+        odd_passes<L, DIR, P + 1, NS * R>(x, tw, j);
     }
 }
 
-template <int L, int DIR, int P, int NS, typename T>
-__device__ __forceinline__ void fft_passes(cpx<T> *v, cpx<T> *lds, const cpx<T> *__restrict__ tw, int j)
+template <int L, int DIR, int P, int NS, typename X, typename T>
+__device__ __forceinline__ void fft_passes(cpx<T> *v, X &x, const cpx<T> *__restrict__ tw, int j)
 {
     constexpr int NP = num_passes(L);
     if constexpr (P < NP) {
         constexpr int R = pass_radix(L, P);
         constexpr bool LAST = (P == NP - 1);
-        stockham_pass<L, R, NS, DIR, LAST>(v, lds, tw, j);
+        stockham_pass<L, R, NS, DIR, LAST>(v, x, tw, j);
         if constexpr (!LAST) {
             constexpr int TPL = L / 8;
-            line_sync<TPL>();
+            x.publish();
 #pragma unroll
-            for (int s = 0; s < 8; s++) v[s] = lds[lpad(j + TPL * s)];
-            line_sync<TPL>();
-            fft_passes<L, DIR, P + 1, NS * R>(v, lds, tw, j);
+            for (int s = 0; s < 8; s++) v[s] = x.r(j + TPL * s);
+            x.release();
+            fft_passes<L, DIR, P + 1, NS * R>(v, x, tw, j);
         }
     }
 }
 
 // Full line FFT of L = 8*TPL points (line_length_ok(L), up to 4096), values
 // in registers at positions j + TPL*s.  Exponent sign DIR (-1 forward, +1
-// inverse), unnormalised.  tw[k] = exp(-2 pi i k / L).  Uses the LDS line
-// buffer (lpad_len(L) entries) for the exchanges between passes; every
-// thread of the line must call it (line_sync); the caller must have
-// synchronised if the LDS line was in use before.  The radix-3/5 passes run
-// first, through LDS; the power-of-two passes follow, the last one leaving
-// the results in registers.
-template <int L, int DIR, typename T>
-__device__ __forceinline__ void fft_line(cpx<T> *v, cpx<T> *lds, const cpx<T> *__restrict__ tw, int j)
+// inverse), unnormalised.  tw[k] = exp(-2 pi i k / L).  Uses the exchange x
+// between passes; every thread of the line (ColX: of the block) must call it;
+// the caller must have synchronised if the exchange buffer was in use
+// before.  The radix-3/5 passes run first, through LDS; the power-of-two
+// passes follow, the last one leaving the results in registers.
+template <int L, int DIR, typename X, typename T>
+__device__ __forceinline__ void fft_exchange(cpx<T> *v, X &x, const cpx<T> *__restrict__ tw, int j)
 {
     static_assert(line_length_ok(L), "line length must be 2^a 3^b 5^c with 8 | L");
     if constexpr (odd_part(L) > 1) {
         constexpr int TPL = L / 8;
 #pragma unroll
-        for (int s = 0; s < 8; s++) lds[lpad(j + TPL * s)] = v[s];
-        line_sync<TPL>();
-        odd_passes<L, DIR, 0, 1>(lds, tw, j);
+        for (int s = 0; s < 8; s++) x.w(j + TPL * s) = v[s];
+        x.publish();
+        odd_passes<L, DIR, 0, 1>(x, tw, j);
 #pragma unroll
-        for (int s = 0; s < 8; s++) v[s] = lds[lpad(j + TPL * s)];
-        line_sync<TPL>();
-        fft_passes<L, DIR, 0, odd_part(L)>(v, lds, tw, j);
+        for (int s = 0; s < 8; s++) v[s] = x.r(j + TPL * s);
+        x.release();
+        fft_passes<L, DIR, 0, odd_part(L)>(v, x, tw, j);
     } else {
-        fft_passes<L, DIR, 0, 1>(v, lds, tw, j);
+        fft_passes<L, DIR, 0, 1>(v, x, tw, j);
     }
+}
+
+// fft_exchange on consecutive points in LDS (the z lines and the sin/cos lines).
+template <int L, int DIR, typename T>
+__device__ __forceinline__ void fft_line(cpx<T> *v, cpx<T> *lds, const cpx<T> *__restrict__ tw, int j)
+{
+    LineX<T, L> x{lds};
+    fft_exchange<L, DIR>(v, x, tw, j);
 }
 
 }  // namespace tg

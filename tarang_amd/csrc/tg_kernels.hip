@@ -38,12 +38,17 @@ struct ColArgs {
     int nouter;
 };
 
-template <typename T, int L, int DIR, int CB>
+// Bound by HBM (each field read and written once).  A thread's row segment and
+// its share of the transform are the same points (ColX), so LDS carries only
+// the exchanges between the radix passes; 512^3 FP64, per field: 476 us with
+// the tile staged through LDS both ways, 381 us (5.7 TB/s, a copy's 6.2) with
+// this layout, whole rows and non-temporal access.
+template <typename T, int L, int DIR, int CB, bool NT>
 __global__ void __launch_bounds__(CB *(L / 8)) k_colfft(ColArgs a)
 {
     constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    __shared__ cpx<T> lds[CB * LP];
+    using X = ColX<T, L, CB, 1>;
+    __shared__ cpx<T> lds[X::SIZE];
     // xcd_tile: the column blocks of one outer index run in turn on one XCD,
     // so the rows' 128-byte lines that two blocks share (CB columns of fewer
     // than 128 bytes) are fetched into one L2
@@ -52,40 +57,19 @@ __global__ void __launch_bounds__(CB *(L / 8)) k_colfft(ColArgs a)
     if (b >= a.nouter * nblk) return;
     const int outer = b / nblk;
     const int c0 = (b % nblk) * CB;
-    cpx<T> *f = (cpx<T> *)a.f[blockIdx.y] + (size_t)outer * a.outer_stride;
-    const cpx<T> *tw = (const cpx<T> *)a.tw;
-    // thread t moves column t % CB, rows t / CB + TPL i: the eight loads are
-    // issued before the first LDS write (a column past the last one loads
-    // the last one, stages zeros and is not stored)
-    const int sc = threadIdx.x % CB, sr = threadIdx.x / CB, scol = c0 + sc;
-    const bool live = scol < a.ncol;
-    {
-        const cpx<T> *p = f + (size_t)sr * a.row_stride + min(scol, a.ncol - 1);
-        const size_t step = (size_t)TPL * a.row_stride;
-        cpx<T> x[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) x[i] = mk<T>(p[i * step].x, p[i * step].y);
-#pragma unroll
-        for (int i = 0; i < 8; i++) lds[sc * LP + lpad(sr + TPL * i)] = live ? x[i] : mk<T>(0, 0);
-    }
-    lds_barrier();
-    const int c = threadIdx.x / TPL, j = threadIdx.x % TPL;
+    const int c = threadIdx.x % CB, j = threadIdx.x / CB, col = c0 + c;
+    // a column past the last one transforms the last one and is not stored
+    cpx<T> *p = (cpx<T> *)a.f[blockIdx.y] + (size_t)outer * a.outer_stride + (size_t)j * a.row_stride +
+                min(col, a.ncol - 1);
+    const size_t step = (size_t)TPL * a.row_stride;
     cpx<T> v[8];
 #pragma unroll
-    for (int s = 0; s < 8; s++) v[s] = lds[c * LP + lpad(j + TPL * s)];
-    lds_barrier();
-    fft_line<L, DIR>(v, lds + c * LP, tw, j);
+    for (int s = 0; s < 8; s++) v[s] = gload<NT>(p + s * step);
+    X x(lds, c);
+    fft_exchange<L, DIR>(v, x, (const cpx<T> *)a.tw, j);
+    if (col < a.ncol) {
 #pragma unroll
-    for (int s = 0; s < 8; s++) lds[c * LP + lpad(j + TPL * s)] = v[s];
-    lds_barrier();
-    if (live) {
-        cpx<T> *p = f + (size_t)sr * a.row_stride + scol;
-        const size_t step = (size_t)TPL * a.row_stride;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const cpx<T> v = lds[sc * LP + lpad(sr + TPL * i)];
-            p[i * step] = mk<T>(v.x, v.y);
-        }
+        for (int s = 0; s < 8; s++) gstore<NT>(p + s * step, v[s]);
     }
 }
 
@@ -868,14 +852,27 @@ __global__ void k_dealias(PlaneArgs a)
 template <typename T, int LL>
 hipError_t colfft_len(const ColArgs &a, int dir, int nfields, hipStream_t st)
 {
-    // at most 512 threads a block, except FP32 lines of 512 points and
-    // more: 1024-thread blocks (16 columns at 512 points, 8 at 1024) run
-    // 2% and 9% faster than the 512-thread tiles of half the width
-    constexpr int CB = std::min(col_block<T>(LL, sizeof(cpx<T>)),
-                                std::max(1, (sizeof(T) == 4 && LL >= 512 ? 1024 : 512) / (LL / 8)));
+    // Tiles of 128-byte rows (8 FP64 or 16 FP32 columns), fewer only where a
+    // block would pass 1024 threads: with rows of 64 bytes the in-place pass of
+    // five 512^3 FP64 fields takes 2461 us against 2017, and at 1024 points,
+    // where the wide tile leaves one block per CU, 2485 against 2152.
+    constexpr int CB = std::max(1, std::min(128 / (int)sizeof(cpx<T>), 1024 / (LL / 8)));
+    // Non-temporal loads and stores where the pass streams more than the 256
+    // MiB memory-side cache holds (five 512^3 FP64 fields 2017 -> 1892 us in a
+    // loop of the pass alone, 445 -> 381 us per field within the step); 128^3
+    // FP32 lost 5% in the z pass that follows.  Not where a CU holds one block
+    // (1024 points FP64 2152 against 2226 us) or the rows are half lines.
+    constexpr bool STREAM = CB * sizeof(cpx<T>) == 128 && 2 * ColX<T, LL, CB, 1>::SIZE * sizeof(cpx<T>) <= 160 * 1024;
     dim3 grid(x_grid(a.nouter * ((a.ncol + CB - 1) / CB)), nfields);
-    if (dir < 0) hipLaunchKernelGGL((k_colfft<T, LL, -1, CB>), grid, dim3(CB * (LL / 8)), 0, st, a);
-    else hipLaunchKernelGGL((k_colfft<T, LL, +1, CB>), grid, dim3(CB * (LL / 8)), 0, st, a);
+    const dim3 block(CB * (LL / 8));
+    const bool nt = STREAM && stream_bytes((size_t)nfields * a.nouter * a.outer_stride * sizeof(cpx<T>));
+    if (dir < 0) {
+        if (nt) hipLaunchKernelGGL((k_colfft<T, LL, -1, CB, STREAM>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_colfft<T, LL, -1, CB, false>), grid, block, 0, st, a);
+    } else {
+        if (nt) hipLaunchKernelGGL((k_colfft<T, LL, +1, CB, STREAM>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_colfft<T, LL, +1, CB, false>), grid, block, 0, st, a);
+    }
     return hipGetLastError();
 }
 
@@ -980,7 +977,10 @@ hipError_t launch_colfft(const Grid &g, int axis, int dir, void *const *fields, 
         a.nouter = g.nx;
         a.outer_stride = (long long)g.ny * g.nzp;
         a.row_stride = g.nzp;
-        a.ncol = g.nzc;
+        // the pad columns too (they hold zeros): a row's last 128-byte line is
+        // written whole (257 of 264 columns written: 1903 us a launch at 512^3
+        // FP64, all 264: 1780)
+        a.ncol = g.nzp;
     } else {
         L = g.nx;
         a.nouter = 1;

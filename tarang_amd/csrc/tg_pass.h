@@ -9,6 +9,10 @@ namespace tg {
 
 static constexpr int kLdsBudget = 73728;  // bytes; two blocks fit the 160 KB LDS of a CU
 
+// Whether a pass over `bytes` of fields streams past the 256 MiB memory-side
+// cache, so that nothing it writes is still there for the next pass.
+inline bool stream_bytes(size_t bytes) { return bytes > ((size_t)256 << 20); }
+
 __device__ __forceinline__ int kwave(int l, int n) { return l <= n / 2 ? l : l - n; }
 
 __device__ __forceinline__ bool dealias_zero(const Grid &g, int lx, int ly, int lz)
