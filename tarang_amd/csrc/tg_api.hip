@@ -1580,7 +1580,7 @@ int tg_energy_transfer(tg_plan *plan, double *const V_dev[3], const double *radi
     // T[m][k]: transfer from giver shell m into receiver shell k, all modes
     // (the flux's receiver includes the modes beyond the largest inscribed
     // sphere, which the shell-to-shell matrix leaves out)
-    std::vector<double> row(nr), T((size_t)nr * nr, 0.0);
+    std::vector<double> row(2 * (size_t)nr), T((size_t)nr * nr, 0.0);
     const int kin = max_radius_inside(plan->g);
     for (int m = 1; m < n; m++) {
         rc = DISPATCH_PREC(plan, run_giver_nlin)(plan, V_dev, V_dev, 8, radii[m - 1], radii[m], plan->acc,
@@ -1588,12 +1588,12 @@ int tg_energy_transfer(tg_plan *plan, double *const V_dev[3], const double *radi
         if (rc) return rc;
         const double *A[3] = {plan->acc[0], plan->acc[1], plan->acc[2]};
         const double *B[3] = {V_dev[0], V_dev[1], V_dev[2]};
-        rc = reduce_to_host(plan, RED_SHELL_ALL, A, B, 3, 0, radii, nr, 1, kin, 0, 0, row.data());
+        rc = reduce_to_host(plan, RED_SHELL_PAIR, A, B, 3, 0, radii, nr, 2, kin, 0, 0, row.data());
         if (rc) return rc;
-        for (int k = 0; k < nr; k++) S[(size_t)m * nr + k] = -row[k];
-        rc = reduce_to_host(plan, RED_SHELL_ALL_NOCUT, A, B, 3, 0, radii, nr, 1, kin, 0, 0, row.data());
-        if (rc) return rc;
-        for (int k = 0; k < nr; k++) T[(size_t)m * nr + k] = -row[k];
+        for (int k = 0; k < nr; k++) {
+            T[(size_t)m * nr + k] = -row[k];
+            S[(size_t)m * nr + k] = -row[(size_t)nr + k];
+        }
     }
     // flux through sphere s: givers inside (shells 1..s), receivers outside
     flux[0] = 0.0;

@@ -11,7 +11,7 @@ enum {
     RED_SN = 1,              // sum m K^n |A|^2 (K <= kcut; origin skipped for n = 0)
     RED_SPECTRUM = 2,        // bins ceil(K) <= kcut: [m K^n |A|^2 K^2, 2m]
     RED_SHELL_ALL = 3,       // bins first radii >= K, K <= kcut: 2m Re(A.B*)
-    RED_SHELL_ALL_NOCUT = 4, // same without the K cut
+    RED_SHELL_PAIR = 4,      // same over all modes, and over K <= kcut
     RED_SHELL_SINGLE = 5,    // sum over r_lo < K <= r_hi of 2m Re(A.B*)
     RED_CROSS = 6,           // sum w Re(A B*), w = 1/2 on kz = 0
     // anisotropic bins (RedAniso): shell-major, (sub-bins + 1) per shell
