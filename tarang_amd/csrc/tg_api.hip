@@ -75,6 +75,8 @@ struct tg_plan {
     double *force_eh = nullptr;
     int force_eh_n = 0;
     double force_key[4] = {};  // eps, helicity, r_in, r_out of the table
+    double *force_tab = nullptr;   // the force of the band's slots for the call's seed
+    size_t force_tab_bytes = 0;
     // chaining of RK4 steps: valid for the same state pointers and band
     bool unext_valid = false;
     double *unext_V[3] = {};
@@ -85,7 +87,6 @@ struct tg_plan {
     int *nonfinite_host = nullptr;
     // host-side band config for the current step
     Band band{};
-    int x_tile_columns = 0;  // fused x-pass tile width (0 = LDS-budget width)
     // SFF: quarter-wave twiddles exp(-i pi k / (2 Nx)), k < Nx
     void *twq = nullptr;
     // RBC buffers, allocated on first use: [0] theta accumulator (FP64 padded
@@ -226,7 +227,7 @@ void free_plan(tg_plan *p)
     for (void *q : p->mhd)
         if (q) (void)hipFree(q);
     void *aptrs[] = {p->adj.ckpt, p->adj.tape, p->adj.vw, p->adj.lg, p->adj.acc, p->nonfinite_dev, p->rfield,
-                     p->umax_dev, p->force_eh};
+                     p->umax_dev, p->force_eh, p->force_tab};
     for (void *q : aptrs)
         if (q) (void)hipFree(q);
     void *cptrs[] = {p->ch.tmp, p->ch.D, p->ch.S, p->ch.NL[0], p->ch.NL[1], p->ch.NL[2], p->ch.R[0], p->ch.R[1],
@@ -296,7 +297,7 @@ int ensure_slots(tg_plan *p, const tg_fluid *f)
         if (kb > p->g.nx / 2 - 1 || kb > p->g.ny / 2 - 1 || kb > p->g.nz / 2 - 1 || kb > 64)
             return fail(TG_ERR_ARG, "forcing band r_out=%g too large for this grid", f->force_r_out);
         b.kind = 1;
-        b.kb = kb;
+        b.h[0] = b.h[1] = b.h[2] = kb;
         b.r_in = f->force_r_in;
         b.r_out = f->force_r_out;
         b.eps = f->force_eps;
@@ -340,23 +341,41 @@ int ensure_slots(tg_plan *p, const tg_fluid *f)
         b.shell_eh = p->force_eh;
         b.tau = f->force_tau;
         b.seed = f->force_seed;
+        const int n[3] = {p->g.nx, p->g.ny, p->g.nz};
+        for (int d = 0; d < 3; d++)
+            b.h[d] = (int)std::min<double>(std::ceil(f->force_r_out / p->g.kf[d]), n[d] / 2);
+        const size_t bytes = (size_t)(2 * b.h[0] + 1) * (2 * b.h[1] + 1) * (b.h[2] + 1) * 3 * 16;
+        if (bytes > p->force_tab_bytes) {
+            HIPCHK(hipStreamSynchronize(p->stream));
+            if (p->force_tab) {
+                (void)hipFree(p->force_tab);
+                p->dev_bytes -= (int64_t)p->force_tab_bytes;
+                p->force_tab = nullptr;
+                p->force_tab_bytes = 0;
+            }
+            int rc = dmalloc(p, (void **)&p->force_tab, bytes);
+            if (rc) return rc;
+            p->force_tab_bytes = bytes;
+        }
+        b.force = p->force_tab;
+        HIPCHK(launch_random_force(p->g, b, p->force_tab, p->stream));
     } else if (f && f->force_kind != 0) {
         return fail(TG_ERR_ARG, "unknown force_kind %d", f->force_kind);
     }
     p->band = b;
     if (b.kind != 1) return TG_OK;
-    if (p->slot_kb != b.kb) {
+    if (p->slot_kb != b.h[0]) {
         // the stage-1 transform prepared for a continuation has no slots here
         p->unext_valid = false;
         for (int i = 0; i < 2; i++)
             if (p->slots[i]) { (void)hipFree(p->slots[i]); p->slots[i] = nullptr; }
-        p->nslots = (size_t)band_nslots(b.kb);
+        p->nslots = (size_t)band_nslots(b);
         for (int i = 0; i < 2; i++) {
             int rc = dmalloc(p, (void **)&p->slots[i], p->nslots * 3 * 16);
             if (rc) return rc;
             HIPCHK(hipMemsetAsync(p->slots[i], 0, p->nslots * 3 * 16, p->stream));
         }
-        p->slot_kb = b.kb;
+        p->slot_kb = b.h[0];
     }
     return TG_OK;
 }
@@ -518,7 +537,7 @@ int run_rk4(tg_plan *p, double *const V[3], const tg_fluid *f, int nsteps, int f
     int rc = ensure_slots(p, f);
     if (rc) return rc;
     const Band &ob = p->unext_band, &nb = p->band;
-    const bool same_band = ob.kind == nb.kind && ob.kb == nb.kb && ob.r_in == nb.r_in && ob.r_out == nb.r_out &&
+    const bool same_band = ob.kind == nb.kind && ob.h[0] == nb.h[0] && ob.r_in == nb.r_in && ob.r_out == nb.r_out &&
                            ob.eps == nb.eps;
     const bool cont = (flags & TG_STEP_CONTINUE) && p->unext_valid && same_band && p->unext_V[0] == V[0] &&
                       p->unext_V[1] == V[1] && p->unext_V[2] == V[2];
@@ -538,7 +557,7 @@ int run_rk4(tg_plan *p, double *const V[3], const tg_fluid *f, int nsteps, int f
             if (s == 4) rk.nonfinite = p->nonfinite_dev;
             Prof pr(p, TG_KERNEL_X_NLIN_RK);
             HIPCHK(launch_x_nlin<T>(p->g, p->band, rk, p->P, V, p->acc, p->U, p->slots[(s - 1) & 1],
-                                    p->slots[s & 1], nullptr, p->twx, p->stream, p->x_tile_columns));
+                                    p->slots[s & 1], nullptr, p->twx, p->stream));
         }
         if (p->cfg.strong_reality) {
             Prof pr(p, TG_KERNEL_REALITY);
@@ -748,7 +767,7 @@ int record_steps(tg_plan *p, double *const V[3], const tg_fluid *f, int nsteps)
             rk.trace_free = 1;
             Prof pr(p, TG_KERNEL_X_NLIN_RK);
             HIPCHK(launch_x_nlin<T>(p->g, nb, rk, p->P, V, p->acc, p->U, nullptr, nullptr, nullptr, p->twx,
-                                    p->stream, p->x_tile_columns));
+                                    p->stream));
         }
     p->unext_valid = false;
     return TG_OK;
@@ -1148,7 +1167,6 @@ int tg_plan_create(const tg_config *cfg, tg_plan **plan)
         const int per_line = 128 / (int)p->elem;  // elements per 128-byte line
         p->g.nzp = (p->g.nzc + per_line - 1) / per_line * per_line;
     }
-    if (const char *e = getenv("TG_X_TILE_COLUMNS")) p->x_tile_columns = atoi(e);
     p->nc = (size_t)cfg->nx * cfg->ny * (cfg->nz / 2 + 1);
     p->ncw = (size_t)cfg->nx * cfg->ny * p->g.nzp;
     int rc = set_device(p);

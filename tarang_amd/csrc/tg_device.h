@@ -303,32 +303,18 @@ struct LineX {
 // to registers and back without passing through LDS; only the exchanges
 // between the FFT passes do, behind block barriers.  Rows of fewer than 128
 // bytes take one pad row in 8 (the first radix-8 pass writes rows 8 apart).
-// NBUF 2: a second buffer, so that an exchange takes one barrier instead of
-// two (a buffer is written again only after the other one's barrier, which
-// every thread reaches after its reads of the first).
-template <typename T, int L, int CB, int NBUF>
+// (Two buffers, which save every other barrier, gained nothing in the x pass:
+// 4750 against 4795 us a launch at 512^3 FP64.)
+template <typename T, int L, int CB>
 struct ColX {
     static constexpr bool PAD = CB * sizeof(cpx<T>) < 128;
-    static constexpr int ROWS = PAD ? L + L / 8 : L;
-    static constexpr int SIZE = ROWS * CB;   // entries of one buffer
-    cpx<T> *a, *b;   // buffer to write next, buffer to read (NBUF 1: the same)
-    __device__ __forceinline__ ColX(cpx<T> *lds, int c) : a(lds + c), b(NBUF == 2 ? lds + SIZE + c : lds + c) {}
+    static constexpr int SIZE = (PAD ? L + L / 8 : L) * CB;   // entries
+    cpx<T> *p;   // column c of the buffer
     static __device__ __forceinline__ int row(int i) { return (PAD ? i + (i >> 3) : i) * CB; }
-    __device__ __forceinline__ cpx<T> &w(int i) const { return a[row(i)]; }
-    __device__ __forceinline__ cpx<T> &r(int i) const { return b[row(i)]; }
-    __device__ __forceinline__ void publish()
-    {
-        lds_barrier();
-        if constexpr (NBUF == 2) {
-            cpx<T> *t = a;
-            a = b;
-            b = t;
-        }
-    }
-    __device__ __forceinline__ void release() const
-    {
-        if constexpr (NBUF == 1) lds_barrier();
-    }
+    __device__ __forceinline__ cpx<T> &w(int i) const { return p[row(i)]; }
+    __device__ __forceinline__ cpx<T> &r(int i) const { return p[row(i)]; }
+    __device__ __forceinline__ void publish() const { lds_barrier(); }
+    __device__ __forceinline__ void release() const { lds_barrier(); }
 };
 
 // One Stockham pass, radix R, stride NS (product of the earlier radices),
@@ -369,7 +355,7 @@ __device__ __forceinline__ void stockham_pass(cpx<T> *v, const X &x, const cpx<T
 // are spread over the TPL threads (ceil(8/R) each, the last round partial);
 // every input is read before the first output is written.
 template <int L, int R, int NS, int DIR, typename X, typename T>
-__device__ __forceinline__ void odd_pass(X &x, const cpx<T> *__restrict__ tw, int j)
+__device__ __forceinline__ void odd_pass(const X &x, const cpx<T> *__restrict__ tw, int j)
 {
     constexpr int TPL = L / 8, NB = L / R, QM = (NB + TPL - 1) / TPL;
     cpx<T> a[QM][R];
@@ -402,7 +388,7 @@ __device__ __forceinline__ void odd_pass(X &x, const cpx<T> *__restrict__ tw, in
 }
 
 template <int L, int DIR, int P, int NS, typename X, typename T>
-__device__ __forceinline__ void odd_passes(X &x, const cpx<T> *__restrict__ tw, int j)
+__device__ __forceinline__ void odd_passes(const X &x, const cpx<T> *__restrict__ tw, int j)
 {
     if constexpr (P < num_odd_passes(L)) {
         constexpr int R = odd_radix(L, P);
@@ -412,7 +398,7 @@ __device__ __forceinline__ void odd_passes(X &x, const cpx<T> *__restrict__ tw, 
 }
 
 template <int L, int DIR, int P, int NS, typename X, typename T>
-__device__ __forceinline__ void fft_passes(cpx<T> *v, X &x, const cpx<T> *__restrict__ tw, int j)
+__device__ __forceinline__ void fft_passes(cpx<T> *v, const X &x, const cpx<T> *__restrict__ tw, int j)
 {
     constexpr int NP = num_passes(L);
     if constexpr (P < NP) {
@@ -438,7 +424,7 @@ __device__ __forceinline__ void fft_passes(cpx<T> *v, X &x, const cpx<T> *__rest
 // before.  The radix-3/5 passes run first, through LDS; the power-of-two
 // passes follow, the last one leaving the results in registers.
 template <int L, int DIR, typename X, typename T>
-__device__ __forceinline__ void fft_exchange(cpx<T> *v, X &x, const cpx<T> *__restrict__ tw, int j)
+__device__ __forceinline__ void fft_exchange(cpx<T> *v, const X &x, const cpx<T> *__restrict__ tw, int j)
 {
     static_assert(line_length_ok(L), "line length must be 2^a 3^b 5^c with 8 | L");
     if constexpr (odd_part(L) > 1) {
@@ -460,7 +446,7 @@ __device__ __forceinline__ void fft_exchange(cpx<T> *v, X &x, const cpx<T> *__re
 template <int L, int DIR, typename T>
 __device__ __forceinline__ void fft_line(cpx<T> *v, cpx<T> *lds, const cpx<T> *__restrict__ tw, int j)
 {
-    LineX<T, L> x{lds};
+    const LineX<T, L> x{lds};
     fft_exchange<L, DIR>(v, x, tw, j);
 }
 

@@ -16,19 +16,22 @@ struct Grid {
     int basis;            // 0 FFF; 1 SFF (sin/cos along x: kx = lx, K_x = lx*kf[0])
 };
 
-// Forcing band slots: modes with |kx|,|ky| <= kb and 0 <= kz <= kb.
+// Forcing band: slots for the modes of the box |kx| <= h[0], |ky| <= h[1],
+// 0 <= kz <= h[2].
 struct Band {
     int kind;             // 0 none, 1 constant energy supply alpha-forcing, 2 random band forcing
-    int kb;               // slot box half-width
+    int h[3];             // box half-widths
     double r_in, r_out, eps;
-    // kind 2: per-mode supplies (e_k, h_k) of shells 0..ceil(r_out), random
+    // kind 2: the force of every slot (launch_random_force), made from the
+    // per-mode supplies (e_k, h_k) of shells 0..ceil(r_out), the random
     // interval and the seed of the phases
+    const double *force;
     const double *shell_eh;
     double tau;
     unsigned long long seed;
 };
 
-__host__ __device__ inline int band_nslots(int kb) { return (2 * kb + 1) * (2 * kb + 1) * (kb + 1); }
+__host__ __device__ inline int band_nslots(const Band &b) { return (2 * b.h[0] + 1) * (2 * b.h[1] + 1) * (b.h[2] + 1); }
 
 // Launch helpers (defined in tg_kernels.hip).  All return hipError_t.
 // T is float or double (transform precision).
@@ -91,13 +94,13 @@ struct RkParams {
 
 // Fused x pass: forward x-FFT of the 6 (giver: 9) products, nonlinear term, RHS and the
 // Lawson RK4 stage algebra, next stage input, dealias, inverse x-FFT.
-// x_tile_columns selects the tile width: the LDS-budget width, or half of it
-// (smaller blocks, more of them resident per CU).
 template <typename T>
 hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void *const *P, double *const *V,
                          double *const *acc, void *const *U, const double *slots_in, double *slots_out,
-                         double *const *out, const void *twx, hipStream_t st, int x_tile_columns = 0);
+                         double *const *out, const void *twx, hipStream_t st);
 
+// the random force (kind 2) of the band's slots, 3 complex values each
+hipError_t launch_random_force(const Grid &g, const Band &b, double *out, hipStream_t st);
 hipError_t launch_reality(const Grid &g, double *const *V, int ncomp, hipStream_t st);
 // n ints at p set to v by a kernel (no memset node, so it may be captured)
 hipError_t launch_fill_int(int *p, int n, int v, hipStream_t st);

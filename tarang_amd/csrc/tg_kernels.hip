@@ -47,7 +47,7 @@ template <typename T, int L, int DIR, int CB, bool NT>
 __global__ void __launch_bounds__(CB *(L / 8)) k_colfft(ColArgs a)
 {
     constexpr int TPL = L / 8;
-    using X = ColX<T, L, CB, 1>;
+    using X = ColX<T, L, CB>;
     __shared__ cpx<T> lds[X::SIZE];
     // xcd_tile: the column blocks of one outer index run in turn on one XCD,
     // so the rows' 128-byte lines that two blocks share (CB columns of fewer
@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(CB *(L / 8)) k_colfft(ColArgs a)
     cpx<T> v[8];
 #pragma unroll
     for (int s = 0; s < 8; s++) v[s] = gload<NT>(p + s * step);
-    X x(lds, c);
+    const X x{lds + c};
     fft_exchange<L, DIR>(v, x, (const cpx<T> *)a.tw, j);
     if (col < a.ncol) {
 #pragma unroll
@@ -396,16 +396,19 @@ struct XnlArgs {
     RkParams rk;
 };
 
-__device__ double band_alpha(const Grid &g, const Band &b, const double *slots)
+// alpha = eps / (2 E_band) with E_band = sum w |V|^2 over the band modes,
+// w = 1/2 on kz = 0 (Get_local_energy weights, FFF_pencil_energy.cc:59-67),
+// summed by the NT threads of the block in a fixed order (red: 16 values of
+// LDS; every thread of the block calls it).
+template <int NT>
+__device__ __forceinline__ double band_alpha(const Grid &g, const Band &b, const double *slots, double *red)
 {
-    // alpha = eps / (2 E_band) with E_band = sum w |V|^2 over the band modes,
-    // w = 1/2 on kz = 0 (Get_local_energy weights, FFF_pencil_energy.cc:59-67)
-    const int n = band_nslots(b.kb);
+    const int n = band_nslots(b);
     double e = 0.0;
-    for (int s = 0; s < n; s++) {
-        const int kz = s % (b.kb + 1);
-        const int ky = (s / (b.kb + 1)) % (2 * b.kb + 1) - b.kb;
-        const int kx = s / ((b.kb + 1) * (2 * b.kb + 1)) - b.kb;
+    for (int s = threadIdx.x; s < n; s += NT) {
+        const int kz = s % (b.h[2] + 1);
+        const int ky = (s / (b.h[2] + 1)) % (2 * b.h[1] + 1) - b.h[1];
+        const int kx = s / ((b.h[2] + 1) * (2 * b.h[1] + 1)) - b.h[0];
         const double K = kmag(g, kx, ky, kz);
         if (K > b.r_in && K <= b.r_out) {
             const double w = kz == 0 ? 0.5 : 1.0;
@@ -415,7 +418,17 @@ __device__ double band_alpha(const Grid &g, const Band &b, const double *slots)
             }
         }
     }
-    return e > 0.0 ? b.eps / (2.0 * e) : 0.0;
+    // lanes past the block's last thread hold nothing to add
+    constexpr int NW = (NT + 63) / 64;
+    for (int off = 32; off > 0; off >>= 1) {
+        const double t = __shfl_down(e, off, 64);
+        if ((int)(threadIdx.x & 63) + off < 64 && (int)threadIdx.x + off < NT) e += t;
+    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64] = e;
+    lds_barrier();
+    double t = 0.0;
+    for (int w = 0; w < NW; w++) t += red[w];
+    return t > 0.0 ? b.eps / (2.0 * t) : 0.0;
 }
 
 // Random band forcing of one mode (kind 2; compute_force_random.cc:65-130,
@@ -442,173 +455,241 @@ __device__ void random_force_mode(const Grid &g, const Band &b, int lx, int ly, 
     F[2] = (-st) * U2;
 }
 
-// Order in which the product spectra are folded into N, following the
-// reference's diag/offdiag accumulation (compute_diag_offdiag.cc:47-112 for
-// NS, :329-414 for the giver form with P[3i+j] = FT[u_j w_i]).
-static __constant__ int kNsOrder[6] = {0, 1, 2, 3, 4, 5};
-// NS products xx, yy, zz, xy, yz, zx: derivative applied for N_0, N_1, N_2
-// (Compute_nlin_diag, then Compute_nlin_offdiag's Add_*deriv calls).
-static __constant__ int kNsSel[6][3] = {{1, 0, 0}, {0, 2, 0}, {0, 0, 3}, {2, 1, 0}, {0, 3, 2}, {3, 0, 1}};
-// The trace-shifted five (xx - zz, yy - zz, xy, yz, zx; projected stages only).
-static __constant__ int kNsSel5[5][3] = {{1, 0, 0}, {0, 2, 0}, {2, 1, 0}, {0, 3, 2}, {3, 0, 1}};
-static __constant__ int kGiverOrder[9] = {0, 4, 8, 3, 1, 7, 5, 2, 6};
+#if TG_LEN_UNIT == 0
+// The random force of every mode of the box |k_d| <= h_d in band_slot order,
+// zero outside r_in < K <= r_out.  The phases hold for a whole call, so they
+// are drawn once here: within the x pass their sines and cosines were most of
+// its instructions (0.5 ms of a 512^3 FP64 step).
+__global__ void k_random_force(Grid g, Band b, double *out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= band_nslots(b)) return;
+    const int kz = i % (b.h[2] + 1);
+    const int ky = (i / (b.h[2] + 1)) % (2 * b.h[1] + 1) - b.h[1];
+    const int kx = i / ((b.h[2] + 1) * (2 * b.h[1] + 1)) - b.h[0];
+    // the indices of the mode; k = -N/2 is not one
+    const int lx = kx >= 0 ? kx : kx + g.nx, ly = ky >= 0 ? ky : ky + g.ny;
+    const double K = kmag(g, kx, ky, kz);
+    cpx<double> F[3] = {mk<double>(0, 0), mk<double>(0, 0), mk<double>(0, 0)};
+    if (K > b.r_in && K <= b.r_out && kwave(lx, g.nx) == kx && kwave(ly, g.ny) == ky && kz < g.nzc)
+        random_force_mode(g, b, lx, ly, kz, kx, ky, K, F);
+    for (int c = 0; c < 3; c++) ((cpx<double> *)out)[3 * (size_t)i + c] = F[c];
+}
 
-template <typename T, int L, int CB, int MODE>
+hipError_t launch_random_force(const Grid &g, const Band &b, double *out, hipStream_t st)
+{
+    const int n = band_nslots(b);
+    hipLaunchKernelGGL(k_random_force, dim3((n + 63) / 64), dim3(64), 0, st, g, b, out);
+    return hipGetLastError();
+}
+#endif
+
+// The x pass's products, in the reference's accumulation order
+// (compute_diag_offdiag.cc:47-112 for NS, :329-414 for the giver form).
+enum {
+    XNL_SIX = 0,    // NS products xx, yy, zz, xy, yz, zx
+    XNL_GIVER = 1,  // P[3i+j] = FT[u_j w_i]: i K_j P to N_i
+    XNL_TRANS = 2,  // transposed (MHD: N-_j = sum_i d_i(Z+_i Z-_j)): i K_i P to N_j
+    XNL_FIVE = 3,   // trace-shifted xx - zz, yy - zz, xy, yz, zx, where the nonlinear
+                    // term is only used projected (its gradient part i K F[u_z^2]
+                    // drops out)
+};
+constexpr int xnl_products(int mode) { return mode == XNL_SIX ? 6 : (mode == XNL_FIVE ? 5 : 9); }
+constexpr int xnl_index(int mode, int pi)
+{
+    constexpr int giver[9] = {0, 4, 8, 3, 1, 7, 5, 2, 6};
+    return mode == XNL_SIX || mode == XNL_FIVE ? pi : giver[pi];
+}
+// product index p of mode: the axis d whose i K_d FT[p] is added to N_i, -1: none
+constexpr int xnl_axis(int mode, int p, int i)
+{
+    if (mode == XNL_GIVER) return p / 3 == i ? p % 3 : -1;
+    if (mode == XNL_TRANS) return p % 3 == i ? p / 3 : -1;
+    constexpr int sel[6][3] = {{0, -1, -1}, {-1, 1, -1}, {-1, -1, 2}, {1, 0, -1}, {-1, 2, 1}, {2, -1, 0}};
+    return sel[mode == XNL_FIVE && p >= 2 ? p + 1 : p][i];
+}
+
+// Keeps loads and stores on their side of it (no wait): without it the loads of
+// all the later products move up to the first one and spill.
+__device__ __forceinline__ void pin_memory_order()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// A value formed at this point: the sums and factors below would otherwise be
+// moved to their uses (inside a later branch) and everything that they are
+// formed from kept in registers until then (1.3 KB a lane spilled).
+__device__ __forceinline__ void settle(double &x) { asm volatile("" : "+v"(x)); }
+template <typename T>
+__device__ __forceinline__ void settle(cpx<T> &z) { asm volatile("" : "+v"(z.x), "+v"(z.y)); }
+
+// An index hidden from loop-invariant code motion: the twiddles, wavenumbers
+// and LDS addresses formed from it are formed again at each use instead of
+// staying in registers over the whole kernel (the twiddles alone are 56).
+__device__ __forceinline__ int hidden(int j)
+{
+    asm volatile("" : "+v"(j));
+    return j;
+}
+
+// This thread's 8 points of a column (ColX order): rows j + TPL s.  p is the
+// same for the whole block (its first row and column), off this thread's byte
+// offset from it (under 4 GB: an eighth of a field), so that an address is a
+// scalar base and one 32-bit register however many rows and fields there are.
+template <bool NT, typename T>
+__device__ __forceinline__ void col_load(cpx<T> *v, const cpx<T> *p, size_t step, uint32_t off)
+{
+#pragma unroll
+    for (int s = 0; s < 8; s++) v[s] = gload<NT>((const cpx<T> *)((const char *)(p + s * step) + off));
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void col_store(const cpx<T> *v, cpx<T> *p, size_t step, uint32_t off)
+{
+#pragma unroll
+    for (int s = 0; s < 8; s++) gstore<NT>((cpx<T> *)((char *)(p + s * step) + off), v[s]);
+}
+
+// Bound by HBM and by the one block of two waves a SIMD that its registers
+// leave: the next tile is always in flight.  Columns go from memory to
+// registers in the transform's own order (ColX) and back; LDS holds the
+// exchanges, the twiddles and the viscous factors.  Every value is settled
+// where it is formed, and each stage has its own code after a common forward
+// part: with the four stages, the hyperviscosity loops and the random phases
+// inlined per point the kernel was 300 KB of instructions, mostly fetched
+// from L2.  512^3, per launch: FP64 5170 -> 3770 us (4.7 TB/s), FP32 4550 ->
+// 3150 us; 64^3 FP64 54 -> 21 us, 240x160x96 348 -> 161 us.
+template <typename T, int L, int CB, int MODE, bool NT>
 __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
 {
     constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    // two FP64 tile buffers (separate LDS objects, so that the compiler can
-    // tell accesses to one from the direct-to-LDS loads into the other): A
-    // hosts the FFT exchanges and stages state inputs; B receives the next
-    // product while the current one is transformed, then holds the
-    // state/accumulator tile of the RK update
-    __shared__ __attribute__((aligned(16))) char rawA[CB * LP * sizeof(cpx<double>)];
-    __shared__ __attribute__((aligned(16))) char rawB[CB * LP * sizeof(cpx<double>)];
-    __shared__ int colw[CB], cols[CB];
-    // twiddles are read from LDS: kept out of registers across the product loop
-    // (1024-point lines: from global memory, L1-resident, so that two
-    // blocks fit the LDS of a CU)
-    constexpr bool TWL = L < 1024;
-    __shared__ cpx<T> twl[TWL ? L : 1];
-    cpx<double> *ldd = (cpx<double> *)rawA;
-    cpx<T> *ldt = (cpx<T> *)rawA;
-    cpx<double> *ldb = (cpx<double> *)rawB;
+    // non-temporal access of whole 128-byte lines only (the unpadded state rows
+    // share their lines with the neighbouring tiles)
+    constexpr bool NTW = NT && CB * sizeof(cpx<T>) >= 128, NTA = NT && CB * sizeof(cpx<double>) >= 128;
+    using X = ColX<T, L, CB>;
+    __shared__ cpx<T> lds[X::SIZE];
+    // twiddles are read from LDS: a load from global memory between the FFT
+    // passes would wait for the next tile's loads in flight
+    __shared__ cpx<T> tw[L];
+    __shared__ double red[16];
+    // the viscous factors exp(-nu K^2 dt/2), exp(-nu K^2 dt) of this thread's
+    // points (their registers would spill)
+    __shared__ double visc[MODE == XNL_FIVE ? 2 : 1][MODE == XNL_FIVE ? 8 * CB * TPL : 1];
     const Grid &g = a.g;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     if (tile >= x_tiles(g, CB, false)) return;
-    tile_columns<CB>(colw, cols, g, false, tile);
-    lds_barrier();
-    const int c = threadIdx.x / TPL, j = threadIdx.x % TPL;
-    const int cw = colw[c];
-    const int ly = cw >= 0 ? cw / g.nzp : 0, lz = cw >= 0 ? cw % g.nzp : 0;
+    // Tiles of 128-byte rows divide nzp and lie within one ky row, the same for
+    // the whole block; the wider ones of short lines do not, and the last one
+    // may run past the last column (those threads move the last column and
+    // store nothing).
+    constexpr bool WIDE = CB * sizeof(cpx<T>) > 128;
+    const int c = threadIdx.x % CB, j = threadIdx.x / CB;
+    const int ncol = g.ny * g.nzp;
+    const int cw0 = tile * CB;
+    const int cwt = WIDE ? min(cw0 + c, ncol - 1) : cw0;
+    const bool inside = !WIDE || cw0 + c < ncol;
+    const int ly = cwt / g.nzp, lz0 = WIDE ? 0 : cwt % g.nzp;
+    const int lz = WIDE ? cwt % g.nzp : lz0 + c;
+    const bool live = inside && lz < g.nzc;   // the pad columns carry zeros
     const int ky = kwave(ly, g.ny);
     const double Ky = ky * g.kf[1], Kz = lz * g.kf[2];
-    if constexpr (TWL)
-        for (int i = threadIdx.x; i < L; i += CB * TPL) twl[i] = ((const cpx<T> *)a.tw)[i];
-    const cpx<T> *tw = TWL ? (const cpx<T> *)twl : (const cpx<T> *)a.tw;
-    const int ncw = g.ny * g.nzp, ncs = g.ny * g.nzc;
+    const size_t ncw = (size_t)ncol, ncs = (size_t)g.ny * g.nzc;
+    const size_t stepw = (size_t)TPL * ncw, steps = (size_t)TPL * ncs;
+    const size_t state0 = WIDE ? 0 : (size_t)ly * g.nzc + min(lz0, g.nzc - 1);
+    const uint32_t colt = WIDE ? cwt - cw0 : c;
+    const uint32_t offt = (uint32_t)(j * ncw + colt) * sizeof(cpx<T>), offw = (uint32_t)(j * ncw + colt) * 16;
+    // (a pad column reads the last one; a tile may hold pad columns only)
+    const uint32_t offs = (uint32_t)(j * ncs + (WIDE ? ly * g.nzc + min(lz, g.nzc - 1)
+                                                     : max(min(c, g.nzc - 1 - lz0), 0))) * 16;
     const T sc = (T)a.rk.scale;
     const T Kyt = (T)Ky, Kzt = (T)Kz;
+    constexpr bool NS = MODE == XNL_SIX || MODE == XNL_FIVE;
+    constexpr int NP = xnl_products(MODE);
+    const int stage = MODE == XNL_FIVE ? a.rk.stage : 0;
+    const bool want_rhs = NS && (stage > 0 || a.rk.write_rhs);
+
+    cpx<T> cur[8];
+    col_load<NTW>(cur, (const cpx<T> *)a.P[0] + cw0, stepw, offt);
+    for (int i = threadIdx.x; i < L; i += CB * TPL) tw[i] = ((const cpx<T> *)a.tw)[i];
+    // whether a column of this tile can hold forced modes; the alpha forcing's
+    // coefficient is summed by the block (one thread summing all the slots
+    // took 70 us of a 128^3 stage)
+    const bool band_tile = NS && a.b.kind != 0 && (WIDE || (abs(ky) <= a.b.h[1] && lz0 <= a.b.h[2]));
+    double alpha = 0.0;
+    if (band_tile && a.b.kind == 1 && want_rhs) alpha = band_alpha<CB * TPL>(g, a.b, a.slots_in, red);
+    unsigned forced = 0;   // bit s: row j + TPL s of this column is forced
+    if (band_tile && live)
+        for (int s = 0; s < 8; s++) {
+            const int kx = kwave(j + TPL * s, g.nx);
+            if (band_slot(a.b, kx, ky, lz) >= 0 && in_band(g, a.b, kx, ky, lz)) forced |= 1u << s;
+        }
+    lds_barrier();
+    const X x{lds + c};
 
     // --- forward x-FFT of the products and the divergence-form sum ---
-    // Product p adds i K_d FT[p] to N_i for the (i, d) pairs of the
-    // divergence form; sel_i = 0 (none), 1 (Kx), 2 (Ky), 3 (Kz).  Summing
-    // from zero in this order reproduces the reference's accumulation order.
-    constexpr bool GIVER = MODE != 0;
+    // Unrolled over the products: each adds to the one or two components its
+    // derivatives belong to, and the next one (at the end the state of the
+    // first component) is in flight while it is transformed.
     cpx<T> N[3][8];
 #pragma unroll
     for (int s = 0; s < 8; s++) N[0][s] = N[1][s] = N[2][s] = mk<T>(0, 0);
-    // five trace-shifted products when the nonlinear term is only used
-    // projected (its gradient part i K F[u_z^2] drops out)
-    const bool tf = !GIVER && a.rk.trace_free;
-    const int nprod = GIVER ? 9 : (tf ? 5 : 6);
-    constexpr bool DMA = tile_dma_ok<T, L, CB>();
-    const int cw0 = tile * CB;  // first padded work column of the tile
-    if constexpr (DMA) dma_tile<T, L, CB>((const cpx<T> *)a.P[GIVER ? kGiverOrder[0] : kNsOrder[0]], cw0, ncw, rawB);
-#pragma unroll 1
-    for (int pi = 0; pi < nprod; pi++) {
-        const int p = GIVER ? kGiverOrder[pi] : kNsOrder[pi];
-        int sel0, sel1, sel2;
-        if (MODE == 1) {
-            // P[3i+j] = FT[u_j w_i] contributes i K_j to N_i
-            sel0 = p / 3 == 0 ? p % 3 + 1 : 0;
-            sel1 = p / 3 == 1 ? p % 3 + 1 : 0;
-            sel2 = p / 3 == 2 ? p % 3 + 1 : 0;
-        } else if (MODE == 2) {
-            // transposed: P[3i+j] contributes i K_i to N_j (MHD: N-_j = sum_i d_i(Z+_i Z-_j))
-            sel0 = p % 3 == 0 ? p / 3 + 1 : 0;
-            sel1 = p % 3 == 1 ? p / 3 + 1 : 0;
-            sel2 = p % 3 == 2 ? p / 3 + 1 : 0;
-        } else if (tf) {
-            sel0 = kNsSel5[p][0];
-            sel1 = kNsSel5[p][1];
-            sel2 = kNsSel5[p][2];
-        } else {
-            sel0 = kNsSel[p][0];
-            sel1 = kNsSel[p][1];
-            sel2 = kNsSel[p][2];
-        }
-        // the line index, hidden from loop-invariant code motion: the LDS
-        // addresses of the FFT passes are recomputed each product (a few
-        // integer ops) rather than held in registers across the loop, where
-        // their spill reloads would wait for the in-flight prefetch
-        int jj = j;
-        asm volatile("" : "+v"(jj));
-        cpx<T> v[8];
-        if constexpr (DMA) {
-            // product p has landed in B; read it, then start the next one
-            dma_wait();
-            lds_barrier();
-#pragma unroll
-            for (int s = 0; s < 8; s++) v[s] = dma_tile_read<T, L, CB>(rawB, jj + TPL * s, c);
-            lds_barrier();
-            if (pi + 1 < nprod)
-                dma_tile<T, L, CB>((const cpx<T> *)a.P[GIVER ? kGiverOrder[pi + 1] : kNsOrder[pi + 1]], cw0, ncw,
-                                   rawB);
-            else if (a.rk.stage > 0)
-                // the state of the first component, for the RK update below
-                dma_state_tile<L, CB>((const cpx<double> *)a.V[0], cols, ncs, rawB);
-        } else {
-            stage_in<L, CB>(ldt, (const cpx<T> *)a.P[p], colw, ncw);
-            lds_barrier();
-#pragma unroll
-            for (int s = 0; s < 8; s++) v[s] = ldt[c * LP + lpad(j + TPL * s)];
-            lds_barrier();
-        }
-        fft_line<L, -1>(v, ldt + c * LP, tw, jj);
+    cpx<double> v0[8];
+    auto product = [&](auto pc, cpx<T> *v, cpx<T> *next) {
+        constexpr int PI = decltype(pc)::value;
+        pin_memory_order();
+        if constexpr (PI + 1 < NP) col_load<NTW>(next, (const cpx<T> *)a.P[xnl_index(MODE, PI + 1)] + cw0, stepw, offt);
+        else if (stage > 0) col_load<false>(v0, (const cpx<double> *)a.V[0] + state0, steps, offs);
+        pin_memory_order();
+        const int jh = hidden(j);
+        fft_exchange<L, -1>(v, x, tw, jh);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int s = 0; s < 8; s++) {
-            const T Kx = (T)(kwave(jj + TPL * s, g.nx) * g.kf[0]);
+            const T Kx = (T)(kwave(jh + TPL * s, g.nx) * g.kf[0]);
             const cpx<T> q = sc * v[s];
-            const T K0 = sel0 == 1 ? Kx : (sel0 == 2 ? Kyt : (sel0 == 3 ? Kzt : (T)0));
-            const T K1 = sel1 == 1 ? Kx : (sel1 == 2 ? Kyt : (sel1 == 3 ? Kzt : (T)0));
-            const T K2 = sel2 == 1 ? Kx : (sel2 == 2 ? Kyt : (sel2 == 3 ? Kzt : (T)0));
-            N[0][s] = N[0][s] + mul_i(K0, q);
-            N[1][s] = N[1][s] + mul_i(K1, q);
-            N[2][s] = N[2][s] + mul_i(K2, q);
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                constexpr int P = xnl_index(MODE, PI);
+                const int d = xnl_axis(MODE, P, i);
+                if (d >= 0) {
+                    N[i][s] = N[i][s] + mul_i(d == 0 ? Kx : (d == 1 ? Kyt : Kzt), q);
+                    settle(N[i][s]);
+                }
+            }
         }
-        if constexpr (!DMA) lds_barrier();
-    }
-    // the FFT exchanges in A are done before A and B are reused below (B may
-    // be receiving the first state component)
-    if constexpr (DMA) lds_barrier_async();
+    };
+    cpx<T> alt[8];
+    auto pair = [&](auto pc) {
+        constexpr int PI = decltype(pc)::value;
+        if constexpr (PI < NP) product(std::integral_constant<int, PI>{}, cur, alt);
+        if constexpr (PI + 1 < NP) product(std::integral_constant<int, PI + 1>{}, alt, cur);
+    };
+    pair(std::integral_constant<int, 0>{});
+    pair(std::integral_constant<int, 2>{});
+    pair(std::integral_constant<int, 4>{});
+    pair(std::integral_constant<int, 6>{});
+    pair(std::integral_constant<int, 8>{});
 
-    const int stage = a.rk.stage;
-    const bool want_rhs = stage > 0 || a.rk.write_rhs;
     // --- force, pressure projection, negation (Compute_force_TO_rhs), in
     // place on N: N <- -(N - F + i K p), p = i K.(N - F) / K^2 (computed in
     // FP64, stored in the transform precision) ---
-    double alpha = 0.0;
-    bool alpha_done = false;
-    if (want_rhs) {
+    auto project = [&](auto fc) {
+        constexpr bool FORCED = decltype(fc)::value;
+        const int jh = hidden(j);
 #pragma unroll
         for (int s = 0; s < 8; s++) {
-            const int lx = j + TPL * s;
+            const int lx = jh + TPL * s;
             const int kx = kwave(lx, g.nx);
             const double Kx = kx * g.kf[0];
             cpx<double> n0 = cvt<double>(N[0][s]), n1 = cvt<double>(N[1][s]), n2 = cvt<double>(N[2][s]);
-            if (a.b.kind == 1 && cw >= 0) {
-                const int sl = band_slot(a.b, kx, ky, lz);
-                if (sl >= 0) {
-                    const double K = kmag(g, kx, ky, lz);
-                    if (K > a.b.r_in && K <= a.b.r_out) {
-                        if (!alpha_done) { alpha = band_alpha(g, a.b, a.slots_in); alpha_done = true; }
-                        const cpx<double> *sv = (const cpx<double> *)a.slots_in + sl * 3;
-                        n0 = n0 - alpha * sv[0];
-                        n1 = n1 - alpha * sv[1];
-                        n2 = n2 - alpha * sv[2];
-                    }
-                }
-            } else if (a.b.kind == 2 && cw >= 0) {
-                const double K = kmag(g, kx, ky, lz);
-                if (K > a.b.r_in && K <= a.b.r_out) {
-                    cpx<double> F[3];
-                    random_force_mode(g, a.b, lx, ly, lz, kx, ky, K, F);
-                    n0 = n0 - F[0];
-                    n1 = n1 - F[1];
-                    n2 = n2 - F[2];
-                }
+            if (FORCED && (forced & (1u << s))) {
+                // the stage input's band modes, or the random force itself
+                const cpx<double> *sv =
+                    (const cpx<double> *)(a.b.kind == 1 ? a.slots_in : a.b.force) + band_slot(a.b, kx, ky, lz) * 3;
+                const double f = a.b.kind == 1 ? alpha : 1.0;
+                n0 = n0 - f * sv[0];
+                n1 = n1 - f * sv[1];
+                n2 = n2 - f * sv[2];
             }
             cpx<double> div = mul_i(Kx, n0);
             div = div + mul_i(Ky, n1);
@@ -623,178 +704,129 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
             N[0][s] = cvt<T>(mk<double>(-n0.x, -n0.y));
             N[1][s] = cvt<T>(mk<double>(-n1.x, -n1.y));
             N[2][s] = cvt<T>(mk<double>(-n2.x, -n2.y));
+#pragma unroll
+            for (int i = 0; i < 3; i++) settle(N[i][s]);
+            if (s % 2) __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    if (want_rhs) {
+        if (band_tile) project(std::true_type{});
+        else project(std::false_type{});
     }
-#define TG_TAKE(comp, nc)                                                           \
-    do {                                                                            \
-        if ((comp) == 0) {                                                          \
-            _Pragma("unroll") for (int s_ = 0; s_ < 8; s_++) nc[s_] = N[0][s_];    \
-        } else if ((comp) == 1) {                                                   \
-            _Pragma("unroll") for (int s_ = 0; s_ < 8; s_++) nc[s_] = N[1][s_];    \
-        } else {                                                                    \
-            _Pragma("unroll") for (int s_ = 0; s_ < 8; s_++) nc[s_] = N[2][s_];    \
-        }                                                                           \
-    } while (0)
 
     if (stage == 0) {
         // Compute_nlin (and optionally Compute_rhs) output, FP64 boundary layout
-#pragma unroll 1
-        for (int comp = 0; comp < 3; comp++) {
-            cpx<T> nc[8];
-            TG_TAKE(comp, nc);
+        if (live) {
 #pragma unroll
-            for (int s = 0; s < 8; s++) ldd[c * LP + lpad(j + TPL * s)] = cvt<double>(nc[s]);
-            lds_barrier();
-            stage_out<L, CB>(ldd, (cpx<double> *)a.out[comp], cols, ncs);
-            lds_barrier();
+            for (int comp = 0; comp < 3; comp++) {
+                cpx<double> o[8];
+#pragma unroll
+                for (int s = 0; s < 8; s++) o[s] = cvt<double>(N[comp][s]);
+                col_store<false>(o, (cpx<double> *)a.out[comp] + state0, steps, offs);
+            }
         }
         return;
     }
 
     // --- Lawson RK4 stage algebra (RK.cc:91-170, Tadvance_functions.cc:298-324,566-570) ---
     // V: FP64 state, boundary layout; acc: FP64, padded work layout (the RK
-    // state accumulation stays FP64 whatever the transform precision).
+    // state accumulation stays FP64 whatever the transform precision).  The
+    // next component's state is loaded before this one's results are stored
+    // (loads and stores retire in order, so that the wait for it does not
+    // wait for those stores).
     const double dt = a.rk.dt;
     const double c_half = 0.5 * dt, c_one = 1.0 * dt;
     const double c_sixth = (1.0 / 6) * dt, c_third = (1.0 / 3) * dt;
-    if constexpr (DMA) {
-        // Component K: its state V[K] sits in tile X (direct-to-LDS load,
-        // column-major chunks), the accumulator is staged into tile Y, which
-        // then takes the updated accumulator (or state); the next stage input
-        // is x-inverted with X as the exchange buffer, and V[K+1] is loaded
-        // into Y while that input is stored.  The components are unrolled so
-        // that X and Y are known LDS objects (the waits for the direct-to-LDS
-        // loads then cover only the tile they write).
-        auto rk_comp = [&](auto kc, char *X, char *Y) {
-            constexpr int K = decltype(kc)::value;
-            cpx<double> *Yd = (cpx<double> *)Y;
-            cpx<T> *Xt = (cpx<T> *)X;
-            if (stage >= 2) stage_in<L, CB>(Yd, (const cpx<double> *)a.acc[K], colw, ncw);
-            dma_wait();
-            lds_barrier();
-            cpx<T> v[8];
-#pragma unroll
+    int zx0, zx1;   // rows of this column that the dealias mask zeroes (a pad column: all)
+    dealias_rows(g, ly, lz, zx0, zx1);
+    if (!live) { zx0 = 0; zx1 = L - 1; }
+    // One instance per stage: only the stage that runs occupies the
+    // instruction cache, and the viscous factors are formed once for the three
+    // components.
+    auto rk_stage = [&](auto stc) {
+        constexpr int ST = decltype(stc)::value;
+        {
+            const int jh = hidden(j);
+#pragma unroll 2
             for (int s = 0; s < 8; s++) {
-                const int lx = j + TPL * s;
-                const int li = c * LP + lpad(lx);
-                const double Kx = kwave(lx, g.nx) * g.kf[0];
+                const double Kx = kwave(jh + TPL * s, g.nx) * g.kf[0];
                 const double kxs = Kx * Kx;
                 const double ks = (kxs + Ky * Ky) + Kz * Kz;
-                const double Eh = visc_exp(a.rk.fh, a.rk.fhh, a.rk.hq, ks);
+                const double kp = hyper_power(a.rk.hq, ks);
+                if (ST < 4) visc[0][s * CB * TPL + threadIdx.x] = exp((a.rk.fh + a.rk.fhh * kp) * ks);
+                if (ST == 1 || ST == 4) visc[1][s * CB * TPL + threadIdx.x] = exp((a.rk.f1 + a.rk.f1h * kp) * ks);
+            }
+        }
+        // (each thread reads its own entries only)
+        auto Eh = [&](int s) { return visc[0][s * CB * TPL + threadIdx.x]; };
+        auto E1 = [&](int s) { return visc[1][s * CB * TPL + threadIdx.x]; };
+        cpx<double> ac[8];
+        if (ST >= 2) col_load<NTA>(ac, (const cpx<double> *)a.acc[0] + cw0, stepw, offw);
+        bool bad = false;
+        // SLOTS: the undealiased stage input of forced modes goes to the slots
+        auto algebra = [&](auto kc, auto slc, cpx<T> *v) {
+            constexpr int K = decltype(kc)::value;
+            constexpr bool SLOTS = decltype(slc)::value;
+            const int jh = hidden(j);
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                const int lx = jh + TPL * s;
                 const cpx<double> r = cvt<double>(N[K][s]);
-                const cpx<double> v0 = dma_tile_read<double, L, CB>(X, lx, c);
-                cpx<double> vn, ac;
-                if (stage == 1) {
-                    cpx<double> d0 = v0;
-                    if (dealias_zero(g, lx, ly, lz)) d0 = mk<double>(0, 0);
-                    const double E1 = visc_exp(a.rk.f1, a.rk.f1h, a.rk.hq, ks);
-                    ac = c_sixth * (E1 * r);
-                    vn = Eh * (d0 + c_half * r);
-                } else if (stage == 2) {
-                    ac = Yd[li] + c_third * (Eh * r);
-                    vn = Eh * v0 + c_half * r;
-                } else if (stage == 3) {
-                    ac = Yd[li] + c_third * (Eh * r);
-                    vn = Eh * (Eh * v0 + c_one * r);
+                cpx<double> vn;
+                if constexpr (ST == 1) {
+                    cpx<double> d0 = v0[s];
+                    if (lx >= zx0 && lx <= zx1) d0 = mk<double>(0, 0);
+                    ac[s] = c_sixth * (E1(s) * r);
+                    vn = Eh(s) * (d0 + c_half * r);
+                } else if constexpr (ST == 2) {
+                    ac[s] = ac[s] + c_third * (Eh(s) * r);
+                    vn = Eh(s) * v0[s] + c_half * r;
+                } else if constexpr (ST == 3) {
+                    ac[s] = ac[s] + c_third * (Eh(s) * r);
+                    vn = Eh(s) * (Eh(s) * v0[s] + c_one * r);
                 } else {
-                    ac = Yd[li] + c_sixth * r;
-                    const double E1 = visc_exp(a.rk.f1, a.rk.f1h, a.rk.hq, ks);
-                    vn = E1 * v0 + ac;
+                    ac[s] = ac[s] + c_sixth * r;
+                    vn = E1(s) * v0[s] + ac[s];
+                    ac[s] = vn;   // the new state
+                    bad = bad || !(isfinite(vn.x) && isfinite(vn.y));
                 }
-                Yd[li] = mk<double>(stage == 4 ? vn.x : ac.x, stage == 4 ? vn.y : ac.y);
-                if (stage == 4 && !(isfinite(vn.x) && isfinite(vn.y)) && a.rk.nonfinite) *a.rk.nonfinite = 1;
-                if (a.b.kind == 1 && cw >= 0) {
-                    const int kx = kwave(lx, g.nx);
-                    const int sl = band_slot(a.b, kx, ky, lz);
-                    if (sl >= 0) {
-                        const double Kb = kmag(g, kx, ky, lz);
-                        if (Kb > a.b.r_in && Kb <= a.b.r_out) ((cpx<double> *)a.slots_out)[sl * 3 + K] = vn;
-                    }
-                }
-                if (dealias_zero(g, lx, ly, lz)) vn = mk<double>(0, 0);
+                if (SLOTS && (forced & (1u << s)))
+                    ((cpx<double> *)a.slots_out)[band_slot(a.b, kwave(lx, g.nx), ky, lz) * 3 + K] = vn;
+                if (lx >= zx0 && lx <= zx1) vn = mk<double>(0, 0);
                 v[s] = cvt<T>(vn);
             }
-            lds_barrier();
-            if (stage == 4) stage_out<L, CB>(Yd, (cpx<double> *)a.V[K], cols, ncs);
-            else stage_out<L, CB>(Yd, (cpx<double> *)a.acc[K], colw, ncw);
-            fft_line<L, +1>(v, Xt + c * LP, tw, j);
-#pragma unroll
-            for (int s = 0; s < 8; s++) Xt[c * LP + lpad(j + TPL * s)] = v[s];
-            lds_barrier();
-            if constexpr (K < 2) dma_state_tile<L, CB>((const cpx<double> *)a.V[K + 1], cols, ncs, Y);
-            stage_out<L, CB>(Xt, (cpx<T> *)a.U[K], colw, ncw);
-            lds_barrier_async();
         };
-        rk_comp(std::integral_constant<int, 0>{}, rawB, rawA);
-        rk_comp(std::integral_constant<int, 1>{}, rawA, rawB);
-        rk_comp(std::integral_constant<int, 2>{}, rawB, rawA);
-        return;
-    }
-#pragma unroll 1
-    for (int comp = 0; comp < 3; comp++) {
-        cpx<T> nc[8];
-        TG_TAKE(comp, nc);
-        stage_in<L, CB>(ldd, (const cpx<double> *)a.V[comp], cols, ncs);
-        if (stage >= 2) stage_in<L, CB>(ldb, (const cpx<double> *)a.acc[comp], colw, ncw);
-        lds_barrier();
-        cpx<T> v[8];
-#pragma unroll
-        for (int s = 0; s < 8; s++) {
-            const int lx = j + TPL * s;
-            const int li = c * LP + lpad(lx);
-            const double Kx = kwave(lx, g.nx) * g.kf[0];
-            const double kxs = Kx * Kx;
-            const double ks = (kxs + Ky * Ky) + Kz * Kz;
-            const double Eh = visc_exp(a.rk.fh, a.rk.fhh, a.rk.hq, ks);
-            const cpx<double> r = cvt<double>(nc[s]);
-            const cpx<double> v0 = ldd[li];
-            cpx<double> vn, ac;
-            if (stage == 1) {
-                cpx<double> d0 = v0;
-                if (dealias_zero(g, lx, ly, lz)) d0 = mk<double>(0, 0);
-                const double E1 = visc_exp(a.rk.f1, a.rk.f1h, a.rk.hq, ks);
-                ac = c_sixth * (E1 * r);
-                vn = Eh * (d0 + c_half * r);
-            } else if (stage == 2) {
-                ac = ldb[li] + c_third * (Eh * r);
-                vn = Eh * v0 + c_half * r;
-            } else if (stage == 3) {
-                ac = ldb[li] + c_third * (Eh * r);
-                vn = Eh * (Eh * v0 + c_one * r);
+        auto rk_comp = [&](auto kc) {
+            constexpr int K = decltype(kc)::value;
+            cpx<T> v[8];
+            if (band_tile && a.b.kind == 1) algebra(kc, std::true_type{}, v);
+            else algebra(kc, std::false_type{}, v);
+            pin_memory_order();
+            if constexpr (K < 2) col_load<false>(v0, (const cpx<double> *)a.V[K + 1] + state0, steps, offs);
+            if (ST == 4) {
+                if (live) col_store<false>(ac, (cpx<double> *)a.V[K] + state0, steps, offs);
             } else {
-                ac = ldb[li] + c_sixth * r;
-                const double E1 = visc_exp(a.rk.f1, a.rk.f1h, a.rk.hq, ks);
-                vn = E1 * v0 + ac;
+                if (inside) col_store<NTA>(ac, (cpx<double> *)a.acc[K] + cw0, stepw, offw);
             }
-            // accumulator (stages 1-3) or the new state (stage 4) back to B
-            // (component-wise select: selecting the objects keeps them in memory)
-            ldb[li] = mk<double>(stage == 4 ? vn.x : ac.x, stage == 4 ? vn.y : ac.y);
-            if (stage == 4 && !(isfinite(vn.x) && isfinite(vn.y)) && a.rk.nonfinite) *a.rk.nonfinite = 1;
-            // next stage input: band slots, dealias
-            if (a.b.kind == 1 && cw >= 0) {
-                const int kx = kwave(lx, g.nx);
-                const int sl = band_slot(a.b, kx, ky, lz);
-                if (sl >= 0) {
-                    const double K = kmag(g, kx, ky, lz);
-                    if (K > a.b.r_in && K <= a.b.r_out) ((cpx<double> *)a.slots_out)[sl * 3 + comp] = vn;
-                }
-            }
-            if (dealias_zero(g, lx, ly, lz)) vn = mk<double>(0, 0);
-            v[s] = cvt<T>(vn);
-        }
-        lds_barrier();
-        if (stage == 4) stage_out<L, CB>(ldb, (cpx<double> *)a.V[comp], cols, ncs);
-        else stage_out<L, CB>(ldb, (cpx<double> *)a.acc[comp], colw, ncw);
-        // inverse x-FFT of the next stage input (exchanges in buffer A)
-        fft_line<L, +1>(v, ldt + c * LP, tw, j);
-#pragma unroll
-        for (int s = 0; s < 8; s++) ldt[c * LP + lpad(j + TPL * s)] = v[s];
-        lds_barrier();
-        stage_out<L, CB>(ldt, (cpx<T> *)a.U[comp], colw, ncw);
-        lds_barrier();
+            if (ST >= 2 && K < 2)
+                col_load<NTA>(ac, (const cpx<double> *)a.acc[K < 2 ? K + 1 : 2] + cw0, stepw, offw);
+            pin_memory_order();
+            fft_exchange<L, +1>(v, x, tw, hidden(j));
+            pin_memory_order();
+            if (inside) col_store<NTW>(v, (cpx<T> *)a.U[K] + cw0, stepw, offt);
+        };
+        rk_comp(std::integral_constant<int, 0>{});
+        rk_comp(std::integral_constant<int, 1>{});
+        rk_comp(std::integral_constant<int, 2>{});
+        if (ST == 4 && bad && live && a.rk.nonfinite) *a.rk.nonfinite = 1;
+    };
+    if constexpr (MODE == XNL_FIVE) {
+        if (stage == 1) rk_stage(std::integral_constant<int, 1>{});
+        else if (stage == 2) rk_stage(std::integral_constant<int, 2>{});
+        else if (stage == 3) rk_stage(std::integral_constant<int, 3>{});
+        else rk_stage(std::integral_constant<int, 4>{});
     }
 }
-#undef TG_TAKE
 
 #if TG_LEN_UNIT == 0
 // ---------------------------------------------------------------------------
@@ -856,13 +888,13 @@ hipError_t colfft_len(const ColArgs &a, int dir, int nfields, hipStream_t st)
     // block would pass 1024 threads: with rows of 64 bytes the in-place pass of
     // five 512^3 FP64 fields takes 2461 us against 2017, and at 1024 points,
     // where the wide tile leaves one block per CU, 2485 against 2152.
-    constexpr int CB = std::max(1, std::min(128 / (int)sizeof(cpx<T>), 1024 / (LL / 8)));
+    constexpr int CB = colx_block<T>(LL, 1024);
     // Non-temporal loads and stores where the pass streams more than the 256
     // MiB memory-side cache holds (five 512^3 FP64 fields 2017 -> 1892 us in a
     // loop of the pass alone, 445 -> 381 us per field within the step); 128^3
     // FP32 lost 5% in the z pass that follows.  Not where a CU holds one block
     // (1024 points FP64 2152 against 2226 us) or the rows are half lines.
-    constexpr bool STREAM = CB * sizeof(cpx<T>) == 128 && 2 * ColX<T, LL, CB, 1>::SIZE * sizeof(cpx<T>) <= 160 * 1024;
+    constexpr bool STREAM = CB * sizeof(cpx<T>) >= 128 && 2 * ColX<T, LL, CB>::SIZE * sizeof(cpx<T>) <= 160 * 1024;
     dim3 grid(x_grid(a.nouter * ((a.ncol + CB - 1) / CB)), nfields);
     const dim3 block(CB * (LL / 8));
     const bool nt = STREAM && stream_bytes((size_t)nfields * a.nouter * a.outer_stride * sizeof(cpx<T>));
@@ -927,35 +959,36 @@ hipError_t z_products_len(const ZArgs &a, int giver, hipStream_t st)
     return hipGetLastError();
 }
 
-#define TG_XNL(CBV, M) \
-    hipLaunchKernelGGL((k_x_nlin<T, LL, CBV, M>), dim3(x_grid(x_tiles(a.g, CBV, false))), dim3(CBV * (LL / 8)), 0, st, a)
-
-template <typename T, int LL>
-hipError_t x_nlin_len(const XnlArgs &a, int mode, int x_tile_columns, hipStream_t st)
+template <typename T, int LL, int MODE>
+hipError_t x_nlin_launch(const XnlArgs &a, hipStream_t st)
 {
-    // two FP64 tile buffers per block: the LDS-budget width (two blocks
-    // per CU), or twice that width (one block per CU)
-    constexpr int CB = col_block<T>(LL, 2 * sizeof(cpx<double>));
-    constexpr int CBW = 2 * CB * (LL / 8) <= 1024 ? 2 * CB : CB;
-    const bool wide = x_tile_columns == CBW && CBW != CB;
-    if (wide) {
-        if (mode == 1) TG_XNL(CBW, 1);
-        else if (mode == 2) TG_XNL(CBW, 2);
-        else TG_XNL(CBW, 0);
-    } else {
-        if (mode == 1) TG_XNL(CB, 1);
-        else if (mode == 2) TG_XNL(CB, 2);
-        else TG_XNL(CB, 0);
-    }
+    // One block of 512 threads fills a CU's registers (the three sums, a
+    // product and the next one): 128-byte rows up to 512-point FP64 and
+    // 256-point FP32 lines.  64-byte rows of 512-point FP64 lines in two blocks
+    // a CU took 5041 us a launch against 4828 (before the instruction cache
+    // was relieved).
+    constexpr int CB = colx_block<T>(LL, 512);
+    const bool nt = stream_bytes((size_t)8 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
+    const dim3 grid(x_grid(x_tiles(a.g, CB, false))), block(CB * (LL / 8));
+    if (nt) hipLaunchKernelGGL((k_x_nlin<T, LL, CB, MODE, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_x_nlin<T, LL, CB, MODE, false>), grid, block, 0, st, a);
     return hipGetLastError();
 }
-#undef TG_XNL
+
+template <typename T, int LL>
+hipError_t x_nlin_len(const XnlArgs &a, int mode, hipStream_t st)
+{
+    if (mode == XNL_GIVER) return x_nlin_launch<T, LL, XNL_GIVER>(a, st);
+    if (mode == XNL_TRANS) return x_nlin_launch<T, LL, XNL_TRANS>(a, st);
+    if (mode == XNL_FIVE) return x_nlin_launch<T, LL, XNL_FIVE>(a, st);
+    return x_nlin_launch<T, LL, XNL_SIX>(a, st);
+}
 
 #define TG_KERNELS_L(N, T, P)                                                                  \
     P template hipError_t colfft_len<T, N>(const ColArgs &, int, int, hipStream_t);           \
     P template hipError_t xinv_state_len<T, N>(const XinvArgs &, hipStream_t);                \
     P template hipError_t xfwd_spec_len<T, N>(const XfwdArgs &, hipStream_t);                 \
-    P template hipError_t x_nlin_len<T, N>(const XnlArgs &, int, int, hipStream_t);
+    P template hipError_t x_nlin_len<T, N>(const XnlArgs &, int, hipStream_t);
 #define TG_KERNELS_M(N, T, P)                                                                  \
     P template hipError_t z_c2r_len<T, N>(const ZArgs &, hipStream_t);                        \
     P template hipError_t z_r2c_len<T, N>(const ZArgs &, hipStream_t);                        \
@@ -1079,7 +1112,7 @@ hipError_t launch_z_products(const Grid &g, void *const *U, void *const *P, int 
 template <typename T>
 hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void *const *P, double *const *V,
                          double *const *acc, void *const *U, const double *slots_in, double *slots_out,
-                         double *const *out, const void *twx, hipStream_t st, int x_tile_columns)
+                         double *const *out, const void *twx, hipStream_t st)
 {
     XnlArgs a{};
     // rk.stage -1: giver form, -2: transposed giver form (nonlinear term only)
@@ -1101,7 +1134,9 @@ hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void 
         a.rk.stage = 0;
         a.rk.write_rhs = 0;
     }
-    TG_DISPATCH_L(T, g.nx, return (x_nlin_len<T, LL>)(a, giver, x_tile_columns, st));
+    const int mode = giver == 1 ? XNL_GIVER : (giver == 2 ? XNL_TRANS : (rk.trace_free ? XNL_FIVE : XNL_SIX));
+    if (mode != XNL_FIVE && a.rk.stage > 0) return hipErrorInvalidValue;
+    TG_DISPATCH_L(T, g.nx, return (x_nlin_len<T, LL>)(a, mode, st));
     return hipErrorInvalidValue;
 }
 
@@ -1153,7 +1188,7 @@ hipError_t launch_dealias(const Grid &g, double *const *V, int ncomp, hipStream_
                                              const void *, hipStream_t, void *const *);                        \
     template hipError_t launch_x_nlin<T>(const Grid &, const Band &, const RkParams &, void *const *,           \
                                          double *const *, double *const *, void *const *, const double *,      \
-                                         double *, double *const *, const void *, hipStream_t, int);
+                                         double *, double *const *, const void *, hipStream_t);
 
 TG_INST(double)
 TG_INST(float)

@@ -49,17 +49,57 @@ __device__ __forceinline__ bool dealias_zero(const Grid &g, int lx, int ly, int 
     return false;
 }
 
+// The rows lx of column (ly, lz) that dealias_zero zeroes: x0 <= lx <= x1
+// (x0 > x1: none).  |kx| > n/3 is n/3 < lx < n - n/3.
+__device__ __forceinline__ void dealias_rows(const Grid &g, int ly, int lz, int &x0, int &x1)
+{
+    x0 = 1;
+    x1 = 0;
+    if (g.dealias == 1) {
+        const int ylo = g.ny / 3 + 1, yhi = max(2 * g.ny / 3 - 1, ylo);
+        const int zlo = g.nz / 3 + 1, zhi = max(g.nz / 2, zlo);
+        if (ly >= ylo && ly <= yhi && lz >= zlo && lz <= zhi) {
+            x0 = g.basis == 1 ? 2 * g.nx / 3 + 1 : g.nx / 3 + 1;
+            x1 = g.basis == 1 ? g.nx - 1 : 2 * g.nx / 3 - 1;
+        }
+    } else if (g.dealias == 2) {
+        const bool all = abs(kwave(ly, g.ny)) > g.ny / 3 || lz > g.nz / 3;
+        x0 = all ? 0 : (g.basis == 1 ? 2 * g.nx / 3 + 1 : g.nx / 3 + 1);
+        x1 = all || g.basis == 1 ? g.nx - 1 : g.nx - g.nx / 3 - 1;
+    }
+}
+
+// K^(q-2) = (K^2)^((q-2)/2) of the hyperviscosity, integer division (q = 4:
+// K^2), by repeated multiplication; q = 0 (none): 1.
+__device__ __forceinline__ double hyper_power(int q, double ks)
+{
+    const int n = q == 0 ? 0 : (q == 4 ? 1 : (q - 2) / 2);
+    double kp = 1.0;
+#pragma unroll 1
+    for (int i = 0; i < n; i++) kp *= ks;
+    return kp;
+}
+
 // Viscous factor exp(exponent) of Array_exp_ksqr: exponent f K^2, or with
 // hyperviscosity (f + fh K^(q-2)) K^2 (universal_basic.cc:265-291), K^(q-2) =
 // (K^2)^((q-2)/2) with integer division (q = 4: K^2), by repeated
 // multiplication; q = 0: none.  ks = K^2.
 __device__ __forceinline__ double visc_exp(double f, double fh, int q, double ks)
 {
-    if (q == 0) return exp(f * ks);
-    const int n = q == 4 ? 1 : (q - 2) / 2;
-    double kp = 1.0;
-    for (int i = 0; i < n; i++) kp *= ks;
-    return exp((f + fh * kp) * ks);
+    return exp((f + fh * hyper_power(q, ks)) * ks);
+}
+
+// Columns of a ColX tile of L-point lines, a power of two: rows of 128 bytes (8
+// FP64 or 16 FP32 columns), more where a block would have less than a
+// wavefront, fewer where it would pass `threads`.
+template <typename T>
+__host__ __device__ constexpr int colx_block(int L, int threads)
+{
+    const int tpl = L / 8;
+    int cb = 128 / (int)sizeof(cpx<T>);
+    while (cb * tpl < 64) cb *= 2;
+    while (cb > 1 && cb * tpl > threads) cb /= 2;
+    return cb;
 }
 
 template <typename T>
@@ -263,16 +303,23 @@ __device__ __forceinline__ cpx<T> dma_tile_read(const char *lds, int r, int c)
 // insertion see that the loads have retired.
 __device__ __forceinline__ void dma_wait() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// the slot of a mode, -1 outside the box
 __device__ __forceinline__ int band_slot(const Band &b, int kx, int ky, int kz)
 {
-    if (kx < -b.kb || kx > b.kb || ky < -b.kb || ky > b.kb || kz > b.kb) return -1;
-    return ((kx + b.kb) * (2 * b.kb + 1) + (ky + b.kb)) * (b.kb + 1) + kz;
+    if (abs(kx) > b.h[0] || abs(ky) > b.h[1] || kz > b.h[2]) return -1;
+    return ((kx + b.h[0]) * (2 * b.h[1] + 1) + (ky + b.h[1])) * (b.h[2] + 1) + kz;
 }
 
 __device__ __forceinline__ double kmag(const Grid &g, int kx, int ky, int kz)
 {
     const double a = kx * g.kf[0], b = ky * g.kf[1], c = kz * g.kf[2];
     return sqrt(a * a + b * b + c * c);
+}
+
+__device__ __forceinline__ bool in_band(const Grid &g, const Band &b, int kx, int ky, int kz)
+{
+    const double K = kmag(g, kx, ky, kz);
+    return K > b.r_in && K <= b.r_out;
 }
 
 // ---------------------------------------------------------------------------
