@@ -134,19 +134,19 @@ __device__ __forceinline__ void tape_mac(cpx<T> *q, const cpx<T> *v, const cpx<T
 // and, as its share of sigma_zz, subtracts u_z sigma_jj from q_z; an
 // off-diagonal line sigma_jm adds u_j sigma_jm to q_m and u_m sigma_jm to
 // q_j.  Five c2r and three r2c per line.
-template <typename T, int M>
+template <typename T, int M, bool NT>
 __global__ void __launch_bounds__(256) k_z_adj(ZArgs a)
 {
     constexpr int TPL = M / 8;
     constexpr int LPB = z_lines_per_block<M>();
     constexpr int LP = lpad_len(M);
-    __shared__ cpx<T> lds[LPB * LP];
+    __shared__ cpx<T> lds[LPB * LP], ldw[2 * M];
+    const ZTwiddles<T, M> tw(ldw, a.twm, a.twn);
     const int li = threadIdx.x / TPL, j = threadIdx.x % TPL;
     const size_t line = (size_t)blockIdx.x * LPB + li;
     const size_t nlines = (size_t)a.g.nx * a.g.ny;
     const bool valid = line < nlines;
     const size_t lsafe = valid ? line : nlines - 1;
-    const cpx<T> *twm = (const cpx<T> *)a.twm, *twn = (const cpx<T> *)a.twn;
     cpx<T> *L = lds + li * LP;
     const size_t off = lsafe * a.g.nzp;
     cpx<T> q[3][8];
@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(256) k_z_adj(ZArgs a)
         const cpx<T> *X = (const cpx<T> *)(t == 0 ? a.in[0] : t == 1 ? a.in[1] : t == 2 ? a.in[2] :
                                             t == 3 ? a.in[3] : a.in[4]);
         cpx<T> v[8];
-        zline_c2r<T, M>(v, X + off, L, twm, twn, j);
+        zline_c2r<T, M, NT>(v, X + off, L, tw, j);
         line_sync<M / 8>();
         const cpx<T> *uj = (const cpx<T> *)(jt == 0 ? a.tape[0] : jt == 1 ? a.tape[1] : a.tape[2]) + lsafe * M;
         const cpx<T> *um = (const cpx<T> *)(mt == 0 ? a.tape[0] : mt == 1 ? a.tape[1] : a.tape[2]) + lsafe * M;
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(256) k_z_adj(ZArgs a)
 #pragma unroll
     for (int m = 0; m < 3; m++) {
         cpx<T> *Q = (cpx<T> *)(m == 0 ? a.out[0] : m == 1 ? a.out[1] : a.out[2]);
-        zline_r2c_post<T, M>(q[m], Q + off, L, twm, twn, j, valid);
+        zline_r2c_post<T, M, NT>(q[m], Q + off, L, tw, j, valid, a.g.nzp - M);
     }
 }
 
@@ -300,7 +300,10 @@ hipError_t z_adj_len(const ZArgs &a, hipStream_t st)
     constexpr int LPB = z_lines_per_block<MM>();
     const size_t nlines = (size_t)a.g.nx * a.g.ny;
     dim3 grid((unsigned)((nlines + LPB - 1) / LPB));
-    hipLaunchKernelGGL((k_z_adj<T, MM>), grid, dim3(LPB * (MM / 8)), 0, st, a);
+    const dim3 block(LPB * (MM / 8));
+    const bool nt = stream_bytes((size_t)8 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
+    if (nt) hipLaunchKernelGGL((k_z_adj<T, MM, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_z_adj<T, MM, false>), grid, block, 0, st, a);
     return hipGetLastError();
 }
 

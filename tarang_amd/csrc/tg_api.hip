@@ -57,7 +57,8 @@ struct tg_plan {
     size_t nc = 0;        // complex modes per field
     size_t ncw = 0;       // complex entries of one padded work field
     int64_t dev_bytes = 0;
-    // twiddle tables in the transform precision: x (Nx), y (Ny), m (Nz/2), n (Nz, k = 0..Nz/2)
+    // twiddle tables in the transform precision: x (Nx), y (Ny), m (Nz/2) in
+    // pass order (twiddle_order), n (Nz, k = 0..Nz/2)
     void *twx = nullptr, *twy = nullptr, *twm = nullptr, *twn = nullptr;
     void *U[6] = {};      // x/y-transformed velocity (0..2) and giver (3..5) lines
     void *P[9] = {};      // product spectra
@@ -185,12 +186,18 @@ int prof_collect(tg_plan *p)
     return TG_OK;
 }
 
+// count factors exp(-2 pi i k / L), in pass order (twiddle_order; count = L) for
+// the line transforms, otherwise k = 0..count-1
 template <typename T>
-int upload_twiddles(tg_plan *p, void **dst, int L, int count)
+int upload_twiddles(tg_plan *p, void **dst, int L, int count, bool pass_order)
 {
     std::vector<T> h(2 * (size_t)count);
+    std::vector<int> order(count);
+    if (pass_order) twiddle_order(L, order.data());
+    else
+        for (int k = 0; k < count; k++) order[k] = k;
     for (int k = 0; k < count; k++) {
-        const double a = -2.0 * M_PI * (double)k / (double)L;
+        const double a = -2.0 * M_PI * (double)order[k] / (double)L;
         h[2 * k] = (T)std::cos(a);
         h[2 * k + 1] = (T)std::sin(a);
     }
@@ -1172,17 +1179,17 @@ int tg_plan_create(const tg_config *cfg, tg_plan **plan)
     int rc = set_device(p);
     if (rc) { free_plan(p); return rc; }
     if (p->prec == TG_PREC_FP32) {
-        rc = upload_twiddles<float>(p, &p->twx, cfg->nx, cfg->nx);
-        if (!rc) rc = upload_twiddles<float>(p, &p->twy, cfg->ny, cfg->ny);
-        if (!rc) rc = upload_twiddles<float>(p, &p->twm, cfg->nz / 2, cfg->nz / 2);
-        if (!rc) rc = upload_twiddles<float>(p, &p->twn, cfg->nz, cfg->nz / 2 + 1);
-        if (!rc && p->g.basis == 1) rc = upload_twiddles<float>(p, &p->twq, 4 * cfg->nx, cfg->nx);
+        rc = upload_twiddles<float>(p, &p->twx, cfg->nx, cfg->nx, true);
+        if (!rc) rc = upload_twiddles<float>(p, &p->twy, cfg->ny, cfg->ny, true);
+        if (!rc) rc = upload_twiddles<float>(p, &p->twm, cfg->nz / 2, cfg->nz / 2, true);
+        if (!rc) rc = upload_twiddles<float>(p, &p->twn, cfg->nz, cfg->nz / 2 + 1, false);
+        if (!rc && p->g.basis == 1) rc = upload_twiddles<float>(p, &p->twq, 4 * cfg->nx, cfg->nx, false);
     } else {
-        rc = upload_twiddles<double>(p, &p->twx, cfg->nx, cfg->nx);
-        if (!rc) rc = upload_twiddles<double>(p, &p->twy, cfg->ny, cfg->ny);
-        if (!rc) rc = upload_twiddles<double>(p, &p->twm, cfg->nz / 2, cfg->nz / 2);
-        if (!rc) rc = upload_twiddles<double>(p, &p->twn, cfg->nz, cfg->nz / 2 + 1);
-        if (!rc && p->g.basis == 1) rc = upload_twiddles<double>(p, &p->twq, 4 * cfg->nx, cfg->nx);
+        rc = upload_twiddles<double>(p, &p->twx, cfg->nx, cfg->nx, true);
+        if (!rc) rc = upload_twiddles<double>(p, &p->twy, cfg->ny, cfg->ny, true);
+        if (!rc) rc = upload_twiddles<double>(p, &p->twm, cfg->nz / 2, cfg->nz / 2, true);
+        if (!rc) rc = upload_twiddles<double>(p, &p->twn, cfg->nz, cfg->nz / 2 + 1, false);
+        if (!rc && p->g.basis == 1) rc = upload_twiddles<double>(p, &p->twq, 4 * cfg->nx, cfg->nx, false);
     }
     for (int i = 0; i < 6 && !rc; i++) rc = dmalloc(p, &p->U[i], p->ncw * p->elem);
     for (int i = 0; i < 9 && !rc; i++) rc = dmalloc(p, &p->P[i], p->ncw * p->elem);

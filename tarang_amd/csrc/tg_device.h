@@ -224,6 +224,25 @@ __host__ __device__ constexpr int num_passes(int L)
     return n;
 }
 
+// Pass order of the twiddle table of a line of L points: the pass of radix R
+// and stride NS reads entries r NS + k (1 <= r < R, k < NS), the factor
+// exp(-2 pi i m / L) with m = r k L / (NS R).  The passes' ranges [NS, NS R)
+// follow each other, so the table has L entries (entry 0 unused).  order[i]
+// receives m.  (In natural order a pass's threads read entries up to 4 r
+// apart, which LDS serves 8 to a bank.)
+inline void twiddle_order(int L, int *order)
+{
+    order[0] = 0;
+    int NS = 1;
+    auto pass = [&](int R) {
+        for (int r = 1; r < R; r++)
+            for (int k = 0; k < NS; k++) order[r * NS + k] = (int)((long long)r * k * L / ((long long)NS * R));
+        NS *= R;
+    };
+    for (int p = 0; p < num_odd_passes(L); p++) pass(odd_radix(L, p));
+    for (int p = 0; p < num_passes(L); p++) pass(pass_radix(L, p));
+}
+
 // Block barrier that orders LDS accesses only.  The pass kernels exchange
 // data between threads through LDS alone, so their barriers need not wait
 // for global memory: __syncthreads' fence waits for every outstanding global
@@ -335,9 +354,8 @@ __device__ __forceinline__ void stockham_pass(cpx<T> *v, const X &x, const cpx<T
 #pragma unroll
         for (int r = 0; r < R; r++) a[r] = v[q + r * Q];
         if constexpr (NS > 1) {
-            const int step = (L / (NS * R)) * k;
 #pragma unroll
-            for (int r = 1; r < R; r++) a[r] = twmul<DIR>(a[r], tw[r * step]);
+            for (int r = 1; r < R; r++) a[r] = twmul<DIR>(a[r], tw[r * NS + k]);
         }
         dftR<R, DIR>(a);
         if constexpr (LAST) {
@@ -374,9 +392,8 @@ __device__ __forceinline__ void odd_pass(const X &x, const cpx<T> *__restrict__ 
         if (b < NB) {
             const int k = b % NS;
             if constexpr (NS > 1) {
-                const int step = (L / (NS * R)) * k;
 #pragma unroll
-                for (int r = 1; r < R; r++) a[q][r] = twmul<DIR>(a[q][r], tw[r * step]);
+                for (int r = 1; r < R; r++) a[q][r] = twmul<DIR>(a[q][r], tw[r * NS + k]);
             }
             dftR<R, DIR>(a[q]);
             const int base = (b / NS) * NS * R + k;
@@ -418,7 +435,8 @@ __device__ __forceinline__ void fft_passes(cpx<T> *v, const X &x, const cpx<T> *
 
 // Full line FFT of L = 8*TPL points (line_length_ok(L), up to 4096), values
 // in registers at positions j + TPL*s.  Exponent sign DIR (-1 forward, +1
-// inverse), unnormalised.  tw[k] = exp(-2 pi i k / L).  Uses the exchange x
+// inverse), unnormalised.  tw: the twiddles in pass order (twiddle_order), so
+// that the threads of a pass read consecutive entries.  Uses the exchange x
 // between passes; every thread of the line (ColX: of the block) must call it;
 // the caller must have synchronised if the exchange buffer was in use
 // before.  The radix-3/5 passes run first, through LDS; the power-of-two

@@ -208,7 +208,8 @@ __global__ void __launch_bounds__(256) k_z_c2r(ZArgs a)
     constexpr int TPL = M / 8;
     constexpr int LPB = z_lines_per_block<M>();
     constexpr int LP = lpad_len(M);
-    __shared__ cpx<T> lds[LPB * LP];
+    __shared__ cpx<T> lds[LPB * LP], ldw[2 * M];
+    const ZTwiddles<T, M> tw(ldw, a.twm, a.twn);
     const int li = threadIdx.x / TPL, j = threadIdx.x % TPL;
     const size_t line = (size_t)blockIdx.x * LPB + li;
     const size_t nlines = (size_t)a.g.nx * a.g.ny;
@@ -216,7 +217,7 @@ __global__ void __launch_bounds__(256) k_z_c2r(ZArgs a)
     for (int comp = 0; comp < a.ncomp; comp++) {
         const cpx<T> *X = (const cpx<T> *)a.in[comp] + lsafe * a.g.nzp;
         cpx<T> v[8];
-        zline_c2r<T, M>(v, X, lds + li * LP, (const cpx<T> *)a.twm, (const cpx<T> *)a.twn, j);
+        zline_c2r<T, M>(v, X, lds + li * LP, tw, j);
         if (line < nlines) {
             double *R = (double *)a.out[comp] + line * (size_t)(2 * M + 2);
 #pragma unroll
@@ -236,7 +237,8 @@ __global__ void __launch_bounds__(256) k_z_r2c(ZArgs a)
     constexpr int TPL = M / 8;
     constexpr int LPB = z_lines_per_block<M>();
     constexpr int LP = lpad_len(M);
-    __shared__ cpx<T> lds[LPB * LP];
+    __shared__ cpx<T> lds[LPB * LP], ldw[2 * M];
+    const ZTwiddles<T, M> tw(ldw, a.twm, a.twn);
     const int li = threadIdx.x / TPL, j = threadIdx.x % TPL;
     const size_t line = (size_t)blockIdx.x * LPB + li;
     const size_t nlines = (size_t)a.g.nx * a.g.ny;
@@ -247,7 +249,7 @@ __global__ void __launch_bounds__(256) k_z_r2c(ZArgs a)
 #pragma unroll
         for (int s = 0; s < 8; s++) v[s] = cvt<T>(R[j + TPL * s]);
         cpx<T> *X = (cpx<T> *)a.out[comp] + lsafe * a.g.nzp;
-        zline_r2c_post<T, M>(v, X, lds + li * LP, (const cpx<T> *)a.twm, (const cpx<T> *)a.twn, j, line < nlines);
+        zline_r2c_post<T, M>(v, X, lds + li * LP, tw, j, line < nlines, a.g.nzp - M);
     }
 }
 
@@ -258,36 +260,41 @@ __global__ void __launch_bounds__(256) k_z_r2c(ZArgs a)
 // u_y u_z, u_z u_x (the nonlinear term less the gradient i K F[u_z^2], which
 // the pressure projection removes).
 // Giver: out[3*i + j] = u_j w_i (compute_diag_offdiag.cc:329-414).
+// Bound by HBM.  The twiddles sit in LDS: read from global memory, those of
+// each product waited for the stores of the one before (loads and stores
+// retire in order) and took 168 of the 264 memory instructions of a wave.
+// Rows are written whole, and non-temporally where the fields pass the
+// memory-side cache.  512^3, per launch: FP64 2125 -> 1736 us (5.0 TB/s), FP32
+// 1363 -> 830 us (5.2 TB/s).
 // FP32 lines of 256 points (512-point z axis): four waves per SIMD (the
-// allocation fits 128 VGPRs without spills and the pass runs 6% faster at
-// 512^3 than with the three waves the unconstrained allocation gives).
+// allocation fits 128 VGPRs without spills).
 // FIVE: the NS form with the five trace-shifted products (an instance of its
 // own: with both NS forms in one kernel the FP32 instance spilled under its
 // four-wave bound); with GIVER, the eight trace-shifted products of the MHD
 // stage: P_xx - P_zz, P_yy - P_zz and the six off-diagonal ones (P_zz is
 // not stored).
-template <typename T, int M, bool GIVER, bool FIVE = false>
+template <typename T, int M, bool GIVER, bool FIVE, bool NT>
 __global__ void __launch_bounds__(256, (sizeof(T) == 4 && !GIVER && M == 256) ? 4 : 1) k_z_products(ZArgs a)
 {
     constexpr int TPL = M / 8;
     constexpr int LPB = z_lines_per_block<M>();
     constexpr int LP = lpad_len(M);
-    __shared__ cpx<T> lds[LPB * LP];
+    __shared__ cpx<T> lds[LPB * LP], ldw[2 * M];
     const int li = threadIdx.x / TPL, j = threadIdx.x % TPL;
     const size_t line = (size_t)blockIdx.x * LPB + li;
     const size_t nlines = (size_t)a.g.nx * a.g.ny;
     const bool valid = line < nlines;
     const size_t lsafe = valid ? line : nlines - 1;
-    const cpx<T> *twm = (const cpx<T> *)a.twm, *twn = (const cpx<T> *)a.twn;
     cpx<T> *L = lds + li * LP;
     // the three input lines are loaded before the first transform: their
     // loads are in flight together
     cpx<T> u[3][8], xm[3];
 #pragma unroll
-    for (int c = 0; c < 3; c++) zline_load<T, M>(u[c], xm[c], (const cpx<T> *)a.in[c] + lsafe * a.g.nzp, j);
+    for (int c = 0; c < 3; c++) zline_load<T, M, NT>(u[c], xm[c], (const cpx<T> *)a.in[c] + lsafe * a.g.nzp, j);
+    const ZTwiddles<T, M> tw(ldw, a.twm, a.twn);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        zline_c2r_from<T, M>(u[c], xm[c], L, twm, twn, j);
+        zline_c2r_from<T, M>(u[c], xm[c], L, tw, j);
         line_sync<M / 8>();
     }
     if (!GIVER && a.tape[0] && valid) {
@@ -301,7 +308,7 @@ __global__ void __launch_bounds__(256, (sizeof(T) == 4 && !GIVER && M == 256) ? 
     }
     auto emit = [&](cpx<T> *p, int o) {
         cpx<T> *X = (cpx<T> *)a.out[o] + lsafe * a.g.nzp;
-        zline_r2c_post<T, M>(p, X, L, twm, twn, j, valid);
+        zline_r2c_post<T, M, NT>(p, X, L, tw, j, valid, a.g.nzp - M);
     };
     if constexpr (!GIVER && FIVE) {
         // the cross products first, then the two shifted squares (u_z is
@@ -344,7 +351,7 @@ __global__ void __launch_bounds__(256, (sizeof(T) == 4 && !GIVER && M == 256) ? 
         for (int ii = 0; ii < 3; ii++) {
             const int i = ii == 0 ? 2 : ii - 1;
             cpx<T> w[8];
-            zline_c2r<T, M>(w, (const cpx<T> *)a.in[3 + i] + lsafe * a.g.nzp, L, twm, twn, j);
+            zline_c2r<T, M, NT>(w, (const cpx<T> *)a.in[3 + i] + lsafe * a.g.nzp, L, tw, j);
             line_sync<M / 8>();
             if (ii == 0) {
 #pragma unroll
@@ -366,7 +373,7 @@ __global__ void __launch_bounds__(256, (sizeof(T) == 4 && !GIVER && M == 256) ? 
 #pragma unroll 1
         for (int i = 0; i < 3; i++) {
             cpx<T> w[8];
-            zline_c2r<T, M>(w, (const cpx<T> *)a.in[3 + i] + lsafe * a.g.nzp, L, twm, twn, j);
+            zline_c2r<T, M, NT>(w, (const cpx<T> *)a.in[3 + i] + lsafe * a.g.nzp, L, tw, j);
             line_sync<M / 8>();
 #pragma unroll
             for (int jj = 0; jj < 3; jj++) {
@@ -948,15 +955,25 @@ hipError_t z_r2c_len(const ZArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
+template <typename T, int MM, bool GIVER, bool FIVE>
+hipError_t z_products_launch(const ZArgs &a, hipStream_t st)
+{
+    const dim3 grid = z_grid<MM>(a.g), block(z_lines_per_block<MM>() * (MM / 8));
+    const int fields = (GIVER ? 6 : 3) + a.ncomp;
+    constexpr bool STREAM = GIVER || FIVE;
+    const bool nt = STREAM && stream_bytes((size_t)fields * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
+    if (nt) hipLaunchKernelGGL((k_z_products<T, MM, GIVER, FIVE, STREAM>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_z_products<T, MM, GIVER, FIVE, false>), grid, block, 0, st, a);
+    return hipGetLastError();
+}
+
 template <typename T, int MM>
 hipError_t z_products_len(const ZArgs &a, int giver, hipStream_t st)
 {
-    const dim3 grid = z_grid<MM>(a.g), block(z_lines_per_block<MM>() * (MM / 8));
-    if (giver && a.ncomp == 8) hipLaunchKernelGGL((k_z_products<T, MM, true, true>), grid, block, 0, st, a);
-    else if (giver) hipLaunchKernelGGL((k_z_products<T, MM, true>), grid, block, 0, st, a);
-    else if (a.ncomp == 5) hipLaunchKernelGGL((k_z_products<T, MM, false, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((k_z_products<T, MM, false>), grid, block, 0, st, a);
-    return hipGetLastError();
+    if (giver && a.ncomp == 8) return z_products_launch<T, MM, true, true>(a, st);
+    if (giver) return z_products_launch<T, MM, true, false>(a, st);
+    if (a.ncomp == 5) return z_products_launch<T, MM, false, true>(a, st);
+    return z_products_launch<T, MM, false, false>(a, st);
 }
 
 template <typename T, int LL, int MODE>

@@ -331,24 +331,40 @@ __device__ __forceinline__ bool in_band(const Grid &g, const Band &b, int kx, in
 // r2c: Z = DFT_M(z); X[k] = ((Z[k] + conj Z[M-k]) - i W^k (Z[k] - conj Z[M-k]))/2.
 // W = exp(-2 pi i / N); twn holds W^k for k = 0..M.
 // ---------------------------------------------------------------------------
+// The twiddles of a z kernel in LDS (2 M entries: m in pass order, then n): read
+// from global memory between two lines' stores, each would wait for the stores
+// before it (loads and stores retire in order).
+template <typename T, int M>
+struct ZTwiddles {
+    const cpx<T> *m, *n;
+    // all threads of the block; ends in a barrier
+    __device__ __forceinline__ ZTwiddles(cpx<T> *lds, const void *twm, const void *twn) : m(lds), n(lds + M)
+    {
+        for (int i = threadIdx.x; i < M; i += blockDim.x) {
+            lds[i] = ((const cpx<T> *)twm)[i];
+            lds[M + i] = ((const cpx<T> *)twn)[i];
+        }
+        lds_barrier();
+    }
+};
+
 // The M+1 points of a complex line: v[s] = X[j + TPL*s], xm = X[M] (read by
 // every thread of the line; member-wise copies keep v in registers).
-template <typename T, int M>
+template <typename T, int M, bool NT = false>
 __device__ __forceinline__ void zline_load(cpx<T> *v, cpx<T> &xm, const cpx<T> *__restrict__ X, int j)
 {
     constexpr int TPL = M / 8;
 #pragma unroll
-    for (int s = 0; s < 8; s++) v[s] = mk<T>(X[j + TPL * s].x, X[j + TPL * s].y);
-    xm = mk<T>(X[M].x, X[M].y);
+    for (int s = 0; s < 8; s++) v[s] = gload<NT>(X + j + TPL * s);
+    xm = gload<false>(X + M);
 }
 
 // c2r of a line already loaded by zline_load (v in, samples out in v).
 template <typename T, int M>
-__device__ __forceinline__ void zline_c2r_from(cpx<T> *v, cpx<T> xm, cpx<T> *lds, const cpx<T> *__restrict__ twm,
-                                               const cpx<T> *__restrict__ twn, int j)
+__device__ __forceinline__ void zline_c2r_from(cpx<T> *v, cpx<T> xm, cpx<T> *lds, const ZTwiddles<T, M> &tw, int j)
 {
     constexpr int TPL = M / 8;
-    // stage the line (M+1 points) in LDS
+    // the line (M+1 points) in LDS, for the mirrored points
 #pragma unroll
     for (int s = 0; s < 8; s++) lds[lpad(j + TPL * s)] = mk<T>(v[s].x, v[s].y);
     if (j == 0) lds[lpad(M)] = xm;
@@ -356,39 +372,41 @@ __device__ __forceinline__ void zline_c2r_from(cpx<T> *v, cpx<T> xm, cpx<T> *lds
 #pragma unroll
     for (int s = 0; s < 8; s++) {
         const int k = j + TPL * s;
-        cpx<T> xk = lds[lpad(k)];
+        cpx<T> xk = v[s];
         cpx<T> xm = lds[lpad(M - k)];
         if (k == 0) { xk.y = 0; xm.y = 0; }
         const cpx<T> a = xk + conj(xm);
         const cpx<T> d = xk - conj(xm);
-        const cpx<T> w = twn[k];  // W^k ; we need W^-k = conj(w)
+        const cpx<T> w = tw.n[k];  // W^k ; we need W^-k = conj(w)
         const cpx<T> e = mk<T>(d.x * w.x + d.y * w.y, d.y * w.x - d.x * w.y);
         v[s] = a + mk<T>(-e.y, e.x);
     }
     line_sync<M / 8>();
-    fft_line<M, +1>(v, lds, twm, j);
+    fft_line<M, +1>(v, lds, tw.m, j);
 }
 
-template <typename T, int M>
+template <typename T, int M, bool NT = false>
 __device__ __forceinline__ void zline_c2r(cpx<T> *v, const cpx<T> *__restrict__ X, cpx<T> *lds,
-                                          const cpx<T> *__restrict__ twm, const cpx<T> *__restrict__ twn, int j)
+                                          const ZTwiddles<T, M> &tw, int j)
 {
     cpx<T> xm;
-    zline_load<T, M>(v, xm, X, j);
-    zline_c2r_from<T, M>(v, xm, lds, twm, twn, j);
+    zline_load<T, M, NT>(v, xm, X, j);
+    zline_c2r_from<T, M>(v, xm, lds, tw, j);
 }
 
-template <typename T, int M>
+// The line's npad = nzp - M entries from X[M] on are written too (zeros after
+// X[M]): whole 128-byte lines.
+template <typename T, int M, bool NT = false>
 __device__ __forceinline__ void zline_r2c_post(cpx<T> *v, cpx<T> *__restrict__ X, cpx<T> *lds,
-                                               const cpx<T> *__restrict__ twm, const cpx<T> *__restrict__ twn, int j,
-                                               bool store)
+                                               const ZTwiddles<T, M> &tw, int j, bool store, int npad)
 {
     constexpr int TPL = M / 8;
-    fft_line<M, -1>(v, lds, twm, j);
+    fft_line<M, -1>(v, lds, tw.m, j);
 #pragma unroll
     for (int s = 0; s < 8; s++) lds[lpad(j + TPL * s)] = v[s];
     line_sync<M / 8>();
     const T h = (T)0.5;
+    const cpx<T> z0 = lds[0];
 #pragma unroll
     for (int s = 0; s < 8; s++) {
         const int k = j + TPL * s;
@@ -396,11 +414,12 @@ __device__ __forceinline__ void zline_r2c_post(cpx<T> *v, cpx<T> *__restrict__ X
         const cpx<T> zm = lds[lpad(k == 0 ? 0 : M - k)];
         const cpx<T> a = zk + conj(zm);
         const cpx<T> d = zk - conj(zm);
-        const cpx<T> w = twn[k];
+        const cpx<T> w = tw.n[k];
         const cpx<T> e = d * w;  // W^k d
-        if (store) X[k] = mk<T>(h * (a.x + e.y), h * (a.y - e.x));
+        if (store) gstore<NT>(X + k, mk<T>(h * (a.x + e.y), h * (a.y - e.x)));
     }
-    if (store && j == 0) X[M] = mk<T>(v[0].x - v[0].y, (T)0);
+    if (store)
+        for (int i = j; i < npad; i += TPL) gstore<NT>(X + M + i, mk<T>(i == 0 ? z0.x - z0.y : (T)0, (T)0));
     line_sync<M / 8>();
 }
 

@@ -241,34 +241,34 @@ __device__ __forceinline__ void *sel_ptr(void *const *p, int i, int n)
 // u_y^2 - u_z^2 and the off-diagonal ones (out[2], zz, not written): the stage
 // uses the velocity term only projected, and the SFF projection removes the
 // gradient of u_z^2 that the shift adds.
-template <typename T, int M, bool SHIFT = false>
+template <typename T, int M, bool SHIFT, bool NT>
 __global__ void __launch_bounds__(256, 2) k_z_rbc(ZArgs a)
 {
     constexpr int TPL = M / 8;
     constexpr int LPB = z_lines_per_block<M>();
     constexpr int LP = lpad_len(M);
-    __shared__ cpx<T> lds[LPB * LP];
+    __shared__ cpx<T> lds[LPB * LP], ldw[2 * M];
     const int li = threadIdx.x / TPL, j = threadIdx.x % TPL;
     const size_t line = (size_t)blockIdx.x * LPB + li;
     const size_t nlines = (size_t)a.g.nx * a.g.ny;
     const bool valid = line < nlines;
     const size_t lsafe = valid ? line : nlines - 1;
-    const cpx<T> *twm = (const cpx<T> *)a.twm, *twn = (const cpx<T> *)a.twn;
     cpx<T> *L = lds + li * LP;
     const size_t off = lsafe * a.g.nzp;
     cpx<T> u[3][8], xm[3];
 #pragma unroll
-    for (int c = 0; c < 3; c++) zline_load<T, M>(u[c], xm[c], (const cpx<T> *)a.in[c] + off, j);
+    for (int c = 0; c < 3; c++) zline_load<T, M, NT>(u[c], xm[c], (const cpx<T> *)a.in[c] + off, j);
+    const ZTwiddles<T, M> tw(ldw, a.twm, a.twn);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        zline_c2r_from<T, M>(u[c], xm[c], L, twm, twn, j);
+        zline_c2r_from<T, M>(u[c], xm[c], L, tw, j);
         line_sync<M / 8>();
     }
     auto emit = [&](const cpx<T> *x, const cpx<T> *y, int o) {
         cpx<T> p[8];
 #pragma unroll
         for (int s = 0; s < 8; s++) p[s] = mk<T>(x[s].x * y[s].x, x[s].y * y[s].y);
-        zline_r2c_post<T, M>(p, (cpx<T> *)a.out[o] + off, L, twm, twn, j, valid);
+        zline_r2c_post<T, M, NT>(p, (cpx<T> *)a.out[o] + off, L, tw, j, valid, a.g.nzp - M);
     };
     if constexpr (SHIFT) {
         // the off-diagonal products first, then the shifted squares (u_z is
@@ -283,7 +283,7 @@ __global__ void __launch_bounds__(256, 2) k_z_rbc(ZArgs a)
             for (int s = 0; s < 8; s++)
                 p[s] = mk<T>(u[ia][s].x * u[ia][s].x - u[2][s].x * u[2][s].x,
                              u[ia][s].y * u[ia][s].y - u[2][s].y * u[2][s].y);
-            zline_r2c_post<T, M>(p, (cpx<T> *)a.out[ia] + off, L, twm, twn, j, valid);
+            zline_r2c_post<T, M, NT>(p, (cpx<T> *)a.out[ia] + off, L, tw, j, valid, a.g.nzp - M);
         }
     } else {
 #pragma unroll
@@ -292,7 +292,7 @@ __global__ void __launch_bounds__(256, 2) k_z_rbc(ZArgs a)
             for (int ib = ia; ib < 3; ib++) emit(u[ia], u[ib], rbc_pair(ia, ib));
     }
     cpx<T> t[8];
-    zline_c2r<T, M>(t, (const cpx<T> *)a.in[3] + off, L, twm, twn, j);
+    zline_c2r<T, M, NT>(t, (const cpx<T> *)a.in[3] + off, L, tw, j);
     line_sync<M / 8>();
 #pragma unroll
     for (int ia = 0; ia < 3; ia++) emit(u[ia], t, rbc_pair(ia, 3));
@@ -662,8 +662,11 @@ hipError_t z_rbc_len(const ZArgs &a, hipStream_t st)
     constexpr int LPB = z_lines_per_block<MM>();
     const size_t nlines = (size_t)a.g.nx * a.g.ny;
     dim3 grid((unsigned)((nlines + LPB - 1) / LPB));
-    if (a.ncomp == 8) hipLaunchKernelGGL((k_z_rbc<T, MM, true>), grid, dim3(LPB * (MM / 8)), 0, st, a);
-    else hipLaunchKernelGGL((k_z_rbc<T, MM>), grid, dim3(LPB * (MM / 8)), 0, st, a);
+    const dim3 block(LPB * (MM / 8));
+    const bool nt = stream_bytes((size_t)12 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
+    if (a.ncomp != 8) hipLaunchKernelGGL((k_z_rbc<T, MM, false, false>), grid, block, 0, st, a);
+    else if (nt) hipLaunchKernelGGL((k_z_rbc<T, MM, true, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_z_rbc<T, MM, true, false>), grid, block, 0, st, a);
     return hipGetLastError();
 }
 
