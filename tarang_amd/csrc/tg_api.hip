@@ -94,9 +94,8 @@ struct tg_plan {
     // work layout), [1..4] force inputs theta, u_x of two stage parities
     // (FP64 boundary layout)
     double *rbc[5] = {};
-    // MHD buffers (FP64), allocated on first use: [0..2] accW (padded work
-    // layout), [3..5] Z+, [6..8] Z- (boundary layout)
-    double *mhd[9] = {};
+    // MHD: accW (FP64, padded work layout), allocated on first use
+    double *mhd[3] = {};
     // adjoint: checkpoints (FP64 spectral, 3 components each), tape of the
     // real-space stage velocities (every x 4 stages x 3 components, packed
     // z lines in the transform precision), recompute state, cotangent and
@@ -581,9 +580,9 @@ int run_rk4(tg_plan *p, double *const V[3], const tg_fluid *f, int nsteps, int f
 
 int ensure_mhd(tg_plan *p)
 {
-    for (int i = 0; i < 9; i++)
+    for (int i = 0; i < 3; i++)
         if (!p->mhd[i]) {
-            int rc = dmalloc(p, (void **)&p->mhd[i], (i < 3 ? p->ncw : p->nc) * 16);
+            int rc = dmalloc(p, (void **)&p->mhd[i], p->ncw * 16);
             if (rc) return rc;
         }
     return TG_OK;
@@ -607,12 +606,10 @@ int mhd_nonlinear(tg_plan *p, double *const *Np, double *const *Nm)
 }
 
 template <typename T>
-int mhd_xinv(tg_plan *p, double *const *Zp, double *const *Zm)
+int mhd_xinv(tg_plan *p, double *const V[3], double *const W[3], bool patch)
 {
-    Band nb{};
     Prof pr(p, TG_KERNEL_X_INV);
-    HIPCHK(launch_xinv_state<T>(p->g, nb, Zm, 3, p->U, nullptr, 0, p->twx, p->stream));
-    HIPCHK(launch_xinv_state<T>(p->g, nb, Zp, 3, p->U + 3, nullptr, 0, p->twx, p->stream));
+    HIPCHK(launch_xinv_elsasser<T>(p->g, V, W, p->U, patch, p->twx, p->stream));
     return TG_OK;
 }
 
@@ -622,15 +619,12 @@ int run_rk4_mhd(tg_plan *p, double *const V[3], double *const W[3], const tg_flu
     int rc = ensure_mhd(p);
     if (rc) return rc;
     double *accW[3] = {p->mhd[0], p->mhd[1], p->mhd[2]};
-    double *Zp[3] = {p->mhd[3], p->mhd[4], p->mhd[5]};
-    double *Zm[3] = {p->mhd[6], p->mhd[7], p->mhd[8]};
     p->unext_valid = false;
     rc = nonfinite_begin(p);
     if (rc) return rc;
     // stage-1 input of the first step; the stage-4 x pass of each step leaves
     // that of the next
-    HIPCHK(launch_mhd_elsasser(p->g, V, W, Zp, Zm, p->stream));
-    rc = mhd_xinv<T>(p, Zp, Zm);
+    rc = mhd_xinv<T>(p, V, W, false);
     if (rc) return rc;
     for (int step = 0; step < nsteps; step++) {
         for (int s = 1; s <= 4; s++) {
@@ -670,10 +664,8 @@ int run_rk4_mhd(tg_plan *p, double *const V[3], double *const W[3], const tg_flu
             HIPCHK(launch_reality(p->g, W, 3, p->stream));
             if (step + 1 < nsteps) {
                 // the next stage-1 input on the two planes the condition rewrote
-                Band nb{};
-                HIPCHK(launch_mhd_elsasser_planes(p->g, V, W, Zp, Zm, p->stream));
-                HIPCHK(launch_xinv_state<T>(p->g, nb, Zm, 3, p->U, nullptr, 4, p->twx, p->stream));
-                HIPCHK(launch_xinv_state<T>(p->g, nb, Zp, 3, p->U + 3, nullptr, 4, p->twx, p->stream));
+                rc = mhd_xinv<T>(p, V, W, true);
+                if (rc) return rc;
             }
         }
     }
@@ -683,17 +675,12 @@ int run_rk4_mhd(tg_plan *p, double *const V[3], double *const W[3], const tg_flu
 template <typename T>
 int run_nlin_mhd(tg_plan *p, double *const V[3], double *const W[3], double *const NU[3], double *const NW[3])
 {
-    int rc = ensure_mhd(p);
-    if (rc) return rc;
-    double *Zp[3] = {p->mhd[3], p->mhd[4], p->mhd[5]};
-    double *Zm[3] = {p->mhd[6], p->mhd[7], p->mhd[8]};
     p->unext_valid = false;
     if (p->g.dealias) {
         HIPCHK(launch_dealias(p->g, V, 3, p->stream));
         HIPCHK(launch_dealias(p->g, W, 3, p->stream));
     }
-    HIPCHK(launch_mhd_elsasser(p->g, V, W, Zp, Zm, p->stream));
-    rc = mhd_xinv<T>(p, Zp, Zm);
+    int rc = mhd_xinv<T>(p, V, W, false);
     if (!rc) rc = mhd_nonlinear<T>(p, NU, NW);
     if (rc) return rc;
     HIPCHK(launch_mhd_combine(p->g, NU, NW, p->stream));

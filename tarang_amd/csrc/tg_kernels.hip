@@ -516,57 +516,17 @@ constexpr int xnl_axis(int mode, int p, int i)
     return sel[mode == XNL_FIVE && p >= 2 ? p + 1 : p][i];
 }
 
-// Keeps loads and stores on their side of it (no wait): without it the loads of
-// all the later products move up to the first one and spill.
-__device__ __forceinline__ void pin_memory_order()
-{
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-// A value formed at this point: the sums and factors below would otherwise be
-// moved to their uses (inside a later branch) and everything that they are
-// formed from kept in registers until then (1.3 KB a lane spilled).
-__device__ __forceinline__ void settle(double &x) { asm volatile("" : "+v"(x)); }
-template <typename T>
-__device__ __forceinline__ void settle(cpx<T> &z) { asm volatile("" : "+v"(z.x), "+v"(z.y)); }
-
-// An index hidden from loop-invariant code motion: the twiddles, wavenumbers
-// and LDS addresses formed from it are formed again at each use instead of
-// staying in registers over the whole kernel (the twiddles alone are 56).
-__device__ __forceinline__ int hidden(int j)
-{
-    asm volatile("" : "+v"(j));
-    return j;
-}
-
-// This thread's 8 points of a column (ColX order): rows j + TPL s.  p is the
-// same for the whole block (its first row and column), off this thread's byte
-// offset from it (under 4 GB: an eighth of a field), so that an address is a
-// scalar base and one 32-bit register however many rows and fields there are.
-template <bool NT, typename T>
-__device__ __forceinline__ void col_load(cpx<T> *v, const cpx<T> *p, size_t step, uint32_t off)
-{
-#pragma unroll
-    for (int s = 0; s < 8; s++) v[s] = gload<NT>((const cpx<T> *)((const char *)(p + s * step) + off));
-}
-template <bool NT, typename T>
-__device__ __forceinline__ void col_store(const cpx<T> *v, cpx<T> *p, size_t step, uint32_t off)
-{
-#pragma unroll
-    for (int s = 0; s < 8; s++) gstore<NT>((cpx<T> *)((char *)(p + s * step) + off), v[s]);
-}
-
 // Bound by HBM and by the one block of two waves a SIMD that its registers
 // leave: the next tile is always in flight.  Columns go from memory to
 // registers in the transform's own order (ColX) and back; LDS holds the
 // exchanges, the twiddles and the viscous factors.  Every value is settled
-// where it is formed, and each stage has its own code after a common forward
-// part: with the four stages, the hyperviscosity loops and the random phases
-// inlined per point the kernel was 300 KB of instructions, mostly fetched
-// from L2.  512^3, per launch: FP64 5170 -> 3770 us (4.7 TB/s), FP32 4550 ->
-// 3150 us; 64^3 FP64 54 -> 21 us, 240x160x96 348 -> 161 us.
-template <typename T, int L, int CB, int MODE, bool NT>
+// where it is formed, and each stage is an instance of its own: with the four
+// stages, the hyperviscosity loops and the random phases inlined per point the
+// kernel was 300 KB of instructions, mostly fetched from L2 (and the stages'
+// registers, allocated together, spilled).  512^3, per launch: FP64 5170 ->
+// 3606 us (4.9 TB/s), FP32 4550 -> 3150 us; 64^3 FP64 54 -> 19 us, 240x160x96
+// 348 -> 137 us.
+template <typename T, int L, int CB, int MODE, int ST, bool NT>
 __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
 {
     constexpr int TPL = L / 8;
@@ -579,41 +539,24 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
     // passes would wait for the next tile's loads in flight
     __shared__ cpx<T> tw[L];
     __shared__ double red[16];
-    // the viscous factors exp(-nu K^2 dt/2), exp(-nu K^2 dt) of this thread's
-    // points (their registers would spill)
-    __shared__ double visc[MODE == XNL_FIVE ? 2 : 1][MODE == XNL_FIVE ? 8 * CB * TPL : 1];
+    // the viscous factors of this thread's points (their registers would
+    // spill): exp(-nu K^2 dt/2), stage 4 exp(-nu K^2 dt), stage 1 both
+    __shared__ double visc[ST == 1 ? 2 : 1][ST ? 8 * CB * TPL : 1];
     const Grid &g = a.g;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     if (tile >= x_tiles(g, CB, false)) return;
-    // Tiles of 128-byte rows divide nzp and lie within one ky row, the same for
-    // the whole block; the wider ones of short lines do not, and the last one
-    // may run past the last column (those threads move the last column and
-    // store nothing).
-    constexpr bool WIDE = CB * sizeof(cpx<T>) > 128;
-    const int c = threadIdx.x % CB, j = threadIdx.x / CB;
-    const int ncol = g.ny * g.nzp;
-    const int cw0 = tile * CB;
-    const int cwt = WIDE ? min(cw0 + c, ncol - 1) : cw0;
-    const bool inside = !WIDE || cw0 + c < ncol;
-    const int ly = cwt / g.nzp, lz0 = WIDE ? 0 : cwt % g.nzp;
-    const int lz = WIDE ? cwt % g.nzp : lz0 + c;
-    const bool live = inside && lz < g.nzc;   // the pad columns carry zeros
+    const ColTile<T, L, CB> t(g, tile);
+    const int j = t.j, ly = t.ly, lz = t.lz, cw0 = t.cw0;
+    const bool live = t.live;
+    const size_t stepw = t.stepw, steps = t.steps, state0 = t.state0;
+    const uint32_t offt = t.offt, offw = t.offw, offs = t.offs;
     const int ky = kwave(ly, g.ny);
     const double Ky = ky * g.kf[1], Kz = lz * g.kf[2];
-    const size_t ncw = (size_t)ncol, ncs = (size_t)g.ny * g.nzc;
-    const size_t stepw = (size_t)TPL * ncw, steps = (size_t)TPL * ncs;
-    const size_t state0 = WIDE ? 0 : (size_t)ly * g.nzc + min(lz0, g.nzc - 1);
-    const uint32_t colt = WIDE ? cwt - cw0 : c;
-    const uint32_t offt = (uint32_t)(j * ncw + colt) * sizeof(cpx<T>), offw = (uint32_t)(j * ncw + colt) * 16;
-    // (a pad column reads the last one; a tile may hold pad columns only)
-    const uint32_t offs = (uint32_t)(j * ncs + (WIDE ? ly * g.nzc + min(lz, g.nzc - 1)
-                                                     : max(min(c, g.nzc - 1 - lz0), 0))) * 16;
     const T sc = (T)a.rk.scale;
     const T Kyt = (T)Ky, Kzt = (T)Kz;
     constexpr bool NS = MODE == XNL_SIX || MODE == XNL_FIVE;
     constexpr int NP = xnl_products(MODE);
-    const int stage = MODE == XNL_FIVE ? a.rk.stage : 0;
-    const bool want_rhs = NS && (stage > 0 || a.rk.write_rhs);
+    const bool want_rhs = NS && (ST > 0 || a.rk.write_rhs);
 
     cpx<T> cur[8];
     col_load<NTW>(cur, (const cpx<T> *)a.P[0] + cw0, stepw, offt);
@@ -621,7 +564,7 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
     // whether a column of this tile can hold forced modes; the alpha forcing's
     // coefficient is summed by the block (one thread summing all the slots
     // took 70 us of a 128^3 stage)
-    const bool band_tile = NS && a.b.kind != 0 && (WIDE || (abs(ky) <= a.b.h[1] && lz0 <= a.b.h[2]));
+    const bool band_tile = NS && a.b.kind != 0 && (t.WIDE || (abs(ky) <= a.b.h[1] && t.lz0 <= a.b.h[2]));
     double alpha = 0.0;
     if (band_tile && a.b.kind == 1 && want_rhs) alpha = band_alpha<CB * TPL>(g, a.b, a.slots_in, red);
     unsigned forced = 0;   // bit s: row j + TPL s of this column is forced
@@ -631,7 +574,7 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
             if (band_slot(a.b, kx, ky, lz) >= 0 && in_band(g, a.b, kx, ky, lz)) forced |= 1u << s;
         }
     lds_barrier();
-    const X x{lds + c};
+    const X x{lds + t.c};
 
     // --- forward x-FFT of the products and the divergence-form sum ---
     // Unrolled over the products: each adds to the one or two components its
@@ -645,7 +588,7 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
         constexpr int PI = decltype(pc)::value;
         pin_memory_order();
         if constexpr (PI + 1 < NP) col_load<NTW>(next, (const cpx<T> *)a.P[xnl_index(MODE, PI + 1)] + cw0, stepw, offt);
-        else if (stage > 0) col_load<false>(v0, (const cpx<double> *)a.V[0] + state0, steps, offs);
+        else if (ST > 0) col_load<false>(v0, (const cpx<double> *)a.V[0] + state0, steps, offs);
         pin_memory_order();
         const int jh = hidden(j);
         fft_exchange<L, -1>(v, x, tw, jh);
@@ -721,7 +664,7 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
         else project(std::false_type{});
     }
 
-    if (stage == 0) {
+    if constexpr (ST == 0) {
         // Compute_nlin (and optionally Compute_rhs) output, FP64 boundary layout
         if (live) {
 #pragma unroll
@@ -747,11 +690,7 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
     int zx0, zx1;   // rows of this column that the dealias mask zeroes (a pad column: all)
     dealias_rows(g, ly, lz, zx0, zx1);
     if (!live) { zx0 = 0; zx1 = L - 1; }
-    // One instance per stage: only the stage that runs occupies the
-    // instruction cache, and the viscous factors are formed once for the three
-    // components.
-    auto rk_stage = [&](auto stc) {
-        constexpr int ST = decltype(stc)::value;
+    if constexpr (ST > 0) {
         {
             const int jh = hidden(j);
 #pragma unroll 2
@@ -761,15 +700,16 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
                 const double ks = (kxs + Ky * Ky) + Kz * Kz;
                 const double kp = hyper_power(a.rk.hq, ks);
                 if (ST < 4) visc[0][s * CB * TPL + threadIdx.x] = exp((a.rk.fh + a.rk.fhh * kp) * ks);
-                if (ST == 1 || ST == 4) visc[1][s * CB * TPL + threadIdx.x] = exp((a.rk.f1 + a.rk.f1h * kp) * ks);
+                if (ST == 1 || ST == 4)
+                    visc[ST == 1][s * CB * TPL + threadIdx.x] = exp((a.rk.f1 + a.rk.f1h * kp) * ks);
             }
         }
         // (each thread reads its own entries only)
         auto Eh = [&](int s) { return visc[0][s * CB * TPL + threadIdx.x]; };
-        auto E1 = [&](int s) { return visc[1][s * CB * TPL + threadIdx.x]; };
+        auto E1 = [&](int s) { return visc[ST == 1][s * CB * TPL + threadIdx.x]; };
         cpx<double> ac[8];
         if (ST >= 2) col_load<NTA>(ac, (const cpx<double> *)a.acc[0] + cw0, stepw, offw);
-        bool bad = false;
+        double chk = 0.0;   // stage 4: NaN after a non-finite value
         // SLOTS: the undealiased stage input of forced modes goes to the slots
         auto algebra = [&](auto kc, auto slc, cpx<T> *v) {
             constexpr int K = decltype(kc)::value;
@@ -795,7 +735,7 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
                     ac[s] = ac[s] + c_sixth * r;
                     vn = E1(s) * v0[s] + ac[s];
                     ac[s] = vn;   // the new state
-                    bad = bad || !(isfinite(vn.x) && isfinite(vn.y));
+                    chk += 0.0 * vn.x + 0.0 * vn.y;
                 }
                 if (SLOTS && (forced & (1u << s)))
                     ((cpx<double> *)a.slots_out)[band_slot(a.b, kwave(lx, g.nx), ky, lz) * 3 + K] = vn;
@@ -813,25 +753,19 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
             if (ST == 4) {
                 if (live) col_store<false>(ac, (cpx<double> *)a.V[K] + state0, steps, offs);
             } else {
-                if (inside) col_store<NTA>(ac, (cpx<double> *)a.acc[K] + cw0, stepw, offw);
+                if (t.inside) col_store<NTA>(ac, (cpx<double> *)a.acc[K] + cw0, stepw, offw);
             }
             if (ST >= 2 && K < 2)
                 col_load<NTA>(ac, (const cpx<double> *)a.acc[K < 2 ? K + 1 : 2] + cw0, stepw, offw);
             pin_memory_order();
             fft_exchange<L, +1>(v, x, tw, hidden(j));
             pin_memory_order();
-            if (inside) col_store<NTW>(v, (cpx<T> *)a.U[K] + cw0, stepw, offt);
+            if (t.inside) col_store<NTW>(v, (cpx<T> *)a.U[K] + cw0, stepw, offt);
         };
         rk_comp(std::integral_constant<int, 0>{});
         rk_comp(std::integral_constant<int, 1>{});
         rk_comp(std::integral_constant<int, 2>{});
-        if (ST == 4 && bad && live && a.rk.nonfinite) *a.rk.nonfinite = 1;
-    };
-    if constexpr (MODE == XNL_FIVE) {
-        if (stage == 1) rk_stage(std::integral_constant<int, 1>{});
-        else if (stage == 2) rk_stage(std::integral_constant<int, 2>{});
-        else if (stage == 3) rk_stage(std::integral_constant<int, 3>{});
-        else rk_stage(std::integral_constant<int, 4>{});
+        if (ST == 4 && chk != 0.0 && live && a.rk.nonfinite) *a.rk.nonfinite = 1;
     }
 }
 
@@ -901,7 +835,8 @@ hipError_t colfft_len(const ColArgs &a, int dir, int nfields, hipStream_t st)
     // loop of the pass alone, 445 -> 381 us per field within the step); 128^3
     // FP32 lost 5% in the z pass that follows.  Not where a CU holds one block
     // (1024 points FP64 2152 against 2226 us) or the rows are half lines.
-    constexpr bool STREAM = CB * sizeof(cpx<T>) >= 128 && 2 * ColX<T, LL, CB>::SIZE * sizeof(cpx<T>) <= 160 * 1024;
+    constexpr bool STREAM = LL >= kStreamLength && CB * sizeof(cpx<T>) >= 128 &&
+                            2 * ColX<T, LL, CB>::SIZE * sizeof(cpx<T>) <= 160 * 1024;
     dim3 grid(x_grid(a.nouter * ((a.ncol + CB - 1) / CB)), nfields);
     const dim3 block(CB * (LL / 8));
     const bool nt = STREAM && stream_bytes((size_t)nfields * a.nouter * a.outer_stride * sizeof(cpx<T>));
@@ -960,7 +895,7 @@ hipError_t z_products_launch(const ZArgs &a, hipStream_t st)
 {
     const dim3 grid = z_grid<MM>(a.g), block(z_lines_per_block<MM>() * (MM / 8));
     const int fields = (GIVER ? 6 : 3) + a.ncomp;
-    constexpr bool STREAM = GIVER || FIVE;
+    constexpr bool STREAM = (GIVER || FIVE) && MM >= kStreamLength / 2;
     const bool nt = STREAM && stream_bytes((size_t)fields * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
     if (nt) hipLaunchKernelGGL((k_z_products<T, MM, GIVER, FIVE, STREAM>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((k_z_products<T, MM, GIVER, FIVE, false>), grid, block, 0, st, a);
@@ -976,7 +911,7 @@ hipError_t z_products_len(const ZArgs &a, int giver, hipStream_t st)
     return z_products_launch<T, MM, false, false>(a, st);
 }
 
-template <typename T, int LL, int MODE>
+template <typename T, int LL, int MODE, int ST>
 hipError_t x_nlin_launch(const XnlArgs &a, hipStream_t st)
 {
     // One block of 512 threads fills a CU's registers (the three sums, a
@@ -987,18 +922,25 @@ hipError_t x_nlin_launch(const XnlArgs &a, hipStream_t st)
     constexpr int CB = colx_block<T>(LL, 512);
     const bool nt = stream_bytes((size_t)8 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
     const dim3 grid(x_grid(x_tiles(a.g, CB, false))), block(CB * (LL / 8));
-    if (nt) hipLaunchKernelGGL((k_x_nlin<T, LL, CB, MODE, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((k_x_nlin<T, LL, CB, MODE, false>), grid, block, 0, st, a);
+    constexpr bool NT = LL >= kStreamLength && (ST > 0 || MODE == XNL_GIVER);
+    if (NT && nt) hipLaunchKernelGGL((k_x_nlin<T, LL, CB, MODE, ST, NT>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_x_nlin<T, LL, CB, MODE, ST, false>), grid, block, 0, st, a);
     return hipGetLastError();
 }
 
 template <typename T, int LL>
 hipError_t x_nlin_len(const XnlArgs &a, int mode, hipStream_t st)
 {
-    if (mode == XNL_GIVER) return x_nlin_launch<T, LL, XNL_GIVER>(a, st);
-    if (mode == XNL_TRANS) return x_nlin_launch<T, LL, XNL_TRANS>(a, st);
-    if (mode == XNL_FIVE) return x_nlin_launch<T, LL, XNL_FIVE>(a, st);
-    return x_nlin_launch<T, LL, XNL_SIX>(a, st);
+    if (mode == XNL_GIVER) return x_nlin_launch<T, LL, XNL_GIVER, 0>(a, st);
+    if (mode == XNL_TRANS) return x_nlin_launch<T, LL, XNL_TRANS, 0>(a, st);
+    if (mode == XNL_SIX) return x_nlin_launch<T, LL, XNL_SIX, 0>(a, st);
+    switch (a.rk.stage) {
+        case 1: return x_nlin_launch<T, LL, XNL_FIVE, 1>(a, st);
+        case 2: return x_nlin_launch<T, LL, XNL_FIVE, 2>(a, st);
+        case 3: return x_nlin_launch<T, LL, XNL_FIVE, 3>(a, st);
+        case 4: return x_nlin_launch<T, LL, XNL_FIVE, 4>(a, st);
+        default: return x_nlin_launch<T, LL, XNL_FIVE, 0>(a, st);
+    }
 }
 
 #define TG_KERNELS_L(N, T, P)                                                                  \

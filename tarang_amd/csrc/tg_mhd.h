@@ -5,11 +5,11 @@
 
 namespace tg {
 
-hipError_t launch_mhd_elsasser(const Grid &g, double *const *V, double *const *W, double *const *Zp,
-                               double *const *Zm, hipStream_t st);
-// the same on the kz = 0 and kz = Nz/2 planes only
-hipError_t launch_mhd_elsasser_planes(const Grid &g, double *const *V, double *const *W, double *const *Zp,
-                                      double *const *Zm, hipStream_t st);
+// x-inverse of the Elsasser fields of u = V, b = W (dealiased on read): Z- into
+// U[0..2], Z+ into U[3..5]; patch: the kz = 0 and kz = Nz/2 columns only.
+template <typename T>
+hipError_t launch_xinv_elsasser(const Grid &g, double *const *V, double *const *W, void *const *U, bool patch,
+                                const void *twx, hipStream_t st);
 // NU <- (NU + NW)/2, NW <- (NU - NW)/2 in place (MHD::Elsasser_to_UB_nlin)
 hipError_t launch_mhd_combine(const Grid &g, double *const *NU, double *const *NW, hipStream_t st);
 // Fused x pass of an MHD RK stage (1..4): P[3i+j] = FT[Z-_j Z+_i] (work

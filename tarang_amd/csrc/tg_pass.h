@@ -12,6 +12,9 @@ static constexpr int kLdsBudget = 73728;  // bytes; two blocks fit the 160 KB LD
 // Whether a pass over `bytes` of fields streams past the 256 MiB memory-side
 // cache, so that nothing it writes is still there for the next pass.
 inline bool stream_bytes(size_t bytes) { return bytes > ((size_t)256 << 20); }
+// Shortest x and y lines with non-temporal instances (shorter ones only stream
+// that much on grids of very unequal sides).
+static constexpr int kStreamLength = 64;
 
 __device__ __forceinline__ int kwave(int l, int n) { return l <= n / 2 ? l : l - n; }
 
@@ -222,6 +225,134 @@ __device__ __forceinline__ void tile_columns(int *colw, int *cols, const Grid &g
         cols[c] = st;
     }
 }
+
+// ---------------------------------------------------------------------------
+// Column tiles of the x passes that hold their points in registers (ColX).
+// ---------------------------------------------------------------------------
+// Keeps loads and stores on their side of it (no wait): without it the loads of
+// all the later products move up to the first one and spill.
+__device__ __forceinline__ void pin_memory_order()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// A value formed at this point: the sums and factors below would otherwise be
+// moved to their uses (inside a later branch) and everything that they are
+// formed from kept in registers until then (1.3 KB a lane spilled).
+__device__ __forceinline__ void settle(double &x) { asm volatile("" : "+v"(x)); }
+template <typename T>
+__device__ __forceinline__ void settle(cpx<T> &z) { asm volatile("" : "+v"(z.x), "+v"(z.y)); }
+
+// An index hidden from loop-invariant code motion: the twiddles, wavenumbers
+// and LDS addresses formed from it are formed again at each use instead of
+// staying in registers over the whole kernel (the twiddles alone are 56).
+__device__ __forceinline__ int hidden(int j)
+{
+    asm volatile("" : "+v"(j));
+    return j;
+}
+
+// A global address that is the same for the whole wavefront, in scalar
+// registers (the sum of a field's base, a row and a thread's offset would
+// otherwise be formed the other way round: a 64-bit vector address for each
+// row).
+typedef __attribute__((address_space(1))) char gchar;
+__device__ __forceinline__ gchar *uniform_address(const void *p)
+{
+    const uint64_t v = (uint64_t)(uintptr_t)p;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (gchar *)(((uint64_t)hi << 32) | lo);
+}
+
+// This thread's 8 points of a column (ColX order): rows j + TPL s.  p is the
+// same for the whole block (its first row and column), off this thread's byte
+// offset from it (under 4 GB: an eighth of a field), so that an address is a
+// scalar base and one 32-bit register however many rows and fields there are.
+template <bool NT, typename T>
+__device__ __forceinline__ void col_load(cpx<T> *v, const cpx<T> *p, size_t step, uint32_t off)
+{
+    typedef __attribute__((address_space(1))) const vec2<T> gvec;
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        gvec *q = (gvec *)(uniform_address(p + s * step) + off);
+        vec2<T> x;
+        if constexpr (NT) x = __builtin_nontemporal_load(q);
+        else x = *q;
+        v[s] = mk<T>(x.x, x.y);
+    }
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void col_store(const cpx<T> *v, cpx<T> *p, size_t step, uint32_t off)
+{
+    typedef __attribute__((address_space(1))) vec2<T> gvec;
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        gvec *q = (gvec *)(uniform_address(p + s * step) + off);
+        vec2<T> x;
+        x.x = v[s].x;
+        x.y = v[s].y;
+        if constexpr (NT) __builtin_nontemporal_store(x, q);
+        else *q = x;
+    }
+}
+
+// The CB columns of a block of an x pass, thread t on column t % CB at rows
+// t / CB + TPL s.  Tiles of at most 128-byte rows divide nzp and lie within one
+// ky row, the same for the whole block; the wider ones of short lines do not,
+// and the last one may run past the last column (those threads move the last
+// column and store nothing).  Columns of the work fields (padded layout, T or
+// FP64) are at base + cw0 with byte offsets offt / offw and row step stepw, of
+// the state (boundary layout, FP64) at base + state0 with offs and steps.
+template <typename T, int L, int CB>
+struct ColTile {
+    static constexpr int TPL = L / 8;
+    static constexpr bool WIDE = CB * sizeof(cpx<T>) > 128;
+    int c, j, ly, lz, lz0, cw0;
+    bool inside, live;   // a column of the tile; one that holds modes (pad columns carry zeros)
+    size_t stepw, steps, state0;
+    uint32_t offt, offw, offs;
+
+    // patch: the kz = 0 and Nz/2 columns of every ky (bases at the fields' start)
+    __device__ __forceinline__ ColTile(const Grid &g, int tile, bool patch = false)
+    {
+        c = threadIdx.x % CB;
+        j = threadIdx.x / CB;
+        const int ncol = g.ny * g.nzp;
+        if (patch) {
+            const int p = tile * CB + c, q = min(p, 2 * g.ny - 1);
+            inside = live = p < 2 * g.ny;
+            ly = q >> 1;
+            lz = q & 1 ? g.nz / 2 : 0;
+            lz0 = cw0 = 0;
+            state0 = 0;
+            stepw = (size_t)TPL * ncol;
+            steps = (size_t)TPL * g.ny * g.nzc;
+            const uint32_t cw = (uint32_t)((size_t)j * ncol + ly * g.nzp + lz);
+            offt = cw * (uint32_t)sizeof(cpx<T>);
+            offw = cw * 16u;
+            offs = (uint32_t)((size_t)j * g.ny * g.nzc + ly * g.nzc + lz) * 16u;
+            return;
+        }
+        cw0 = tile * CB;
+        const int cwt = WIDE ? min(cw0 + c, ncol - 1) : cw0;
+        inside = !WIDE || cw0 + c < ncol;
+        ly = cwt / g.nzp;
+        lz0 = WIDE ? 0 : cwt % g.nzp;
+        lz = WIDE ? cwt % g.nzp : lz0 + c;
+        live = inside && lz < g.nzc;
+        const size_t ncw = (size_t)ncol, ncs = (size_t)g.ny * g.nzc;
+        stepw = (size_t)TPL * ncw;
+        steps = (size_t)TPL * ncs;
+        state0 = WIDE ? 0 : (size_t)ly * g.nzc + min(lz0, g.nzc - 1);
+        const uint32_t colt = WIDE ? cwt - cw0 : c;
+        offt = (uint32_t)(j * ncw + colt) * (uint32_t)sizeof(cpx<T>);
+        offw = (uint32_t)(j * ncw + colt) * 16u;
+        // (a pad column reads the last one; a tile may hold pad columns only)
+        offs = (uint32_t)(j * ncs + (WIDE ? ly * g.nzc + min(lz, g.nzc - 1) : max(min(c, g.nzc - 1 - lz0), 0))) * 16u;
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Direct-to-LDS staging of an x tile (global_load_lds_dwordx4): the L x CB
