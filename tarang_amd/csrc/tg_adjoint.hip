@@ -28,90 +28,78 @@ struct XsymArgs {
     Grid g;
 };
 
-// From the cotangent G of a tile (put(k) stages component k of G into the
-// LDS tile in the stage_in layout): M = P G, the five symmetrised fields
+// From a column's cotangent m (consumed): M = P G, the five symmetrised fields
 // xx, yy, xy, yz, zx of (-i K_m M_j - i K_j M_m)/c (zz = -xx - yy), their
-// x-inverse, stored into S.
-template <typename T, int L, int CB, typename Put>
-__device__ __forceinline__ void xsym_tile(const Grid &g, char *raw, const int *colw, const cpx<T> *tw,
-                                          void *const *S, Put put)
+// x-inverse, stored into S.  Pad columns carry zeros.
+template <bool NT, typename T, int L, int CB>
+__device__ __forceinline__ void xsym_columns(const Grid &g, const ColTile<T, L, CB> &t, const ColX<T, L, CB> &x,
+                                             const cpx<T> *tw, void *const *S, cpx<double> (*m)[8])
 {
     constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    cpx<double> *ldd = (cpx<double> *)raw;
-    cpx<T> *ldt = (cpx<T> *)raw;
-    const int c = threadIdx.x / TPL, j = threadIdx.x % TPL;
-    const int cw = colw[c];
-    const int ly = cw >= 0 ? cw / g.nzp : 0, lz = cw >= 0 ? cw % g.nzp : 0;
-    const double Ky = kwave(ly, g.ny) * g.kf[1], Kz = lz * g.kf[2];
-    const int ncw = g.ny * g.nzp;
-    cpx<double> m[3][8];
+    constexpr bool NTW = NT && CB * sizeof(cpx<T>) >= 128;
+    const double Ky = kwave(t.ly, g.ny) * g.kf[1], Kz = t.lz * g.kf[2];
+    {
+        // M = P G (Pressure.cc:56-72 form: G - K (K.G)/K^2, identity at K = 0)
+        const int jh = hidden(t.j);
 #pragma unroll
-    for (int comp = 0; comp < 3; comp++) {
-        put(comp);
-        lds_barrier();
-#pragma unroll
-        for (int s = 0; s < 8; s++) m[comp][s] = ldd[c * LP + lpad(j + TPL * s)];
-        lds_barrier();
-    }
-    // M = P G (Pressure.cc:56-72 form: G - K (K.G)/K^2, identity at K = 0)
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const double Kx = kwave(j + TPL * s, g.nx) * g.kf[0];
-        const double ks = (Kx * Kx + Ky * Ky) + Kz * Kz;
-        if (ks > 0.0) {
-            cpx<double> d = Kx * m[0][s];
-            d = d + Ky * m[1][s];
-            d = d + Kz * m[2][s];
-            const cpx<double> e = mk<double>(d.x / ks, d.y / ks);
-            m[0][s] = m[0][s] - Kx * e;
-            m[1][s] = m[1][s] - Ky * e;
-            m[2][s] = m[2][s] - Kz * e;
+        for (int s = 0; s < 8; s++) {
+            const double Kx = kwave(jh + TPL * s, g.nx) * g.kf[0];
+            const double ks = (Kx * Kx + Ky * Ky) + Kz * Kz;
+            if (ks > 0.0) {
+                cpx<double> d = Kx * m[0][s];
+                d = d + Ky * m[1][s];
+                d = d + Kz * m[2][s];
+                const cpx<double> e = mk<double>(d.x / ks, d.y / ks);
+                m[0][s] = m[0][s] - Kx * e;
+                m[1][s] = m[1][s] - Ky * e;
+                m[2][s] = m[2][s] - Kz * e;
+            }
+            settle(m[0][s]);
+            settle(m[1][s]);
+            settle(m[2][s]);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    const double w = (lz == 0 || lz == g.nz / 2) ? 1.0 : 0.5;
+    const double w = !t.live ? 0.0 : (t.lz == 0 || t.lz == g.nz / 2) ? 1.0 : 0.5;
     constexpr int pa[5] = {0, 1, 0, 1, 2};
     constexpr int pb[5] = {0, 1, 1, 2, 0};
 #pragma unroll
-    for (int t = 0; t < 5; t++) {
+    for (int p = 0; p < 5; p++) {
         cpx<T> v[8];
+        const int jh = hidden(t.j);
 #pragma unroll
         for (int s = 0; s < 8; s++) {
-            const double Kx = kwave(j + TPL * s, g.nx) * g.kf[0];
+            const double Kx = kwave(jh + TPL * s, g.nx) * g.kf[0];
             const double K[3] = {Kx, Ky, Kz};
-            const cpx<double> A = m[pa[t]][s], B = m[pb[t]][s];
+            const cpx<double> A = m[pa[p]][s], B = m[pb[p]][s];
             // -i K_b A - i K_a B, times 1/c
-            const double re = K[pb[t]] * A.y + K[pa[t]] * B.y;
-            const double im = -(K[pb[t]] * A.x + K[pa[t]] * B.x);
-            v[s] = (cw >= 0) ? mk<T>((T)(w * re), (T)(w * im)) : mk<T>(0, 0);
+            const double re = K[pb[p]] * A.y + K[pa[p]] * B.y;
+            const double im = -(K[pb[p]] * A.x + K[pa[p]] * B.x);
+            v[s] = mk<T>((T)(w * re), (T)(w * im));
         }
-        fft_line<L, +1>(v, ldt + c * LP, tw, j);
-#pragma unroll
-        for (int s = 0; s < 8; s++) ldt[c * LP + lpad(j + TPL * s)] = v[s];
-        lds_barrier();
-        stage_out<L, CB>(ldt, (cpx<T> *)S[t], colw, ncw);
-        lds_barrier();
+        fft_exchange<L, +1>(v, x, tw, jh);
+        pin_memory_order();
+        if (t.inside) col_store<NTW>(v, (cpx<T> *)S[p] + t.cw0, t.stepw, t.offt);
     }
 }
 
-template <typename T, int L, int CB>
-__global__ void __launch_bounds__(CB *(L / 8)) k_xinv_sym(XsymArgs a)
+// Column tiles in registers in transform order (ColX), as k_xfwd_adj.
+template <typename T, int L, int CB, bool NT>
+__global__ void __launch_bounds__(CB *(L / 8), 2) k_xinv_sym(XsymArgs a)
 {
-    constexpr int LP = lpad_len(L);
-    __shared__ __attribute__((aligned(16))) char raw[CB * LP * sizeof(cpx<double>)];
-    __shared__ int colw[CB], cols[CB];
+    using X = ColX<T, L, CB>;
+    __shared__ cpx<T> lds[X::SIZE];
+    __shared__ cpx<T> tw[L];
     const Grid &g = a.g;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     if (tile >= x_tiles(g, CB, false)) return;
-    tile_columns<CB>(colw, cols, g, false, tile);
-    lds_barrier();
-    const int ncs = g.ny * g.nzc;
-    // the three cotangent tiles' loads are in flight together
-    cpx<double> gr[3][8];
+    const ColTile<T, L, CB> t(g, tile);
+    cpx<double> m[3][8];
 #pragma unroll
-    for (int comp = 0; comp < 3; comp++) stage_load<L, CB>(gr[comp], (const cpx<double> *)a.G[comp], cols, ncs);
-    xsym_tile<T, L, CB>(g, raw, colw, (const cpx<T> *)a.tw, a.S,
-                        [&](int k) { stage_put<L, CB>((cpx<double> *)raw, gr[k], cols); });
+    for (int c = 0; c < 3; c++) col_load<false>(m[c], (const cpx<double> *)a.G[c] + t.state0, t.steps, t.offs);
+    for (int i = threadIdx.x; i < L; i += CB * (L / 8)) tw[i] = ((const cpx<T> *)a.tw)[i];
+    lds_barrier();
+    xsym_columns<NT>(g, t, X{lds + t.c}, tw, a.S, m);
 }
 
 // q += u * v (SUB: q -= u * v) on the packed real points of this thread (u
@@ -191,106 +179,103 @@ struct XadjArgs {
 
 // FUSE: the next stage's cotangent (lg, or lam after the step's last stage)
 // stays in registers instead of going through HBM, and the next stage's
-// xsym_tile runs on it here (lg is not stored).
-template <typename T, int L, int CB, bool FUSE>
-__global__ void __launch_bounds__(CB *(L / 8)) k_xfwd_adj(XadjArgs a)
+// xsym_columns runs on it here (lg is not stored).
+// Bound by HBM: columns go from memory to registers and back in transform
+// order, one instance per mode (its loads and factors only); with the tiles
+// staged through LDS a launch at 256^3 FP64 took 732 us, now 590 (S1; 4.0 TB/s).
+template <typename T, int L, int CB, int MODE, bool FUSE, bool NT>
+__global__ void __launch_bounds__(CB *(L / 8), 2) k_xfwd_adj(XadjArgs a)
 {
-    constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    __shared__ __attribute__((aligned(16))) char raw[CB * LP * sizeof(cpx<double>)];
-    __shared__ int colw[CB], cols[CB];
-    cpx<double> *ldd = (cpx<double> *)raw;
-    cpx<T> *ldt = (cpx<T> *)raw;
+    constexpr int TPL = L / 8, NTH = CB * TPL;
+    constexpr bool NTW = NT && CB * sizeof(cpx<T>) >= 128;
+    constexpr bool NEED_L = MODE != ADJ_RHS, NEED_A = MODE == ADJ_S2 || MODE == ADJ_S1 || MODE == ADJ_S0;
+    constexpr bool EH = MODE == ADJ_S3 || MODE == ADJ_S2 || MODE == ADJ_S1, E1 = MODE == ADJ_S1 || MODE == ADJ_S0;
+    using X = ColX<T, L, CB>;
+    __shared__ cpx<T> lds[X::SIZE];
+    __shared__ cpx<T> tw[L];
+    // exp(-nu K^2 dt/2) and exp(-nu K^2 dt) at this thread's points
+    __shared__ double visc[(EH ? 1 : 0) + (E1 ? 1 : 0) + (EH || E1 ? 0 : 1)][8 * NTH];
     const Grid &g = a.g;
     const AdjParams &ap = a.ap;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     if (tile >= x_tiles(g, CB, false)) return;
-    tile_columns<CB>(colw, cols, g, false, tile);
-    lds_barrier();
-    const int c = threadIdx.x / TPL, j = threadIdx.x % TPL;
-    const cpx<T> *tw = (const cpx<T> *)a.tw;
-    const int ncw = g.ny * g.nzp, ncs = g.ny * g.nzc;
-    const double c_sixth = (1.0 / 6) * ap.dt, c_third = (1.0 / 3) * ap.dt, c_half = 0.5 * ap.dt;
-    cpx<double> gn[3][8];  // FUSE: next cotangent, stage_in layout
-#pragma unroll
-    for (int comp = 0; comp < 3; comp++) {
-#pragma unroll
-        for (int ii = 0; ii < 8; ii++) gn[comp][ii] = mk<double>(0, 0);
-        stage_in<L, CB>(ldt, (const cpx<T> *)a.Q[comp], colw, ncw);
-        lds_barrier();
-        cpx<T> v[8];
-#pragma unroll
-        for (int s = 0; s < 8; s++) v[s] = ldt[c * LP + lpad(j + TPL * s)];
-        lds_barrier();
-        fft_line<L, -1>(v, ldt + c * LP, tw, j);
-        lds_barrier();
-#pragma unroll
-        for (int s = 0; s < 8; s++) ldd[c * LP + lpad(j + TPL * s)] = ap.scale * cvt<double>(v[s]);
-        lds_barrier();
-        cpx<double> *lam = (cpx<double> *)a.lam[comp], *acc = (cpx<double> *)a.acc[comp];
-        cpx<double> *lg = (cpx<double> *)a.lg[comp];
-        // thread t: column t % CB, rows t / CB + TPL i; the eight elements'
-        // inputs are loaded before the first result is stored
-        const int cc = threadIdx.x % CB, r0 = threadIdx.x / CB, col = cols[cc];
-        if (col >= 0) {
-            const int ly = col / g.nzc, lz = col % g.nzc;
-            const double cw = (lz == 0 || lz == g.nz / 2) ? -1.0 : -2.0;
-            const double Ky = kwave(ly, g.ny) * g.kf[1], Kz = lz * g.kf[2];
-            const bool need_l = ap.mode != ADJ_RHS;
-            const bool need_a = ap.mode == ADJ_S2 || ap.mode == ADJ_S1 || ap.mode == ADJ_S0;
-            cpx<double> l4[8], a4[8];
-#pragma unroll
-            for (int ii = 0; ii < 8; ii++) {
-                const size_t i = (size_t)(r0 + TPL * ii) * ncs + col;
-                l4[ii] = need_l ? mk<double>(lam[i].x, lam[i].y) : mk<double>(0, 0);
-                a4[ii] = need_a ? mk<double>(acc[i].x, acc[i].y) : mk<double>(0, 0);
-            }
-#pragma unroll
-            for (int ii = 0; ii < 8; ii++) {
-                const int lx = r0 + TPL * ii;
-                const size_t i = (size_t)lx * ncs + col;
-                cpx<double> r = ldd[cc * LP + lpad(lx)];
-                r = dealias_zero(g, lx, ly, lz) ? mk<double>(0, 0) : cw * r;
-                if (ap.mode == ADJ_RHS) {
-                    lg[i] = r;
-                    continue;
-                }
-                const double Kx = kwave(lx, g.nx) * g.kf[0];
-                const double ks = (Kx * Kx + Ky * Ky) + Kz * Kz;
-                cpx<double> nx;
-                if (ap.mode == ADJ_S3) {
-                    const double Eh = visc_exp(ap.fh, ap.fhh, ap.hq, ks);
-                    const cpx<double> lv = c_sixth * r;
-                    acc[i] = (Eh * Eh) * lv;
-                    nx = c_third * (Eh * l4[ii]) + ap.dt * (Eh * lv);
-                } else if (ap.mode == ADJ_S2) {
-                    const double Eh = visc_exp(ap.fh, ap.fhh, ap.hq, ks);
-                    acc[i] = a4[ii] + Eh * r;
-                    nx = c_third * (Eh * l4[ii]) + c_half * r;
-                } else if (ap.mode == ADJ_S1) {
-                    const double Eh = visc_exp(ap.fh, ap.fhh, ap.hq, ks), E1 = visc_exp(ap.f1, ap.f1h, ap.hq, ks);
-                    acc[i] = a4[ii] + Eh * r;
-                    nx = c_sixth * (E1 * l4[ii]) + c_half * (Eh * r);
-                } else {
-                    const double E1 = visc_exp(ap.f1, ap.f1h, ap.hq, ks);
-                    nx = (E1 * l4[ii] + a4[ii]) + r;
-                    lam[i] = nx;
-                }
-                if (ap.mode != ADJ_S0 && !FUSE) lg[i] = nx;
-                if constexpr (FUSE) gn[comp][ii] = nx;
-            }
+    const ColTile<T, L, CB> t(g, tile);
+    const int j = t.j;
+    cpx<T> v[8];
+    cpx<double> lm[8], ac[8];
+    col_load<NTW>(v, (const cpx<T> *)a.Q[0] + t.cw0, t.stepw, t.offt);
+    if (NEED_L) col_load<false>(lm, (const cpx<double> *)a.lam[0] + t.state0, t.steps, t.offs);
+    if (NEED_A) col_load<false>(ac, (const cpx<double> *)a.acc[0] + t.state0, t.steps, t.offs);
+    for (int i = threadIdx.x; i < L; i += NTH) tw[i] = ((const cpx<T> *)a.tw)[i];
+    if (EH || E1) {
+        const double Ky = kwave(t.ly, g.ny) * g.kf[1], Kz = t.lz * g.kf[2];
+#pragma unroll 2
+        for (int s = 0; s < 8; s++) {
+            const double Kx = kwave(j + TPL * s, g.nx) * g.kf[0];
+            const double ks = (Kx * Kx + Ky * Ky) + Kz * Kz;
+            const double kp = hyper_power(ap.hq, ks);
+            if (EH) visc[0][s * NTH + threadIdx.x] = exp((ap.fh + ap.fhh * kp) * ks);
+            if (E1) visc[EH ? 1 : 0][s * NTH + threadIdx.x] = exp((ap.f1 + ap.f1h * kp) * ks);
         }
-        lds_barrier();
     }
-    if constexpr (FUSE)
-        xsym_tile<T, L, CB>(g, raw, colw, tw, a.S, [&](int k) { stage_put<L, CB>(ldd, gn[k], cols); });
+    lds_barrier();
+    const X x{lds + t.c};
+    int zx0, zx1;
+    dealias_rows(g, t.ly, t.lz, zx0, zx1);
+    const double cw = (t.lz == 0 || t.lz == g.nz / 2) ? -1.0 : -2.0;
+    const double c_sixth = (1.0 / 6) * ap.dt, c_third = (1.0 / 3) * ap.dt, c_half = 0.5 * ap.dt;
+    cpx<double> gn[3][8];   // the next cotangent
+#pragma unroll
+    for (int K = 0; K < 3; K++) {
+        const int jh = hidden(j);
+        fft_exchange<L, -1>(v, x, tw, jh);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const int lx = jh + TPL * s;
+            cpx<double> r = ap.scale * cvt<double>(v[s]);
+            r = lx >= zx0 && lx <= zx1 ? mk<double>(0, 0) : cw * r;
+            const double Eh = EH ? visc[0][s * NTH + threadIdx.x] : 0.0;
+            const double Ef = E1 ? visc[EH ? 1 : 0][s * NTH + threadIdx.x] : 0.0;
+            cpx<double> nx;
+            if constexpr (MODE == ADJ_RHS) {
+                nx = r;
+            } else if constexpr (MODE == ADJ_S3) {
+                const cpx<double> lv = c_sixth * r;
+                ac[s] = (Eh * Eh) * lv;
+                nx = c_third * (Eh * lm[s]) + ap.dt * (Eh * lv);
+            } else if constexpr (MODE == ADJ_S2) {
+                ac[s] = ac[s] + Eh * r;
+                nx = c_third * (Eh * lm[s]) + c_half * r;
+            } else if constexpr (MODE == ADJ_S1) {
+                ac[s] = ac[s] + Eh * r;
+                nx = c_sixth * (Ef * lm[s]) + c_half * (Eh * r);
+            } else {
+                nx = (Ef * lm[s] + ac[s]) + r;
+            }
+            gn[K][s] = nx;
+            settle(gn[K][s]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        pin_memory_order();
+        if (K < 2) col_load<NTW>(v, (const cpx<T> *)a.Q[K < 2 ? K + 1 : 2] + t.cw0, t.stepw, t.offt);
+        if (NEED_L && K < 2) col_load<false>(lm, (const cpx<double> *)a.lam[K < 2 ? K + 1 : 2] + t.state0, t.steps, t.offs);
+        if (t.live) {
+            if (EH) col_store<false>(ac, (cpx<double> *)a.acc[K] + t.state0, t.steps, t.offs);
+            if (MODE == ADJ_S0) col_store<false>(gn[K], (cpx<double> *)a.lam[K] + t.state0, t.steps, t.offs);
+            else if (!FUSE) col_store<false>(gn[K], (cpx<double> *)a.lg[K] + t.state0, t.steps, t.offs);
+        }
+        if (NEED_A && K < 2) col_load<false>(ac, (const cpx<double> *)a.acc[K < 2 ? K + 1 : 2] + t.state0, t.steps, t.offs);
+        pin_memory_order();
+    }
+    if constexpr (FUSE) xsym_columns<NT>(g, t, x, tw, a.S, gn);
 }
 
 template <typename T, int LL>
 hipError_t xinv_sym_len(const XsymArgs &a, hipStream_t st)
 {
-    constexpr int CB = col_block<T>(LL, sizeof(cpx<double>));
-    hipLaunchKernelGGL((k_xinv_sym<T, LL, CB>), dim3(x_grid(x_tiles(a.g, CB, false))), dim3(CB * (LL / 8)), 0, st, a);
+    constexpr int CB = colx_block<T>(LL, 512);
+    hipLaunchKernelGGL((k_xinv_sym<T, LL, CB, false>), dim3(x_grid(x_tiles(a.g, CB, false))), dim3(CB * (LL / 8)), 0, st, a);
     return hipGetLastError();
 }
 
@@ -307,14 +292,32 @@ hipError_t z_adj_len(const ZArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
+template <typename T, int LL, int MODE, bool FUSE>
+hipError_t xfwd_adj_launch(const XadjArgs &a, hipStream_t st)
+{
+    constexpr int CB = colx_block<T>(LL, 512);
+    const bool nt = stream_bytes((size_t)8 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
+    constexpr bool NT = FUSE && LL >= kStreamLength;
+    const dim3 grid(x_grid(x_tiles(a.g, CB, false))), block(CB * (LL / 8));
+    if (NT && nt) hipLaunchKernelGGL((k_xfwd_adj<T, LL, CB, MODE, FUSE, NT>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_xfwd_adj<T, LL, CB, MODE, FUSE, false>), grid, block, 0, st, a);
+    return hipGetLastError();
+}
+
+// Only the last stage of a sweep and ADJ_RHS end without a next stage.
 template <typename T, int LL>
 hipError_t xfwd_adj_len(const XadjArgs &a, bool fuse, hipStream_t st)
 {
-    constexpr int CB = col_block<T>(LL, sizeof(cpx<double>));
-    const dim3 grid(x_grid(x_tiles(a.g, CB, false))), block(CB * (LL / 8));
-    if (fuse) hipLaunchKernelGGL((k_xfwd_adj<T, LL, CB, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((k_xfwd_adj<T, LL, CB, false>), grid, block, 0, st, a);
-    return hipGetLastError();
+    if (a.ap.mode == ADJ_RHS && !fuse) return xfwd_adj_launch<T, LL, ADJ_RHS, false>(a, st);
+    if (a.ap.mode == ADJ_S0 && !fuse) return xfwd_adj_launch<T, LL, ADJ_S0, false>(a, st);
+    if (!fuse) return hipErrorInvalidValue;
+    switch (a.ap.mode) {
+        case ADJ_S0: return xfwd_adj_launch<T, LL, ADJ_S0, true>(a, st);
+        case ADJ_S1: return xfwd_adj_launch<T, LL, ADJ_S1, true>(a, st);
+        case ADJ_S2: return xfwd_adj_launch<T, LL, ADJ_S2, true>(a, st);
+        case ADJ_S3: return xfwd_adj_launch<T, LL, ADJ_S3, true>(a, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 #define TG_ADJ_L(N, T, P)                                                     \

@@ -38,3 +38,87 @@ def test_mhd_steps(N, prec):
             o.rk4_step_mhd(fl, eta, V, W)
         assert rel_l2_vec([host(v) for v in U.cvf] + [host(w) for w in B.cvf], V + W) <= TOL[prec]
         b.close()
+
+
+def _spec(shape, seed, real_mean):
+    """A smooth random spectrum with the conjugate symmetry left to the step."""
+    r = np.random.default_rng(seed)
+    k = [np.arange(shape[0]), np.minimum(np.arange(shape[1]), shape[1] - np.arange(shape[1])), np.arange(shape[2])]
+    w = np.exp(-0.5 * (k[0][:, None, None] + k[1][None, :, None] + k[2][None, None, :]))
+    s = 0.1 * w * (r.standard_normal(shape) + 1j * r.standard_normal(shape))
+    if real_mean:
+        s[0] = 0.0
+    return s
+
+
+@pytest.mark.parametrize("N,prec", [g for g in GRIDS if g[0][0] <= 640])
+def test_rbc_steps(N, prec):
+    log(f"rbc {N} {prec}")
+    for dealias, reality in ((to.DEALIAS_REF_CORNER, 2), (to.DEALIAS_TWOTHIRDS, 0)):
+        o = to.Oracle(N, kfactor=(np.pi, 1.5, 1.0), dealias=dealias, strong_reality=False)
+        V = [_spec(o.cshape, 50 + c, c == 0) for c in range(3)]
+        T = _spec(o.cshape, 53, True)
+        b = api.SFF_Basis(N, kfactor=(np.pi, 1.5, 1.0), precision=prec, dealias=dealias, reality=reality)
+        U, S = api.FluidVF(b), api.FluidSF(b)
+        U.set_field([dev(v) for v in V])
+        S.set_field(dev(T))
+        api.Time_advance_incompress_RBC(U, S, 1e4, 1.0, 1e-5).Time_advance_step(2)
+        for _ in range(2):
+            o.rk4_step_rbc(to.Rbc(1e4, 1.0, 1e-5, reality), V, T)
+        # the long lines' x-derivatives multiply round-off by K_max = pi L
+        tol = TOL[prec] * max(1.0, (np.pi * N[0] / 1000.0) ** 2)
+        assert rel_l2_vec([host(v) for v in U.cvf] + [host(S.F)], V + [T]) <= tol
+        b.close()
+
+
+@pytest.mark.parametrize("N,prec", GRIDS)
+def test_adjoint_sweep(N, prec):
+    """Two forward steps and the sweep back: each mode of the fused x pass."""
+    log(f"adjoint {N} {prec}")
+    o = to.Oracle(N, dealias=to.DEALIAS_REF_CORNER, strong_reality=False)
+    V = o.init_field(kind=1, kmin=1.0, kmax=max(N) / 3, energy=0.5, seed=41)
+    r_lo, r_hi = 0.5, 5.0
+    loss_ref, grad_ref = o.adjoint_shell_energy(to.Fluid(0.01, 1e-3, 0, 0.0, 0.0, 0.0), V, 2, r_lo, r_hi)
+    b = api.FFF_Basis(N, precision=prec, strong_reality=False)
+    U = api.FluidVF(b, 0.01)
+    U.set_field([dev(v) for v in V])
+    adj = api.Adjoint_incompress(U, 1e-3)
+    adj.Forward(2)
+    k = [np.minimum(np.arange(n), n - np.arange(n)) for n in N[:2]] + [np.arange(N[2] // 2 + 1)]
+    K = np.sqrt(k[0][:, None, None] ** 2.0 + k[1][None, :, None] ** 2 + k[2][None, None, :] ** 2)
+    # the oracle's loss: the energy of the shell, the kz = 0 plane at half weight
+    m = ((K >= r_lo) & (K < r_hi)).astype(np.float64)
+    m[:, :, 0] *= 0.5
+    m = torch.as_tensor(m, device="cuda")
+    lam = [2.0 * m * v for v in U.cvf]
+    adj.Backward(lam)
+    # the bounds of the gradient tests: 1e-11, FP32 transforms 2e-5
+    assert rel_l2_vec([host(x) for x in lam], grad_ref) <= (1e-11 if prec == api.PREC_FP64 else 2e-5)
+    b.close()
+
+
+@pytest.mark.parametrize("N,prec", GRIDS)
+def test_transforms_keep_and_drop_modes(N, prec):
+    """The plain x passes on a random spectrum: transforms, the shell filter of
+    the transfer functions (columns without a mode to keep are not read)."""
+    log(f"transforms {N} {prec}")
+    tol = 1e-12 if prec == api.PREC_FP64 else 1e-5
+    o = to.Oracle(N)
+    b = api.FFF_Basis(N, precision=prec)
+    r = np.random.default_rng(1).standard_normal(o.rshape)
+    r[:, :, -2:] = 0.0
+    A, Ar = b.complex_array(), b.real_array()
+    b.Forward_transform(dev(r), A)
+    b.Inverse_transform(A, Ar)
+    assert rel_l2(host(A), o.forward(r)) <= tol and rel_l2(host(Ar), r) <= tol
+    if prec == api.PREC_FP32:
+        b.close()
+        return
+    V = o.init_field(kind=1, kmin=1.0, kmax=max(N) / 3, energy=0.5, seed=7)
+    radii = np.array([0.0, 1.5, 3.0, np.inf])
+    U = api.FluidVF(b)
+    U.set_field([dev(v) for v in V])
+    got = api.EnergyTr(b, radii, radii).Compute_shell_tr(U)
+    want = o.shell_to_shell([v.copy() for v in V], radii)
+    assert rel_l2(got, want) <= 1e-11
+    b.close()
