@@ -1009,7 +1009,6 @@ int run_rk4_rbc(tg_plan *p, double *const V[3], double *T_, const tg_rbc *r, int
             const double *f_in[2] = {s == 1 ? T_ : p->rbc[1 + 2 * rd], s == 1 ? V[0] : p->rbc[2 + 2 * rd]};
             double *f_out[2] = {p->rbc[1 + 2 * wr], p->rbc[2 + 2 * wr]};
             RbcParams rp = rbc_params(p, r, s);
-            rp.trace_free = 1;
             if (s == 4) rp.nonfinite = p->nonfinite_dev;
             Prof pr(p, TG_KERNEL_X_RBC);
             HIPCHK(launch_x_rbc<T>(p->g, rp, p->P, S, acc, p->U, f_in, f_out, nullptr, p->twx, p->twq, p->stream));

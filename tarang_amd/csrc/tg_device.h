@@ -247,30 +247,13 @@ inline void twiddle_order(int L, int *order)
 // data between threads through LDS alone, so their barriers need not wait
 // for global memory: __syncthreads' fence waits for every outstanding global
 // load and store (stores count in vmcnt on this architecture, so each
-// barrier after a tile store would wait out the write acknowledgements) and
-// for direct-to-LDS loads in flight.  Direct-to-LDS tiles are waited for
-// explicitly (dma_wait) before the barrier that publishes them.
+// barrier after a tile store would wait out the write acknowledgements, and
+// the next tile's loads in flight).
 __device__ __forceinline__ void lds_barrier()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// lds_barrier for a point where a direct-to-LDS load into a tile that no
-// thread touches until its own wait is in flight: the workgroup-scope release
-// fence would wait for that load too (it counts as a pending LDS write).  The
-// wave's own LDS instructions are complete before it reaches the barrier
-// (s_waitcnt lgkmcnt(0)), as with the workgroup fence, and the
-// wavefront-scope fences keep the compiler from moving LDS accesses across
-// the barrier; the direct-to-LDS tile is published later by its own wait
-// (dma_wait) and an lds_barrier.
-__device__ __forceinline__ void lds_barrier_async()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt and expcnt at their maxima
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
 // Synchronisation of the threads that share one line.  A line of L points

@@ -29,31 +29,6 @@ struct MhdArgs {
     Grid g;
 };
 
-// Lawson stage ST of one mode: the accumulator ac (stage 4: the new state),
-// the next stage input vn; E = exp(-nu K^2 dt/2), stage 4 exp(-nu K^2 dt), E1
-// (stage 1) exp(-nu K^2 dt).
-template <int ST>
-__device__ __forceinline__ void lawson(const cpx<double> &v0in, const cpx<double> &r, double E, double E1, double dt,
-                                       cpx<double> &ac, cpx<double> &vn)
-{
-    const double c_half = 0.5 * dt, c_one = 1.0 * dt;
-    const double c_sixth = (1.0 / 6) * dt, c_third = (1.0 / 3) * dt;
-    if constexpr (ST == 1) {
-        ac = c_sixth * (E1 * r);
-        vn = E * (v0in + c_half * r);
-    } else if constexpr (ST == 2) {
-        ac = ac + c_third * (E * r);
-        vn = E * v0in + c_half * r;
-    } else if constexpr (ST == 3) {
-        ac = ac + c_third * (E * r);
-        vn = E * (E * v0in + c_one * r);
-    } else {
-        ac = ac + c_sixth * r;
-        vn = E * v0in + ac;
-        ac = vn;
-    }
-}
-
 // x-inverse of Z- = D(u) - D(b) and Z+ = D(u) + D(b) into U[0..2] and U[3..5]
 // (stage-1 input, Compute_nlin), straight from the state: forming Z+- in
 // fields of their own first took 2.7 + 3.3 ms at 512^3 FP32 transforms.
@@ -147,7 +122,7 @@ constexpr int mhd_index(int pi)
 // flight, products unrolled, code per stage, values settled where they are
 // formed.  The six sums take 192 registers in FP64: 256-thread blocks there
 // (512 registers a thread), 512-thread blocks in FP32.  512^3 FP32, per launch:
-// 11.0 ms, now 5.1 in stage 1, 5.9 in stages 2 and 3 (4.8 TB/s), 8.1 in stage 4.
+// 11.0 ms, now 5.1 in stage 1, 5.9 in stages 2 and 3 (4.8 TB/s), 7.1 in stage 4.
 template <typename T, int L, int CB, int ST, bool NT>
 __global__ void __launch_bounds__(CB *(L / 8), sizeof(T) == 8 ? 1 : 2) k_x_mhd(XmhdArgs a)
 {
@@ -298,9 +273,13 @@ __global__ void __launch_bounds__(CB *(L / 8), sizeof(T) == 8 ? 1 : 2) k_x_mhd(X
                 if (ST == 1 && z) w[s] = mk<double>(0, 0);
                 const double E1 = ST == 1 ? exp(a.f1_u * ksq(lx)) : 0.0;
                 lawson<ST>(w[s], cvt<double>(Np[K][s]), visc[0][s * NTH + threadIdx.x], E1, a.dt, ac[s], un[s]);
-                if (ST == 4) chk += 0.0 * un[s].x + 0.0 * un[s].y;
+                if (ST == 4) {
+                    chk += 0.0 * un[s].x + 0.0 * un[s].y;
+                    settle(chk);
+                }
                 if (z) un[s] = mk<double>(0, 0);
                 settle(un[s]);
+                settle(ac[s]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -323,12 +302,16 @@ __global__ void __launch_bounds__(CB *(L / 8), sizeof(T) == 8 ? 1 : 2) k_x_mhd(X
                 const double E1 = ST == 1 ? exp(a.f1_b * ksq(lx)) : 0.0;
                 cpx<double> bn;
                 lawson<ST>(w[s], cvt<double>(Nm[K][s]), visc[1][s * NTH + threadIdx.x], E1, a.dt, ac[s], bn);
-                if (ST == 4) chk += 0.0 * bn.x + 0.0 * bn.y;
+                if (ST == 4) {
+                    chk += 0.0 * bn.x + 0.0 * bn.y;
+                    settle(chk);
+                }
                 if (z) bn = mk<double>(0, 0);
                 zp[s] = cvt<T>(un[s] + bn);
                 zm[s] = cvt<T>(un[s] - bn);
                 settle(zp[s]);
                 settle(zm[s]);
+                settle(ac[s]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }

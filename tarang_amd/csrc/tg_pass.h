@@ -1,13 +1,11 @@
-// tg_pass.h -- device helpers shared by the x, y and z passes (tiling of the
-// x pass through LDS, z-line real<->complex transforms, wavenumbers and the
-// dealias mask) and the size dispatch of the launchers.
+// tg_pass.h -- device helpers shared by the x, y and z passes (column tiles of
+// the x pass, z-line real<->complex transforms, wavenumbers and the dealias
+// mask) and the size dispatch of the launchers.
 #pragma once
 #include "tg_device.h"
 #include "tg_kernels.h"
 
 namespace tg {
-
-static constexpr int kLdsBudget = 73728;  // bytes; two blocks fit the 160 KB LDS of a CU
 
 // Whether a pass over `bytes` of fields streams past the 256 MiB memory-side
 // cache, so that nothing it writes is still there for the next pass.
@@ -72,8 +70,9 @@ __device__ __forceinline__ void dealias_rows(const Grid &g, int ly, int lz, int 
     }
 }
 
-// K^(q-2) = (K^2)^((q-2)/2) of the hyperviscosity, integer division (q = 4:
-// K^2), by repeated multiplication; q = 0 (none): 1.
+// K^(q-2) = (K^2)^((q-2)/2) of the hyperviscous factor exp((f + fh K^(q-2)) K^2)
+// (Array_exp_ksqr, universal_basic.cc:265-291), integer division (q = 4: K^2),
+// by repeated multiplication; q = 0 (none): 1.
 __device__ __forceinline__ double hyper_power(int q, double ks)
 {
     const int n = q == 0 ? 0 : (q == 4 ? 1 : (q - 2) / 2);
@@ -81,15 +80,6 @@ __device__ __forceinline__ double hyper_power(int q, double ks)
 #pragma unroll 1
     for (int i = 0; i < n; i++) kp *= ks;
     return kp;
-}
-
-// Viscous factor exp(exponent) of Array_exp_ksqr: exponent f K^2, or with
-// hyperviscosity (f + fh K^(q-2)) K^2 (universal_basic.cc:265-291), K^(q-2) =
-// (K^2)^((q-2)/2) with integer division (q = 4: K^2), by repeated
-// multiplication; q = 0: none.  ks = K^2.
-__device__ __forceinline__ double visc_exp(double f, double fh, int q, double ks)
-{
-    return exp((f + fh * hyper_power(q, ks)) * ks);
 }
 
 // Columns of a ColX tile of L-point lines, a power of two: rows of 128 bytes (8
@@ -105,87 +95,39 @@ __host__ __device__ constexpr int colx_block(int L, int threads)
     return cb;
 }
 
-template <typename T>
-__host__ __device__ constexpr int col_block(int L, int elem_bytes)
-{
-    int tpl = L / 8;
-    int cb = 16;
-    while (cb > 1 && (cb * tpl > 1024 || cb * lpad_len(L) * elem_bytes > kLdsBudget)) cb /= 2;
-    return cb;
-}
-
 template <typename A, typename B>
 __device__ __forceinline__ cpx<A> cvt(cpx<B> v) { return mk<A>((A)v.x, (A)v.y); }
 
-// ---------------------------------------------------------------------------
-// x pass helpers: staging of an (Nx x CB) column tile through LDS.
-// ---------------------------------------------------------------------------
-// Thread t moves column t % CB, rows t / CB + TPL i (i < 8): consecutive
-// lanes cover the CB columns of a row.  The eight loads are issued before the
-// first LDS write (a runtime-bounded loop would wait for each load in turn);
-// a column outside the field (cols[c] < 0) loads column 0 and stages zeros.
-template <int L, int CB, typename S, typename G>
-__device__ __forceinline__ void stage_in(cpx<S> *lds, const cpx<G> *__restrict__ f, const int *cols, int ncol_total)
+// Lawson stage ST of one mode: the accumulator ac (stage 4: the new state),
+// the next stage input vn; E = exp(-nu K^2 dt/2), stage 4 exp(-nu K^2 dt), E1
+// (stage 1) exp(-nu K^2 dt).
+template <int ST>
+__device__ __forceinline__ void lawson(const cpx<double> &v0in, const cpx<double> &r, double E, double E1, double dt,
+                                       cpx<double> &ac, cpx<double> &vn)
 {
-    constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    const int c = threadIdx.x % CB, r0 = threadIdx.x / CB, col = cols[c];
-    const cpx<G> *p = f + (size_t)r0 * ncol_total + max(col, 0);
-    const size_t step = (size_t)TPL * ncol_total;
-    cpx<G> x[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) x[i] = mk<G>(p[i * step].x, p[i * step].y);
-#pragma unroll
-    for (int i = 0; i < 8; i++) lds[c * LP + lpad(r0 + TPL * i)] = col >= 0 ? cvt<S>(x[i]) : mk<S>(0, 0);
-}
-
-// stage_in in two halves, so that several tiles' loads can be in flight
-// together: stage_load fills x[8] (this thread's share), stage_put writes it
-// to LDS (zeros for a column outside the field).
-template <int L, int CB, typename G>
-__device__ __forceinline__ void stage_load(cpx<G> *x, const cpx<G> *__restrict__ f, const int *cols, int ncol_total)
-{
-    constexpr int TPL = L / 8;
-    const int c = threadIdx.x % CB, r0 = threadIdx.x / CB;
-    const cpx<G> *p = f + (size_t)r0 * ncol_total + max(cols[c], 0);
-    const size_t step = (size_t)TPL * ncol_total;
-#pragma unroll
-    for (int i = 0; i < 8; i++) x[i] = mk<G>(p[i * step].x, p[i * step].y);
-}
-
-template <int L, int CB, typename S, typename G>
-__device__ __forceinline__ void stage_put(cpx<S> *lds, const cpx<G> *x, const int *cols)
-{
-    constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    const int c = threadIdx.x % CB, r0 = threadIdx.x / CB;
-    const bool in = cols[c] >= 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) lds[c * LP + lpad(r0 + TPL * i)] = in ? cvt<S>(x[i]) : mk<S>(0, 0);
-}
-
-template <int L, int CB, typename S, typename G>
-__device__ __forceinline__ void stage_out(const cpx<S> *lds, cpx<G> *__restrict__ f, const int *cols, int ncol_total)
-{
-    constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    const int c = threadIdx.x % CB, r0 = threadIdx.x / CB, col = cols[c];
-    if (col < 0) return;
-    cpx<G> *p = f + (size_t)r0 * ncol_total + col;
-    const size_t step = (size_t)TPL * ncol_total;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const cpx<S> v = lds[c * LP + lpad(r0 + TPL * i)];
-        p[i * step] = mk<G>((G)v.x, (G)v.y);
+    const double c_half = 0.5 * dt, c_one = 1.0 * dt;
+    const double c_sixth = (1.0 / 6) * dt, c_third = (1.0 / 3) * dt;
+    if constexpr (ST == 1) {
+        ac = c_sixth * (E1 * r);
+        vn = E * (v0in + c_half * r);
+    } else if constexpr (ST == 2) {
+        ac = ac + c_third * (E * r);
+        vn = E * v0in + c_half * r;
+    } else if constexpr (ST == 3) {
+        ac = ac + c_third * (E * r);
+        vn = E * (E * v0in + c_one * r);
+    } else {
+        ac = ac + c_sixth * r;
+        vn = E * v0in + ac;
+        ac = vn;
     }
 }
 
 // Tiles of the x pass.  Work fields store each ky row of kz with the padded
 // stride nzp (a multiple of 128 bytes); the FP64 state in the boundary layout
 // uses nzc = Nz/2+1.  A tile is CB consecutive columns of the padded (ly,lz)
-// space (pad columns lz >= nzc are skipped), or -- patch tiles -- the
-// kz = 0 and kz = Nz/2 columns of every ky.  colw = ly*nzp + lz indexes the
-// work fields, cols = ly*nzc + lz the state.
+// space (pad columns lz >= nzc carry zeros), or -- patch tiles -- the kz = 0
+// and kz = Nz/2 columns of every ky.
 //
 // Blocks are dispatched to the 8 XCDs round-robin; xcd_tile() hands each XCD
 // a contiguous range of tiles so that neighbouring tiles (which share the
@@ -202,29 +144,6 @@ __host__ __device__ inline int x_tiles(const Grid &g, int CB, bool patch)
 }
 
 __host__ inline int x_grid(int ntiles) { return 8 * ((ntiles + 7) / 8); }
-
-template <int CB>
-__device__ __forceinline__ void tile_columns(int *colw, int *cols, const Grid &g, bool patch, int tile)
-{
-    if (threadIdx.x < CB) {
-        const int c = threadIdx.x;
-        int w = -1, st = -1;
-        if (!patch) {
-            const int cw = tile * CB + c;
-            const int ly = cw / g.nzp, lz = cw % g.nzp;
-            if (cw < g.ny * g.nzp && lz < g.nzc) { w = cw; st = ly * g.nzc + lz; }
-        } else {
-            const int p = tile * CB + c;
-            if (p < 2 * g.ny) {
-                const int ly = p >> 1, lz = (p & 1) ? g.nz / 2 : 0;
-                w = ly * g.nzp + lz;
-                st = ly * g.nzc + lz;
-            }
-        }
-        colw[c] = w;
-        cols[c] = st;
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Column tiles of the x passes that hold their points in registers (ColX).
@@ -353,86 +272,6 @@ struct ColTile {
         offs = (uint32_t)(j * ncs + (WIDE ? ly * g.nzc + min(lz, g.nzc - 1) : max(min(c, g.nzc - 1 - lz0), 0))) * 16u;
     }
 };
-
-// ---------------------------------------------------------------------------
-// Direct-to-LDS staging of an x tile (global_load_lds_dwordx4): the L x CB
-// tile of consecutive padded work columns cw0 .. cw0+CB-1 is moved in 1 KB
-// chunks, one per wave instruction (64 lanes x 16 bytes, lane l landing at
-// chunk + 16 l).  Within a chunk the layout is column-major, so the FFT's
-// reads of one column are consecutive:
-//   FP64 (16-byte elements): chunk = RPC = 64/CB rows x CB columns, lane
-//        c*RPC + r%RPC holds element (r, c);
-//   FP32 (8-byte elements): chunk = RPC2 = 128/CB rows x CB columns, lane
-//        (c/2)*RPC2 + r%RPC2 holds the pair (r, c & ~1), (r, c | 1).
-// Lanes of one instruction read CB adjacent columns of RPC (RPC2) rows: the
-// same 64-byte row segments as a row-major staging.  The tile must fill whole
-// waves and whole chunks (tile_dma_ok); the columns are always inside the
-// padded rows, so pad columns are loaded too (and ignored).
-// ---------------------------------------------------------------------------
-template <typename T, int L, int CB>
-__host__ __device__ constexpr bool tile_dma_ok()
-{
-    return (CB * (L / 8)) % 64 == 0 && (L * CB * (int)sizeof(cpx<T>)) % 1024 == 0 &&
-           (sizeof(T) == 8 || CB % 2 == 0);
-}
-
-template <typename T, int L, int CB>
-__device__ __forceinline__ void dma_tile(const cpx<T> *__restrict__ f, int cw0, int ncol_total, char *lds)
-{
-    constexpr int NWAVE = CB * (L / 8) / 64;
-    constexpr int NCHUNK = L * CB * (int)sizeof(cpx<T>) / 1024;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int k = wave; k < NCHUNK; k += NWAVE) {
-        const cpx<T> *src;
-        if constexpr (sizeof(T) == 8) {
-            constexpr int RPC = 64 / CB;
-            src = f + (size_t)(k * RPC + lane % RPC) * ncol_total + cw0 + lane / RPC;
-        } else {
-            constexpr int RPC2 = 128 / CB;
-            src = f + (size_t)(k * RPC2 + lane % RPC2) * ncol_total + cw0 + 2 * (lane / RPC2);
-        }
-        __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(lds + k * 1024),
-                                         16, 0, 0);
-    }
-}
-
-// The same chunk layout for an FP64 tile of the state (boundary layout):
-// column c of the tile is state column cols[c]; a column outside the state
-// (cols[c] < 0, the padding of the work layout) loads state column 0 instead,
-// whose values the caller ignores.
-template <int L, int CB>
-__device__ __forceinline__ void dma_state_tile(const cpx<double> *__restrict__ f, const int *cols, int ncol_total,
-                                               char *lds)
-{
-    constexpr int NWAVE = CB * (L / 8) / 64;
-    constexpr int NCHUNK = L * CB * 16 / 1024;
-    constexpr int RPC = 64 / CB;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int col = max(cols[lane / RPC], 0);
-    for (int k = wave; k < NCHUNK; k += NWAVE) {
-        const cpx<double> *src = f + (size_t)(k * RPC + lane % RPC) * ncol_total + col;
-        __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)(lds + k * 1024),
-                                         16, 0, 0);
-    }
-}
-
-template <typename T, int L, int CB>
-__device__ __forceinline__ cpx<T> dma_tile_read(const char *lds, int r, int c)
-{
-    if constexpr (sizeof(T) == 8) {
-        constexpr int RPC = 64 / CB;
-        return ((const cpx<T> *)lds)[(r / RPC) * 64 + c * RPC + (r % RPC)];
-    } else {
-        constexpr int RPC2 = 128 / CB;
-        return *(const cpx<T> *)(lds + (r / RPC2) * 1024 + ((c / 2) * RPC2 + (r % RPC2)) * 16 + (c % 2) * 8);
-    }
-}
-
-// Waits for this wave's direct-to-LDS loads (the barrier that follows makes
-// every wave's loads visible): s_waitcnt vmcnt(0) with expcnt and lgkmcnt at
-// their maxima.  The builtin (not inline asm) lets the compiler's wait
-// insertion see that the loads have retired.
-__device__ __forceinline__ void dma_wait() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 // the slot of a mode, -1 outside the box
 __device__ __forceinline__ int band_slot(const Band &b, int kx, int ky, int kz)

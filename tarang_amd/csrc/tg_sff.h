@@ -27,7 +27,8 @@ hipError_t launch_z_rbc(const Grid &g, void *const *U, void *const *P, const voi
                         hipStream_t st, bool shift = false);
 
 struct RbcParams {
-    int stage;            // 1..4; 0 = nonlinear terms (or right-hand sides) only
+    int stage;            // 1..4 (velocity products trace-shifted: xx - zz, yy - zz, zz not
+                          // formed); 0 = nonlinear terms (or right-hand sides) only
     int write_rhs;        // stage 0: force, projection and signs of Compute_rhs
     double dt;
     double fh_u, f1_u;    // -nu dt/2, -nu dt
@@ -35,8 +36,6 @@ struct RbcParams {
     double scale;         // 1/(2 Nx Ny Nz)
     int *nonfinite;       // stage 4: set to 1 if the new state holds a
                           // non-finite value (null: not checked)
-    int trace_free;       // velocity products trace-shifted (xx - zz, yy - zz,
-                          // zz not formed): an RK stage
 };
 
 // Fused x pass of an RBC stage: sin/cos x-forward of the 9 products, N and

@@ -15,10 +15,11 @@
 //   cosine inverse   V_k = W^-k (A_k - i A_{N-k}), v = IFFT(V) (unscaled)
 //   sine inverse     V_k = W^-k (A_{N-k} - i A_k), V_0 = 0, then (-1)^j
 // with W = exp(-i pi / (2N)) (table twq) and the (k, N-k) pairs exchanged
-// through the LDS line buffer.  A thread holds k = j + TPL*s (s < 8), and
-// every pass forms W^k = W^j W^(TPL s) from those TPL + 8 table entries
-// (QuarterTw), so all sin/cos passes round alike and the fused kernels keep
-// only 8 + TPL entries in LDS.  Along y and z the FFF passes are reused.
+// through LDS.  A thread holds k = j + TPL*s (s < 8), and every pass forms
+// W^k = W^j W^(TPL s) from those TPL + 8 table entries (QuarterTw), so all
+// sin/cos passes round alike and keep only 8 + TPL entries in LDS.  A thread's
+// samples are loaded and stored at their Makhoul positions directly (rows 2j
+// apart, from both ends), so the reordering costs no pass through LDS.  Along y and z the FFF passes are reused.
 #include <type_traits>
 
 #include "tg_device.h"
@@ -26,9 +27,6 @@
 #include "tg_sff.h"
 
 namespace tg {
-
-// sample index whose value sits at Makhoul position n
-__device__ __forceinline__ int mk_perm(int n, int N) { return n < N / 2 ? 2 * n : 2 * N - 2 * n - 1; }
 
 template <typename T>
 __device__ __forceinline__ cpx<T> times_i(cpx<T> z) { return mk<T>(-z.y, z.x); }
@@ -41,67 +39,47 @@ struct QuarterTw {
     __device__ __forceinline__ cpx<T> operator()(int j, int s) const { return lo[j] * hi[s]; }
 };
 
-// The core: v[s] holds the reordered (and, for sine, sign-alternated) input
-// at Makhoul position j + TPL*s; `col` is a free LDS line buffer.
-template <int L, typename T, typename Q>
-__device__ __forceinline__ void sc_forward_core(cpx<T> *v, cpx<T> *col, const cpx<T> *tw, Q twq, int j, bool sine)
+// Forward transform of a column: v[s] holds the sample at Makhoul position
+// j + TPL*s; on return 2N A_k at k = j + TPL*s.
+template <int L, typename X, typename T>
+__device__ __forceinline__ void sc_forward(cpx<T> *v, const X &x, const cpx<T> *tw, const QuarterTw<T> &twq, int j, bool sine)
 {
     constexpr int TPL = L / 8;
-    fft_line<L, -1>(v, col, tw, j);
+    if (sine) {
 #pragma unroll
-    for (int s = 0; s < 8; s++) col[lpad(j + TPL * s)] = v[s];
-    line_sync<TPL>();
+        for (int s = 4; s < 8; s++) v[s] = mk<T>(-v[s].x, -v[s].y);
+    }
+    fft_exchange<L, -1>(v, x, tw, j);
+#pragma unroll
+    for (int s = 0; s < 8; s++) x.w(j + TPL * s) = v[s];
+    x.publish();
 #pragma unroll
     for (int s = 0; s < 8; s++) {
         const int k = j + TPL * s;
-        const cpx<T> vn = col[lpad(k == 0 ? 0 : L - k)];
+        const cpx<T> vn = x.r(k == 0 ? 0 : L - k);
         const cpx<T> w = twq(j, s);
         const cpx<T> p = w * v[s];
         const cpx<T> q = conj(w) * vn;
         if (!sine) v[s] = p + q;
         else v[s] = k == 0 ? mk<T>(0, 0) : times_i(p - q);
     }
-    line_sync<TPL>();
+    x.release();
 }
 
-// Makhoul input gather of sample mk_perm(n) from `load(sample)`.
-template <int L, typename T, typename Load>
-__device__ __forceinline__ void sc_gather(cpx<T> *v, int j, bool sine, Load load)
+// Inverse: A_k in v[s] (k = j + TPL*s); on return the sample at Makhoul
+// position j + TPL*s.
+template <int L, typename X, typename T>
+__device__ __forceinline__ void sc_inverse(cpx<T> *v, const X &x, const cpx<T> *tw, const QuarterTw<T> &twq, int j, bool sine)
 {
     constexpr int TPL = L / 8;
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const int n = j + TPL * s;
-        cpx<T> x = load(mk_perm(n, L));
-        if (sine && n >= L / 2) x = mk<T>(-x.x, -x.y);
-        v[s] = x;
-    }
-}
-
-// Forward sin/cos transform of the line held in natural order in the LDS
-// line buffer `col`; on return v[s] = 2N A_k at k = j + TPL*s.  The caller
-// synchronises before (col written by other threads) and after (col reused).
-template <int L, typename T, typename Q>
-__device__ __forceinline__ void sc_forward(cpx<T> *v, cpx<T> *col, const cpx<T> *tw, Q twq, int j, bool sine)
-{
-    sc_gather<L, T>(v, j, sine, [&](int r) { return col[lpad(r)]; });
-    line_sync<L / 8>();
-    sc_forward_core<L>(v, col, tw, twq, j, sine);
-}
-
-// Inverse: A_k in v[s] (k = j + TPL*s); on return the samples are in `col`
-// in natural order (the caller synchronises before reading them).
-template <int L, typename T, typename Q>
-__device__ __forceinline__ void sc_inverse(cpx<T> *v, cpx<T> *col, const cpx<T> *tw, Q twq, int j, bool sine)
-{
-    constexpr int TPL = L / 8;
-#pragma unroll
-    for (int s = 0; s < 8; s++) col[lpad(j + TPL * s)] = v[s];
-    line_sync<TPL>();
+    for (int s = 0; s < 8; s++) x.w(j + TPL * s) = v[s];
+    x.publish();
 #pragma unroll
     for (int s = 0; s < 8; s++) {
         const int k = j + TPL * s;
-        const cpx<T> an = k == 0 ? mk<T>(0, 0) : col[lpad(L - k)];
+        cpx<T> an = x.r(k == 0 ? 0 : L - k);
+        if (k == 0) an = mk<T>(0, 0);
         const cpx<T> ak = v[s];
         // component-wise selects (a select of the two values as objects keeps
         // v[] out of registers)
@@ -111,17 +89,74 @@ __device__ __forceinline__ void sc_inverse(cpx<T> *v, cpx<T> *col, const cpx<T> 
         if (sine && k == 0) z = mk<T>(0, 0);
         v[s] = z;
     }
-    line_sync<TPL>();
-    fft_line<L, +1>(v, col, tw, j);
-    line_sync<TPL>();
+    x.release();
+    fft_exchange<L, +1>(v, x, tw, j);
+    if (sine) {
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const int n = j + TPL * s;
-        cpx<T> x = v[s];
-        if (sine && n >= L / 2) x = mk<T>(-x.x, -x.y);
-        col[lpad(mk_perm(n, L))] = x;
+        for (int s = 4; s < 8; s++) v[s] = mk<T>(-v[s].x, -v[s].y);
     }
 }
+
+// A column tile whose T work fields are read and written in Makhoul order:
+// position n = j + TPL s holds sample 2n (s < 4: row 2j of rows 2 TPL s on) or
+// 2(N - n) - 1 (row 2 TPL - 1 - 2j of rows 2 TPL (7 - s) on).  Byte offsets
+// below a quarter of a field.
+template <typename T, int L, int CB>
+struct ScTile : ColTile<T, L, CB> {
+    uint32_t even, odd;
+    __device__ __forceinline__ ScTile(const Grid &g, int tile, bool patch = false) : ColTile<T, L, CB>(g, tile, patch)
+    {
+        const uint32_t row = (uint32_t)(g.ny * g.nzp) * (uint32_t)sizeof(cpx<T>);
+        const uint32_t col = this->offt - this->j * row;
+        even = 2 * this->j * row + col;
+        odd = (2 * ColTile<T, L, CB>::TPL - 1 - 2 * this->j) * row + col;
+    }
+    template <bool NT>
+    __device__ __forceinline__ void load(cpx<T> *v, const void *f) const
+    {
+        typedef __attribute__((address_space(1))) const vec2<T> gvec;
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const cpx<T> *p = (const cpx<T> *)f + this->cw0 + 2 * (s < 4 ? s : 7 - s) * this->stepw;
+            gvec *q = (gvec *)(uniform_address(p) + (s < 4 ? even : odd));
+            vec2<T> x;
+            if constexpr (NT) x = __builtin_nontemporal_load(q);
+            else x = *q;
+            v[s] = mk<T>(x.x, x.y);
+        }
+    }
+    template <bool NT>
+    __device__ __forceinline__ void store(const cpx<T> *v, void *f) const
+    {
+        typedef __attribute__((address_space(1))) vec2<T> gvec;
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            cpx<T> *p = (cpx<T> *)f + this->cw0 + 2 * (s < 4 ? s : 7 - s) * this->stepw;
+            gvec *q = (gvec *)(uniform_address(p) + (s < 4 ? even : odd));
+            vec2<T> x;
+            x.x = v[s].x;
+            x.y = v[s].y;
+            if constexpr (NT) __builtin_nontemporal_store(x, q);
+            else *q = x;
+        }
+    }
+};
+
+// The twiddles of a sin/cos x kernel in LDS (L + L/8 + 8 entries).
+template <typename T, int L>
+struct ScTwiddles {
+    const cpx<T> *tw;
+    QuarterTw<T> twq;
+    // all threads of the block; ends in a barrier
+    __device__ __forceinline__ ScTwiddles(cpx<T> *lds, const void *twx, const void *q) : tw(lds), twq{lds + L, lds + L + L / 8}
+    {
+        constexpr int TPL = L / 8;
+        for (int i = threadIdx.x; i < L; i += blockDim.x) lds[i] = ((const cpx<T> *)twx)[i];
+        for (int i = threadIdx.x; i < TPL; i += blockDim.x) lds[L + i] = ((const cpx<T> *)q)[i];
+        if (threadIdx.x < 8) lds[L + TPL + threadIdx.x] = ((const cpx<T> *)q)[TPL * threadIdx.x];
+        lds_barrier();
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Plain x passes (tg_forward / tg_inverse, stage-1 inputs, reality patches)
@@ -139,75 +174,64 @@ template <typename T, int L, int CB>
 __global__ void __launch_bounds__(CB *(L / 8)) k_xinv_sc(XscArgs a)
 {
     constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    __shared__ __attribute__((aligned(16))) char raw[CB * LP * sizeof(cpx<double>)];
-    __shared__ int colw[CB], cols[CB];
-    cpx<double> *ldd = (cpx<double> *)raw;
-    cpx<T> *ldt = (cpx<T> *)raw;
+    using X = ColX<T, L, CB>;
+    __shared__ cpx<T> lds[X::SIZE];
+    __shared__ cpx<T> ldw[L + TPL + 8];
     const Grid &g = a.g;
-    __shared__ cpx<T> qhi[8];
     const bool patch = (a.flags & 4) != 0;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     if (tile >= x_tiles(g, CB, patch)) return;
-    tile_columns<CB>(colw, cols, g, patch, tile);
-    if (threadIdx.x < 8) qhi[threadIdx.x] = ((const cpx<T> *)a.twq)[(L / 8) * threadIdx.x];
-    lds_barrier();
-    const int c = threadIdx.x / TPL, j = threadIdx.x % TPL;
-    const int cw = colw[c];
-    const int ly = cw >= 0 ? cw / g.nzp : 0, lz = cw >= 0 ? cw % g.nzp : 0;
-    const cpx<T> *tw = (const cpx<T> *)a.tw;
-    const QuarterTw<T> twq{(const cpx<T> *)a.twq, qhi};
-    const int ncw = g.ny * g.nzp, ncs = g.ny * g.nzc;
+    const ScTile<T, L, CB> t(g, tile, patch);
+    const int j = t.j;
+    cpx<double> d[8];
+    col_load<false>(d, (const cpx<double> *)a.V[0] + t.state0, t.steps, t.offs);
+    const ScTwiddles<T, L> tw(ldw, a.tw, a.twq);
+    const X x{lds + t.c};
+    int zx0 = 1, zx1 = 0;
+    if (a.flags & 1) dealias_rows(g, t.ly, t.lz, zx0, zx1);
+    if (!t.live) { zx0 = 0; zx1 = L - 1; }
+#pragma unroll 1
     for (int comp = 0; comp < a.ncomp; comp++) {
-        stage_in<L, CB>(ldd, (const cpx<double> *)a.V[comp], cols, ncs);
-        lds_barrier();
         cpx<T> v[8];
+        const int jh = hidden(j);
 #pragma unroll
         for (int s = 0; s < 8; s++) {
-            const int lx = j + TPL * s;
-            cpx<double> d = ldd[c * LP + lpad(lx)];
-            if ((a.flags & 1) && dealias_zero(g, lx, ly, lz)) d = mk<double>(0, 0);
-            v[s] = cvt<T>(d);
+            const int lx = jh + TPL * s;
+            v[s] = lx >= zx0 && lx <= zx1 ? mk<T>(0, 0) : cvt<T>(d[s]);
+            settle(v[s]);
         }
-        lds_barrier();
-        sc_inverse<L>(v, ldt + c * LP, tw, twq, j, ((a.parity >> comp) & 1) != 0);
-        lds_barrier();
-        stage_out<L, CB>(ldt, (cpx<T> *)a.U[comp], colw, ncw);
-        lds_barrier();
+        pin_memory_order();
+        if (comp + 1 < a.ncomp) col_load<false>(d, (const cpx<double> *)a.V[comp + 1] + t.state0, t.steps, t.offs);
+        pin_memory_order();
+        sc_inverse<L>(v, x, tw.tw, tw.twq, jh, ((a.parity >> comp) & 1) != 0);
+        pin_memory_order();
+        if (t.inside) t.template store<false>(v, a.U[comp]);
     }
 }
 
 template <typename T, int L, int CB>
 __global__ void __launch_bounds__(CB *(L / 8)) k_xfwd_sc(XscArgs a)
 {
-    constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    __shared__ __attribute__((aligned(16))) char raw[CB * LP * sizeof(cpx<double>)];
-    __shared__ int colw[CB], cols[CB];
-    cpx<double> *ldd = (cpx<double> *)raw;
-    cpx<T> *ldt = (cpx<T> *)raw;
-    const Grid &g = a.g;
-    __shared__ cpx<T> qhi[8];
+    using X = ColX<T, L, CB>;
+    __shared__ cpx<T> lds[X::SIZE];
+    __shared__ cpx<T> ldw[L + L / 8 + 8];
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    if (tile >= x_tiles(g, CB, false)) return;
-    tile_columns<CB>(colw, cols, g, false, tile);
-    if (threadIdx.x < 8) qhi[threadIdx.x] = ((const cpx<T> *)a.twq)[(L / 8) * threadIdx.x];
-    lds_barrier();
-    const int c = threadIdx.x / TPL, j = threadIdx.x % TPL;
-    const cpx<T> *tw = (const cpx<T> *)a.tw;
-    const QuarterTw<T> twq{(const cpx<T> *)a.twq, qhi};
-    const int ncw = g.ny * g.nzp, ncs = g.ny * g.nzc;
+    if (tile >= x_tiles(a.g, CB, false)) return;
+    const ScTile<T, L, CB> t(a.g, tile);
+    cpx<T> v[8];
+    t.template load<false>(v, a.U[0]);
+    const ScTwiddles<T, L> tw(ldw, a.tw, a.twq);
+    const X x{lds + t.c};
+#pragma unroll 1
     for (int comp = 0; comp < a.ncomp; comp++) {
-        stage_in<L, CB>(ldt, (const cpx<T> *)a.U[comp], colw, ncw);
-        lds_barrier();
-        cpx<T> v[8];
-        sc_forward<L>(v, ldt + c * LP, tw, twq, j, ((a.parity >> comp) & 1) != 0);
-        lds_barrier();
+        sc_forward<L>(v, x, tw.tw, tw.twq, hidden(t.j), ((a.parity >> comp) & 1) != 0);
+        cpx<double> o[8];
 #pragma unroll
-        for (int s = 0; s < 8; s++) ldd[c * LP + lpad(j + TPL * s)] = a.scale * cvt<double>(v[s]);
-        lds_barrier();
-        stage_out<L, CB>(ldd, (cpx<double> *)a.V[comp], cols, ncs);
-        lds_barrier();
+        for (int s = 0; s < 8; s++) o[s] = a.scale * cvt<double>(v[s]);
+        pin_memory_order();
+        if (comp + 1 < a.ncomp) t.template load<false>(v, a.U[comp + 1]);
+        pin_memory_order();
+        if (t.live) col_store<false>(o, (cpx<double> *)a.V[comp] + t.state0, t.steps, t.offs);
     }
 }
 
@@ -225,14 +249,6 @@ __device__ __forceinline__ int rbc_pair(int ia, int ib)
     if (ia == 0) return ib == 1 ? 3 : (ib == 2 ? 5 : 6);
     if (ia == 1) return ib == 2 ? 4 : 7;
     return 8;
-}
-
-__device__ __forceinline__ void *sel_ptr(void *const *p, int i, int n)
-{
-    void *r = p[0];
-    for (int k = 1; k < n; k++)
-        if (i == k) r = p[k];
-    return r;
 }
 
 // Two waves per SIMD also for FP64 512-point lines (a few spilled registers
@@ -314,255 +330,132 @@ struct XrbcArgs {
     RbcParams rp;
 };
 
-// Contribution of a transformed product q to one output component:
-// sel 0 none, 1 +Kx q (d/dx of an 'S' product), 2 -Kx q ('C' product),
-// 3 i Ky q, 4 i Kz q (SFF_pencil_tr.cc:77-151).  Branch-free form: the
-// term is a q + i b q with a = ax Kx, b = ay Ky + az Kz and one of ax, ay,
-// az equal to +-1 (the others 0), so every term keeps its exact value.
-template <typename T>
-struct RbcTerm {
-    T ax, b;
-    __device__ __forceinline__ RbcTerm(int sel, T Ky, T Kz)
-        : ax(sel == 1 ? T(1) : (sel == 2 ? T(-1) : T(0))), b(sel == 3 ? Ky : (sel == 4 ? Kz : T(0)))
-    {
-    }
-    __device__ __forceinline__ cpx<T> operator()(T Kx, cpx<T> q) const
-    {
-        const T a = ax * Kx;
-        return mk<T>(a * q.x - b * q.y, a * q.y + b * q.x);
-    }
-};
-
-// Selectors of the velocity products (xx C, yy C, zz C, xy S, yz C, zx S)
-// for N_x, N_y, N_z in the reference's accumulation order.
-__device__ __forceinline__ int rbc_sel(int p, int comp)
+// Terms of the nonlinear terms (SFF_pencil_tr.cc:77-151): the derivative of a
+// transformed product q along axis D (x: +Kx q of an 'S' product, -Kx q of a
+// 'C' one), added to n.  The term is settled before it is added: the passes
+// round it on its own.
+template <int D, bool SINE, typename T>
+__device__ __forceinline__ void add_term(cpx<T> &n, T Kx, T Ky, T Kz, cpx<T> q)
 {
-    switch (p) {
-        case 0: return comp == 0 ? 2 : 0;                      // xx: N_x = -Kx F_C
-        case 1: return comp == 1 ? 3 : 0;                      // yy: N_y = i Ky F_C
-        case 2: return comp == 2 ? 4 : 0;                      // zz: N_z = i Kz F_C
-        case 3: return comp == 0 ? 3 : (comp == 1 ? 1 : 0);    // xy: N_x += i Ky, N_y += Kx (F_S)
-        case 4: return comp == 1 ? 4 : (comp == 2 ? 3 : 0);    // yz: N_y += i Kz, N_z += i Ky (F_C)
-        default: return comp == 0 ? 4 : (comp == 2 ? 1 : 0);  // zx: N_x += i Kz, N_z += Kx (F_S)
-    }
+    cpx<T> d;
+    if constexpr (D == 0) d = SINE ? mk<T>(Kx * q.x, Kx * q.y) : mk<T>(-Kx * q.x, -Kx * q.y);
+    else d = mul_i(D == 1 ? Ky : Kz, q);
+    settle(d);
+    n = n + d;
+    settle(n);
 }
 
-// One component of the Lawson stage (RK_SF.cc:97-215 with
-// Tadvance_functions.cc:298-324, 566-570): r = right-hand side (FP64).
-template <typename T, int L, int CB>
-__device__ __forceinline__ void rbc_lawson(const Grid &g, const RbcParams &rp, int c, int j, int ly, int lz,
-                                           double Ky, double Kz, const int *colw, const int *cols,
-                                           cpx<double> *ldd, cpx<double> *ldb, cpx<T> *ldt, const cpx<T> *tw,
-                                           QuarterTw<T> twq, const cpx<double> *r, double fh, double f1,
-                                           double *V, double *acc, void *U, double *fo, bool sine)
-{
-    constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    const int stage = rp.stage;
-    const int ncw = g.ny * g.nzp, ncs = g.ny * g.nzc;
-    const double dt = rp.dt;
-    const double c_half = 0.5 * dt, c_one = 1.0 * dt;
-    const double c_sixth = (1.0 / 6) * dt, c_third = (1.0 / 3) * dt;
-    stage_in<L, CB>(ldd, (const cpx<double> *)V, cols, ncs);
-    if (stage >= 2) stage_in<L, CB>(ldb, (const cpx<double> *)acc, colw, ncw);
-    lds_barrier();
-    cpx<T> v[8];
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const int lx = j + TPL * s;
-        const int li = c * LP + lpad(lx);
-        const double Kx = lx * g.kf[0];
-        const double ks = (Kx * Kx + Ky * Ky) + Kz * Kz;
-        const double Eh = exp(fh * ks);
-        const cpx<double> v0 = ldd[li];
-        cpx<double> vn, ac;
-        if (stage == 1) {
-            cpx<double> d0 = v0;
-            if (dealias_zero(g, lx, ly, lz)) d0 = mk<double>(0, 0);
-            const double E1 = exp(f1 * ks);
-            ac = c_sixth * (E1 * r[s]);
-            vn = Eh * (d0 + c_half * r[s]);
-        } else if (stage == 2) {
-            ac = ldb[li] + c_third * (Eh * r[s]);
-            vn = Eh * v0 + c_half * r[s];
-        } else if (stage == 3) {
-            ac = ldb[li] + c_third * (Eh * r[s]);
-            vn = Eh * (Eh * v0 + c_one * r[s]);
-        } else {
-            ac = ldb[li] + c_sixth * r[s];
-            const double E1 = exp(f1 * ks);
-            vn = E1 * v0 + ac;
-        }
-        // component-wise select (selecting the objects keeps them in memory)
-        ldb[li] = mk<double>(stage == 4 ? vn.x : ac.x, stage == 4 ? vn.y : ac.y);
-        if (stage == 4 && !(isfinite(vn.x) && isfinite(vn.y)) && rp.nonfinite) *rp.nonfinite = 1;
-        // the undealiased next-stage value (this field's share of the next
-        // force) replaces v0 in the thread's own slot of the state tile
-        if (fo) ldd[li] = vn;
-        if (dealias_zero(g, lx, ly, lz)) vn = mk<double>(0, 0);
-        v[s] = cvt<T>(vn);
-    }
-    lds_barrier();
-    if (stage == 4) stage_out<L, CB>(ldb, (cpx<double> *)V, cols, ncs);
-    else stage_out<L, CB>(ldb, (cpx<double> *)acc, colw, ncw);
-    if (fo) {
-        stage_out<L, CB>(ldd, (cpx<double> *)fo, cols, ncs);
-        lds_barrier();
-    }
-    sc_inverse<L>(v, ldt + c * LP, tw, twq, j, sine);
-    lds_barrier();
-    stage_out<L, CB>(ldt, (cpx<T> *)U, colw, ncw);
-    lds_barrier();
-}
-
-// PHASE 0: temperature (N_T, its right-hand side, Lawson for theta);
-// PHASE 1: velocity.  The two launches of a stage touch disjoint data (the
-// force inputs they read are the other field's, of this stage's input).
-template <typename T, int L, int CB, int PHASE>
+// PHASE 0: temperature (N_T, its right-hand side, Lawson for theta, nu =
+// kappa); PHASE 1: velocity.  The two launches of a stage touch disjoint data
+// (the force inputs they read are the other field's, of this stage's input).
+// ST: RK stage 1..4 (velocity products trace-shifted: xx - zz, yy - zz, zz not
+// formed), 0 nonlinear terms or right-hand sides only (six products).
+//
+// Bound by HBM.  Columns go from memory to registers and back in transform
+// order (the products and the next stage input in Makhoul order), the next
+// load is in flight behind each transform, products and components are
+// unrolled and each stage has its code: with the tiles staged through LDS the
+// launches of a stage at 256 x 512 x 512 FP32 took 1.0 and 2.2 ms, now 0.85 and 1.83 (4.6 TB/s).
+template <typename T, int L, int CB, int PHASE, int ST, bool NT>
 __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_rbc(XrbcArgs a)
 {
-    constexpr int TPL = L / 8;
-    constexpr int LP = lpad_len(L);
-    // A: FFT exchanges and state staging; B: products arriving by
-    // direct-to-LDS loads, then the accumulator tile (separate LDS objects)
-    __shared__ __attribute__((aligned(16))) char rawA[CB * LP * sizeof(cpx<double>)];
-    __shared__ __attribute__((aligned(16))) char rawB[CB * LP * sizeof(cpx<double>)];
-    __shared__ int colw[CB], cols[CB];
-    __shared__ cpx<T> twl[L], twqlo[L / 8], twqhi[8];
-    cpx<double> *ldd = (cpx<double> *)rawA;
-    cpx<T> *ldt = (cpx<T> *)rawA;
-    cpx<double> *ldb = (cpx<double> *)rawB;
-    constexpr bool DMA = tile_dma_ok<T, L, CB>();
+    constexpr int TPL = L / 8, NTH = CB * TPL;
+    constexpr bool NTW = NT && CB * sizeof(cpx<T>) >= 128, NTA = NT && CB * sizeof(cpx<double>) >= 128;
+    constexpr int NC = PHASE == 0 ? 1 : 3;   // components of the phase
+    constexpr int C0 = PHASE == 0 ? 3 : 0;   // the first one (u_x, u_y, u_z, theta)
+    using X = ColX<T, L, CB>;
+    __shared__ cpx<T> lds[X::SIZE];
+    __shared__ cpx<T> ldw[L + TPL + 8];
+    // the viscous factors at this thread's points: exp(-nu K^2 dt/2) (not in
+    // stage 4), exp(-nu K^2 dt) (stages 1 and 4)
+    __shared__ double visc[ST == 1 ? 2 : 1][ST > 0 ? 8 * NTH : 1];
     const Grid &g = a.g;
     const RbcParams &rp = a.rp;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     if (tile >= x_tiles(g, CB, false)) return;
-    tile_columns<CB>(colw, cols, g, false, tile);
-    for (int i = threadIdx.x; i < L; i += CB * TPL) twl[i] = ((const cpx<T> *)a.tw)[i];
-    if (threadIdx.x < TPL) twqlo[threadIdx.x] = ((const cpx<T> *)a.twq)[threadIdx.x];
-    if (threadIdx.x < 8) twqhi[threadIdx.x] = ((const cpx<T> *)a.twq)[TPL * threadIdx.x];
-    const QuarterTw<T> twql{twqlo, twqhi};
-    lds_barrier();
-    const int c = threadIdx.x / TPL, j = threadIdx.x % TPL;
-    const int cw = colw[c];
-    const int ly = cw >= 0 ? cw / g.nzp : 0, lz = cw >= 0 ? cw % g.nzp : 0;
+    const ScTile<T, L, CB> t(g, tile);
+    const int j = t.j, ly = t.ly, lz = t.lz;
     const double Ky = kwave(ly, g.ny) * g.kf[1], Kz = lz * g.kf[2];
     const T Kyt = (T)Ky, Kzt = (T)Kz;
     const T sc = (T)rp.scale;
-    const int ncw = g.ny * g.nzp, ncs = g.ny * g.nzc;
-    const int stage = rp.stage;
-    const bool want_rhs = stage > 0 || rp.write_rhs;
-    const int cw0 = tile * CB;
-    // Product p of a phase into registers v (Makhoul order, sign-alternated
-    // for sine products): from B after its direct-to-LDS load (then the load
-    // of product p_next starts), or staged through A.
-    auto load_product = [&](cpx<T> *v, int p, int p_next, int jj, bool sine) {
-        if constexpr (DMA) {
-            dma_wait();
-            lds_barrier();
-            sc_gather<L, T>(v, jj, sine, [&](int r) { return dma_tile_read<T, L, CB>(rawB, r, c); });
-            lds_barrier();
-            if (p_next >= 0) dma_tile<T, L, CB>((const cpx<T> *)sel_ptr(a.P, p_next, 9), cw0, ncw, rawB);
-        } else {
-            stage_in<L, CB>(ldt, (const cpx<T> *)sel_ptr(a.P, p, 9), colw, ncw);
-            lds_barrier();
-            sc_gather<L, T>(v, jj, sine, [&](int r) { return ldt[c * LP + lpad(r)]; });
-            lds_barrier();
+    const bool want_rhs = ST > 0 || rp.write_rhs;
+    // the products of the phase: x theta C, y theta S, z theta S; xx C, yy C,
+    // (zz C), xy S, yz C, zx S
+    constexpr int NP = PHASE == 0 ? 3 : (ST > 0 ? 5 : 6);
+    constexpr int first = PHASE == 0 ? 6 : 0;
+    auto index = [](int q) { return PHASE == 1 && ST > 0 && q >= 2 ? q + 1 : first + q; };
+    cpx<T> cur[8], alt[8];
+    t.template load<NTW>(cur, a.P[first]);
+    const ScTwiddles<T, L> tw(ldw, a.tw, a.twq);
+    const X x{lds + t.c};
+    cpx<T> N[NC][8];
+#pragma unroll
+    for (int k = 0; k < NC; k++)
+#pragma unroll
+        for (int s = 0; s < 8; s++) N[k][s] = mk<T>(0, 0);
+    cpx<double> w[8];
+    auto product = [&](auto qc, cpx<T> *v, cpx<T> *next) {
+        constexpr int Q = decltype(qc)::value;
+        if constexpr (Q < NP) {
+            constexpr int P = PHASE == 1 && ST > 0 && Q >= 2 ? Q + 1 : first + Q;
+            constexpr bool SINE = P == 3 || P == 5 || P > 6;
+            pin_memory_order();
+            if constexpr (Q + 1 < NP) t.template load<NTW>(next, a.P[index(Q + 1)]);
+            else if (want_rhs) col_load<false>(w, (const cpx<double> *)a.f_in[PHASE == 0 ? 1 : 0] + t.state0, t.steps, t.offs);
+            pin_memory_order();
+            const int jh = hidden(j);
+            sc_forward<L>(v, x, tw.tw, tw.twq, jh, SINE);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                const T Kx = (T)((jh + TPL * s) * g.kf[0]);
+                const cpx<T> q = sc * v[s];
+                if constexpr (P >= 6) {
+                    add_term<P - 6, SINE>(N[0][s], Kx, Kyt, Kzt, q);
+                } else if constexpr (P < 3) {
+                    add_term<P, SINE>(N[P % NC][s], Kx, Kyt, Kzt, q);
+                } else {
+                    constexpr int A = P - 3, B = (P - 2) % 3;   // xy, yz, zx
+                    add_term<B, SINE>(N[A % NC][s], Kx, Kyt, Kzt, q);
+                    add_term<A, SINE>(N[B % NC][s], Kx, Kyt, Kzt, q);
+                }
+            }
         }
     };
+    product(std::integral_constant<int, 0>{}, cur, alt);
+    product(std::integral_constant<int, 1>{}, alt, cur);
+    product(std::integral_constant<int, 2>{}, cur, alt);
+    product(std::integral_constant<int, 3>{}, alt, cur);
+    product(std::integral_constant<int, 4>{}, cur, alt);
+    product(std::integral_constant<int, 5>{}, alt, cur);
 
-    // ===== temperature: N_T = -Kx F_C(u_x T) + i Ky F_S(u_y T) + i Kz F_S(u_z T) =====
+    // --- right-hand sides (in place, negated) ---
+    cpx<double> ac[8], v0[8];
+    if (ST > 0) col_load<false>(v0, (const cpx<double> *)a.V[C0] + t.state0, t.steps, t.offs);
+    pin_memory_order();
+    cpx<double> rt[PHASE == 0 ? 8 : 1];   // RHS_T stays in FP64
     if constexpr (PHASE == 0) {
-        cpx<T> nt[8];
-#pragma unroll
-        for (int s = 0; s < 8; s++) nt[s] = mk<T>(0, 0);
-        if constexpr (DMA) dma_tile<T, L, CB>((const cpx<T> *)a.P[6], cw0, ncw, rawB);
-#pragma unroll 1
-        for (int p = 6; p < 9; p++) {
-            int jj = j;  // hidden from loop-invariant code motion (see k_x_nlin)
-            asm volatile("" : "+v"(jj));
-            cpx<T> v[8];
-            load_product(v, p, p < 8 ? p + 1 : -1, jj, p != 6);
-            sc_forward_core<L>(v, ldt + c * LP, twl, twql, jj, p != 6);
-            const RbcTerm<T> tt(p == 6 ? 2 : (p == 7 ? 3 : 4), Kyt, Kzt);
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const T Kx = (T)((jj + TPL * s) * g.kf[0]);
-                nt[s] = nt[s] + tt(Kx, sc * v[s]);
-            }
-            if constexpr (!DMA) lds_barrier();
-        }
-        if constexpr (DMA) lds_barrier();
-        cpx<double> r[8];
-        if (want_rhs) {
-            // RHS_T = -(N_T - F_T), F_T = u_x of the stage input
-            stage_in<L, CB>(ldb, (const cpx<double> *)a.f_in[1], cols, ncs);
-            lds_barrier();
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const cpx<double> n = cvt<double>(nt[s]) - ldb[c * LP + lpad(j + TPL * s)];
-                r[s] = mk<double>(-n.x, -n.y);
-            }
-            lds_barrier();
-        } else {
-#pragma unroll
-            for (int s = 0; s < 8; s++) r[s] = cvt<double>(nt[s]);
-        }
-        if (stage == 0) {
-#pragma unroll
-            for (int s = 0; s < 8; s++) ldd[c * LP + lpad(j + TPL * s)] = r[s];
-            lds_barrier();
-            stage_out<L, CB>(ldd, (cpx<double> *)a.out[3], cols, ncs);
-            lds_barrier();
-        } else {
-            rbc_lawson<T, L, CB>(g, rp, c, j, ly, lz, Ky, Kz, colw, cols, ldd, ldb, ldt, twl, twql, r, rp.fh_t, rp.f1_t,
-                                 a.V[3], a.acc[3], a.U[3], stage < 4 ? a.f_out[0] : nullptr, true);
-        }
-    }
-
-    if constexpr (PHASE == 0) return;
-    // ===== velocity: divergence-form N with the SFF parities =====
-    cpx<T> N[3][8];
-#pragma unroll
-    for (int s = 0; s < 8; s++) N[0][s] = N[1][s] = N[2][s] = mk<T>(0, 0);
-    if constexpr (DMA) dma_tile<T, L, CB>((const cpx<T> *)a.P[0], cw0, ncw, rawB);
-    // trace-shifted products (an RK stage): xx - zz, yy - zz, xy, yz, zx, the
-    // zz slot skipped
-    const bool shift = rp.trace_free != 0;
-    const int nvp = shift ? 5 : 6;
-#pragma unroll 1
-    for (int q = 0; q < nvp; q++) {
-        const int p = shift && q >= 2 ? q + 1 : q;
-        const int pn = q + 1 < nvp ? (shift && q + 1 >= 2 ? q + 2 : q + 1) : -1;
-        int jj = j;
-        asm volatile("" : "+v"(jj));
-        cpx<T> v[8];
-        load_product(v, p, pn, jj, p == 3 || p == 5);
-        sc_forward_core<L>(v, ldt + c * LP, twl, twql, jj, p == 3 || p == 5);
-        const RbcTerm<T> t0(rbc_sel(p, 0), Kyt, Kzt), t1(rbc_sel(p, 1), Kyt, Kzt), t2(rbc_sel(p, 2), Kyt, Kzt);
+        // RHS_T = -(N_T - F_T), F_T = u_x of the stage input
 #pragma unroll
         for (int s = 0; s < 8; s++) {
-            const T Kx = (T)((jj + TPL * s) * g.kf[0]);
-            const cpx<T> q = sc * v[s];
-            N[0][s] = N[0][s] + t0(Kx, q);
-            N[1][s] = N[1][s] + t1(Kx, q);
-            N[2][s] = N[2][s] + t2(Kx, q);
+            rt[s] = cvt<double>(N[0][s]);
+            if (want_rhs) {
+                const cpx<double> n = rt[s] - w[s];
+                rt[s] = mk<double>(-n.x, -n.y);
+            }
+            settle(rt[s]);
         }
-        if constexpr (!DMA) lds_barrier();
-    }
-    if constexpr (DMA) lds_barrier();
-    if (want_rhs) {
+    } else if (want_rhs) {
         // nlin -= F (F_x = theta of the stage input); p = div/K^2 with the SFF
         // divergence (+Kx on the 'S' x component); nlin += grad p ('C' parity:
         // -Kx p); negate (Compute_rhs_scalar)
-        stage_in<L, CB>(ldd, (const cpx<double> *)a.f_in[0], cols, ncs);
-        lds_barrier();
+        const int jh = hidden(j);
 #pragma unroll
         for (int s = 0; s < 8; s++) {
-            const int lx = j + TPL * s;
+            const int lx = jh + TPL * s;
             const double Kx = lx * g.kf[0];
-            cpx<double> n0 = cvt<double>(N[0][s]) - ldd[c * LP + lpad(lx)];
-            cpx<double> n1 = cvt<double>(N[1][s]), n2 = cvt<double>(N[2][s]);
+            cpx<double> n0 = cvt<double>(N[0][s]) - w[s];
+            cpx<double> n1 = cvt<double>(N[1 % NC][s]), n2 = cvt<double>(N[2 % NC][s]);
             cpx<double> div = Kx * n0;
             div = div + mul_i(Ky, n1);
             div = div + mul_i(Kz, n2);
@@ -573,35 +466,92 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_rbc(XrbcArgs a)
             n1 = n1 + mul_i(Ky, pr);
             n2 = n2 + mul_i(Kz, pr);
             N[0][s] = cvt<T>(mk<double>(-n0.x, -n0.y));
-            N[1][s] = cvt<T>(mk<double>(-n1.x, -n1.y));
-            N[2][s] = cvt<T>(mk<double>(-n2.x, -n2.y));
+            N[1 % NC][s] = cvt<T>(mk<double>(-n1.x, -n1.y));
+            N[2 % NC][s] = cvt<T>(mk<double>(-n2.x, -n2.y));
+            settle(N[0][s]);
+            settle(N[1 % NC][s]);
+            settle(N[2 % NC][s]);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        lds_barrier();
     }
-    // the three components unrolled: N[K] and the field pointers are static
-    // (a runtime component index put N in scratch memory)
-    auto vel_comp = [&](auto kc) {
-        constexpr int K = decltype(kc)::value;
-        cpx<double> r[8];
+    if constexpr (ST == 0) {
 #pragma unroll
-        for (int s = 0; s < 8; s++) r[s] = cvt<double>(N[K][s]);
-        if (stage == 0) {
+        for (int k = 0; k < NC; k++) {
+            cpx<double> o[8];
 #pragma unroll
-            for (int s = 0; s < 8; s++) ldd[c * LP + lpad(j + TPL * s)] = r[s];
-            lds_barrier();
-            stage_out<L, CB>(ldd, (cpx<double> *)a.out[K], cols, ncs);
-            lds_barrier();
-        } else {
-            int jj = j;  // keeps the per-thread LDS addresses inside each component
-            asm volatile("" : "+v"(jj));
-            rbc_lawson<T, L, CB>(g, rp, c, jj, ly, lz, Ky, Kz, colw, cols, ldd, ldb, ldt, twl, twql, r, rp.fh_u,
-                                 rp.f1_u, a.V[K], a.acc[K], a.U[K], (K == 0 && stage < 4) ? a.f_out[1] : nullptr,
-                                 K == 0);
+            for (int s = 0; s < 8; s++) o[s] = PHASE == 0 ? rt[PHASE == 0 ? s : 0] : cvt<double>(N[k][s]);
+            if (t.live) col_store<false>(o, (cpx<double> *)a.out[C0 + k] + t.state0, t.steps, t.offs);
         }
-    };
-    vel_comp(std::integral_constant<int, 0>{});
-    vel_comp(std::integral_constant<int, 1>{});
-    vel_comp(std::integral_constant<int, 2>{});
+    } else {
+        // --- Lawson stage (RK_SF.cc:97-215 with Tadvance_functions.cc:298-324,
+        // 566-570), next stage input ---
+        int zx0, zx1;
+        dealias_rows(g, ly, lz, zx0, zx1);
+        if (!t.live) { zx0 = 0; zx1 = L - 1; }
+        {
+            const int jh = hidden(j);
+            const double fh = PHASE == 0 ? rp.fh_t : rp.fh_u, f1 = PHASE == 0 ? rp.f1_t : rp.f1_u;
+#pragma unroll 2
+            for (int s = 0; s < 8; s++) {
+                const double Kx = (jh + TPL * s) * g.kf[0];
+                const double ks = (Kx * Kx + Ky * Ky) + Kz * Kz;
+                visc[0][s * NTH + threadIdx.x] = exp((ST == 4 ? f1 : fh) * ks);
+                if (ST == 1) visc[ST == 1][s * NTH + threadIdx.x] = exp(f1 * ks);
+            }
+        }
+        if (ST >= 2) col_load<NTA>(ac, (const cpx<double> *)a.acc[C0] + t.cw0, t.stepw, t.offw);
+        double chk = 0.0;   // stage 4: NaN after a non-finite value
+        auto comp = [&](auto kc) {
+            constexpr int K = decltype(kc)::value;
+            constexpr int C = C0 + K;
+            constexpr bool FORCE = ST < 4 && (C == 0 || C == 3);   // feeds the next stage's force
+            cpx<T> v[8];
+            {
+                const int jh = hidden(j);
+#pragma unroll
+                for (int s = 0; s < 8; s++) {
+                    const int lx = jh + TPL * s;
+                    const bool z = lx >= zx0 && lx <= zx1;
+                    if (ST == 1 && z) v0[s] = mk<double>(0, 0);
+                    const double E = visc[0][s * NTH + threadIdx.x];
+                    const double E1 = ST == 1 ? visc[ST == 1][s * NTH + threadIdx.x] : 0.0;
+                    cpx<double> vn;
+                    lawson<ST>(v0[s], PHASE == 0 ? rt[PHASE == 0 ? s : 0] : cvt<double>(N[K][s]), E, E1, rp.dt, ac[s], vn);
+                    if (ST == 4) {
+                        chk += 0.0 * vn.x + 0.0 * vn.y;
+                        settle(chk);
+                    }
+                    // the undealiased value is this field's share of the next force
+                    if (FORCE) v0[s] = vn;
+                    v[s] = z ? mk<T>(0, 0) : cvt<T>(vn);
+                    settle(v[s]);
+                    settle(ac[s]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            pin_memory_order();
+            if (FORCE && t.live)
+                col_store<false>(v0, (cpx<double> *)a.f_out[PHASE == 0 ? 0 : 1] + t.state0, t.steps, t.offs);
+            if (K + 1 < NC) col_load<false>(v0, (const cpx<double> *)a.V[K + 1 < NC ? C + 1 : C] + t.state0, t.steps, t.offs);
+            if (ST == 4) {
+                if (t.live) col_store<false>(ac, (cpx<double> *)a.V[C] + t.state0, t.steps, t.offs);
+            } else if (t.inside) {
+                col_store<NTA>(ac, (cpx<double> *)a.acc[C] + t.cw0, t.stepw, t.offw);
+            }
+            if (ST >= 2 && K + 1 < NC)
+                col_load<NTA>(ac, (const cpx<double> *)a.acc[K + 1 < NC ? C + 1 : C] + t.cw0, t.stepw, t.offw);
+            pin_memory_order();
+            sc_inverse<L>(v, x, tw.tw, tw.twq, hidden(j), C == 0 || C == 3);
+            pin_memory_order();
+            if (t.inside) t.template store<NTW>(v, a.U[C]);
+        };
+        comp(std::integral_constant<int, 0>{});
+        if constexpr (NC > 1) {
+            comp(std::integral_constant<int, (NC > 1 ? 1 : 0)>{});
+            comp(std::integral_constant<int, (NC > 2 ? 2 : 0)>{});
+        }
+        if (ST == 4 && chk != 0.0 && t.live && rp.nonfinite) *rp.nonfinite = 1;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -642,7 +592,7 @@ __global__ void k_sff_reality(SffPlaneArgs a)
 template <typename T, int LL>
 hipError_t xinv_sc_len(const XscArgs &a, hipStream_t st)
 {
-    constexpr int CB = col_block<T>(LL, sizeof(cpx<double>));
+    constexpr int CB = colx_block<T>(LL, 512);
     hipLaunchKernelGGL((k_xinv_sc<T, LL, CB>), dim3(x_grid(x_tiles(a.g, CB, (a.flags & 4) != 0))),
                        dim3(CB * (LL / 8)), 0, st, a);
     return hipGetLastError();
@@ -651,7 +601,7 @@ hipError_t xinv_sc_len(const XscArgs &a, hipStream_t st)
 template <typename T, int LL>
 hipError_t xfwd_sc_len(const XscArgs &a, hipStream_t st)
 {
-    constexpr int CB = col_block<T>(LL, sizeof(cpx<double>));
+    constexpr int CB = colx_block<T>(LL, 512);
     hipLaunchKernelGGL((k_xfwd_sc<T, LL, CB>), dim3(x_grid(x_tiles(a.g, CB, false))), dim3(CB * (LL / 8)), 0, st, a);
     return hipGetLastError();
 }
@@ -670,14 +620,33 @@ hipError_t z_rbc_len(const ZArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
+template <typename T, int LL, int ST>
+hipError_t x_rbc_launch(const XrbcArgs &a, hipStream_t st)
+{
+    constexpr int CB = colx_block<T>(LL, 512);
+    const bool nt = stream_bytes((size_t)12 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
+    constexpr bool NT = ST > 0 && LL >= kStreamLength;
+    const dim3 grid(x_grid(x_tiles(a.g, CB, false))), block(CB * (LL / 8));
+    if (NT && nt) {
+        hipLaunchKernelGGL((k_x_rbc<T, LL, CB, 0, ST, NT>), grid, block, 0, st, a);
+        hipLaunchKernelGGL((k_x_rbc<T, LL, CB, 1, ST, NT>), grid, block, 0, st, a);
+    } else {
+        hipLaunchKernelGGL((k_x_rbc<T, LL, CB, 0, ST, false>), grid, block, 0, st, a);
+        hipLaunchKernelGGL((k_x_rbc<T, LL, CB, 1, ST, false>), grid, block, 0, st, a);
+    }
+    return hipGetLastError();
+}
+
 template <typename T, int LL>
 hipError_t x_rbc_len(const XrbcArgs &a, hipStream_t st)
 {
-    constexpr int CB = col_block<T>(LL, 2 * sizeof(cpx<double>));
-    const dim3 grid(x_grid(x_tiles(a.g, CB, false)));
-    hipLaunchKernelGGL((k_x_rbc<T, LL, CB, 0>), grid, dim3(CB * (LL / 8)), 0, st, a);
-    hipLaunchKernelGGL((k_x_rbc<T, LL, CB, 1>), grid, dim3(CB * (LL / 8)), 0, st, a);
-    return hipGetLastError();
+    switch (a.rp.stage) {
+        case 1: return x_rbc_launch<T, LL, 1>(a, st);
+        case 2: return x_rbc_launch<T, LL, 2>(a, st);
+        case 3: return x_rbc_launch<T, LL, 3>(a, st);
+        case 4: return x_rbc_launch<T, LL, 4>(a, st);
+        default: return x_rbc_launch<T, LL, 0>(a, st);
+    }
 }
 
 #define TG_SFF_L(N, T, P)                                                   \
