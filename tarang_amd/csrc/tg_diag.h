@@ -33,10 +33,11 @@ struct RedAniso {
     int bin_lo;
 };
 
+// cut (the modes with B): of the modes beyond it neither field is read.
 hipError_t launch_reduce(const Grid &g, int mode, const double *const *A, const double *const *B, int ncomp, int n,
                          const double *radii_dev, int nbins, int nq, int kcut, double r_lo, double r_hi,
                          double *partial, int nblocks, double *out_dev, hipStream_t st,
-                         const RedAniso *an = nullptr);
+                         const RedAniso *an = nullptr, const Cut *cut = nullptr);
 
 hipError_t launch_init_field(const Grid &g, double *const *V, int kind, double k0, double kmin, double kmax,
                              uint64_t seed, hipStream_t st);

@@ -65,6 +65,7 @@ struct RedArgs {
     int mode, ncomp, n, nbins, nq, kcut;  // kcut: Max_radius_inside (mode SHELL_ALL) / Min_radius_outside
     double r_lo, r_hi;
     RedAniso an;
+    Cut cut;
 };
 
 constexpr int kRedThreads = 256;
@@ -145,11 +146,13 @@ __global__ void __launch_bounds__(kRedThreads) k_reduce(RedArgs a)
     // across the wavefront)
     for (size_t i0 = beg; i0 < end; i0 += blockDim.x) {
         const size_t i = i0 + threadIdx.x;
-        const bool valid = i < end;
+        bool valid = i < end;
         const size_t ii = valid ? i : beg;
         const int lz = ii % g.nzc;
         const int ly = (ii / g.nzc) % g.ny;
         const int lx = ii / ((size_t)g.nzc * g.ny);
+        if (MODE == RED_SHELL_SINGLE || MODE == RED_RING_MULT || MODE == RED_CYL_MULT)
+            valid = valid && abs(kw(lx, g.nx)) <= a.cut.x && abs(kw(ly, g.ny)) <= a.cut.y && lz <= a.cut.z;
         // FFF: w = 1/2 on kz = 0 (FFF_pencil_energy.cc:59-68); SFF: 2 sum - kz=0
         // plane - kx=0 plane + half the kx=0,kz=0 line (SFF_pencil_energy.cc:
         // 88-104), i.e. w = (lx ? 2 : 1)(lz ? 2 : 1)/2
@@ -282,15 +285,17 @@ __global__ void __launch_bounds__(kRedThreads) k_reduce_rows(RedArgs a)
     for (int i = threadIdx.x; i < 2 * NW * NQ * nb; i += blockDim.x) dyn[i] = 0.0;
     __syncthreads();
     double *bsum = dyn + (size_t)wave * NQ * nb, *bcmp = dyn + (size_t)(NW + wave) * NQ * nb;
-    const long long nrows = (long long)g.nx * g.ny;
+    const int ny = kept(g.ny, a.cut.y), nzc = min(g.nzc, a.cut.z + 1);
+    const long long nrows = (long long)kept(g.nx, a.cut.x) * ny;
     const long long chunk = (nrows + gridDim.x - 1) / gridDim.x;
     const long long end = min(nrows, (long long)(blockIdx.x + 1) * chunk);
-    for (long long row = blockIdx.x * chunk + wave; row < end; row += NW) {
-        const int lx = (int)(row / g.ny), ly = (int)(row % g.ny);
-        for (int l0 = 0; l0 < g.nzc; l0 += 64) {
+    for (long long r = blockIdx.x * chunk + wave; r < end; r += NW) {
+        const int lx = kept_index((int)(r / ny), g.nx, a.cut.x), ly = kept_index((int)(r % ny), g.ny, a.cut.y);
+        const size_t row = (size_t)lx * g.ny + ly;
+        for (int l0 = 0; l0 < nzc; l0 += 64) {
             const int lz = l0 + lane;
-            const bool valid = lz < g.nzc;
-            const size_t ii = (size_t)row * g.nzc + min(lz, g.nzc - 1);
+            const bool valid = lz < nzc;
+            const size_t ii = row * g.nzc + min(lz, nzc - 1);
             const double K = kmag_l(g, lx, ly, lz);
             const double m = multiplicity(g, lx, ly, lz);
             int bin;
@@ -362,9 +367,12 @@ __global__ void __launch_bounds__(256) k_reduce_final(const double *partial, int
 
 hipError_t launch_reduce(const Grid &g, int mode, const double *const *A, const double *const *B, int ncomp,
                          int n, const double *radii_dev, int nbins, int nq, int kcut, double r_lo, double r_hi,
-                         double *partial, int nblocks, double *out_dev, hipStream_t st, const RedAniso *an)
+                         double *partial, int nblocks, double *out_dev, hipStream_t st, const RedAniso *an,
+                         const Cut *cut)
 {
     RedArgs a{};
+    if (cut && !B) return hipErrorInvalidValue;
+    a.cut = cut ? *cut : cut_none(g);
     if (an) a.an = *an;
     for (int c = 0; c < ncomp; c++) {
         a.A[c] = A[c];

@@ -16,6 +16,25 @@ struct Grid {
     int basis;            // 0 FFF; 1 SFF (sin/cos along x: kx = lx, K_x = lx*kf[0])
 };
 
+// The modes that a pass has to deal with: beyond |kx| <= x, |ky| <= y, kz <= z
+// its input is zero (and need not be there), or its output is not used (and is
+// not written).  The lines beyond the box cost nothing; rows of kz are cut at
+// 128-byte lines.
+struct Cut {
+    int x, y, z;
+};
+__host__ inline Cut cut_none(const Grid &g) { return {g.nx / 2, g.ny / 2, g.nz / 2}; }
+// the indices of an axis of n with |k| <= c: their number, and the i-th of them
+__host__ __device__ inline int kept(int n, int c) { return c >= n / 2 ? n : 2 * c + 1; }
+__host__ __device__ inline int kept_index(int i, int n, int c) { return i <= c ? i : i + n - kept(n, c); }
+// columns of a row of a work field of cpx<T> (whole 128-byte lines)
+template <typename T>
+__host__ __device__ inline int kept_columns(const Grid &g, int z)
+{
+    constexpr int line = 128 / (2 * (int)sizeof(T));
+    return z >= g.nz / 2 ? g.nzp : (z / line + 1) * line;
+}
+
 // Forcing band: slots for the modes of the box |kx| <= h[0], |ky| <= h[1],
 // 0 <= kz <= h[2].
 struct Band {
@@ -35,9 +54,11 @@ __host__ __device__ inline int band_nslots(const Band &b) { return (2 * b.h[0] +
 
 // Launch helpers (defined in tg_kernels.hip).  All return hipError_t.
 // T is float or double (transform precision).
+// cut: along y (axis 1), inverse: the rows and columns beyond it are zero and
+// not read; forward: they are not written.
 template <typename T>
 hipError_t launch_colfft(const Grid &g, int axis, int dir, void *const *fields, int nfields,
-                         const void *tw, hipStream_t st);
+                         const void *tw, hipStream_t st, const Cut *cut = nullptr);
 
 // x-inverse of an FP64 spectral field set into the T work layout.
 //   flags: 1 = dealias on read, 2 = write band slots, 4 = reality patch
@@ -45,10 +66,12 @@ hipError_t launch_colfft(const Grid &g, int axis, int dir, void *const *fields, 
 //   16 = keep the ring r_lo < K <= r_hi, a_lo < theta <= a_hi (polar angle
 //   to the axis dirn), 32 = keep the cylindrical ring r_lo < K <= r_hi,
 //   a_lo < Kpll <= a_hi.
+// cut: nothing is kept beyond it, and nothing written there.
 template <typename T>
 hipError_t launch_xinv_state(const Grid &g, const Band &b, double *const *V, int ncomp, void *const *U,
                              double *slots, int flags, const void *twx, hipStream_t st, double r_lo = 0.0,
-                             double r_hi = 0.0, double a_lo = 0.0, double a_hi = 0.0, int dirn = 3);
+                             double r_hi = 0.0, double a_lo = 0.0, double a_hi = 0.0, int dirn = 3,
+                             const Cut *cut = nullptr);
 
 // x-forward of T work fields into FP64 spectral outputs, scaled.
 template <typename T>
@@ -74,9 +97,11 @@ hipError_t launch_z_r2c(const Grid &g, const double *const *R, int ncomp, void *
 // only used projected).
 // tape (NS form only): also store the three real velocity lines, each line as
 // Nz/2 packed points (x[2n] + i x[2n+1]) at line*(Nz/2).
+// in_u, in_w, out (giver 1): cuts of the two fields and of the products in kz.
 template <typename T>
 hipError_t launch_z_products(const Grid &g, void *const *U, void *const *P, int giver, const void *twm,
-                             const void *twn, hipStream_t st, void *const *tape = nullptr);
+                             const void *twn, hipStream_t st, void *const *tape = nullptr, const Cut *in_u = nullptr,
+                             const Cut *in_w = nullptr, const Cut *out = nullptr);
 
 struct RkParams {
     int stage;            // 1..4; 0 = write the nonlinear term only; -1 = giver
@@ -94,10 +119,11 @@ struct RkParams {
 
 // Fused x pass: forward x-FFT of the 6 (giver: 9) products, nonlinear term, RHS and the
 // Lawson RK4 stage algebra, next stage input, dealias, inverse x-FFT.
+// cut (giver form): only the columns within it are read and written.
 template <typename T>
 hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void *const *P, double *const *V,
                          double *const *acc, void *const *U, const double *slots_in, double *slots_out,
-                         double *const *out, const void *twx, hipStream_t st);
+                         double *const *out, const void *twx, hipStream_t st, const Cut *cut = nullptr);
 
 // the random force (kind 2) of the band's slots, 3 complex values each
 hipError_t launch_random_force(const Grid &g, const Band &b, double *out, hipStream_t st);

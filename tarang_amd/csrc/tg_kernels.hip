@@ -36,6 +36,7 @@ struct ColArgs {
     long long row_stride;    // elements between consecutive rows (transform axis)
     int ncol;                // contiguous columns per row
     int nouter;
+    int keep;                // CUT: rows |k| <= keep
 };
 
 // Bound by HBM (each field read and written once).  A thread's row segment and
@@ -43,7 +44,8 @@ struct ColArgs {
 // the exchanges between the radix passes; 512^3 FP64, per field: 476 us with
 // the tile staged through LDS both ways, 381 us (5.7 TB/s, a copy's 6.2) with
 // this layout, whole rows and non-temporal access.
-template <typename T, int L, int DIR, int CB, bool NT>
+// CUT: of the rows |k| > keep nothing is read (inverse) or written (forward).
+template <typename T, int L, int DIR, int CB, bool NT, bool CUT>
 __global__ void __launch_bounds__(CB *(L / 8)) k_colfft(ColArgs a)
 {
     constexpr int TPL = L / 8;
@@ -64,12 +66,16 @@ __global__ void __launch_bounds__(CB *(L / 8)) k_colfft(ColArgs a)
     const size_t step = (size_t)TPL * a.row_stride;
     cpx<T> v[8];
 #pragma unroll
-    for (int s = 0; s < 8; s++) v[s] = gload<NT>(p + s * step);
+    for (int s = 0; s < 8; s++) {
+        v[s] = mk<T>(0, 0);
+        if (!CUT || DIR < 0 || abs(kwave(j + TPL * s, L)) <= a.keep) v[s] = gload<NT>(p + s * step);
+    }
     const X x{lds + c};
     fft_exchange<L, DIR>(v, x, (const cpx<T> *)a.tw, j);
     if (col < a.ncol) {
 #pragma unroll
-        for (int s = 0; s < 8; s++) gstore<NT>(p + s * step, v[s]);
+        for (int s = 0; s < 8; s++)
+            if (!CUT || DIR > 0 || abs(kwave(j + TPL * s, L)) <= a.keep) gstore<NT>(p + s * step, v[s]);
     }
 }
 
@@ -91,11 +97,12 @@ struct XinvArgs {
     // (Fill_array_cylindrical_ring); theta, Kpll about the axis dirn
     double a_lo, a_hi;
     int dirn;
+    Cut cut;
 };
 
 // Columns go from memory to registers and back in transform order; a column
 // without a mode to keep is not read.  One field at 256^3 FP64: 123 us with the
-// tiles staged through LDS, now 85.  FILTER: flags & (8 | 16 | 32).
+// tiles staged through LDS, now 85.  FILTER: flags & (8 | 16 | 32), cut.
 template <typename T, int L, int CB, bool FILTER>
 __global__ void __launch_bounds__(CB *(L / 8)) k_xinv_state(XinvArgs a)
 {
@@ -106,8 +113,8 @@ __global__ void __launch_bounds__(CB *(L / 8)) k_xinv_state(XinvArgs a)
     const Grid &g = a.g;
     const bool patch = (a.flags & 4) != 0;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    if (tile >= x_tiles(g, CB, patch)) return;
-    const ColTile<T, L, CB> t(g, tile, patch);
+    if (tile >= (FILTER ? x_tiles_cut<T>(g, CB, a.cut) : x_tiles(g, CB, patch))) return;
+    const ColTile<T, L, CB> t(g, FILTER ? x_tile_cut<T>(g, CB, a.cut, tile) : tile, patch);
     const int j = t.j, ky = kwave(t.ly, g.ny), lz = t.lz;
     int zx0 = 1, zx1 = 0;
     if (a.flags & 1) dealias_rows(g, t.ly, lz, zx0, zx1);
@@ -294,9 +301,11 @@ __global__ void __launch_bounds__(256, (sizeof(T) == 4 && !GIVER && M == 256) ? 
     cpx<T> *L = lds + li * LP;
     // the three input lines are loaded before the first transform: their
     // loads are in flight together
+    constexpr bool LIM = GIVER && !FIVE;
     cpx<T> u[3][8], xm[3];
 #pragma unroll
-    for (int c = 0; c < 3; c++) zline_load<T, M, NT>(u[c], xm[c], (const cpx<T> *)a.in[c] + lsafe * a.g.nzp, j);
+    for (int c = 0; c < 3; c++)
+        zline_load<T, M, NT, LIM>(u[c], xm[c], (const cpx<T> *)a.in[c] + lsafe * a.g.nzp, j, a.lim_u);
     const ZTwiddles<T, M> tw(ldw, a.twm, a.twn);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
@@ -314,7 +323,7 @@ __global__ void __launch_bounds__(256, (sizeof(T) == 4 && !GIVER && M == 256) ? 
     }
     auto emit = [&](cpx<T> *p, int o) {
         cpx<T> *X = (cpx<T> *)a.out[o] + lsafe * a.g.nzp;
-        zline_r2c_post<T, M, NT>(p, X, L, tw, j, valid, a.g.nzp - M);
+        zline_r2c_post<T, M, NT, LIM>(p, X, L, tw, j, valid, a.g.nzp - M, a.lim_out);
     };
     if constexpr (!GIVER && FIVE) {
         // the cross products first, then the two shifted squares (u_z is
@@ -379,7 +388,7 @@ __global__ void __launch_bounds__(256, (sizeof(T) == 4 && !GIVER && M == 256) ? 
 #pragma unroll 1
         for (int i = 0; i < 3; i++) {
             cpx<T> w[8];
-            zline_c2r<T, M, NT>(w, (const cpx<T> *)a.in[3 + i] + lsafe * a.g.nzp, L, tw, j);
+            zline_c2r<T, M, NT, LIM>(w, (const cpx<T> *)a.in[3 + i] + lsafe * a.g.nzp, L, tw, j, a.lim_w);
             line_sync<M / 8>();
 #pragma unroll
             for (int jj = 0; jj < 3; jj++) {
@@ -407,6 +416,7 @@ struct XnlArgs {
     Grid g;
     Band b;
     RkParams rk;
+    Cut cut;   // giver form
 };
 
 // alpha = eps / (2 E_band) with E_band = sum w |V|^2 over the band modes,
@@ -550,8 +560,9 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
     __shared__ double visc[ST == 1 ? 2 : 1][ST ? 8 * CB * TPL : 1];
     const Grid &g = a.g;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    if (tile >= x_tiles(g, CB, false)) return;
-    const ColTile<T, L, CB> t(g, tile);
+    constexpr bool CUT = MODE == XNL_GIVER;
+    if (tile >= (CUT ? x_tiles_cut<T>(g, CB, a.cut) : x_tiles(g, CB, false))) return;
+    const ColTile<T, L, CB> t(g, CUT ? x_tile_cut<T>(g, CB, a.cut, tile) : tile);
     const int j = t.j, ly = t.ly, lz = t.lz, cw0 = t.cw0;
     const bool live = t.live;
     const size_t stepw = t.stepw, steps = t.steps, state0 = t.state0;
@@ -846,13 +857,20 @@ hipError_t colfft_len(const ColArgs &a, int dir, int nfields, hipStream_t st)
     dim3 grid(x_grid(a.nouter * ((a.ncol + CB - 1) / CB)), nfields);
     const dim3 block(CB * (LL / 8));
     const bool nt = STREAM && stream_bytes((size_t)nfields * a.nouter * a.outer_stride * sizeof(cpx<T>));
-    if (dir < 0) {
-        if (nt) hipLaunchKernelGGL((k_colfft<T, LL, -1, CB, STREAM>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((k_colfft<T, LL, -1, CB, false>), grid, block, 0, st, a);
-    } else {
-        if (nt) hipLaunchKernelGGL((k_colfft<T, LL, +1, CB, STREAM>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((k_colfft<T, LL, +1, CB, false>), grid, block, 0, st, a);
-    }
+    const bool cut = a.keep < LL / 2;
+    auto go = [&](auto dc, auto ntc) {
+        constexpr int DIR = decltype(dc)::value;
+        constexpr bool NT = decltype(ntc)::value;
+        if (cut) hipLaunchKernelGGL((k_colfft<T, LL, DIR, CB, NT, true>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_colfft<T, LL, DIR, CB, NT, false>), grid, block, 0, st, a);
+    };
+    using fwd = std::integral_constant<int, -1>;
+    using inv = std::integral_constant<int, +1>;
+    using stream = std::bool_constant<STREAM>;
+    if (dir < 0 && nt) go(fwd{}, stream{});
+    else if (dir < 0) go(fwd{}, std::false_type{});
+    else if (nt) go(inv{}, stream{});
+    else go(inv{}, std::false_type{});
     return hipGetLastError();
 }
 
@@ -861,7 +879,8 @@ hipError_t xinv_state_len(const XinvArgs &a, hipStream_t st)
 {
     constexpr int CB = colx_block<T>(LL, 512);
     const dim3 grid(x_grid(x_tiles(a.g, CB, (a.flags & 4) != 0))), block(CB * (LL / 8));
-    if (a.flags & 56) hipLaunchKernelGGL((k_xinv_state<T, LL, CB, true>), grid, block, 0, st, a);
+    if (a.flags & 56)
+        hipLaunchKernelGGL((k_xinv_state<T, LL, CB, true>), dim3(x_grid(x_tiles_cut<T>(a.g, CB, a.cut))), block, 0, st, a);
     else hipLaunchKernelGGL((k_xinv_state<T, LL, CB, false>), grid, block, 0, st, a);
     return hipGetLastError();
 }
@@ -928,7 +947,7 @@ hipError_t x_nlin_launch(const XnlArgs &a, hipStream_t st)
     // was relieved).
     constexpr int CB = colx_block<T>(LL, 512);
     const bool nt = stream_bytes((size_t)8 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
-    const dim3 grid(x_grid(x_tiles(a.g, CB, false))), block(CB * (LL / 8));
+    const dim3 grid(x_grid(MODE == XNL_GIVER ? x_tiles_cut<T>(a.g, CB, a.cut) : x_tiles(a.g, CB, false))), block(CB * (LL / 8));
     constexpr bool NT = LL >= kStreamLength && (ST > 0 || MODE == XNL_GIVER);
     if (NT && nt) hipLaunchKernelGGL((k_x_nlin<T, LL, CB, MODE, ST, NT>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((k_x_nlin<T, LL, CB, MODE, ST, false>), grid, block, 0, st, a);
@@ -965,7 +984,7 @@ TG_ALL_UNITS(TG_KERNELS_L, TG_KERNELS_M, extern)
 
 template <typename T>
 hipError_t launch_colfft(const Grid &g, int axis, int dir, void *const *fields, int nfields, const void *tw,
-                         hipStream_t st)
+                         hipStream_t st, const Cut *cut)
 {
     ColArgs a{};
     for (int i = 0; i < nfields; i++) a.f[i] = fields[i];
@@ -979,9 +998,12 @@ hipError_t launch_colfft(const Grid &g, int axis, int dir, void *const *fields, 
         // the pad columns too (they hold zeros): a row's last 128-byte line is
         // written whole (257 of 264 columns written: 1903 us a launch at 512^3
         // FP64, all 264: 1780)
-        a.ncol = g.nzp;
+        a.ncol = cut ? kept_columns<T>(g, cut->z) : g.nzp;
+        a.keep = cut ? cut->y : L;
     } else {
+        if (cut) return hipErrorInvalidValue;
         L = g.nx;
+        a.keep = L;
         a.nouter = 1;
         a.outer_stride = 0;
         a.row_stride = (long long)g.ny * g.nzp;
@@ -994,9 +1016,11 @@ hipError_t launch_colfft(const Grid &g, int axis, int dir, void *const *fields, 
 template <typename T>
 hipError_t launch_xinv_state(const Grid &g, const Band &b, double *const *V, int ncomp, void *const *U,
                              double *slots, int flags, const void *twx, hipStream_t st, double r_lo, double r_hi,
-                             double a_lo, double a_hi, int dirn)
+                             double a_lo, double a_hi, int dirn, const Cut *cut)
 {
     XinvArgs a{};
+    if (cut && !(flags & 56)) return hipErrorInvalidValue;
+    a.cut = cut ? *cut : cut_none(g);
     a.r_lo = r_lo;
     a.r_hi = r_hi;
     a.a_lo = a_lo;
@@ -1057,9 +1081,14 @@ hipError_t launch_z_r2c(const Grid &g, const double *const *R, int ncomp, void *
 
 template <typename T>
 hipError_t launch_z_products(const Grid &g, void *const *U, void *const *P, int giver, const void *twm,
-                             const void *twn, hipStream_t st, void *const *tape)
+                             const void *twn, hipStream_t st, void *const *tape, const Cut *in_u, const Cut *in_w,
+                             const Cut *out)
 {
     ZArgs a{};
+    if ((in_u || in_w || out) && giver != 1) return hipErrorInvalidValue;
+    a.lim_u = in_u ? kept_columns<T>(g, in_u->z) : g.nzp;
+    a.lim_w = in_w ? kept_columns<T>(g, in_w->z) : g.nzp;
+    a.lim_out = out ? kept_columns<T>(g, out->z) : g.nzp;
     // giver 2: the NS form with the five trace-shifted products; 3: the giver
     // form with the eight trace-shifted ones (MHD stage)
     a.ncomp = giver == 2 ? 5 : (giver == 3 ? 8 : (giver == 1 ? 9 : 6));
@@ -1078,9 +1107,11 @@ hipError_t launch_z_products(const Grid &g, void *const *U, void *const *P, int 
 template <typename T>
 hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void *const *P, double *const *V,
                          double *const *acc, void *const *U, const double *slots_in, double *slots_out,
-                         double *const *out, const void *twx, hipStream_t st)
+                         double *const *out, const void *twx, hipStream_t st, const Cut *cut)
 {
     XnlArgs a{};
+    if (cut && rk.stage != -1) return hipErrorInvalidValue;
+    a.cut = cut ? *cut : cut_none(g);
     // rk.stage -1: giver form, -2: transposed giver form (nonlinear term only)
     const int giver = rk.stage == -1 ? 1 : (rk.stage == -2 ? 2 : 0);
     for (int i = 0; i < (giver ? 9 : 6); i++) a.P[i] = P[i];
@@ -1140,10 +1171,11 @@ hipError_t launch_dealias(const Grid &g, double *const *V, int ncomp, hipStream_
 }
 
 #define TG_INST(T)                                                                                              \
-    template hipError_t launch_colfft<T>(const Grid &, int, int, void *const *, int, const void *, hipStream_t); \
+    template hipError_t launch_colfft<T>(const Grid &, int, int, void *const *, int, const void *, hipStream_t, \
+                                         const Cut *);                                                         \
     template hipError_t launch_xinv_state<T>(const Grid &, const Band &, double *const *, int, void *const *,   \
                                              double *, int, const void *, hipStream_t, double, double, double, \
-                                             double, int);                                                     \
+                                             double, int, const Cut *);                                                     \
     template hipError_t launch_xfwd_spec<T>(const Grid &, void *const *, int, double *const *, double,          \
                                             const void *, hipStream_t);                                        \
     template hipError_t launch_z_c2r<T>(const Grid &, void *const *, int, double *const *, const void *,        \
@@ -1151,10 +1183,11 @@ hipError_t launch_dealias(const Grid &g, double *const *V, int ncomp, hipStream_
     template hipError_t launch_z_r2c<T>(const Grid &, const double *const *, int, void *const *, const void *,  \
                                         const void *, hipStream_t);                                            \
     template hipError_t launch_z_products<T>(const Grid &, void *const *, void *const *, int, const void *,     \
-                                             const void *, hipStream_t, void *const *);                        \
+                                             const void *, hipStream_t, void *const *, const Cut *, const Cut *, \
+                                             const Cut *);                        \
     template hipError_t launch_x_nlin<T>(const Grid &, const Band &, const RkParams &, void *const *,           \
                                          double *const *, double *const *, void *const *, const double *,      \
-                                         double *, double *const *, const void *, hipStream_t);
+                                         double *, double *const *, const void *, hipStream_t, const Cut *);
 
 TG_INST(double)
 TG_INST(float)

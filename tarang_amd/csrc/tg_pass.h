@@ -143,6 +143,22 @@ __host__ __device__ inline int x_tiles(const Grid &g, int CB, bool patch)
     return patch ? (2 * g.ny + CB - 1) / CB : (g.ny * g.nzp + CB - 1) / CB;
 }
 
+// Tiles of the columns that a cut keeps, and the place of one of them among
+// all tiles.  Tiles wider than a row's 128-byte lines are not cut.
+template <typename T>
+__host__ __device__ inline int x_tiles_cut(const Grid &g, int CB, const Cut &c)
+{
+    if (CB * (int)sizeof(cpx<T>) > 128) return x_tiles(g, CB, false);
+    return kept(g.ny, c.y) * (kept_columns<T>(g, c.z) / CB);
+}
+template <typename T>
+__device__ __forceinline__ int x_tile_cut(const Grid &g, int CB, const Cut &c, int tile)
+{
+    if (CB * (int)sizeof(cpx<T>) > 128) return tile;
+    const int per = kept_columns<T>(g, c.z) / CB;
+    return kept_index(tile / per, g.ny, c.y) * (g.nzp / CB) + tile % per;
+}
+
 __host__ inline int x_grid(int ntiles) { return 8 * ((ntiles + 7) / 8); }
 
 // ---------------------------------------------------------------------------
@@ -320,13 +336,18 @@ struct ZTwiddles {
 
 // The M+1 points of a complex line: v[s] = X[j + TPL*s], xm = X[M] (read by
 // every thread of the line; member-wise copies keep v in registers).
-template <typename T, int M, bool NT = false>
-__device__ __forceinline__ void zline_load(cpx<T> *v, cpx<T> &xm, const cpx<T> *__restrict__ X, int j)
+// LIM: the points from lim on are zero and not read.
+template <typename T, int M, bool NT = false, bool LIM = false>
+__device__ __forceinline__ void zline_load(cpx<T> *v, cpx<T> &xm, const cpx<T> *__restrict__ X, int j, int lim = 0)
 {
     constexpr int TPL = M / 8;
 #pragma unroll
-    for (int s = 0; s < 8; s++) v[s] = gload<NT>(X + j + TPL * s);
-    xm = gload<false>(X + M);
+    for (int s = 0; s < 8; s++) {
+        v[s] = mk<T>(0, 0);
+        if (!LIM || j + TPL * s < lim) v[s] = gload<NT>(X + j + TPL * s);
+    }
+    xm = mk<T>(0, 0);
+    if (!LIM || M < lim) xm = gload<false>(X + M);
 }
 
 // c2r of a line already loaded by zline_load (v in, samples out in v).
@@ -355,20 +376,20 @@ __device__ __forceinline__ void zline_c2r_from(cpx<T> *v, cpx<T> xm, cpx<T> *lds
     fft_line<M, +1>(v, lds, tw.m, j);
 }
 
-template <typename T, int M, bool NT = false>
+template <typename T, int M, bool NT = false, bool LIM = false>
 __device__ __forceinline__ void zline_c2r(cpx<T> *v, const cpx<T> *__restrict__ X, cpx<T> *lds,
-                                          const ZTwiddles<T, M> &tw, int j)
+                                          const ZTwiddles<T, M> &tw, int j, int lim = 0)
 {
     cpx<T> xm;
-    zline_load<T, M, NT>(v, xm, X, j);
+    zline_load<T, M, NT, LIM>(v, xm, X, j, lim);
     zline_c2r_from<T, M>(v, xm, lds, tw, j);
 }
 
 // The line's npad = nzp - M entries from X[M] on are written too (zeros after
-// X[M]): whole 128-byte lines.
-template <typename T, int M, bool NT = false>
+// X[M]): whole 128-byte lines.  LIM: only the points before lim are written.
+template <typename T, int M, bool NT = false, bool LIM = false>
 __device__ __forceinline__ void zline_r2c_post(cpx<T> *v, cpx<T> *__restrict__ X, cpx<T> *lds,
-                                               const ZTwiddles<T, M> &tw, int j, bool store, int npad)
+                                               const ZTwiddles<T, M> &tw, int j, bool store, int npad, int lim = 0)
 {
     constexpr int TPL = M / 8;
     fft_line<M, -1>(v, lds, tw.m, j);
@@ -386,9 +407,9 @@ __device__ __forceinline__ void zline_r2c_post(cpx<T> *v, cpx<T> *__restrict__ X
         const cpx<T> d = zk - conj(zm);
         const cpx<T> w = tw.n[k];
         const cpx<T> e = d * w;  // W^k d
-        if (store) gstore<NT>(X + k, mk<T>(h * (a.x + e.y), h * (a.y - e.x)));
+        if (store && (!LIM || k < lim)) gstore<NT>(X + k, mk<T>(h * (a.x + e.y), h * (a.y - e.x)));
     }
-    if (store)
+    if (store && (!LIM || M < lim))
         for (int i = j; i < npad; i += TPL) gstore<NT>(X + M + i, mk<T>(i == 0 ? z0.x - z0.y : (T)0, (T)0));
     line_sync<M / 8>();
 }
@@ -400,6 +421,7 @@ struct ZArgs {
     const void *twm, *twn;
     Grid g;
     int ncomp;
+    int lim_u, lim_w, lim_out;  // giver form: columns of the fields and products that are dealt with
 };
 
 template <int M>

@@ -122,3 +122,29 @@ def test_transforms_keep_and_drop_modes(N, prec):
     want = o.shell_to_shell([v.copy() for v in V], radii)
     assert rel_l2(got, want) <= 1e-11
     b.close()
+
+
+@pytest.mark.parametrize("N,prec,kf", [((64, 24, 48), api.PREC_FP64, (1.0, 1.0, 1.0)), ((120, 40, 80), api.PREC_FP64, (1.0, 2.0, 0.5)),
+                                       ((32, 16, 16), api.PREC_FP64, (1.0, 1.0, 1.0)), ((64, 16, 128), api.PREC_FP64, (1.0, 1.0, 1.0)),
+                                       ((128, 32, 64), api.PREC_FP32, (1.0, 1.0, 1.0))])
+def test_transfers_of_cut_fields(N, prec, kf):
+    """Flux, shell and ring transfers only form the modes that the 2/3 rule and
+    the giver's radius keep; without the rule, the giver's radius alone."""
+    log(f"cut transfers {N} {prec} {kf}")
+    # FP64 as the other transfer tests; FP32 products round at 1e-7 of a term, the sums cancel some digits
+    tol = 1e-11 if prec == api.PREC_FP64 else 1e-4
+    for dealias in (to.DEALIAS_TWOTHIRDS, to.DEALIAS_REF_CORNER):
+        o = to.Oracle(N, kfactor=kf, dealias=dealias)
+        V = o.init_field(kind=1, kmin=0.5, kmax=max(N), energy=0.5, seed=9)
+        b = api.FFF_Basis(N, kfactor=kf, precision=prec, dealias=dealias)
+        U = api.FluidVF(b)
+        U.set_field([dev(v) for v in V])
+        radii = np.array([0.0, 0.75, 2.0, 5.0, 9.0, np.inf])
+        # work buffers of an earlier call hold what they like
+        b.Inverse_transform(dev(np.full(o.cshape, 1e200 + 0j)), b.real_array())
+        et = api.EnergyTr(b, radii, radii)
+        flux, S = et.Compute_flux_and_shell_tr(U)
+        assert rel_l2(S, o.shell_to_shell([v.copy() for v in V], radii)) <= tol
+        assert rel_l2(flux, o.flux([v.copy() for v in V], radii)) <= tol
+        assert rel_l2(et.Compute_flux(U), o.flux([v.copy() for v in V], radii)) <= tol
+        b.close()
