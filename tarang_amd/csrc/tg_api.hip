@@ -115,7 +115,7 @@ struct tg_plan {
     // product arrays, Helmholtz scratch, the homogeneous solutions p+-,
     // u_x+- and the influence matrix (for the stored nu, dt)
     struct Chff {
-        double *tmp = nullptr, *D = nullptr, *S = nullptr, *NL[3] = {}, *R[4] = {}, *X = nullptr, *Y = nullptr;
+        double *D = nullptr, *NL[3] = {}, *X = nullptr, *Y = nullptr;
         double *pp = nullptr, *pm = nullptr, *vxp = nullptr, *vxm = nullptr, *M = nullptr;
         double infl_nu = -1.0, infl_dt = -1.0;
     } ch;
@@ -236,8 +236,8 @@ void free_plan(tg_plan *p)
                      p->umax_dev, p->force_eh, p->force_tab};
     for (void *q : aptrs)
         if (q) (void)hipFree(q);
-    void *cptrs[] = {p->ch.tmp, p->ch.D, p->ch.S, p->ch.NL[0], p->ch.NL[1], p->ch.NL[2], p->ch.R[0], p->ch.R[1],
-                     p->ch.R[2], p->ch.R[3], p->ch.X, p->ch.Y, p->ch.pp, p->ch.pm, p->ch.vxp, p->ch.vxm, p->ch.M};
+    void *cptrs[] = {p->ch.D, p->ch.NL[0], p->ch.NL[1], p->ch.NL[2], p->ch.X, p->ch.Y, p->ch.pp, p->ch.pm,
+                     p->ch.vxp, p->ch.vxm, p->ch.M};
     for (void *q : cptrs)
         if (q) (void)hipFree(q);
     if (p->nonfinite_host) (void)hipHostFree(p->nonfinite_host);
@@ -398,9 +398,8 @@ int run_forward(tg_plan *p, const double *real_dev, double *spec_dev, int sincos
     if (p->g.basis == 1) {
         const double scale = 1.0 / (2.0 * p->g.nx * (double)p->g.ny * p->g.nz);
         Prof pr(p, TG_KERNEL_X_SC);
-        HIPCHK(launch_xfwd_sc<T>(p->g, W, 1, sincos == TG_SC_SIN ? 1 : 0, O, scale, p->twx, p->twq, p->stream));
-        // Chebyshev coefficients: a_0 = A_0, a_k = 2 A_k of the cosine transform
-        if (sincos == TG_SC_CHEB) HIPCHK(launch_cheb_scale(p->g, spec_dev, spec_dev, 2.0, p->stream));
+        HIPCHK(launch_xfwd_sc<T>(p->g, W, 1, sincos == TG_SC_SIN ? 1 : 0, O, scale, p->twx, p->twq, p->stream,
+                                 sincos == TG_SC_CHEB ? 8 : 0));
         return TG_OK;
     }
     const double scale = 1.0 / ((double)p->g.nx * p->g.ny * p->g.nz);
@@ -414,14 +413,10 @@ int run_inverse(tg_plan *p, const double *spec_dev, double *real_dev, int sincos
     double *V[1] = {const_cast<double *>(spec_dev)};
     void *W[1] = {p->U[0]};
     Band nb{};
-    if (sincos == TG_SC_CHEB) {
-        // the cosine coefficients A_0 = a_0, A_k = a_k / 2, into a copy (input preserved)
-        HIPCHK(launch_cheb_scale(p->g, spec_dev, p->ch.tmp, 0.5, p->stream));
-        V[0] = p->ch.tmp;
-    }
     if (p->g.basis == 1) {
         Prof pr(p, TG_KERNEL_X_SC);
-        HIPCHK(launch_xinv_sc<T>(p->g, V, 1, sincos == TG_SC_SIN ? 1 : 0, W, 0, p->twx, p->twq, p->stream));
+        HIPCHK(launch_xinv_sc<T>(p->g, V, 1, sincos == TG_SC_SIN ? 1 : 0, W, sincos == TG_SC_CHEB ? 8 : 0, p->twx, p->twq,
+                                 p->stream));
     } else {
         Prof pr(p, TG_KERNEL_X_INV);
         HIPCHK(launch_xinv_state<T>(p->g, nb, V, 1, W, nullptr, 0, p->twx, p->stream));
@@ -1935,13 +1930,12 @@ int tg_init_field(tg_plan *plan, int kind, double k0, double kmin, double kmax, 
 // ---------------------------------------------------------------------------
 static int ensure_chff(tg_plan *p)
 {
-    const size_t nc16 = p->nc * 16, nr8 = (size_t)p->g.nx * p->g.ny * (p->g.nz + 2) * 8;
-    const size_t ncol = (size_t)p->g.ny * p->g.nzc;
+    const size_t nc16 = p->nc * 16, ncol = (size_t)p->g.ny * p->g.nzc;
+    // X, Y: of two components' solves
     struct { double **q; size_t bytes; } need[] = {
-        {&p->ch.tmp, nc16}, {&p->ch.D, nc16}, {&p->ch.S, nc16}, {&p->ch.NL[0], nc16}, {&p->ch.NL[1], nc16},
-        {&p->ch.NL[2], nc16}, {&p->ch.R[0], nr8}, {&p->ch.R[1], nr8}, {&p->ch.R[2], nr8}, {&p->ch.R[3], nr8},
-        {&p->ch.X, nc16}, {&p->ch.Y, nc16}, {&p->ch.pp, p->nc * 8}, {&p->ch.pm, p->nc * 8},
-        {&p->ch.vxp, p->nc * 8}, {&p->ch.vxm, p->nc * 8}, {&p->ch.M, ncol * 4 * 8}};
+        {&p->ch.D, nc16}, {&p->ch.NL[0], nc16}, {&p->ch.NL[1], nc16}, {&p->ch.NL[2], nc16}, {&p->ch.X, nc16},
+        {&p->ch.Y, 2 * nc16}, {&p->ch.pp, p->nc * 8}, {&p->ch.pm, p->nc * 8}, {&p->ch.vxp, p->nc * 8},
+        {&p->ch.vxm, p->nc * 8}, {&p->ch.M, ncol * 4 * 8}};
     for (auto &n : need)
         if (!*n.q) {
             int rc = dmalloc(p, (void **)n.q, n.bytes);
@@ -1969,28 +1963,23 @@ static HelmArgs helm_args(tg_plan *p, const double *R, double *U, double lam_sup
     return h;
 }
 
-// N_i = sum_j d_j (u_j u_i), Chebyshev x-derivatives (no dealiasing)
-static int chff_nlin(tg_plan *p, double *const V[3], double *const N[3])
+// N_i = sum_j d_j (u_j u_i), Chebyshev x-derivatives (no dealiasing); div: its
+// divergence, if wanted
+static int chff_nlin(tg_plan *p, double *const V[3], double *const N[3], double *div)
 {
-    for (int c = 0; c < 3; c++) {
-        int rc = run_inverse<double>(p, V[c], p->ch.R[c], TG_SC_CHEB);
-        if (rc) return rc;
+    {
+        Prof pr(p, TG_KERNEL_X_SC);
+        HIPCHK(launch_xinv_sc<double>(p->g, V, 3, 0, p->U, 8, p->twx, p->twq, p->stream));
     }
-    static const int pa[6] = {0, 1, 2, 0, 1, 2}, pb[6] = {0, 1, 2, 1, 2, 0};
-    const size_t nr = (size_t)p->g.nx * p->g.ny * (p->g.nz + 2);
-    bool assigned[3] = {false, false, false};
-    for (int q = 0; q < 6; q++) {
-        const int a = pa[q], b = pb[q];
-        HIPCHK(launch_real_product(p->ch.R[a], p->ch.R[b], p->ch.R[3], nr, p->stream));
-        int rc = run_forward<double>(p, p->ch.R[3], p->ch.S, TG_SC_CHEB);
-        if (rc) return rc;
-        for (int t = 0; t < (a == b ? 1 : 2); t++) {
-            const int dst = t == 0 ? a : b, dir = t == 0 ? b : a;
-            if (dir == 0) HIPCHK(launch_cheb_deriv(p->g, p->ch.S, p->ch.D, true, p->stream));
-            HIPCHK(launch_add_deriv(p->g, N[dst], p->ch.S, p->ch.D, dir, !assigned[dst], p->stream));
-            assigned[dst] = true;
-        }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<double>(p->g, 1, +1, p->U, 3, p->twy, p->stream)); }
+    {
+        Prof pr(p, TG_KERNEL_Z_PRODUCTS);
+        HIPCHK(launch_z_products<double>(p->g, p->U, p->P, 0, p->twm, p->twn, p->stream));
     }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<double>(p->g, 1, -1, p->P, 6, p->twy, p->stream)); }
+    Prof pr(p, TG_KERNEL_X_SC);
+    const double scale = 1.0 / (2.0 * p->g.nx * (double)p->g.ny * p->g.nz);
+    HIPCHK(launch_xfwd_chff(p->g, p->P, N, div, scale, p->twx, p->twq, p->stream));
     return TG_OK;
 }
 
@@ -1998,7 +1987,7 @@ static int chff_nlin(tg_plan *p, double *const V[3], double *const N[3])
 static int chff_influence(tg_plan *p, double nu, double dt)
 {
     if (p->ch.infl_nu == nu && p->ch.infl_dt == dt) return TG_OK;
-    double *zero = p->ch.R[3];
+    double *zero = p->ch.NL[0];
     HIPCHK(launch_fill_double(zero, p->nc, 0.0, p->stream));
     const double one[2] = {1.0, 0.0}, nil[2] = {0.0, 0.0};
     double *tmp = p->ch.D;  // real scratch (nc doubles)
@@ -2052,7 +2041,7 @@ int tg_compute_nlin_chff(tg_plan *plan, double *const V_dev[3], double *const nl
     if (!rc) rc = set_device(plan);
     if (!rc) rc = ensure_chff(plan);
     if (rc) return rc;
-    return chff_nlin(plan, V_dev, nlin_dev);
+    return chff_nlin(plan, V_dev, nlin_dev, nullptr);
 }
 
 int tg_bdf1_step(tg_plan *plan, double *const V_dev[3], double *P_dev, const tg_fluid *fluid, int nsteps)
@@ -2071,33 +2060,35 @@ int tg_bdf1_step(tg_plan *plan, double *const V_dev[3], double *P_dev, const tg_
     const double nu = fluid->nu, dt = fluid->dt, nil[2] = {0.0, 0.0};
     tg_plan::Chff &c = plan->ch;
     for (int step = 0; step < nsteps; step++) {
-        rc = chff_nlin(plan, V_dev, c.NL);
+        // N and div N, then the pressure with zero wall values (BDF1.cc:69-75)
+        rc = chff_nlin(plan, V_dev, c.NL, c.D);
         if (rc) return rc;
-        // div N, then the pressure with zero wall values (BDF1.cc:69-75)
-        HIPCHK(launch_cheb_deriv(plan->g, c.NL[0], c.D, true, plan->stream));
-        HIPCHK(launch_add_deriv(plan->g, c.D, c.NL[1], nullptr, 1, false, plan->stream));
-        HIPCHK(launch_add_deriv(plan->g, c.D, c.NL[2], nullptr, 2, false, plan->stream));
         HIPCHK(launch_helmholtz(helm_args(plan, c.D, P_dev, 0.0, nil, nil, 2, 0), plan->stream));
+        // the velocity, its x component first: it corrects the pressure
+        HelmArgs h = helm_args(plan, nullptr, nullptr, 1 / (dt * nu), nil, nil, 2, 0);
         for (int k = 0; k < 3; k++) {
-            if (k == 0) HIPCHK(launch_cheb_deriv(plan->g, P_dev, c.D, true, plan->stream));
-            HIPCHK(launch_bdf1_rhs(plan->g, c.NL[k], V_dev[k], P_dev, c.D, k, dt, nu, plan->stream));
-            HIPCHK(launch_helmholtz(helm_args(plan, c.NL[k], V_dev[k], 1 / (dt * nu), nil, nil, 2, 0), plan->stream));
-            if (k == 0) {
-                InflArgs ia{};
-                ia.P = P_dev;
-                ia.V1 = V_dev[0];
-                ia.pp = c.pp;
-                ia.pm = c.pm;
-                ia.vxp = c.vxp;
-                ia.vxm = c.vxm;
-                ia.M = c.M;
-                ia.nx = plan->g.nx;
-                ia.ny = plan->g.ny;
-                ia.nzc = plan->g.nzc;
-                ia.kf = plan->g.kf[0];
-                HIPCHK(launch_influence_correct(ia, plan->stream));
-            }
+            h.N[k] = c.NL[k];
+            h.V[k] = V_dev[k];
         }
+        h.P = P_dev;
+        h.dt = dt;
+        h.nu = nu;
+        HIPCHK(launch_helmholtz(h, plan->stream, 1));
+        InflArgs ia{};
+        ia.P = P_dev;
+        ia.V1 = V_dev[0];
+        ia.pp = c.pp;
+        ia.pm = c.pm;
+        ia.vxp = c.vxp;
+        ia.vxm = c.vxm;
+        ia.M = c.M;
+        ia.nx = plan->g.nx;
+        ia.ny = plan->g.ny;
+        ia.nzc = plan->g.nzc;
+        ia.kf = plan->g.kf[0];
+        HIPCHK(launch_influence_correct(ia, plan->stream));
+        h.comp = 1;
+        HIPCHK(launch_helmholtz(h, plan->stream, 2));
     }
     return TG_OK;
 }

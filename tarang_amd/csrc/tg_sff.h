@@ -10,15 +10,24 @@ namespace tg {
 constexpr int kRbcStateParity = 0x9;
 
 // x-inverse (sin/cos) of FP64 spectral fields into T work fields.
-//   flags: 1 = dealias on read, 4 = only the kz = 0 and kz = Nz/2 columns.
+//   flags: 1 = dealias on read, 4 = only the kz = 0 and kz = Nz/2 columns, 8 =
+//   Chebyshev coefficients (a_k = 2 A_k of the cosine transform, k > 0).
 template <typename T>
 hipError_t launch_xinv_sc(const Grid &g, double *const *V, int ncomp, int parity, void *const *U, int flags,
                           const void *twx, const void *twq, hipStream_t st);
 
-// x-forward (sin/cos) of T work fields into FP64 spectral fields, scaled.
+// x-forward (sin/cos) of T work fields into FP64 spectral fields, scaled (flags:
+// 8 as above).
 template <typename T>
 hipError_t launch_xfwd_sc(const Grid &g, void *const *W, int ncomp, int parity, double *const *out, double scale,
-                          const void *twx, const void *twq, hipStream_t st);
+                          const void *twx, const void *twq, hipStream_t st, int flags = 0);
+
+// The nonlinear term of the Chebyshev basis from its six products (y-forward
+// done: xx, yy, zz, xy, yz, zx): cosine transform along x to Chebyshev
+// coefficients, N_i = sum_j d_j (u_j u_i) into N and, if wanted, the
+// divergence of N into div (boundary layout).
+hipError_t launch_xfwd_chff(const Grid &g, void *const *P, double *const *N, double *div, double scale, const void *twx,
+                            const void *twq, hipStream_t st);
 
 // z pass of the RBC nonlinear terms: 4 lines in (u_x, u_y, u_z, theta), 9
 // products out: xx, yy, zz, xy, yz, zx, x theta, y theta, z theta.

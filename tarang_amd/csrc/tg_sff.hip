@@ -190,6 +190,7 @@ __global__ void __launch_bounds__(CB *(L / 8)) k_xinv_sc(XscArgs a)
     int zx0 = 1, zx1 = 0;
     if (a.flags & 1) dealias_rows(g, t.ly, t.lz, zx0, zx1);
     if (!t.live) { zx0 = 0; zx1 = L - 1; }
+    const double w = (a.flags & 8) ? 0.5 : 1.0;   // a_k = 2 A_k of Chebyshev coefficients, k > 0
 #pragma unroll 1
     for (int comp = 0; comp < a.ncomp; comp++) {
         cpx<T> v[8];
@@ -197,7 +198,7 @@ __global__ void __launch_bounds__(CB *(L / 8)) k_xinv_sc(XscArgs a)
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const int lx = jh + TPL * s;
-            v[s] = lx >= zx0 && lx <= zx1 ? mk<T>(0, 0) : cvt<T>(d[s]);
+            v[s] = lx >= zx0 && lx <= zx1 ? mk<T>(0, 0) : cvt<T>(lx > 0 ? w * d[s] : d[s]);
             settle(v[s]);
         }
         pin_memory_order();
@@ -227,11 +228,139 @@ __global__ void __launch_bounds__(CB *(L / 8)) k_xfwd_sc(XscArgs a)
         sc_forward<L>(v, x, tw.tw, tw.twq, hidden(t.j), ((a.parity >> comp) & 1) != 0);
         cpx<double> o[8];
 #pragma unroll
-        for (int s = 0; s < 8; s++) o[s] = a.scale * cvt<double>(v[s]);
+        for (int s = 0; s < 8; s++) {
+            o[s] = a.scale * cvt<double>(v[s]);
+            if ((a.flags & 8) && t.j + (L / 8) * s > 0) o[s] = 2.0 * o[s];
+        }
         pin_memory_order();
         if (comp + 1 < a.ncomp) t.template load<false>(v, a.U[comp + 1]);
         pin_memory_order();
         if (t.live) col_store<false>(o, (cpx<double> *)a.V[comp] + t.state0, t.steps, t.offs);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// x pass of the Chebyshev basis' nonlinear term
+// ---------------------------------------------------------------------------
+struct XchArgs {
+    void *P[6];
+    double *N[3], *div;
+    const void *tw, *twq;
+    Grid g;
+    double scale;
+};
+
+// Chebyshev derivative of a column, a_k in v (k = j + TPL s) in, b_k out:
+// c_k b_k = b_{k+2} + 2 (k+1) a_{k+1}, i.e. sums of 2 p a_p over p > k of the
+// other parity.  Each thread sums 8 consecutive k and takes the sums of the
+// chunks above from LDS (tot: 2 TPL CB entries).
+template <int L, int CB, typename X>
+__device__ __forceinline__ void cheb_deriv_column(cpx<double> *v, const X &x, cpx<double> *tot, int c, int j, double kf)
+{
+    constexpr int TPL = L / 8;
+#pragma unroll
+    for (int s = 0; s < 8; s++) x.w(j + TPL * s) = (2.0 * (j + TPL * s)) * v[s];
+    x.publish();
+    cpx<double> e = mk<double>(0, 0), o = e;   // sums over even and odd p
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        v[i] = x.r(8 * j + i);
+        if (i % 2) o = o + v[i];
+        else e = e + v[i];
+    }
+    tot[(2 * j) * CB + c] = e;
+    tot[(2 * j + 1) * CB + c] = o;
+    x.release();
+    e = o = mk<double>(0, 0);
+    for (int q = TPL - 1; q > j; q--) {
+        e = e + tot[(2 * q) * CB + c];
+        o = o + tot[(2 * q + 1) * CB + c];
+    }
+#pragma unroll
+    for (int i = 7; i >= 0; i--) {
+        cpx<double> b = i % 2 ? e : o;
+        if (i % 2) o = o + v[i];
+        else e = e + v[i];
+        if (i == 0 && j == 0) b = 0.5 * b;
+        x.w(8 * j + i) = kf * b;
+    }
+    x.publish();
+#pragma unroll
+    for (int s = 0; s < 8; s++) v[s] = x.r(j + TPL * s);
+    x.release();
+}
+
+// One pass over the six products: with the transforms field by field and the
+// products, derivatives and sums in kernels of their own, the nonlinear term
+// took 56 launches, now five (105 us at 64 x 128 x 128, this kernel 35).
+template <typename T, int L, int CB>
+__global__ void __launch_bounds__(CB *(L / 8)) k_xfwd_chff(XchArgs a)
+{
+    constexpr int TPL = L / 8;
+    using X = ColX<T, L, CB>;
+    __shared__ cpx<T> lds[X::SIZE];
+    __shared__ cpx<T> ldw[L + TPL + 8];
+    __shared__ cpx<T> tot[2 * TPL * CB];
+    const Grid &g = a.g;
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    if (tile >= x_tiles(g, CB, false)) return;
+    const ScTile<T, L, CB> t(g, tile);
+    const int j = t.j;
+    const double Ky = kwave(t.ly, g.ny) * g.kf[1], Kz = t.lz * g.kf[2];
+    cpx<T> v[8], next[8];
+    t.template load<false>(next, a.P[0]);
+    const ScTwiddles<T, L> tw(ldw, a.tw, a.twq);
+    const X x{lds + t.c};
+    cpx<T> N[3][8];
+    // product P of axes A and B: N_A += d_B, N_B += d_A; the next one's load is
+    // in flight behind the transform
+    auto product = [&](auto pc, auto nc) {
+        constexpr int P = decltype(pc)::value, PN = decltype(nc)::value;
+        constexpr int A = P < 3 ? P : P - 3, B = P < 3 ? P : (P - 2) % 3;
+#pragma unroll
+        for (int s = 0; s < 8; s++) v[s] = next[s];
+        pin_memory_order();
+        if (PN >= 0) t.template load<false>(next, a.P[PN < 0 ? 0 : PN]);
+        pin_memory_order();
+        sc_forward<L>(v, x, tw.tw, tw.twq, j, false);
+#pragma unroll
+        for (int s = 0; s < 8; s++) v[s] = (j + TPL * s > 0 ? 2.0 * a.scale : a.scale) * v[s];
+        // d_y and d_z first: the x derivative replaces v
+        auto add = [&](auto dst, auto dir) {
+            constexpr int D = decltype(dst)::value, R = decltype(dir)::value;
+            if constexpr (R > 0) {
+#pragma unroll
+                for (int s = 0; s < 8; s++) N[D][s] = N[D][s] + mul_i(R == 1 ? Ky : Kz, v[s]);
+            }
+        };
+        add(std::integral_constant<int, A>{}, std::integral_constant<int, B>{});
+        if constexpr (A != B) add(std::integral_constant<int, B>{}, std::integral_constant<int, A>{});
+        if constexpr (A == 0 || B == 0) {
+            constexpr int D = A == 0 ? B : A;
+            cheb_deriv_column<L, CB>(v, x, tot, t.c, j, g.kf[0]);
+#pragma unroll
+            for (int s = 0; s < 8; s++) N[D][s] = N[D][s] + v[s];
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int s = 0; s < 8; s++) N[i][s] = mk<T>(0, 0);
+    product(std::integral_constant<int, 0>{}, std::integral_constant<int, 3>{});
+    product(std::integral_constant<int, 3>{}, std::integral_constant<int, 5>{});
+    product(std::integral_constant<int, 5>{}, std::integral_constant<int, 1>{});
+    product(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
+    product(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
+    product(std::integral_constant<int, 2>{}, std::integral_constant<int, -1>{});
+    if (t.live) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) col_store<false>(N[i], (cpx<double> *)a.N[i] + t.state0, t.steps, t.offs);
+    }
+    if (a.div) {
+        cheb_deriv_column<L, CB>(N[0], x, tot, t.c, j, g.kf[0]);
+#pragma unroll
+        for (int s = 0; s < 8; s++) N[0][s] = N[0][s] + mul_i(Ky, N[1][s]) + mul_i(Kz, N[2][s]);
+        if (t.live) col_store<false>(N[0], (cpx<double> *)a.div + t.state0, t.steps, t.offs);
     }
 }
 
@@ -606,6 +735,16 @@ hipError_t xfwd_sc_len(const XscArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
+template <typename T, int LL>
+hipError_t xfwd_chff_len(const XchArgs &a, hipStream_t st)
+{
+    constexpr int CB = colx_block<T>(LL, 512);
+    if constexpr (sizeof(T) == 8)
+        hipLaunchKernelGGL((k_xfwd_chff<T, LL, CB>), dim3(x_grid(x_tiles(a.g, CB, false))), dim3(CB * (LL / 8)), 0, st, a);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
 template <typename T, int MM>
 hipError_t z_rbc_len(const ZArgs &a, hipStream_t st)
 {
@@ -652,6 +791,7 @@ hipError_t x_rbc_len(const XrbcArgs &a, hipStream_t st)
 #define TG_SFF_L(N, T, P)                                                   \
     P template hipError_t xinv_sc_len<T, N>(const XscArgs &, hipStream_t); \
     P template hipError_t xfwd_sc_len<T, N>(const XscArgs &, hipStream_t); \
+    P template hipError_t xfwd_chff_len<T, N>(const XchArgs &, hipStream_t); \
     P template hipError_t x_rbc_len<T, N>(const XrbcArgs &, hipStream_t);
 #define TG_SFF_M(N, T, P) P template hipError_t z_rbc_len<T, N>(const ZArgs &, hipStream_t);
 
@@ -679,9 +819,10 @@ hipError_t launch_xinv_sc(const Grid &g, double *const *V, int ncomp, int parity
 
 template <typename T>
 hipError_t launch_xfwd_sc(const Grid &g, void *const *W, int ncomp, int parity, double *const *out, double scale,
-                          const void *twx, const void *twq, hipStream_t st)
+                          const void *twx, const void *twq, hipStream_t st, int flags)
 {
     XscArgs a{};
+    a.flags = flags;
     for (int i = 0; i < ncomp; i++) {
         a.U[i] = W[i];
         a.V[i] = out[i];
@@ -693,6 +834,21 @@ hipError_t launch_xfwd_sc(const Grid &g, void *const *W, int ncomp, int parity, 
     a.parity = parity;
     a.scale = scale;
     TG_DISPATCH_L(T, g.nx, return (xfwd_sc_len<T, LL>)(a, st));
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_xfwd_chff(const Grid &g, void *const *P, double *const *N, double *div, double scale, const void *twx,
+                            const void *twq, hipStream_t st)
+{
+    XchArgs a{};
+    for (int i = 0; i < 6; i++) a.P[i] = P[i];
+    for (int i = 0; i < 3; i++) a.N[i] = N[i];
+    a.div = div;
+    a.tw = twx;
+    a.twq = twq;
+    a.g = g;
+    a.scale = scale;
+    TG_DISPATCH_L(double, g.nx, return (xfwd_chff_len<double, LL>)(a, st));
     return hipErrorInvalidValue;
 }
 
@@ -752,7 +908,7 @@ hipError_t launch_sff_reality(const Grid &g, double *const *V, int ncomp, int mo
     template hipError_t launch_xinv_sc<T>(const Grid &, double *const *, int, int, void *const *, int, const void *, \
                                           const void *, hipStream_t);                                               \
     template hipError_t launch_xfwd_sc<T>(const Grid &, void *const *, int, int, double *const *, double,           \
-                                          const void *, const void *, hipStream_t);                                 \
+                                          const void *, const void *, hipStream_t, int);                            \
     template hipError_t launch_z_rbc<T>(const Grid &, void *const *, void *const *, const void *, const void *,     \
                                         hipStream_t, bool);                                                         \
     template hipError_t launch_x_rbc<T>(const Grid &, const RbcParams &, void *const *, double *const *,            \
