@@ -122,19 +122,19 @@ __device__ __forceinline__ void tape_mac(cpx<T> *q, const cpx<T> *v, const cpx<T
 // and, as its share of sigma_zz, subtracts u_z sigma_jj from q_z; an
 // off-diagonal line sigma_jm adds u_j sigma_jm to q_m and u_m sigma_jm to
 // q_j.  Five c2r and three r2c per line.
-template <typename T, int M, bool NT>
-__global__ void __launch_bounds__(256) k_z_adj(ZArgs a)
+template <typename T, int M, bool NT, int W>
+__global__ void __launch_bounds__(64 * W) k_z_adj(ZArgs a)
 {
     constexpr int TPL = M / 8;
-    constexpr int LPB = z_lines_per_block<M>();
+    constexpr int LPB = ZLines<M, W>::LPB;
     constexpr int LP = lpad_len(M);
     __shared__ cpx<T> lds[LPB * LP], ldw[2 * M];
     const ZTwiddles<T, M> tw(ldw, a.twm, a.twn);
-    const int li = threadIdx.x / TPL, j = threadIdx.x % TPL;
-    const size_t line = (size_t)blockIdx.x * LPB + li;
-    const size_t nlines = (size_t)a.g.nx * a.g.ny;
-    const bool valid = line < nlines;
-    const size_t lsafe = valid ? line : nlines - 1;
+    const ZLines<M, W> z(a.g);
+    const int li = z.li, j = z.j;
+    const size_t lsafe = z.safe;
+    const bool valid = z.valid;
+    if (z.spare) return;
     cpx<T> *L = lds + li * LP;
     const size_t off = lsafe * a.g.nzp;
     cpx<T> q[3][8];
@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(256) k_z_adj(ZArgs a)
                                             t == 3 ? a.in[3] : a.in[4]);
         cpx<T> v[8];
         zline_c2r<T, M, NT>(v, X + off, L, tw, j);
-        line_sync<M / 8>();
+        line_sync();
         const cpx<T> *uj = (const cpx<T> *)(jt == 0 ? a.tape[0] : jt == 1 ? a.tape[1] : a.tape[2]) + lsafe * M;
         const cpx<T> *um = (const cpx<T> *)(mt == 0 ? a.tape[0] : mt == 1 ? a.tape[1] : a.tape[2]) + lsafe * M;
         const cpx<T> *uz = (const cpx<T> *)a.tape[2] + lsafe * M;
@@ -282,13 +282,11 @@ hipError_t xinv_sym_len(const XsymArgs &a, hipStream_t st)
 template <typename T, int MM>
 hipError_t z_adj_len(const ZArgs &a, hipStream_t st)
 {
-    constexpr int LPB = z_lines_per_block<MM>();
-    const size_t nlines = (size_t)a.g.nx * a.g.ny;
-    dim3 grid((unsigned)((nlines + LPB - 1) / LPB));
-    const dim3 block(LPB * (MM / 8));
+    const dim3 grid = ZLines<MM, 4>::grid(a.g), grid1 = ZLines<MM, 1>::grid(a.g);
     const bool nt = stream_bytes((size_t)8 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
-    if (nt) hipLaunchKernelGGL((k_z_adj<T, MM, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((k_z_adj<T, MM, false>), grid, block, 0, st, a);
+    if (nt) hipLaunchKernelGGL((k_z_adj<T, MM, true, 4>), grid, dim3(256), 0, st, a);
+    else if (z_small<MM>(a.g)) hipLaunchKernelGGL((k_z_adj<T, MM, false, 1>), grid1, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL((k_z_adj<T, MM, false, 4>), grid, dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

@@ -586,7 +586,6 @@ int run_rk4(tg_plan *p, double *const V[3], const tg_fluid *f, int nsteps, int f
         }
         if (p->cfg.strong_reality) {
             Prof pr(p, TG_KERNEL_REALITY);
-            HIPCHK(launch_reality(p->g, V, 3, p->stream));
             HIPCHK(launch_xinv_state<T>(p->g, p->band, V, 3, p->U, p->slots[0], 1 | 4 | (p->band.kind == 1 ? 2 : 0),
                                         p->twx, p->stream));
         }

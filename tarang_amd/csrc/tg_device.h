@@ -256,25 +256,16 @@ __device__ __forceinline__ void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Synchronisation of the threads that share one line.  A line of L points
-// is handled by TPL = L/8 consecutive threads; when TPL divides 64 the line
-// lives inside one wavefront, whose LDS operations execute in order, so only
-// the compiler has to be kept from moving LDS accesses across the exchange
-// (wavefront-scope fence on LDS only: global loads and stores may still be
-// moved across it, e.g. the next line's loads ahead of this line's FFT).
-// Longer lines span waves, and lines of 3 or 5 times a power of two
-// straddle them: those need the block barrier (every thread of the block
-// takes part in every line transform, so the barriers match).
-template <int TPL>
+// Synchronisation of the threads that share one line, all of one wavefront: its
+// LDS operations execute in order, so only the compiler has to be kept from
+// moving LDS accesses across the exchange (wavefront-scope fence on LDS only:
+// global loads and stores may still be moved across it, e.g. the next line's
+// loads ahead of this line's FFT).
 __device__ __forceinline__ void line_sync()
 {
-    if constexpr (TPL <= 64 && 64 % TPL == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-    } else {
-        lds_barrier();
-    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
 }
 
 // LDS position with one pad entry every 16 points (breaks the stride-8
@@ -294,8 +285,8 @@ struct LineX {
     cpx<T> *p;
     __device__ __forceinline__ cpx<T> &w(int i) const { return p[lpad(i)]; }
     __device__ __forceinline__ cpx<T> &r(int i) const { return p[lpad(i)]; }
-    __device__ __forceinline__ void publish() const { line_sync<L / 8>(); }
-    __device__ __forceinline__ void release() const { line_sync<L / 8>(); }
+    __device__ __forceinline__ void publish() const { line_sync(); }
+    __device__ __forceinline__ void release() const { line_sync(); }
 };
 
 // ColX: the CB lines of a block interleaved (point i of line c at row i,
@@ -443,7 +434,7 @@ __device__ __forceinline__ void fft_exchange(cpx<T> *v, const X &x, const cpx<T>
     }
 }
 
-// fft_exchange on consecutive points in LDS (the z lines and the sin/cos lines).
+// fft_exchange on consecutive points in LDS (the z lines).
 template <int L, int DIR, typename T>
 __device__ __forceinline__ void fft_line(cpx<T> *v, cpx<T> *lds, const cpx<T> *__restrict__ tw, int j)
 {

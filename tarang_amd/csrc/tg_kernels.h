@@ -61,8 +61,9 @@ hipError_t launch_colfft(const Grid &g, int axis, int dir, void *const *fields, 
                          const void *tw, hipStream_t st, const Cut *cut = nullptr);
 
 // x-inverse of an FP64 spectral field set into the T work layout.
-//   flags: 1 = dealias on read, 2 = write band slots, 4 = reality patch
-//   columns only (kz = 0 and kz = Nz/2), 8 = keep only r_lo < K <= r_hi,
+//   flags: 1 = dealias on read, 2 = write band slots, 4 = the kz = 0 and Nz/2
+//   columns only, the strong reality condition applied to them first (in V
+//   too), 8 = keep only r_lo < K <= r_hi,
 //   16 = keep the ring r_lo < K <= r_hi, a_lo < theta <= a_hi (polar angle
 //   to the axis dirn), 32 = keep the cylindrical ring r_lo < K <= r_hi,
 //   a_lo < Kpll <= a_hi.

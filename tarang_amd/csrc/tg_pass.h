@@ -359,7 +359,7 @@ __device__ __forceinline__ void zline_c2r_from(cpx<T> *v, cpx<T> xm, cpx<T> *lds
 #pragma unroll
     for (int s = 0; s < 8; s++) lds[lpad(j + TPL * s)] = mk<T>(v[s].x, v[s].y);
     if (j == 0) lds[lpad(M)] = xm;
-    line_sync<M / 8>();
+    line_sync();
 #pragma unroll
     for (int s = 0; s < 8; s++) {
         const int k = j + TPL * s;
@@ -372,7 +372,7 @@ __device__ __forceinline__ void zline_c2r_from(cpx<T> *v, cpx<T> xm, cpx<T> *lds
         const cpx<T> e = mk<T>(d.x * w.x + d.y * w.y, d.y * w.x - d.x * w.y);
         v[s] = a + mk<T>(-e.y, e.x);
     }
-    line_sync<M / 8>();
+    line_sync();
     fft_line<M, +1>(v, lds, tw.m, j);
 }
 
@@ -395,7 +395,7 @@ __device__ __forceinline__ void zline_r2c_post(cpx<T> *v, cpx<T> *__restrict__ X
     fft_line<M, -1>(v, lds, tw.m, j);
 #pragma unroll
     for (int s = 0; s < 8; s++) lds[lpad(j + TPL * s)] = v[s];
-    line_sync<M / 8>();
+    line_sync();
     const T h = (T)0.5;
     const cpx<T> z0 = lds[0];
 #pragma unroll
@@ -411,7 +411,7 @@ __device__ __forceinline__ void zline_r2c_post(cpx<T> *v, cpx<T> *__restrict__ X
     }
     if (store && (!LIM || M < lim))
         for (int i = j; i < npad; i += TPL) gstore<NT>(X + M + i, mk<T>(i == 0 ? z0.x - z0.y : (T)0, (T)0));
-    line_sync<M / 8>();
+    line_sync();
 }
 
 struct ZArgs {
@@ -424,11 +424,36 @@ struct ZArgs {
     int lim_u, lim_w, lim_out;  // giver form: columns of the fields and products that are dealt with
 };
 
+// The lines of a block of a z pass: M/8 threads a line, as many lines a wavefront
+// as fit (of the lengths with factors 3 and 5 a few lanes are left over: with
+// their lines across wavefronts, behind block barriers, the products of a
+// 240 x 160 x 96 FP64 step took 96 us, now 87), W wavefronts.
+template <int M, int W>
+struct ZLines {
+    static constexpr int TPL = M / 8, LPW = 64 / TPL, LPB = LPW * W, THREADS = 64 * W;
+    static_assert(TPL <= 64, "a z line lies in one wavefront");
+    int li, j;
+    bool spare;   // a lane without a line (it ends after the last block barrier)
+    size_t line, safe;
+    bool valid;
+    __device__ __forceinline__ ZLines(const Grid &g)
+    {
+        const int lane = threadIdx.x & 63, l = lane / TPL;
+        spare = l >= LPW;
+        li = (threadIdx.x / 64) * LPW + (l < LPW ? l : LPW - 1);
+        j = lane % TPL;
+        line = (size_t)blockIdx.x * LPB + li;
+        const size_t n = (size_t)g.nx * g.ny;
+        valid = line < n;
+        safe = valid ? line : n - 1;
+    }
+    static dim3 grid(const Grid &g) { return dim3((unsigned)(((size_t)g.nx * g.ny + LPB - 1) / LPB)); }
+};
+// Blocks of one wavefront where blocks of four would leave CUs idle: 64 of them
+// at 64^3 FP64, 19.8 us a launch of the products against 15.8; with two a CU and
+// more (128^3 and larger) nothing changes.
 template <int M>
-__host__ __device__ constexpr int z_lines_per_block()
-{
-    return (M / 8) >= 256 ? 1 : 256 / (M / 8);
-}
+inline bool z_small(const Grid &g) { return (size_t)g.nx * g.ny < (size_t)256 * ZLines<M, 4>::LPB; }
 
 // ---------------------------------------------------------------------------
 // Transform lengths with compiled kernels, and the size dispatch of the

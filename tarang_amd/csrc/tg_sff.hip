@@ -386,28 +386,28 @@ __device__ __forceinline__ int rbc_pair(int ia, int ib)
 // u_y^2 - u_z^2 and the off-diagonal ones (out[2], zz, not written): the stage
 // uses the velocity term only projected, and the SFF projection removes the
 // gradient of u_z^2 that the shift adds.
-template <typename T, int M, bool SHIFT, bool NT>
-__global__ void __launch_bounds__(256, 2) k_z_rbc(ZArgs a)
+template <typename T, int M, bool SHIFT, bool NT, int W>
+__global__ void __launch_bounds__(64 * W, 2) k_z_rbc(ZArgs a)
 {
     constexpr int TPL = M / 8;
-    constexpr int LPB = z_lines_per_block<M>();
+    constexpr int LPB = ZLines<M, W>::LPB;
     constexpr int LP = lpad_len(M);
     __shared__ cpx<T> lds[LPB * LP], ldw[2 * M];
-    const int li = threadIdx.x / TPL, j = threadIdx.x % TPL;
-    const size_t line = (size_t)blockIdx.x * LPB + li;
-    const size_t nlines = (size_t)a.g.nx * a.g.ny;
-    const bool valid = line < nlines;
-    const size_t lsafe = valid ? line : nlines - 1;
+    const ZLines<M, W> z(a.g);
+    const int li = z.li, j = z.j;
+    const size_t lsafe = z.safe;
+    const bool valid = z.valid;
     cpx<T> *L = lds + li * LP;
     const size_t off = lsafe * a.g.nzp;
     cpx<T> u[3][8], xm[3];
 #pragma unroll
     for (int c = 0; c < 3; c++) zline_load<T, M, NT>(u[c], xm[c], (const cpx<T> *)a.in[c] + off, j);
     const ZTwiddles<T, M> tw(ldw, a.twm, a.twn);
+    if (z.spare) return;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         zline_c2r_from<T, M>(u[c], xm[c], L, tw, j);
-        line_sync<M / 8>();
+        line_sync();
     }
     auto emit = [&](const cpx<T> *x, const cpx<T> *y, int o) {
         cpx<T> p[8];
@@ -438,7 +438,7 @@ __global__ void __launch_bounds__(256, 2) k_z_rbc(ZArgs a)
     }
     cpx<T> t[8];
     zline_c2r<T, M, NT>(t, (const cpx<T> *)a.in[3] + off, L, tw, j);
-    line_sync<M / 8>();
+    line_sync();
 #pragma unroll
     for (int ia = 0; ia < 3; ia++) emit(u[ia], t, rbc_pair(ia, 3));
 }
@@ -748,14 +748,12 @@ hipError_t xfwd_chff_len(const XchArgs &a, hipStream_t st)
 template <typename T, int MM>
 hipError_t z_rbc_len(const ZArgs &a, hipStream_t st)
 {
-    constexpr int LPB = z_lines_per_block<MM>();
-    const size_t nlines = (size_t)a.g.nx * a.g.ny;
-    dim3 grid((unsigned)((nlines + LPB - 1) / LPB));
-    const dim3 block(LPB * (MM / 8));
+    const dim3 grid = ZLines<MM, 4>::grid(a.g), grid1 = ZLines<MM, 1>::grid(a.g);
     const bool nt = stream_bytes((size_t)12 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
-    if (a.ncomp != 8) hipLaunchKernelGGL((k_z_rbc<T, MM, false, false>), grid, block, 0, st, a);
-    else if (nt) hipLaunchKernelGGL((k_z_rbc<T, MM, true, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((k_z_rbc<T, MM, true, false>), grid, block, 0, st, a);
+    if (a.ncomp != 8) hipLaunchKernelGGL((k_z_rbc<T, MM, false, false, 4>), grid, dim3(256), 0, st, a);
+    else if (nt) hipLaunchKernelGGL((k_z_rbc<T, MM, true, true, 4>), grid, dim3(256), 0, st, a);
+    else if (z_small<MM>(a.g)) hipLaunchKernelGGL((k_z_rbc<T, MM, true, false, 1>), grid1, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL((k_z_rbc<T, MM, true, false, 4>), grid, dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
