@@ -48,6 +48,9 @@ int fail(int code, const char *fmt, ...)
 
 }  // namespace
 
+// bytes of the pinned results (the bins of any one reduction)
+static constexpr size_t kHostOut = 65536;
+
 struct tg_plan {
     tg_config cfg{};
     Grid g{};
@@ -82,10 +85,11 @@ struct tg_plan {
     bool unext_valid = false;
     double *unext_V[3] = {};
     Band unext_band{};
-    // non-finite state detection: device flag set by the stage-4 kernels,
-    // read back into pinned host memory at the end of every time-advance call
-    int *nonfinite_dev = nullptr;
-    int *nonfinite_host = nullptr;
+    // pinned host memory that kernels write to: the results of reductions, and
+    // the flag of a non-finite state
+    double *host_out = nullptr;
+    int *nonfinite = nullptr;
+    bool nonfinite_open = false;
     // host-side band config for the current step
     Band band{};
     // SFF: quarter-wave twiddles exp(-i pi k / (2 Nx)), k < Nx
@@ -232,7 +236,7 @@ void free_plan(tg_plan *p)
         if (q) (void)hipFree(q);
     for (void *q : p->mhd)
         if (q) (void)hipFree(q);
-    void *aptrs[] = {p->adj.ckpt, p->adj.tape, p->adj.vw, p->adj.lg, p->adj.acc, p->nonfinite_dev, p->rfield,
+    void *aptrs[] = {p->adj.ckpt, p->adj.tape, p->adj.vw, p->adj.lg, p->adj.acc, p->rfield,
                      p->umax_dev, p->force_eh, p->force_tab};
     for (void *q : aptrs)
         if (q) (void)hipFree(q);
@@ -240,7 +244,7 @@ void free_plan(tg_plan *p)
                      p->ch.vxp, p->ch.vxm, p->ch.M};
     for (void *q : cptrs)
         if (q) (void)hipFree(q);
-    if (p->nonfinite_host) (void)hipHostFree(p->nonfinite_host);
+    if (p->host_out) (void)hipHostFree(p->host_out);
     for (auto &r : p->prof_recs) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
     for (auto e : p->prof_pool) (void)hipEventDestroy(e);
     delete p;
@@ -253,15 +257,18 @@ int set_device(tg_plan *p) { HIPCHK(hipSetDevice(p->cfg.device)); return TG_OK; 
 // stage-4 kernels flag any non-finite value they write into the state.
 int nonfinite_begin(tg_plan *p)
 {
-    HIPCHK(launch_fill_int(p->nonfinite_dev, 1, 0, p->stream));
+    // (after a call that an error ended, kernels that may set it can be left)
+    if (p->nonfinite_open) HIPCHK(hipStreamSynchronize(p->stream));
+    *p->nonfinite = 0;
+    p->nonfinite_open = true;
     return TG_OK;
 }
 
 int nonfinite_end(tg_plan *p, const char *what)
 {
-    HIPCHK(hipMemcpyAsync(p->nonfinite_host, p->nonfinite_dev, sizeof(int), hipMemcpyDeviceToHost, p->stream));
     HIPCHK(hipStreamSynchronize(p->stream));
-    if (*p->nonfinite_host)
+    p->nonfinite_open = false;
+    if (*(volatile int *)p->nonfinite)
         return fail(TG_ERR_NAN, "%s: the state holds non-finite values after the step (NaN or Inf)", what);
     return TG_OK;
 }
@@ -579,7 +586,7 @@ int run_rk4(tg_plan *p, double *const V[3], const tg_fluid *f, int nsteps, int f
             if (rc) return rc;
             RkParams rk = rk_params(p, f, s);
             rk.trace_free = 1;
-            if (s == 4) rk.nonfinite = p->nonfinite_dev;
+            if (s == 4) rk.nonfinite = p->nonfinite;
             Prof pr(p, TG_KERNEL_X_NLIN_RK);
             HIPCHK(launch_x_nlin<T>(p->g, p->band, rk, p->P, V, p->acc, p->U, p->slots[(s - 1) & 1],
                                     p->slots[s & 1], nullptr, p->twx, p->stream));
@@ -672,7 +679,7 @@ int run_rk4_mhd(tg_plan *p, double *const V[3], double *const W[3], const tg_flu
             xa.fh_b = -eta * 0.5 * f->dt;
             xa.f1_b = -eta * 1.0 * f->dt;
             xa.scale = 1.0 / ((double)p->g.nx * p->g.ny * p->g.nz);
-            xa.nonfinite = s == 4 ? p->nonfinite_dev : nullptr;
+            xa.nonfinite = s == 4 ? p->nonfinite : nullptr;
             Prof pr(p, TG_KERNEL_X_NLIN_RK);
             HIPCHK(launch_x_mhd<T>(xa, p->stream));
         }
@@ -1027,7 +1034,7 @@ int run_rk4_rbc(tg_plan *p, double *const V[3], double *T_, const tg_rbc *r, int
             const double *f_in[2] = {s == 1 ? T_ : p->rbc[1 + 2 * rd], s == 1 ? V[0] : p->rbc[2 + 2 * rd]};
             double *f_out[2] = {p->rbc[1 + 2 * wr], p->rbc[2 + 2 * wr]};
             RbcParams rp = rbc_params(p, r, s);
-            if (s == 4) rp.nonfinite = p->nonfinite_dev;
+            if (s == 4) rp.nonfinite = p->nonfinite;
             Prof pr(p, TG_KERNEL_X_RBC);
             HIPCHK(launch_x_rbc<T>(p->g, rp, p->P, S, acc, p->U, f_in, f_out, nullptr, p->twx, p->twq, p->stream));
         }
@@ -1041,6 +1048,8 @@ int run_rk4_rbc(tg_plan *p, double *const V[3], double *T_, const tg_rbc *r, int
     return nonfinite_end(p, "tg_rk4_step_rbc");
 }
 
+// The last kernel of a reduction writes its result to pinned host memory (a copy
+// back to the caller's own memory took 10 us more a call).
 int reduce_to_host(tg_plan *p, int mode, const double *const *A, const double *const *B, int ncomp, int n,
                    const double *radii_host, int nbins, int nq, int kcut, double r_lo, double r_hi, double *out,
                    const Cut *cut = nullptr)
@@ -1049,7 +1058,6 @@ int reduce_to_host(tg_plan *p, int mode, const double *const *A, const double *c
     double *radii_dev = nullptr;
     size_t need_small = sizeof(double) * (size_t)(width + nbins + 8);
     if (need_small > 65536) return fail(TG_ERR_ARG, "too many bins (%d)", nbins);
-    double *outd = p->small;
     if (radii_host) {
         radii_dev = p->small + width + 4;
         HIPCHK(hipMemcpyAsync(radii_dev, radii_host, sizeof(double) * nbins, hipMemcpyHostToDevice, p->stream));
@@ -1057,9 +1065,9 @@ int reduce_to_host(tg_plan *p, int mode, const double *const *A, const double *c
     const size_t need = (size_t)p->red_blocks * width * sizeof(double);
     if (need > p->partial_bytes) return fail(TG_ERR_ARG, "reduction needs %zu bytes of partials", need);
     HIPCHK(launch_reduce(p->g, mode, A, B, ncomp, n, radii_dev, nbins, nq, kcut, r_lo, r_hi, p->partial,
-                         p->red_blocks, outd, p->stream, nullptr, cut));
-    HIPCHK(hipMemcpyAsync(out, outd, sizeof(double) * width, hipMemcpyDeviceToHost, p->stream));
+                         p->red_blocks, p->host_out, p->stream, nullptr, cut));
     HIPCHK(hipStreamSynchronize(p->stream));
+    std::memcpy(out, p->host_out, sizeof(double) * width);
     return TG_OK;
 }
 
@@ -1096,17 +1104,16 @@ int reduce_aniso_to_host(tg_plan *p, int mode, const double *const *A, const dou
     const size_t off_aux = (size_t)nq * win + 8, off_radii = off_aux + (size_t)nsub + 8;
     const size_t need = sizeof(double) * (off_radii + (size_t)nshell + 8);
     if (need > 65536) return fail(TG_ERR_ARG, "too many shells or sub-bins (%d, %d)", nshell, nsub);
-    double *outd = p->small, *auxd = p->small + off_aux, *radd = radii_host ? p->small + off_radii : nullptr;
+    double *auxd = p->small + off_aux, *radd = radii_host ? p->small + off_radii : nullptr;
     HIPCHK(hipMemcpyAsync(auxd, aux_host, sizeof(double) * (nsub + 1), hipMemcpyHostToDevice, p->stream));
     if (radii_host)
         HIPCHK(hipMemcpyAsync(radd, radii_host, sizeof(double) * (nshell + 1), hipMemcpyHostToDevice, p->stream));
-    std::vector<double> tmp((size_t)nq * win);
+    const double *tmp = p->host_out;
     for (int lo = 0; lo < nbins_total; lo += win) {
         const int nb = std::min(win, nbins_total - lo);
         RedAniso an{auxd, nsub, nshell, dirn, lo};
         HIPCHK(launch_reduce(p->g, mode, A, B, ncomp, n, radd, nb, nq, kcut, 0.0, 0.0, p->partial, p->red_blocks,
-                             outd, p->stream, &an, cut));
-        HIPCHK(hipMemcpyAsync(tmp.data(), outd, sizeof(double) * nq * nb, hipMemcpyDeviceToHost, p->stream));
+                             p->host_out, p->stream, &an, cut));
         HIPCHK(hipStreamSynchronize(p->stream));
         for (int q = 0; q < nq; q++)
             for (int b = 0; b < nb; b++) out[(size_t)q * nbins_total + lo + b] = tmp[(size_t)q * nb + b];
@@ -1212,10 +1219,13 @@ int tg_plan_create(const tg_config *cfg, tg_plan **plan)
     p->partial_bytes = (size_t)p->red_blocks * 2 * 1100 * sizeof(double);
     if (!rc) rc = dmalloc(p, (void **)&p->partial, p->partial_bytes);
     if (!rc) rc = dmalloc(p, (void **)&p->small, 65536);
-    if (!rc) rc = dmalloc(p, (void **)&p->nonfinite_dev, 256);
-    if (!rc && hipHostMalloc((void **)&p->nonfinite_host, sizeof(int), hipHostMallocDefault) != hipSuccess) {
-        p->nonfinite_host = nullptr;
+    if (!rc && hipHostMalloc((void **)&p->host_out, kHostOut + 256, hipHostMallocDefault) != hipSuccess) {
+        p->host_out = nullptr;
         rc = fail(TG_ERR_OOM, "hipHostMalloc failed");
+    }
+    if (!rc) {
+        p->nonfinite = (int *)((char *)p->host_out + kHostOut);
+        *p->nonfinite = 0;
     }
     if (rc) { free_plan(p); return rc; }
     *plan = p;

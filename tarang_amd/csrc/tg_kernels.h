@@ -129,8 +129,6 @@ hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void 
 // the random force (kind 2) of the band's slots, 3 complex values each
 hipError_t launch_random_force(const Grid &g, const Band &b, double *out, hipStream_t st);
 hipError_t launch_reality(const Grid &g, double *const *V, int ncomp, hipStream_t st);
-// n ints at p set to v by a kernel (no memset node, so it may be captured)
-hipError_t launch_fill_int(int *p, int n, int v, hipStream_t st);
 hipError_t launch_dealias(const Grid &g, double *const *V, int ncomp, hipStream_t st);
 
 }  // namespace tg

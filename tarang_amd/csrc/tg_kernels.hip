@@ -1185,18 +1185,6 @@ hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void 
     return hipErrorInvalidValue;
 }
 
-__global__ void k_fill_int(int *p, int n, int v)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-hipError_t launch_fill_int(int *p, int n, int v, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_fill_int, dim3((n + 63) / 64), dim3(64), 0, st, p, n, v);
-    return hipGetLastError();
-}
-
 hipError_t launch_reality(const Grid &g, double *const *V, int ncomp, hipStream_t st)
 {
     PlaneArgs a{};
