@@ -102,7 +102,7 @@ struct XinvArgs {
 
 // Columns go from memory to registers and back in transform order; a column
 // without a mode to keep is not read.  One field at 256^3 FP64: 123 us with the
-// tiles staged through LDS, now 85.  FILTER: flags & (8 | 16 | 32), cut.
+// tiles staged through LDS, now 76.  FILTER: flags & (8 | 16 | 32), cut.
 template <typename T, int L, int CB, bool FILTER>
 __global__ void __launch_bounds__(CB *(L / 8)) k_xinv_state(XinvArgs a)
 {
@@ -925,22 +925,36 @@ hipError_t colfft_len(const ColArgs &a, int dir, int nfields, hipStream_t st)
     return hipGetLastError();
 }
 
+// Columns of the plain x passes' tiles: 16, whose 256 bytes of an unpadded state
+// row lie in three 128-byte lines (8 columns in two, half of each another
+// tile's), while a block has at most 1024 threads.  256^3 FP64, 8 columns: inverse
+// 85 us, forward 60; 16: 76 and 53; 512 x 256 x 256: 161 and 151 us, 148 and 128.
+// (The filtered inverse needs more registers than such a block has.)
+__host__ __device__ constexpr int plain_block(int L)
+{
+    int cb = 16;
+    while (cb * (L / 8) < 64) cb *= 2;
+    while (cb * (L / 8) > 1024) cb /= 2;
+    return cb;
+}
+
 template <typename T, int LL>
 hipError_t xinv_state_len(const XinvArgs &a, hipStream_t st)
 {
-    constexpr int CB = colx_block<T>(LL, 512);
+    constexpr int CB = colx_block<T>(LL, 512), PB = plain_block(LL);
     const dim3 grid(x_grid(x_tiles(a.g, CB, (a.flags & 4) != 0))), block(CB * (LL / 8));
     if (a.flags & 4) hipLaunchKernelGGL((k_xinv_reality<T, LL, CB>), dim3(grid.x, a.ncomp), block, 0, st, a);
     else if (a.flags & 56)
         hipLaunchKernelGGL((k_xinv_state<T, LL, CB, true>), dim3(x_grid(x_tiles_cut<T>(a.g, CB, a.cut))), block, 0, st, a);
-    else hipLaunchKernelGGL((k_xinv_state<T, LL, CB, false>), grid, block, 0, st, a);
+    else
+        hipLaunchKernelGGL((k_xinv_state<T, LL, PB, false>), dim3(x_grid(x_tiles(a.g, PB, false))), dim3(PB * (LL / 8)), 0, st, a);
     return hipGetLastError();
 }
 
 template <typename T, int LL>
 hipError_t xfwd_spec_len(const XfwdArgs &a, hipStream_t st)
 {
-    constexpr int CB = colx_block<T>(LL, 512);
+    constexpr int CB = plain_block(LL);
     dim3 grid(x_grid(x_tiles(a.g, CB, false)));
     hipLaunchKernelGGL((k_xfwd_spec<T, LL, CB>), grid, dim3(CB * (LL / 8)), 0, st, a);
     return hipGetLastError();
