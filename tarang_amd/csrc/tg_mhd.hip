@@ -120,11 +120,14 @@ constexpr int mhd_index(int pi)
 
 // As k_x_nlin: columns in registers in transform order, the next tile in
 // flight, products unrolled, code per stage, values settled where they are
-// formed.  The six sums take 192 registers in FP64: 256-thread blocks there
-// (512 registers a thread), 512-thread blocks in FP32.  512^3 FP32, per launch:
-// 11.0 ms, now 5.1 in stage 1, 5.9 in stages 2 and 3 (4.8 TB/s), 7.1 in stage 4.
+// formed.  The six sums take 192 registers in FP64: blocks of 512 threads spill
+// about 120 of them a lane, which costs less than 64-byte rows in blocks of 256
+// (512 registers a thread): a step at 320 x 320 x 240 16 ms against 29, 512 x 256 x
+// 512 33 against 34, 1024 x 256 x 512 (64-byte rows, or 32) 124 against 129.
+// 512^3 FP32, per launch: 11.0 ms, now 5.1 in stage 1, 5.9 in stages 2 and 3
+// (4.8 TB/s), 7.1 in stage 4.
 template <typename T, int L, int CB, int ST, bool NT>
-__global__ void __launch_bounds__(CB *(L / 8), sizeof(T) == 8 ? 1 : 2) k_x_mhd(XmhdArgs a)
+__global__ void __launch_bounds__(CB *(L / 8), CB * (L / 8) <= 256 ? 1 : 2) k_x_mhd(XmhdArgs a)
 {
     constexpr int TPL = L / 8, NTH = CB * TPL;
     constexpr bool NTW = NT && CB * sizeof(cpx<T>) >= 128, NTA = NT && CB * sizeof(cpx<double>) >= 128;
@@ -332,7 +335,7 @@ __global__ void __launch_bounds__(CB *(L / 8), sizeof(T) == 8 ? 1 : 2) k_x_mhd(X
 template <typename T, int LL>
 hipError_t x_mhd_len(const XmhdArgs &a, hipStream_t st)
 {
-    constexpr int CB = colx_block<T>(LL, sizeof(T) == 8 ? 256 : 512);
+    constexpr int CB = colx_block<T>(LL, 512);
     const bool nt = stream_bytes((size_t)14 * a.g.nx * a.g.ny * a.g.nzp * sizeof(cpx<T>));
     const dim3 grid(x_grid(x_tiles(a.g, CB, false))), block(CB * (LL / 8));
     auto go = [&](auto sc) {
