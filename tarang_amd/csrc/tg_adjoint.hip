@@ -131,10 +131,15 @@ __global__ void __launch_bounds__(64 * W) k_z_adj(ZArgs a)
     __shared__ cpx<T> lds[LPB * LP], ldw[2 * M];
     const ZTwiddles<T, M> tw(ldw, a.twm, a.twn);
     const ZLines<M, W> z(a.g);
-    const int li = z.li, j = z.j;
-    const size_t lsafe = z.safe;
-    const bool valid = z.valid;
     if (z.spare) return;
+    // (formed anew for powers of two: from z's members the compiler no longer
+    // moved the tape's loads ahead of the transforms, 485 us a launch at 256^3
+    // FP64 against 357)
+    constexpr bool WHOLE = 64 % TPL == 0;
+    const int li = WHOLE ? threadIdx.x / TPL : z.li, j = WHOLE ? threadIdx.x % TPL : z.j;
+    const size_t line = (size_t)blockIdx.x * LPB + li, nlines = (size_t)a.g.nx * a.g.ny;
+    const bool valid = line < nlines;
+    const size_t lsafe = valid ? line : nlines - 1;
     cpx<T> *L = lds + li * LP;
     const size_t off = lsafe * a.g.nzp;
     cpx<T> q[3][8];

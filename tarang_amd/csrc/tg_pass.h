@@ -439,9 +439,15 @@ struct ZLines {
     __device__ __forceinline__ ZLines(const Grid &g)
     {
         const int lane = threadIdx.x & 63, l = lane / TPL;
-        spare = l >= LPW;
-        li = (threadIdx.x / 64) * LPW + (l < LPW ? l : LPW - 1);
-        j = lane % TPL;
+        if constexpr (64 % TPL == 0) {
+            spare = false;
+            li = threadIdx.x / TPL;
+            j = threadIdx.x % TPL;
+        } else {
+            spare = l >= LPW;
+            li = (threadIdx.x / 64) * LPW + (l < LPW ? l : LPW - 1);
+            j = lane % TPL;
+        }
         line = (size_t)blockIdx.x * LPB + li;
         const size_t n = (size_t)g.nx * g.ny;
         valid = line < n;
