@@ -591,7 +591,7 @@ constexpr int xnl_axis(int mode, int p, int i)
 // stages, the hyperviscosity loops and the random phases inlined per point the
 // kernel was 300 KB of instructions, mostly fetched from L2 (and the stages'
 // registers, allocated together, spilled).  512^3, per launch: FP64 5170 ->
-// 3606 us (4.9 TB/s), FP32 4550 -> 3150 us; 64^3 FP64 54 -> 19 us, 240x160x96
+// 3240 us (5.4 TB/s), FP32 4550 -> 2920 us; 64^3 FP64 54 -> 19 us, 240x160x96
 // 348 -> 137 us.
 template <typename T, int L, int CB, int MODE, int ST, bool NT>
 __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
@@ -690,7 +690,8 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
 
     // --- force, pressure projection, negation (Compute_force_TO_rhs), in
     // place on N: N <- -(N - F + i K p), p = i K.(N - F) / K^2 (computed in
-    // FP64, stored in the transform precision) ---
+    // FP64, stored in the transform precision); the forced modes in a second
+    // turn, so that all others take one code in every tile ---
     auto project = [&](auto fc) {
         constexpr bool FORCED = decltype(fc)::value;
         const int jh = hidden(j);
@@ -699,8 +700,10 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
             const int lx = jh + TPL * s;
             const int kx = kwave(lx, g.nx);
             const double Kx = kx * g.kf[0];
+            const bool f_mode = (forced & (1u << s)) != 0;
+            if (FORCED && !f_mode) continue;
             cpx<double> n0 = cvt<double>(N[0][s]), n1 = cvt<double>(N[1][s]), n2 = cvt<double>(N[2][s]);
-            if (FORCED && (forced & (1u << s))) {
+            if constexpr (FORCED) {
                 // the stage input's band modes, or the random force itself
                 const cpx<double> *sv =
                     (const cpx<double> *)(a.b.kind == 1 ? a.slots_in : a.b.force) + band_slot(a.b, kx, ky, lz) * 3;
@@ -719,17 +722,20 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
             n0 = n0 + mul_i(Kx, pr);
             n1 = n1 + mul_i(Ky, pr);
             n2 = n2 + mul_i(Kz, pr);
-            N[0][s] = cvt<T>(mk<double>(-n0.x, -n0.y));
-            N[1][s] = cvt<T>(mk<double>(-n1.x, -n1.y));
-            N[2][s] = cvt<T>(mk<double>(-n2.x, -n2.y));
+            const cpx<T> r0 = cvt<T>(mk<double>(-n0.x, -n0.y)), r1 = cvt<T>(mk<double>(-n1.x, -n1.y)),
+                         r2 = cvt<T>(mk<double>(-n2.x, -n2.y));
+            const bool keep = !FORCED && f_mode;
+            N[0][s] = mk<T>(keep ? N[0][s].x : r0.x, keep ? N[0][s].y : r0.y);
+            N[1][s] = mk<T>(keep ? N[1][s].x : r1.x, keep ? N[1][s].y : r1.y);
+            N[2][s] = mk<T>(keep ? N[2][s].x : r2.x, keep ? N[2][s].y : r2.y);
 #pragma unroll
             for (int i = 0; i < 3; i++) settle(N[i][s]);
             if (s % 2) __builtin_amdgcn_sched_barrier(0);
         }
     };
     if (want_rhs) {
+        project(std::false_type{});
         if (band_tile) project(std::true_type{});
-        else project(std::false_type{});
     }
 
     if constexpr (ST == 0) {
