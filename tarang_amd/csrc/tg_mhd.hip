@@ -121,9 +121,13 @@ constexpr int mhd_index(int pi)
 // As k_x_nlin: columns in registers in transform order, the next tile in
 // flight, products unrolled, code per stage, values settled where they are
 // formed.  The six sums take 192 registers in FP64: blocks of 512 threads spill
-// about 120 of them a lane, which costs less than 64-byte rows in blocks of 256
-// (512 registers a thread): a step at 320 x 320 x 240 16 ms against 29, 512 x 256 x
-// 512 33 against 34, 1024 x 256 x 512 (64-byte rows, or 32) 124 against 129.
+// about 120 of them a lane, which costs less than rows of half the width in
+// blocks of 256 (512 registers a thread): a step at 320 x 320 x 240 16 ms against
+// 29, 512 x 256 x 512 33 against 34, 1024 x 256 x 512 82 against 89.
+// The lambdas are inlined by attribute: left to the compiler, the x-inverse was a
+// function at 240, 384 and 480 points and from 640 on, its columns passed through
+// memory and its caller's registers saved around each call (1024 x 256 x 512: 23 ms a
+// launch and 129 a step, now 11 and 82).
 // 512^3 FP32, per launch: 11.0 ms, now 5.1 in stage 1, 5.9 in stages 2 and 3
 // (4.8 TB/s), 7.1 in stage 4.
 template <typename T, int L, int CB, int ST, bool NT>
@@ -157,7 +161,7 @@ __global__ void __launch_bounds__(CB *(L / 8), CB * (L / 8) <= 256 ? 1 : 2) k_x_
 #pragma unroll
     for (int s = 0; s < 8; s++) Np[0][s] = Np[1][s] = Np[2][s] = Nm[0][s] = Nm[1][s] = Nm[2][s] = mk<T>(0, 0);
     cpx<double> w[8];   // the state of u, then of b, of one component
-    auto product = [&](auto pc, cpx<T> *v, cpx<T> *next) {
+    auto product = [&](auto pc, cpx<T> *v, cpx<T> *next) __attribute__((always_inline)) {
         constexpr int PI = decltype(pc)::value;
         constexpr int P = mhd_index(PI), I = P / 3, J = P % 3;
         pin_memory_order();
@@ -245,7 +249,7 @@ __global__ void __launch_bounds__(CB *(L / 8), CB * (L / 8) <= 256 ? 1 : 2) k_x_
     if (ST >= 2) col_load<NTA>(ac, (const cpx<double> *)a.accV[0] + t.cw0, t.stepw, t.offw);
     double chk = 0.0;   // stage 4: NaN after a non-finite value
     // the accumulator, or the new state
-    auto put = [&](double *acc, double *state) {
+    auto put = [&](double *acc, double *state) __attribute__((always_inline)) {
         if (ST == 4) {
             if (t.live) col_store<false>(ac, (cpx<double> *)state + t.state0, t.steps, t.offs);
         } else if (t.inside) {
@@ -254,7 +258,7 @@ __global__ void __launch_bounds__(CB *(L / 8), CB * (L / 8) <= 256 ? 1 : 2) k_x_
     };
     // x-inverse of the next stage input (stage 4: of the next step's
     // first stage, D(u) +- D(b) of the new state)
-    auto inverse = [&](cpx<T> *z, void *u) {
+    auto inverse = [&](cpx<T> *z, void *u) __attribute__((always_inline)) {
         pin_memory_order();
         fft_exchange<L, +1>(z, x, tw, hidden(j));
         pin_memory_order();
@@ -263,7 +267,7 @@ __global__ void __launch_bounds__(CB *(L / 8), CB * (L / 8) <= 256 ? 1 : 2) k_x_
     // Z+ of component K - 1 is transformed while b of component K is
     // loaded, its Z- while u of component K + 1 is
     cpx<T> zp[8], zm[8], zl[8];
-    auto comp = [&](auto kc) {
+    auto comp = [&](auto kc) __attribute__((always_inline)) {
         constexpr int K = decltype(kc)::value;
         constexpr int K1 = K < 2 ? K + 1 : 2;
         cpx<double> un[8];
