@@ -79,8 +79,6 @@ struct tg_plan {
     double *force_eh = nullptr;
     int force_eh_n = 0;
     double force_key[4] = {};  // eps, helicity, r_in, r_out of the table
-    double *force_tab = nullptr;   // the force of the band's slots for the call's seed
-    size_t force_tab_bytes = 0;
     // chaining of RK4 steps: valid for the same state pointers and band
     bool unext_valid = false;
     double *unext_V[3] = {};
@@ -237,7 +235,7 @@ void free_plan(tg_plan *p)
     for (void *q : p->mhd)
         if (q) (void)hipFree(q);
     void *aptrs[] = {p->adj.ckpt, p->adj.tape, p->adj.vw, p->adj.lg, p->adj.acc, p->rfield,
-                     p->umax_dev, p->force_eh, p->force_tab};
+                     p->umax_dev, p->force_eh};
     for (void *q : aptrs)
         if (q) (void)hipFree(q);
     void *cptrs[] = {p->ch.D, p->ch.NL[0], p->ch.NL[1], p->ch.NL[2], p->ch.X, p->ch.Y, p->ch.pp, p->ch.pm,
@@ -357,21 +355,17 @@ int ensure_slots(tg_plan *p, const tg_fluid *f)
         const int n[3] = {p->g.nx, p->g.ny, p->g.nz};
         for (int d = 0; d < 3; d++)
             b.h[d] = (int)std::min<double>(std::ceil(f->force_r_out / p->g.kf[d]), n[d] / 2);
-        const size_t bytes = (size_t)(2 * b.h[0] + 1) * (2 * b.h[1] + 1) * (b.h[2] + 1) * 3 * 16;
-        if (bytes > p->force_tab_bytes) {
-            HIPCHK(hipStreamSynchronize(p->stream));
-            if (p->force_tab) {
-                (void)hipFree(p->force_tab);
-                p->dev_bytes -= (int64_t)p->force_tab_bytes;
-                p->force_tab = nullptr;
-                p->force_tab_bytes = 0;
-            }
-            int rc = dmalloc(p, (void **)&p->force_tab, bytes);
-            if (rc) return rc;
-            p->force_tab_bytes = bytes;
-        }
-        b.force = p->force_tab;
-        HIPCHK(launch_random_force(p->g, b, p->force_tab, p->stream));
+        // the call's force lies in work fields that an NS step and right-hand side leave
+        // alone (U[0..2], P[0..5] are theirs): the slots in one of them where they fit,
+        // of wider bands a field per component, or two with FP32 work fields
+        void *spare[6] = {p->U[3], p->U[4], p->U[5], p->P[6], p->P[7], p->P[8]};
+        const size_t slots = (size_t)(2 * b.h[0] + 1) * (2 * b.h[1] + 1) * (b.h[2] + 1);
+        b.packed = slots * 48 <= p->ncw * p->elem;
+        for (int half = 0; half < 2; half++)
+            for (int c = 0; c < 3; c++)
+                b.force[half][c] = b.packed ? (double *)spare[0] + 2 * c
+                                   : p->elem == 16 ? (double *)spare[c] + half * p->ncw : (double *)spare[2 * c + half];
+        HIPCHK(launch_random_force(p->g, b, p->stream));
     } else if (f && f->force_kind != 0) {
         return fail(TG_ERR_ARG, "unknown force_kind %d", f->force_kind);
     }

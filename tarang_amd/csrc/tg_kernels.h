@@ -41,10 +41,13 @@ struct Band {
     int kind;             // 0 none, 1 constant energy supply alpha-forcing, 2 random band forcing
     int h[3];             // box half-widths
     double r_in, r_out, eps;
-    // kind 2: the force of every slot (launch_random_force), made from the
-    // per-mode supplies (e_k, h_k) of shells 0..ceil(r_out), the random
-    // interval and the seed of the phases
-    const double *force;
+    // the modes' forces (kind 1: to be scaled by alpha): the three components of
+    // each slot (packed), or a padded FP64 work field per component, in two halves
+    // lx < Nx/2 and lx >= Nx/2
+    double *force[2][3];
+    int packed;
+    // kind 2: made from the per-mode supplies (e_k, h_k) of shells
+    // 0..ceil(r_out), the random interval and the seed of the phases
     const double *shell_eh;
     double tau;
     unsigned long long seed;
@@ -126,8 +129,8 @@ hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void 
                          double *const *acc, void *const *U, const double *slots_in, double *slots_out,
                          double *const *out, const void *twx, hipStream_t st, const Cut *cut = nullptr);
 
-// the random force (kind 2) of the band's slots, 3 complex values each
-hipError_t launch_random_force(const Grid &g, const Band &b, double *out, hipStream_t st);
+// the random force (kind 2) of the band's modes into b.force
+hipError_t launch_random_force(const Grid &g, const Band &b, hipStream_t st);
 hipError_t launch_reality(const Grid &g, double *const *V, int ncomp, hipStream_t st);
 hipError_t launch_dealias(const Grid &g, double *const *V, int ncomp, hipStream_t st);
 

@@ -505,6 +505,23 @@ __device__ __forceinline__ double band_alpha(const Grid &g, const Band &b, const
     return t > 0.0 ? b.eps / (2.0 * t) : 0.0;
 }
 
+// Where the force of row lx of a column lies, in complex values from
+// b.force[lx >= Nx/2][component] on.
+struct ForcePlace {
+    size_t row, col;
+    bool packed;
+    __device__ __forceinline__ ForcePlace(const Grid &g, const Band &b, int ky, int ly, int lz) : packed(b.packed)
+    {
+        row = packed ? (size_t)3 * (2 * b.h[1] + 1) * (b.h[2] + 1) : (size_t)g.ny * g.nzp;
+        col = packed ? (size_t)3 * band_slot(b, 0, ky, lz) : (size_t)ly * g.nzp + lz;
+    }
+    __device__ __forceinline__ size_t operator()(const Grid &g, int lx) const
+    {
+        const int r = packed ? kwave(lx, g.nx) : (lx < g.nx / 2 ? lx : lx - g.nx / 2);
+        return col + r * row;
+    }
+};
+
 // Random band forcing of one mode (kind 2; compute_force_random.cc:65-130,
 // force_amp_phase.cc:119-170, FFF_pencil_inline.h:234-248): helical
 // amplitudes sqrt((e_k +- h_k/K) / tau) with phases 2 pi U(seed, 2m),
@@ -530,11 +547,10 @@ __device__ void random_force_mode(const Grid &g, const Band &b, int lx, int ly, 
 }
 
 #if TG_LEN_UNIT == 0
-// The random force of every mode of the box |k_d| <= h_d in band_slot order,
-// zero outside r_in < K <= r_out.  The phases hold for a whole call, so they
-// are drawn once here: within the x pass their sines and cosines were most of
-// its instructions (0.5 ms of a 512^3 FP64 step).
-__global__ void k_random_force(Grid g, Band b, double *out)
+// The random force of the band's modes (r_in < K <= r_out).  The phases hold for a
+// whole call, so they are drawn once here: within the x pass their sines and
+// cosines were most of its instructions (0.5 ms of a 512^3 FP64 step).
+__global__ void k_random_force(Grid g, Band b)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= band_nslots(b)) return;
@@ -543,17 +559,18 @@ __global__ void k_random_force(Grid g, Band b, double *out)
     const int kx = i / ((b.h[2] + 1) * (2 * b.h[1] + 1)) - b.h[0];
     // the indices of the mode; k = -N/2 is not one
     const int lx = kx >= 0 ? kx : kx + g.nx, ly = ky >= 0 ? ky : ky + g.ny;
-    const double K = kmag(g, kx, ky, kz);
-    cpx<double> F[3] = {mk<double>(0, 0), mk<double>(0, 0), mk<double>(0, 0)};
-    if (K > b.r_in && K <= b.r_out && kwave(lx, g.nx) == kx && kwave(ly, g.ny) == ky && kz < g.nzc)
-        random_force_mode(g, b, lx, ly, kz, kx, ky, K, F);
-    for (int c = 0; c < 3; c++) ((cpx<double> *)out)[3 * (size_t)i + c] = F[c];
+    if (kwave(lx, g.nx) != kx || kwave(ly, g.ny) != ky || kz >= g.nzc || !in_band(g, b, kx, ky, kz)) return;
+    cpx<double> F[3];
+    random_force_mode(g, b, lx, ly, kz, kx, ky, kmag(g, kx, ky, kz), F);
+    const size_t w = ForcePlace(g, b, ky, ly, kz)(g, lx);
+#pragma unroll
+    for (int c = 0; c < 3; c++) ((cpx<double> *)b.force[lx >= g.nx / 2][c])[w] = F[c];
 }
 
-hipError_t launch_random_force(const Grid &g, const Band &b, double *out, hipStream_t st)
+hipError_t launch_random_force(const Grid &g, const Band &b, hipStream_t st)
 {
     const int n = band_nslots(b);
-    hipLaunchKernelGGL(k_random_force, dim3((n + 63) / 64), dim3(64), 0, st, g, b, out);
+    hipLaunchKernelGGL(k_random_force, dim3((n + 63) / 64), dim3(64), 0, st, g, b);
     return hipGetLastError();
 }
 #endif
@@ -695,22 +712,22 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
     auto project = [&](auto fc) {
         constexpr bool FORCED = decltype(fc)::value;
         const int jh = hidden(j);
+        const ForcePlace fp(g, a.b, ky, ly, lz);
+        const double fscale = a.b.kind == 1 ? alpha : 1.0;
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const int lx = jh + TPL * s;
-            const int kx = kwave(lx, g.nx);
-            const double Kx = kx * g.kf[0];
+            const double Kx = kwave(lx, g.nx) * g.kf[0];
             const bool f_mode = (forced & (1u << s)) != 0;
             if (FORCED && !f_mode) continue;
             cpx<double> n0 = cvt<double>(N[0][s]), n1 = cvt<double>(N[1][s]), n2 = cvt<double>(N[2][s]);
             if constexpr (FORCED) {
                 // the stage input's band modes, or the random force itself
-                const cpx<double> *sv =
-                    (const cpx<double> *)(a.b.kind == 1 ? a.slots_in : a.b.force) + band_slot(a.b, kx, ky, lz) * 3;
-                const double f = a.b.kind == 1 ? alpha : 1.0;
-                n0 = n0 - f * sv[0];
-                n1 = n1 - f * sv[1];
-                n2 = n2 - f * sv[2];
+                const size_t w = fp(g, lx);
+                auto sv = [&](int c) { return ((const cpx<double> *)a.b.force[s >= 4][c])[w]; };
+                n0 = n0 - fscale * sv(0);
+                n1 = n1 - fscale * sv(1);
+                n2 = n2 - fscale * sv(2);
             }
             cpx<double> div = mul_i(Kx, n0);
             div = div + mul_i(Ky, n1);
@@ -1194,6 +1211,10 @@ hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void 
     a.tw = twx;
     a.g = g;
     a.b = b;
+    if (b.kind == 1) {
+        a.b.packed = 1;
+        for (int c = 0; c < 3; c++) a.b.force[0][c] = a.b.force[1][c] = const_cast<double *>(slots_in) + 2 * c;
+    }
     a.rk = rk;
     if (giver) {
         a.rk.stage = 0;
