@@ -63,8 +63,10 @@ struct tg_plan {
     // twiddle tables in the transform precision: x (Nx), y (Ny), m (Nz/2) in
     // pass order (twiddle_order), n (Nz, k = 0..Nz/2)
     void *twx = nullptr, *twy = nullptr, *twm = nullptr, *twn = nullptr;
-    void *U[6] = {};      // x/y-transformed velocity (0..2) and giver (3..5) lines
-    void *P[9] = {};      // product spectra
+    // x/y-transformed velocity (0..2) and giver (3..5) lines, product spectra.
+    // U[3..5], with FP32 P[6..8] too, lie behind each other: three FP64 fields.
+    void *U[6] = {};
+    void *P[9] = {};
     double *acc[3] = {};  // RK4 accumulator (tot_Vrhs, RK.cc:96); giver nonlinear term
     double *slots[2] = {};
     size_t nslots = 0;
@@ -228,10 +230,10 @@ void free_plan(tg_plan *p)
         if (q) (void)hipFree(q);
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
-    for (void *q : p->U)
-        if (q) (void)hipFree(q);
-    for (void *q : p->P)
-        if (q) (void)hipFree(q);
+    for (int i = 0; i < 4; i++)
+        if (p->U[i]) (void)hipFree(p->U[i]);
+    for (int i = 0; i < (p->elem == 8 ? 6 : 9); i++)
+        if (p->P[i]) (void)hipFree(p->P[i]);
     for (void *q : p->mhd)
         if (q) (void)hipFree(q);
     void *aptrs[] = {p->adj.ckpt, p->adj.tape, p->adj.vw, p->adj.lg, p->adj.acc, p->rfield,
@@ -356,15 +358,8 @@ int ensure_slots(tg_plan *p, const tg_fluid *f)
         for (int d = 0; d < 3; d++)
             b.h[d] = (int)std::min<double>(std::ceil(f->force_r_out / p->g.kf[d]), n[d] / 2);
         // the call's force lies in work fields that an NS step and right-hand side leave
-        // alone (U[0..2], P[0..5] are theirs): the slots in one of them where they fit,
-        // of wider bands a field per component, or two with FP32 work fields
-        void *spare[6] = {p->U[3], p->U[4], p->U[5], p->P[6], p->P[7], p->P[8]};
-        const size_t slots = (size_t)(2 * b.h[0] + 1) * (2 * b.h[1] + 1) * (b.h[2] + 1);
-        b.packed = slots * 48 <= p->ncw * p->elem;
-        for (int half = 0; half < 2; half++)
-            for (int c = 0; c < 3; c++)
-                b.force[half][c] = b.packed ? (double *)spare[0] + 2 * c
-                                   : p->elem == 16 ? (double *)spare[c] + half * p->ncw : (double *)spare[2 * c + half];
+        // alone (U[0..2], P[0..5] are theirs)
+        b.force = (double *)p->U[3];
         HIPCHK(launch_random_force(p->g, b, p->stream));
     } else if (f && f->force_kind != 0) {
         return fail(TG_ERR_ARG, "unknown force_kind %d", f->force_kind);
@@ -1197,8 +1192,14 @@ int tg_plan_create(const tg_config *cfg, tg_plan **plan)
         if (!rc) rc = upload_twiddles<double>(p, &p->twn, cfg->nz, cfg->nz / 2 + 1, false);
         if (!rc && p->g.basis == 1) rc = upload_twiddles<double>(p, &p->twq, 4 * cfg->nx, cfg->nx, false);
     }
-    for (int i = 0; i < 6 && !rc; i++) rc = dmalloc(p, &p->U[i], p->ncw * p->elem);
-    for (int i = 0; i < 9 && !rc; i++) rc = dmalloc(p, &p->P[i], p->ncw * p->elem);
+    for (int i = 0; i < 3 && !rc; i++) rc = dmalloc(p, &p->U[i], p->ncw * p->elem);
+    if (!rc) rc = dmalloc(p, &p->U[3], 3 * p->ncw * 16);
+    for (int i = 0; i < (p->elem == 8 ? 6 : 9) && !rc; i++) rc = dmalloc(p, &p->P[i], p->ncw * p->elem);
+    if (!rc) {
+        char *u = (char *)p->U[3];
+        for (int i = 1; i < 3; i++) p->U[3 + i] = u + i * p->ncw * p->elem;
+        for (int i = 3; i < 6 && p->elem == 8; i++) p->P[3 + i] = u + i * p->ncw * p->elem;
+    }
     // the pad columns kz >= Nz/2+1 of the work fields are never written; the x
     // passes load them with their tiles (and discard the results): keep them zero
     for (int i = 0; i < 6 && !rc; i++)

@@ -41,11 +41,9 @@ struct Band {
     int kind;             // 0 none, 1 constant energy supply alpha-forcing, 2 random band forcing
     int h[3];             // box half-widths
     double r_in, r_out, eps;
-    // the modes' forces (kind 1: to be scaled by alpha): the three components of
-    // each slot (packed), or a padded FP64 work field per component, in two halves
-    // lx < Nx/2 and lx >= Nx/2
-    double *force[2][3];
-    int packed;
+    // the three components of each mode's force, at force_place: kind 1 (to be
+    // scaled by alpha) of the slots, kind 2 of the grid's modes (48 Nx Ny nzp bytes)
+    double *force;
     // kind 2: made from the per-mode supplies (e_k, h_k) of shells
     // 0..ceil(r_out), the random interval and the seed of the phases
     const double *shell_eh;

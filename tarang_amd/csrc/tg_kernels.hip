@@ -505,22 +505,13 @@ __device__ __forceinline__ double band_alpha(const Grid &g, const Band &b, const
     return t > 0.0 ? b.eps / (2.0 * t) : 0.0;
 }
 
-// Where the force of row lx of a column lies, in complex values from
-// b.force[lx >= Nx/2][component] on.
-struct ForcePlace {
-    size_t row, col;
-    bool packed;
-    __device__ __forceinline__ ForcePlace(const Grid &g, const Band &b, int ky, int ly, int lz) : packed(b.packed)
-    {
-        row = packed ? (size_t)3 * (2 * b.h[1] + 1) * (b.h[2] + 1) : (size_t)g.ny * g.nzp;
-        col = packed ? (size_t)3 * band_slot(b, 0, ky, lz) : (size_t)ly * g.nzp + lz;
-    }
-    __device__ __forceinline__ size_t operator()(const Grid &g, int lx) const
-    {
-        const int r = packed ? kwave(lx, g.nx) : (lx < g.nx / 2 ? lx : lx - g.nx / 2);
-        return col + r * row;
-    }
-};
+// Where the force of the modes of a column lies in b.force, in modes: row kx at
+// place + kx step.
+__device__ __forceinline__ void force_place(const Grid &g, const Band &b, int ky, int ly, int lz, int &place, int &step)
+{
+    step = b.kind == 1 ? (2 * b.h[1] + 1) * (b.h[2] + 1) : g.ny * g.nzp;
+    place = b.kind == 1 ? band_slot(b, 0, ky, lz) : (g.nx / 2 - 1) * step + ly * g.nzp + lz;
+}
 
 // Random band forcing of one mode (kind 2; compute_force_random.cc:65-130,
 // force_amp_phase.cc:119-170, FFF_pencil_inline.h:234-248): helical
@@ -562,9 +553,10 @@ __global__ void k_random_force(Grid g, Band b)
     if (kwave(lx, g.nx) != kx || kwave(ly, g.ny) != ky || kz >= g.nzc || !in_band(g, b, kx, ky, kz)) return;
     cpx<double> F[3];
     random_force_mode(g, b, lx, ly, kz, kx, ky, kmag(g, kx, ky, kz), F);
-    const size_t w = ForcePlace(g, b, ky, ly, kz)(g, lx);
+    int place, step;
+    force_place(g, b, ky, ly, kz, place, step);
 #pragma unroll
-    for (int c = 0; c < 3; c++) ((cpx<double> *)b.force[lx >= g.nx / 2][c])[w] = F[c];
+    for (int c = 0; c < 3; c++) ((cpx<double> *)b.force)[(size_t)3 * (place + kx * step) + c] = F[c];
 }
 
 hipError_t launch_random_force(const Grid &g, const Band &b, hipStream_t st)
@@ -712,22 +704,23 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
     auto project = [&](auto fc) {
         constexpr bool FORCED = decltype(fc)::value;
         const int jh = hidden(j);
-        const ForcePlace fp(g, a.b, ky, ly, lz);
+        int place = 0, step = 0;
+        if constexpr (FORCED) force_place(g, a.b, ky, ly, lz, place, step);
         const double fscale = a.b.kind == 1 ? alpha : 1.0;
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const int lx = jh + TPL * s;
-            const double Kx = kwave(lx, g.nx) * g.kf[0];
+            const int kx = kwave(lx, g.nx);
+            const double Kx = kx * g.kf[0];
             const bool f_mode = (forced & (1u << s)) != 0;
             if (FORCED && !f_mode) continue;
             cpx<double> n0 = cvt<double>(N[0][s]), n1 = cvt<double>(N[1][s]), n2 = cvt<double>(N[2][s]);
             if constexpr (FORCED) {
                 // the stage input's band modes, or the random force itself
-                const size_t w = fp(g, lx);
-                auto sv = [&](int c) { return ((const cpx<double> *)a.b.force[s >= 4][c])[w]; };
-                n0 = n0 - fscale * sv(0);
-                n1 = n1 - fscale * sv(1);
-                n2 = n2 - fscale * sv(2);
+                const cpx<double> *sv = (const cpx<double> *)a.b.force + (size_t)3 * (uint32_t)(place + kx * step);
+                n0 = n0 - fscale * sv[0];
+                n1 = n1 - fscale * sv[1];
+                n2 = n2 - fscale * sv[2];
             }
             cpx<double> div = mul_i(Kx, n0);
             div = div + mul_i(Ky, n1);
@@ -1211,10 +1204,7 @@ hipError_t launch_x_nlin(const Grid &g, const Band &b, const RkParams &rk, void 
     a.tw = twx;
     a.g = g;
     a.b = b;
-    if (b.kind == 1) {
-        a.b.packed = 1;
-        for (int c = 0; c < 3; c++) a.b.force[0][c] = a.b.force[1][c] = const_cast<double *>(slots_in) + 2 * c;
-    }
+    if (b.kind == 1) a.b.force = const_cast<double *>(slots_in);
     a.rk = rk;
     if (giver) {
         a.rk.stage = 0;
