@@ -84,7 +84,7 @@ __device__ __forceinline__ void xsym_columns(const Grid &g, const ColTile<T, L, 
 }
 
 // Column tiles in registers in transform order (ColX), as k_xfwd_adj.
-template <typename T, int L, int CB, bool NT>
+template <typename T, int L, int CB>
 __global__ void __launch_bounds__(CB *(L / 8), 2) k_xinv_sym(XsymArgs a)
 {
     using X = ColX<T, L, CB>;
@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(CB *(L / 8), 2) k_xinv_sym(XsymArgs a)
     for (int c = 0; c < 3; c++) col_load<false>(m[c], (const cpx<double> *)a.G[c] + t.state0, t.steps, t.offs);
     for (int i = threadIdx.x; i < L; i += CB * (L / 8)) tw[i] = ((const cpx<T> *)a.tw)[i];
     lds_barrier();
-    xsym_columns<NT>(g, t, X{lds + t.c}, tw, a.S, m);
+    xsym_columns<false>(g, t, X{lds + t.c}, tw, a.S, m);
 }
 
 // q += u * v (SUB: q -= u * v) on the packed real points of this thread (u
@@ -280,7 +280,7 @@ template <typename T, int LL>
 hipError_t xinv_sym_len(const XsymArgs &a, hipStream_t st)
 {
     constexpr int CB = colx_block<T>(LL, 512);
-    hipLaunchKernelGGL((k_xinv_sym<T, LL, CB, false>), dim3(x_grid(x_tiles(a.g, CB, false))), dim3(CB * (LL / 8)), 0, st, a);
+    hipLaunchKernelGGL((k_xinv_sym<T, LL, CB>), dim3(x_grid(x_tiles(a.g, CB, false))), dim3(CB * (LL / 8)), 0, st, a);
     return hipGetLastError();
 }
 

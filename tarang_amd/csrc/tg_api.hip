@@ -389,7 +389,7 @@ int run_forward(tg_plan *p, const double *real_dev, double *spec_dev, int sincos
     const double *R[1] = {real_dev};
     void *W[1] = {p->U[0]};
     { Prof pr(p, TG_KERNEL_Z_R2C); HIPCHK(launch_z_r2c<T>(p->g, R, 1, W, p->twm, p->twn, p->stream)); }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, -1, W, 1, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, -1, W, 1, p->twy, p->stream)); }
     double *O[1] = {spec_dev};
     if (p->g.basis == 1) {
         const double scale = 1.0 / (2.0 * p->g.nx * (double)p->g.ny * p->g.nz);
@@ -417,7 +417,7 @@ int run_inverse(tg_plan *p, const double *spec_dev, double *real_dev, int sincos
         Prof pr(p, TG_KERNEL_X_INV);
         HIPCHK(launch_xinv_state<T>(p->g, nb, V, 1, W, nullptr, 0, p->twx, p->stream));
     }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, +1, W, 1, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, +1, W, 1, p->twy, p->stream)); }
     double *R[1] = {real_dev};
     { Prof pr(p, TG_KERNEL_Z_C2R); HIPCHK(launch_z_c2r<T>(p->g, W, 1, R, p->twm, p->twn, p->stream)); }
     return TG_OK;
@@ -432,12 +432,12 @@ template <typename T>
 int ns_middle(tg_plan *p, bool trace_free)
 {
     const int np = trace_free ? 5 : 6;
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, +1, p->U, 3, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, +1, p->U, 3, p->twy, p->stream)); }
     {
         Prof pr(p, TG_KERNEL_Z_PRODUCTS);
         HIPCHK(launch_z_products<T>(p->g, p->U, p->P, trace_free ? 2 : 0, p->twm, p->twn, p->stream));
     }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, -1, p->P, np, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, -1, p->P, np, p->twy, p->stream)); }
     return TG_OK;
 }
 
@@ -536,14 +536,14 @@ int run_giver_nlin(tg_plan *p, double *const X[3], double *const Y[3], int filte
     }
     {
         Prof pr(p, TG_KERNEL_Y_FFT);
-        if (!receiver_ready) HIPCHK(launch_colfft<T>(p->g, 1, +1, p->U, 3, p->twy, p->stream, &cut));
-        HIPCHK(launch_colfft<T>(p->g, 1, +1, p->U + 3, 3, p->twy, p->stream, &wc));
+        if (!receiver_ready) HIPCHK(launch_colfft<T>(p->g, +1, p->U, 3, p->twy, p->stream, &cut));
+        HIPCHK(launch_colfft<T>(p->g, +1, p->U + 3, 3, p->twy, p->stream, &wc));
     }
     {
         Prof pr(p, TG_KERNEL_Z_PRODUCTS);
         HIPCHK(launch_z_products<T>(p->g, p->U, p->P, 1, p->twm, p->twn, p->stream, nullptr, &cut, &wc, &cut));
     }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, -1, p->P, 9, p->twy, p->stream, &cut)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, -1, p->P, 9, p->twy, p->stream, &cut)); }
     RkParams rk = rk_params(p, nullptr, -1);
     Prof pr(p, TG_KERNEL_X_NLIN_GIVER);
     HIPCHK(launch_x_nlin<T>(p->g, nb, rk, p->P, nullptr, nullptr, nullptr, nullptr, nullptr, out, p->twx,
@@ -608,9 +608,9 @@ template <typename T>
 int mhd_nonlinear(tg_plan *p, double *const *Np, double *const *Nm)
 {
     Band nb{};
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, +1, p->U, 6, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, +1, p->U, 6, p->twy, p->stream)); }
     { Prof pr(p, TG_KERNEL_Z_PRODUCTS); HIPCHK(launch_z_products<T>(p->g, p->U, p->P, 1, p->twm, p->twn, p->stream)); }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, -1, p->P, 9, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, -1, p->P, 9, p->twy, p->stream)); }
     Prof pr(p, TG_KERNEL_X_NLIN_GIVER);
     RkParams rk = rk_params(p, nullptr, -1);
     HIPCHK(launch_x_nlin<T>(p->g, nb, rk, p->P, nullptr, nullptr, nullptr, nullptr, nullptr, Np, p->twx, p->stream));
@@ -642,13 +642,13 @@ int run_rk4_mhd(tg_plan *p, double *const V[3], double *const W[3], const tg_flu
     if (rc) return rc;
     for (int step = 0; step < nsteps; step++) {
         for (int s = 1; s <= 4; s++) {
-            { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, +1, p->U, 6, p->twy, p->stream)); }
+            { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, +1, p->U, 6, p->twy, p->stream)); }
             {
                 // the eight trace-shifted products (P_zz enters N_u only as a gradient)
                 Prof pr(p, TG_KERNEL_Z_PRODUCTS);
                 HIPCHK(launch_z_products<T>(p->g, p->U, p->P, 3, p->twm, p->twn, p->stream));
             }
-            { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, -1, p->P, 8, p->twy, p->stream)); }
+            { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, -1, p->P, 8, p->twy, p->stream)); }
             // one x pass: both nonlinear terms, the stage for u and b, the next Z+- x-inverse
             XmhdArgs xa{};
             for (int i = 0; i < 9; i++) xa.P[i] = p->P[i];
@@ -765,12 +765,12 @@ int record_steps(tg_plan *p, double *const V[3], const tg_fluid *f, int nsteps)
     for (int step = 0; step < nsteps; step++)
         for (int s = 1; s <= 4; s++) {
             void *tp[3] = {tape_ptr(p, step, s - 1, 0), tape_ptr(p, step, s - 1, 1), tape_ptr(p, step, s - 1, 2)};
-            { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, +1, p->U, 3, p->twy, p->stream)); }
+            { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, +1, p->U, 3, p->twy, p->stream)); }
             {
                 Prof pr(p, TG_KERNEL_Z_PRODUCTS);
                 HIPCHK(launch_z_products<T>(p->g, p->U, p->P, 2, p->twm, p->twn, p->stream, tp));
             }
-            { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, -1, p->P, 5, p->twy, p->stream)); }
+            { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, -1, p->P, 5, p->twy, p->stream)); }
             RkParams rk = rk_params(p, f, s);
             rk.trace_free = 1;
             Prof pr(p, TG_KERNEL_X_NLIN_RK);
@@ -794,9 +794,9 @@ int adj_stage(tg_plan *p, double *const G[3], void *const tp[3], const AdjParams
     void *S[5] = {p->P[0], p->P[1], p->P[2], p->P[3], p->P[4]};
     void *Q[3] = {p->P[6], p->P[7], p->P[8]};
     if (!sym_done) { Prof pr(p, TG_KERNEL_X_INV_SYM); HIPCHK(launch_xinv_sym<T>(p->g, G, S, p->twx, p->stream)); }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, +1, S, 5, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, +1, S, 5, p->twy, p->stream)); }
     { Prof pr(p, TG_KERNEL_Z_ADJ); HIPCHK(launch_z_adj<T>(p->g, S, Q, tp, p->twm, p->twn, p->stream)); }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, -1, Q, 3, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, -1, Q, 3, p->twy, p->stream)); }
     Prof pr(p, TG_KERNEL_X_FWD_ADJ);
     HIPCHK(launch_xfwd_adj<T>(p->g, ap, Q, lam, acc, lg, p->twx, p->stream, fuse_next ? S : nullptr));
     return TG_OK;
@@ -908,7 +908,7 @@ int run_rhs_vjp(tg_plan *p, double *const V[3], double *const lam[3], double *co
     Band nb{};
     void *tp[3] = {tape_ptr(p, 0, 0, 0), tape_ptr(p, 0, 0, 1), tape_ptr(p, 0, 0, 2)};
     { Prof pr(p, TG_KERNEL_X_INV); HIPCHK(launch_xinv_state<T>(p->g, nb, V, 3, p->U, nullptr, 1, p->twx, p->stream)); }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, +1, p->U, 3, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, +1, p->U, 3, p->twy, p->stream)); }
     {
         Prof pr(p, TG_KERNEL_Z_PRODUCTS);
         HIPCHK(launch_z_products<T>(p->g, p->U, p->P, 0, p->twm, p->twn, p->stream, tp));
@@ -961,9 +961,9 @@ int rbc_middle(tg_plan *p, bool shift)
     int nf = 0;
     for (int i = 0; i < 9; i++)
         if (!(shift && i == 2)) F[nf++] = p->P[i];
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, +1, p->U, 4, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, +1, p->U, 4, p->twy, p->stream)); }
     { Prof pr(p, TG_KERNEL_Z_RBC); HIPCHK(launch_z_rbc<T>(p->g, p->U, p->P, p->twm, p->twn, p->stream, shift)); }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, 1, -1, F, nf, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<T>(p->g, -1, F, nf, p->twy, p->stream)); }
     return TG_OK;
 }
 
@@ -1975,12 +1975,12 @@ static int chff_nlin(tg_plan *p, double *const V[3], double *const N[3], double 
         Prof pr(p, TG_KERNEL_X_SC);
         HIPCHK(launch_xinv_sc<double>(p->g, V, 3, 0, p->U, 8, p->twx, p->twq, p->stream));
     }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<double>(p->g, 1, +1, p->U, 3, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<double>(p->g, +1, p->U, 3, p->twy, p->stream)); }
     {
         Prof pr(p, TG_KERNEL_Z_PRODUCTS);
         HIPCHK(launch_z_products<double>(p->g, p->U, p->P, 0, p->twm, p->twn, p->stream));
     }
-    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<double>(p->g, 1, -1, p->P, 6, p->twy, p->stream)); }
+    { Prof pr(p, TG_KERNEL_Y_FFT); HIPCHK(launch_colfft<double>(p->g, -1, p->P, 6, p->twy, p->stream)); }
     Prof pr(p, TG_KERNEL_X_SC);
     const double scale = 1.0 / (2.0 * p->g.nx * (double)p->g.ny * p->g.nz);
     HIPCHK(launch_xfwd_chff(p->g, p->P, N, div, scale, p->twx, p->twq, p->stream));

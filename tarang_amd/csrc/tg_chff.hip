@@ -51,8 +51,6 @@ __global__ void k_cheb_deriv(const double *__restrict__ A, double *__restrict__ 
     }
 }
 
-__device__ __forceinline__ int c_k(int k) { return k == 0 ? 2 : 1; }
-
 // Helmholtz_complex_full_array / Helmholtz_real_full_array (helmholtz.cc:
 // 18-118): one parity of one column per thread, both parts of a complex
 // element (E = 2; the matrix is the same), lambda = Kperp^2 + lam_sup, through

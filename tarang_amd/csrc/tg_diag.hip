@@ -130,10 +130,9 @@ __global__ void __launch_bounds__(kRedThreads) k_reduce(RedArgs a)
     const int nb = a.nbins, nq = a.nq;
     constexpr bool ANIS = MODE == RED_RING_SPEC || MODE == RED_CYL_SPEC || MODE == RED_RING_MULT ||
                           MODE == RED_CYL_MULT;
-    constexpr bool BINNED = ANIS;
     double *bsum = dyn + (size_t)wave * nq * nb;
     double *bcmp = dyn + (size_t)(NW + wave) * nq * nb;
-    if (BINNED) {
+    if (ANIS) {
         for (int i = threadIdx.x; i < 2 * NW * nq * nb; i += blockDim.x) dyn[i] = 0.0;
         __syncthreads();
     }
@@ -248,7 +247,7 @@ __global__ void __launch_bounds__(kRedThreads) k_reduce(RedArgs a)
             }
         }
     }
-    if (!BINNED) {
+    if (!ANIS) {
         // block tree reduction of (s0 + c0)
         double v = s0 + c0;
         for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);

@@ -55,11 +55,11 @@ __host__ __device__ inline int band_nslots(const Band &b) { return (2 * b.h[0] +
 
 // Launch helpers (defined in tg_kernels.hip).  All return hipError_t.
 // T is float or double (transform precision).
-// cut: along y (axis 1), inverse: the rows and columns beyond it are zero and
-// not read; forward: they are not written.
+// The y pass.  cut, inverse: the rows and columns beyond it are zero and not
+// read; forward: they are not written.
 template <typename T>
-hipError_t launch_colfft(const Grid &g, int axis, int dir, void *const *fields, int nfields,
-                         const void *tw, hipStream_t st, const Cut *cut = nullptr);
+hipError_t launch_colfft(const Grid &g, int dir, void *const *fields, int nfields, const void *tw, hipStream_t st,
+                         const Cut *cut = nullptr);
 
 // x-inverse of an FP64 spectral field set into the T work layout.
 //   flags: 1 = dealias on read, 2 = write band slots, 4 = the kz = 0 and Nz/2

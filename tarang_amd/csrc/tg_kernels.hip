@@ -9,10 +9,10 @@
 //   real fields     R(x,y,z)           (Nx, Ny, Nz+2) FP64, z fastest.
 //
 // Passes:
-//   x pass  tiles of all Nx rows x CB contiguous (ly,lz) columns, staged
-//           through LDS (coalesced CB-wide row segments), one line per
-//           TPL = Nx/8 threads.
-//   y pass  tiles of all Ny rows x CB contiguous lz columns of one lx.
+//   x pass  tiles of all Nx rows x CB contiguous (ly,lz) columns, from memory to
+//           registers and back in the transform's order (ColX); LDS carries the
+//           exchanges between the radix passes, one line per TPL = Nx/8 threads.
+//   y pass  tiles of all Ny rows x CB contiguous lz columns of one lx, likewise.
 //   z pass  whole z-lines (contiguous), TPL = Nz/16 threads per line; a
 //           real line of Nz points is packed as Nz/2 complex points.
 #include <algorithm>
@@ -27,7 +27,7 @@
 namespace tg {
 
 // ---------------------------------------------------------------------------
-// Column FFT along a strided axis (the y pass, or a plain x pass).
+// Column FFT along a strided axis (the y pass).
 // ---------------------------------------------------------------------------
 struct ColArgs {
     void *f[9];
@@ -599,9 +599,10 @@ constexpr int xnl_axis(int mode, int p, int i)
 // where it is formed, and each stage is an instance of its own: with the four
 // stages, the hyperviscosity loops and the random phases inlined per point the
 // kernel was 300 KB of instructions, mostly fetched from L2 (and the stages'
-// registers, allocated together, spilled).  512^3, per launch: FP64 5170 ->
-// 3240 us (5.4 TB/s), FP32 4550 -> 2920 us; 64^3 FP64 54 -> 19 us, 240x160x96
-// 348 -> 137 us.
+// registers, allocated together, spilled).  512^3, per launch, mean of the four
+// stages: FP64 5170 -> 3620 us (4.8 TB/s), FP32 4550 -> 3150 us; 64^3 FP64 54 ->
+// 19 us, 240x160x96 348 -> 137 us; a step of 1024 x 256 x 512 (64-byte rows, one
+// block a CU) FP64 58.5 -> 38.2 ms, FP32 42.5 -> 27.2 ms.
 template <typename T, int L, int CB, int MODE, int ST, bool NT>
 __global__ void __launch_bounds__(CB *(L / 8), 2) k_x_nlin(XnlArgs a)
 {
@@ -1061,33 +1062,21 @@ hipError_t x_nlin_len(const XnlArgs &a, int mode, hipStream_t st)
 TG_ALL_UNITS(TG_KERNELS_L, TG_KERNELS_M, extern)
 
 template <typename T>
-hipError_t launch_colfft(const Grid &g, int axis, int dir, void *const *fields, int nfields, const void *tw,
-                         hipStream_t st, const Cut *cut)
+hipError_t launch_colfft(const Grid &g, int dir, void *const *fields, int nfields, const void *tw, hipStream_t st,
+                         const Cut *cut)
 {
     ColArgs a{};
     for (int i = 0; i < nfields; i++) a.f[i] = fields[i];
     a.tw = tw;
-    int L;
-    if (axis == 1) {
-        L = g.ny;
-        a.nouter = g.nx;
-        a.outer_stride = (long long)g.ny * g.nzp;
-        a.row_stride = g.nzp;
-        // the pad columns too (they hold zeros): a row's last 128-byte line is
-        // written whole (257 of 264 columns written: 1903 us a launch at 512^3
-        // FP64, all 264: 1780)
-        a.ncol = cut ? kept_columns<T>(g, cut->z) : g.nzp;
-        a.keep = cut ? cut->y : L;
-    } else {
-        if (cut) return hipErrorInvalidValue;
-        L = g.nx;
-        a.keep = L;
-        a.nouter = 1;
-        a.outer_stride = 0;
-        a.row_stride = (long long)g.ny * g.nzp;
-        a.ncol = g.ny * g.nzp;
-    }
-    TG_DISPATCH_L(T, L, return (colfft_len<T, LL>)(a, dir, nfields, st));
+    a.nouter = g.nx;
+    a.outer_stride = (long long)g.ny * g.nzp;
+    a.row_stride = g.nzp;
+    // the pad columns too (they hold zeros): a row's last 128-byte line is
+    // written whole (257 of 264 columns written: 1903 us a launch at 512^3
+    // FP64, all 264: 1780)
+    a.ncol = cut ? kept_columns<T>(g, cut->z) : g.nzp;
+    a.keep = cut ? cut->y : g.ny;
+    TG_DISPATCH_L(T, g.ny, return (colfft_len<T, LL>)(a, dir, nfields, st));
     return hipErrorInvalidValue;
 }
 
@@ -1238,7 +1227,7 @@ hipError_t launch_dealias(const Grid &g, double *const *V, int ncomp, hipStream_
 }
 
 #define TG_INST(T)                                                                                              \
-    template hipError_t launch_colfft<T>(const Grid &, int, int, void *const *, int, const void *, hipStream_t, \
+    template hipError_t launch_colfft<T>(const Grid &, int, void *const *, int, const void *, hipStream_t,      \
                                          const Cut *);                                                         \
     template hipError_t launch_xinv_state<T>(const Grid &, const Band &, double *const *, int, void *const *,   \
                                              double *, int, const void *, hipStream_t, double, double, double, \
