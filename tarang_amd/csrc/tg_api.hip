@@ -1200,8 +1200,8 @@ int tg_plan_create(const tg_config *cfg, tg_plan **plan)
         for (int i = 1; i < 3; i++) p->U[3 + i] = u + i * p->ncw * p->elem;
         for (int i = 3; i < 6 && p->elem == 8; i++) p->P[3 + i] = u + i * p->ncw * p->elem;
     }
-    // the pad columns kz >= Nz/2+1 of the work fields are never written; the x
-    // passes load them with their tiles (and discard the results): keep them zero
+    // (every pass that fills a work field writes its pad columns kz >= Nz/2+1 too, as
+    // zeros: the x passes load them with their tiles and discard the results)
     for (int i = 0; i < 6 && !rc; i++)
         if (hipMemset(p->U[i], 0, p->ncw * p->elem) != hipSuccess) rc = fail(TG_ERR_HIP, "hipMemset failed");
     for (int i = 0; i < 9 && !rc; i++)
